@@ -315,9 +315,7 @@ int awq_gemm_int4_static(awq_ctx* ctx, uint16_t* out, int ldo, const uint16_t* a
 /* Consume the n_tokens tokens at positions pos .. pos+n_tokens-1 of the shared token list in one batched pass:
  * afterwards the KV cache rows, the logits (of the last token), the token list and the position are those that
  * n_tokens calls of awq_transformer_forward (gen_token false for all but the last, `gen_token` for the last) would
- * leave.  Needs dim, kv_dim and hidden_dim to be multiples of 128.  The batched attention holds a score row per
- * query in LDS and takes contexts of up to 1920 positions with 128-wide heads (5048 / 4856 with 64 / 256); prompt
- * tokens beyond that are run one at a time through the matrix-vector path inside this call. */
+ * leave.  Needs dim, kv_dim and hidden_dim to be multiples of 128. */
 int awq_transformer_prefill(awq_transformer* t, int n_tokens, int gen_token);
 
 /* Diagnostics of the persistent schedule (no counterpart in the reference; its DUMP_PER_TOKEN_TIMINGS switch,

@@ -1,5 +1,6 @@
 // Multi-token prefill: every projection of M prompt tokens as one int4-weight x fp16-activation GEMM on the
-// fp16 matrix cores (weights dequantised into LDS), with batched RMSNorm / RoPE and causal attention around it.
+// fp16 matrix cores (weights dequantised into LDS), with batched RMSNorm and RoPE around it (the causal
+// attention is in prefill_attention.hip).
 //
 // The reference has no such path: it feeds prompt tokens through its matrix-VECTOR kernels one at a time
 // (llama2_q4.cu:716-735).  The contract here is therefore the result of that token-by-token run: after
@@ -61,9 +62,6 @@ __device__ __forceinline__ u32x4 permute8(const u32x4 v) {
     o[3] = __builtin_amdgcn_perm(v[3], v[1], 0x07060302u);
     return o;
 }
-
-// Where element j of a group of 8 sits in that order: (0,4,1,5,2,6,3,7) holds j at ((j & 3) << 1) | (j >> 2).
-__device__ __forceinline__ int permuted_index(int c) { return (c & ~7) | ((c & 3) << 1) | ((c >> 2) & 1); }
 
 // 8 nibbles of one dword -> 8 dequantised fp16 weights in the order (w0,w4)(w1,w5)(w2,w6)(w3,w7).
 // magic = 0x64006400 held in a vector register: v_and_or_b32 takes no literal, and with the constant in a register
@@ -537,385 +535,6 @@ __global__ void rope_rows_kernel(uint16_t* q, uint16_t* kcache_layer, int num_he
     }
 }
 
-// Causal attention for BQ consecutive query tokens of one head (query m attends to cache rows 0..pos0+m), with the
-// reference's rounding points (llama2_q4.cu:410-427): scores -> fp16, probabilities -> fp16, output -> fp16.
-constexpr int BQ = 16;
-
-template <int LP>
-__global__ __launch_bounds__(256) void attn_prefill_kernel(uint16_t* out, const uint16_t* q, const uint16_t* key_cache,
-                                                           const uint16_t* value_cache, int num_heads, int head_size, int kv_mul,
-                                                           int M, int pos0, int out_perm) {
-    extern __shared__ __attribute__((aligned(16))) char smem[];
-    const int h = blockIdx.y;
-    const int mq0 = blockIdx.x * BQ;
-    const int nq = min(BQ, M - mq0);
-    const int nk = pos0 + mq0 + nq;  // keys visible to the last query of the block
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int kv_dim = num_heads * head_size / kv_mul;
-    const float alpha = (float)(1.0 / sqrt((double)head_size));
-    u32x4* qs = reinterpret_cast<u32x4*>(smem);                                            // [BQ][head/8]
-    uint16_t* S = reinterpret_cast<uint16_t*>(smem + BQ * head_size * 2);                    // [BQ][nk_stride] fp16 scores / probs
-    const int nk_stride = (nk + 7) & ~7;
-    float* stat = reinterpret_cast<float*>(smem + BQ * head_size * 2 + BQ * nk_stride * 2);  // [BQ][2]: max, sum
-
-    constexpr int PW = 64 / LP;
-    const int j = lane % LP, pr = lane / LP;
-    for (int i = tid; i < nq * LP; i += 256)
-        qs[i] = *reinterpret_cast<const u32x4*>(q + ((size_t)(mq0 + i / LP) * num_heads + h) * head_size + (i % LP) * 8);
-    __syncthreads();
-
-    // 1. scores
-    const uint16_t* kh = key_cache + (size_t)(h / kv_mul) * head_size + j * 8;
-    for (int t0 = 0; t0 < nk; t0 += 4 * PW) {
-        const int t = t0 + wave * PW + pr;
-        u32x4 kv = {0u, 0u, 0u, 0u};
-        if (t < nk) kv = *reinterpret_cast<const u32x4*>(kh + (size_t)t * kv_dim);
-        for (int qi = 0; qi < nq; qi++) {
-            const u32x4 qv = qs[qi * LP + j];
-            float s = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 4; i++) s = dot2(kv[i], qv[i], s);
-            s = group_sum<LP>(s);
-            if (j == 0 && t < nk) S[qi * nk_stride + t] = float_to_half_bits(s * alpha);
-        }
-    }
-    __syncthreads();
-    // 2. softmax statistics per query row (wave w takes rows w, w+4, ...)
-    for (int qi = wave; qi < nq; qi += 4) {
-        const int size = pos0 + mq0 + qi + 1;
-        float m = (size < 1024) ? 0.0f : -INFINITY;  // the reference's idle-lane seed
-        for (int t = lane; t < size; t += 64) m = fmaxf(m, half_bits_to_float(S[qi * nk_stride + t]));
-        m = wave_max(m);
-        float sum = 0.0f;
-        for (int t = lane; t < size; t += 64) sum += expf(half_bits_to_float(S[qi * nk_stride + t]) - m);
-        sum = wave_sum(sum);
-        for (int t = lane; t < nk; t += 64) {
-            float pv = 0.0f;
-            if (t < size) pv = expf(half_bits_to_float(S[qi * nk_stride + t]) - m) / sum;
-            S[qi * nk_stride + t] = float_to_half_bits(pv);  // probabilities (0 beyond the causal limit)
-        }
-        if (lane == 0) {
-            stat[2 * qi] = m;
-            stat[2 * qi + 1] = sum;
-        }
-    }
-    __syncthreads();
-    // 3. out[q][n] = sum_k P[q][k] * V[k][n]: thread = (dim pair, group of 4 queries)
-    const int npairs = head_size >> 1;
-    const uint16_t* vh = value_cache + (size_t)(h / kv_mul) * head_size;
-    for (int item = tid; item < npairs * 4; item += 256) {
-        const int np = item % npairs, qg = item / npairs;
-        float acc[4][2];
-#pragma unroll
-        for (int a = 0; a < 4; a++) acc[a][0] = acc[a][1] = 0.0f;
-        for (int t = 0; t < nk; t++) {
-            const h16x2 v2 = as_h2(*reinterpret_cast<const uint32_t*>(vh + (size_t)t * kv_dim + np * 2));
-            const float v0 = (float)v2[0], v1 = (float)v2[1];
-#pragma unroll
-            for (int a = 0; a < 4; a++) {
-                const float pv = half_bits_to_float(S[(qg * 4 + a) * nk_stride + t]);
-                acc[a][0] = fmaf(v0, pv, acc[a][0]);
-                acc[a][1] = fmaf(v1, pv, acc[a][1]);
-            }
-        }
-#pragma unroll
-        for (int a = 0; a < 4; a++) {
-            const int qi = qg * 4 + a;
-            if (qi < nq) {
-                uint16_t* o = out + ((size_t)(mq0 + qi) * num_heads + h) * head_size;
-                o[out_perm ? permuted_index(np * 2) : np * 2] = float_to_half_bits(acc[a][0]);
-                o[out_perm ? permuted_index(np * 2 + 1) : np * 2 + 1] = float_to_half_bits(acc[a][1]);
-            }
-        }
-    }
-}
-
-// Causal attention on the matrix cores for 128-wide heads: 32 consecutive query tokens of one head per workgroup.
-// Same rounding points as above.
-//  1. S = Q K^T: both MFMA operands are 8 consecutive head dims of a row, so q and k rows are loaded straight from
-//     memory into fragments; wave w takes key blocks w, w+4, ...; scores go to LDS as fp16.
-//  2. softmax per query row over its causal range, probabilities written back to LDS as fp16 (zero past the range).
-//  3. O = P V: the weights operand needs 8 consecutive keys of one head dim, so value rows are transposed 8 x 8 in
-//     registers on their way into LDS (64 keys per tile, next tile's rows in flight during the multiply); wave w
-//     produces head dims 32w .. 32w+31.
-constexpr int AQ = 32;        // queries per workgroup
-constexpr int VT_STRIDE = 72; // halves per row of the transposed value tile (64 keys + 8 padding)
-constexpr int KT_STRIDE = 136; // halves per row of a wave's key tile (128 dimensions + 8 padding)
-static_assert(4 * 32 * KT_STRIDE <= 2 * 128 * VT_STRIDE, "the four key tiles share the value tiles' space");
-
-// a / b correctly rounded, given rcp = 1 / b correctly rounded: the product a * rcp is within one unit of the quotient,
-// and one step of a - b * q (exact in the fused multiply-add) times rcp puts it right (Markstein's correction; for
-// 0 <= a <= 1 <= b no scaling is needed).  Three instructions where the division takes eleven.
-__device__ __forceinline__ float quotient(float a, float b, float rcp) {
-#pragma clang fp contract(off)
-    const float q = a * rcp;
-    const float e = __builtin_fmaf(-b, q, a);
-    return __builtin_fmaf(e, rcp, q);
-}
-
-__global__ __launch_bounds__(256, 2) void attn_prefill_mfma_kernel(uint16_t* out, const uint16_t* q, const uint16_t* key_cache,
-                                                                const uint16_t* value_cache, int num_heads, int kv_mul, int M,
-                                                                int pos0, int s_stride, int out_perm) {
-    constexpr int HS = 128;
-    extern __shared__ __attribute__((aligned(16))) char smem[];
-    uint16_t* S = reinterpret_cast<uint16_t*>(smem);                          // [AQ][s_stride]
-    uint16_t* Vt = reinterpret_cast<uint16_t*>(smem + AQ * s_stride * 2);     // [2][HS][VT_STRIDE]
-    // Workgroup ids go round-robin over the 8 XCDs: all query blocks of a head run on one XCD, so that the head's key
-    // and value rows come from memory into one L2 only (measured: with a head's blocks spread over all XCDs the score
-    // phase was bound by 8 copies of every row crossing the fabric).  A head's blocks are dealt longest first; the
-    // second half of an XCD's heads shortest first, so that the two workgroups of a compute unit tend to be one long
-    // and one short.
-    const int nqb = (M + AQ - 1) / AQ, hpx = (num_heads + 7) >> 3;
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int h = xcd + 8 * (slot / nqb);
-    if (h >= num_heads) return;
-    const int qb = (slot / nqb) * 2 >= hpx ? slot % nqb : nqb - 1 - slot % nqb;
-    const int mq0 = qb * AQ;
-    const int nq = min(AQ, M - mq0);
-    const int nk = pos0 + mq0 + nq;          // keys visible to the last query of the block
-    const int nk_pad = (nk + 63) & ~63;      // <= s_stride - 8
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int kv_dim = num_heads * HS / kv_mul;
-    const float alpha = (float)(1.0 / sqrt((double)HS));
-    const uint16_t* kh = key_cache + (size_t)(h / kv_mul) * HS;
-    const uint16_t* vh = value_cache + (size_t)(h / kv_mul) * HS;
-    const int l32 = lane & 31, lh = lane >> 5;
-
-    // 1. scores
-    h16x8 qf[8];
-    {
-        const uint16_t* qrow = q + ((size_t)min(mq0 + l32, M - 1) * num_heads + h) * HS + lh * 8;
-#pragma unroll
-        for (int f = 0; f < 8; f++) qf[f] = *reinterpret_cast<const h16x8*>(qrow + f * 16);
-    }
-    {
-        // Each wave takes key blocks wave, wave + 4, ...; the rows of four of them are requested at once (512 keys are
-        // one round trip to memory per wave).  The rows are loaded as they lie in memory, 16 lanes x 16 bytes per
-        // 256-byte row, and turned into MFMA fragments through a tile of LDS private to the wave (the value tiles'
-        // space, idle until phase 3): loaded straight as fragments, an instruction touches 32 rows with 32 bytes each,
-        // and the address path of the compute unit takes twice as long over it (measured: 7 of the kernel's 20 us).
-        // Every load is unconditional, rows past the end clamped to the last one: a load inside a branch is waited
-        // for before the next one is issued.
-        constexpr int KU = 4;
-        uint16_t* kt = Vt + wave * (32 * KT_STRIDE);
-        const int crow = lane >> 4, cpiece = lane & 15;
-        for (int kb0 = wave; kb0 * 32 < nk_pad; kb0 += 4 * KU) {
-            u32x4 kr[KU][8];
-#pragma unroll
-            for (int u = 0; u < KU; u++) {
-#pragma unroll
-                for (int r = 0; r < 8; r++) {
-                    const int key = min((kb0 + 4 * u) * 32 + r * 4 + crow, nk - 1);
-                    kr[u][r] = *reinterpret_cast<const u32x4*>(kh + (size_t)key * kv_dim + cpiece * 8);
-                }
-            }
-            // (the compiler would otherwise move some of these loads down to their use, one wait each)
-#pragma unroll
-            for (int u = 0; u < KU; u++)
-#pragma unroll
-                for (int r = 0; r < 8; r++) asm volatile("" : "+v"(kr[u][r]));
-#pragma unroll
-            for (int u = 0; u < KU; u++) {
-                const int kb = kb0 + 4 * u;
-                if (kb * 32 < nk_pad) {
-#pragma unroll
-                    for (int r = 0; r < 8; r++)
-                        *reinterpret_cast<u32x4*>(kt + (r * 4 + crow) * KT_STRIDE + cpiece * 8) = kr[u][r];
-                    __builtin_amdgcn_wave_barrier();  // LDS serves a wave's accesses in order; this keeps the compiler from reordering them
-                    h16x8 kf[8];
-#pragma unroll
-                    for (int f = 0; f < 8; f++) kf[f] = *reinterpret_cast<const h16x8*>(kt + l32 * KT_STRIDE + f * 16 + lh * 8);
-                    __builtin_amdgcn_wave_barrier();
-                    f32x16 acc;
-#pragma unroll
-                    for (int j = 0; j < 16; j++) acc[j] = 0.0f;
-#pragma unroll
-                    for (int f = 0; f < 8; f++) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(qf[f], kf[f], acc, 0, 0, 0);
-#pragma unroll
-                    for (int j = 0; j < 16; j++) {
-                        const int row = (j >> 2) * 8 + lh * 4 + (j & 3);
-                        S[row * s_stride + kb * 32 + l32] = float_to_half_bits(acc[j] * alpha);
-                    }
-                }
-            }
-        }
-    }
-    // O = P V below stages the value rows through LDS, 8 keys x 8 dimensions per thread transposed in registers: the
-    // waves 0-1 take the first 64 keys of a block of 128, the waves 2-3 the second.  The first two blocks are requested
-    // here, so that they arrive while the softmax runs.
-    const int kg = tid & 7, dc = (tid >> 3) & 15, vhalf = tid >> 7;
-    u32x4 va[8], vb[8];
-    auto load_v = [&](u32x4 (&vr)[8], int t0) {  // unconditional, rows past the end clamped
-#pragma unroll
-        for (int r = 0; r < 8; r++)
-            vr[r] = *reinterpret_cast<const u32x4*>(vh + (size_t)min(t0 + vhalf * 64 + kg * 8 + r, nk - 1) * kv_dim + dc * 8);
-    };
-    load_v(va, 0);
-    load_v(vb, 128);
-    __syncthreads();
-    // 2. softmax per query row; rows past nq get all-zero probabilities
-    if (nk_pad <= 512) {
-        // Eight lanes per row, the eight rows of a wave side by side: a lane holds up to 64 scores of its row in
-        // registers (16-byte LDS accesses, one exponential per score), and the row's maximum and sum are reductions
-        // over 8 lanes.  Row by row with the wave across one row, each row is a chain of dependent reductions with
-        // nothing to overlap it (measured: 7 us for 32 rows of 32 scores).
-        const int r8 = lane >> 3, l8 = lane & 7;
-        const int qi = wave * 8 + r8;
-        const int size = qi < nq ? pos0 + mq0 + qi + 1 : 0;
-        uint16_t* srow = S + qi * s_stride;
-        const int iters = nk_pad >> 6;  // chunks of 8 scores per lane
-        float v[8][8];
-        float m = (size < 1024) ? 0.0f : -INFINITY;  // the reference's idle-lane seed
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            if (i < iters) {
-                const int t0 = (l8 + 8 * i) * 8;
-                const u32x4 raw = *reinterpret_cast<const u32x4*>(srow + t0);
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const h16x2 hh = as_h2(raw[e]);
-                    v[i][2 * e] = t0 + 2 * e < size ? (float)hh[0] : -INFINITY;
-                    v[i][2 * e + 1] = t0 + 2 * e + 1 < size ? (float)hh[1] : -INFINITY;
-                    m = fmaxf(m, fmaxf(v[i][2 * e], v[i][2 * e + 1]));
-                }
-            }
-        }
-        m = fmaxf(m, dpp_mov<0xB1>(m));
-        m = fmaxf(m, dpp_mov<0x4E>(m));
-        m = fmaxf(m, dpp_mov<0x141>(m));
-        float sum = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            if (i < iters) {
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    v[i][e] = expf(v[i][e] - m);  // exp(-inf) = 0 for the masked scores
-                    sum += v[i][e];
-                }
-            }
-        }
-        sum = group_sum<8>(sum);
-        if (size == 0) sum = 1.0f;  // a row past nq: all exponentials are zero, and so are the quotients
-        const float rcp = 1.0f / sum;
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            if (i < iters) {
-                const int t0 = (l8 + 8 * i) * 8;
-                u32x4 o;
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    h16x2 hh;
-                    hh[0] = (h16_t)quotient(v[i][2 * e], sum, rcp);  // masked scores: 0 / sum
-                    hh[1] = (h16_t)quotient(v[i][2 * e + 1], sum, rcp);
-                    o[e] = as_u32(hh);
-                }
-                *reinterpret_cast<u32x4*>(srow + t0) = o;
-            }
-        }
-    } else {
-        // More than 512 keys: the same layout, with the scores read from LDS again in each of the three passes
-        // (maximum, sum of exponentials, probabilities) instead of kept in registers.
-        const int r8 = lane >> 3, l8 = lane & 7;
-        const int qi = wave * 8 + r8;
-        const int size = qi < nq ? pos0 + mq0 + qi + 1 : 0;
-        uint16_t* srow = S + qi * s_stride;
-        const int iters = nk_pad >> 6;
-        auto scores8 = [&](int i, float (&x)[8]) {  // the lane's i-th chunk of 8 scores, masked ones as -inf
-            const int t0 = (l8 + 8 * i) * 8;
-            const u32x4 raw = *reinterpret_cast<const u32x4*>(srow + t0);
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const h16x2 hh = as_h2(raw[e]);
-                x[2 * e] = t0 + 2 * e < size ? (float)hh[0] : -INFINITY;
-                x[2 * e + 1] = t0 + 2 * e + 1 < size ? (float)hh[1] : -INFINITY;
-            }
-        };
-        float m = (size < 1024) ? 0.0f : -INFINITY;  // the reference's idle-lane seed
-#pragma unroll 4
-        for (int i = 0; i < iters; i++) {
-            float x[8];
-            scores8(i, x);
-#pragma unroll
-            for (int e = 0; e < 8; e++) m = fmaxf(m, x[e]);
-        }
-        m = fmaxf(m, dpp_mov<0xB1>(m));
-        m = fmaxf(m, dpp_mov<0x4E>(m));
-        m = fmaxf(m, dpp_mov<0x141>(m));
-        if (size == 0) m = 0.0f;  // a row past nq (with the -inf seed of long contexts): keep exp(-inf - m) defined
-        float sum = 0.0f;
-#pragma unroll 2
-        for (int i = 0; i < iters; i++) {
-            float x[8];
-            scores8(i, x);
-#pragma unroll
-            for (int e = 0; e < 8; e++) sum += expf(x[e] - m);
-        }
-        sum = group_sum<8>(sum);
-        if (size == 0) sum = 1.0f;
-        const float rcp = 1.0f / sum;
-#pragma unroll 2
-        for (int i = 0; i < iters; i++) {
-            float x[8];
-            scores8(i, x);
-            u32x4 o;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                h16x2 hh;
-                hh[0] = (h16_t)quotient(expf(x[2 * e] - m), sum, rcp);
-                hh[1] = (h16_t)quotient(expf(x[2 * e + 1] - m), sum, rcp);
-                o[e] = as_u32(hh);
-            }
-            *reinterpret_cast<u32x4*>(srow + (l8 + 8 * i) * 8) = o;
-        }
-    }
-    // 3. O = P V, 128 keys per round: every thread transposes its 8 x 8 piece into the LDS tile of its half, then
-    // every wave multiplies both tiles.  Value rows travel two rounds ahead of the multiply, in two register sets.
-    auto store_v = [&](const u32x4 (&vr)[8]) {
-        uint16_t* vt = Vt + vhalf * (HS * VT_STRIDE);
-#pragma unroll
-        for (int d = 0; d < 8; d++) {
-            const uint32_t sel = (d & 1) ? 0x07060302u : 0x05040100u;
-            u32x4 o;
-#pragma unroll
-            for (int r2 = 0; r2 < 4; r2++) o[r2] = __builtin_amdgcn_perm(vr[2 * r2 + 1][d >> 1], vr[2 * r2][d >> 1], sel);
-            *reinterpret_cast<u32x4*>(&vt[(dc * 8 + d) * VT_STRIDE + kg * 8]) = o;
-        }
-    };
-    f32x16 oacc;
-#pragma unroll
-    for (int j = 0; j < 16; j++) oacc[j] = 0.0f;
-    auto multiply = [&](int t0, int buf) {
-        const uint16_t* vt = Vt + buf * (HS * VT_STRIDE);
-#pragma unroll
-        for (int kc = 0; kc < 4; kc++) {
-            const h16x8 pf = *reinterpret_cast<const h16x8*>(&S[l32 * s_stride + t0 + kc * 16 + lh * 8]);
-            const h16x8 vf = *reinterpret_cast<const h16x8*>(&vt[(wave * 32 + l32) * VT_STRIDE + kc * 16 + lh * 8]);
-            oacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(pf, vf, oacc, 0, 0, 0);
-        }
-    };
-    for (int t0 = 0; t0 < nk_pad; t0 += 256) {
-        store_v(va);
-        load_v(va, t0 + 256);
-        __syncthreads();  // the first one also orders the probabilities written above
-        multiply(t0, 0);
-        if (t0 + 64 < nk_pad) multiply(t0 + 64, 1);
-        __syncthreads();  // every wave is done with the tiles before they are overwritten
-        if (t0 + 128 >= nk_pad) break;
-        store_v(vb);
-        load_v(vb, t0 + 384);
-        __syncthreads();
-        multiply(t0 + 128, 0);
-        if (t0 + 192 < nk_pad) multiply(t0 + 192, 1);
-        __syncthreads();
-    }
-#pragma unroll
-    for (int j = 0; j < 16; j++) {
-        const int row = (j >> 2) * 8 + lh * 4 + (j & 3);
-        const int d = wave * 32 + l32;
-        if (row < nq) out[((size_t)(mq0 + row) * num_heads + h) * HS + (out_perm ? permuted_index(d) : d)] = float_to_half_bits(oacc[j]);
-    }
-}
-
 __global__ void set_pos_kernel(int* pos_dev, volatile int* pos_host, int value) {
     *pos_dev = value;
     *pos_host = value;
@@ -1119,64 +738,6 @@ int awq_launch_rope_rows(awq_ctx* ctx, uint16_t* q, uint16_t* kcache_layer, int 
     hipLaunchKernelGGL(pf::rope_rows_kernel, dim3(nh, M), dim3(hs / 2), 0, ctx->stream, q, kcache_layer, nh, nkv, hs, pos0, theta,
                        table);
     return awq_check_launch("rope_rows");
-}
-
-// Largest context (pos0 + M) the batched attention kernels take: they hold one fp16 score row per query in LDS.
-int awq_prefill_attention_max_positions(int head_size) {
-    const int lds_cap = 160 * 1024;
-    if (head_size == 128) return ((lds_cap - 2 * 128 * pf::VT_STRIDE * 2) / (pf::AQ * 2) - 8) & ~63;
-    return ((lds_cap - pf::BQ * head_size * 2 - pf::BQ * 8) / (pf::BQ * 2)) & ~7;
-}
-
-int awq_launch_attn_prefill(awq_ctx* ctx, uint16_t* out, const uint16_t* q, const uint16_t* kc, const uint16_t* vc, int nh, int hs,
-                            int kv_mul, int M, int pos0, int out_perm) {
-    if (hs == 128) {
-        const int s_stride = ((pos0 + M + 63) & ~63) + 8;
-        const size_t lds = (size_t)pf::AQ * s_stride * 2 + 2 * 128 * pf::VT_STRIDE * 2;
-        if (lds > 160 * 1024) {
-            awq_set_error("prefill attention: context of %d positions does not fit in LDS", pos0 + M);
-            return AWQ_ERR_SHAPE;
-        }
-        if (lds > 64 * 1024) {
-            hipError_t e = hipFuncSetAttribute((const void*)pf::attn_prefill_mfma_kernel,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-            if (e != hipSuccess) {
-                awq_set_error("hipFuncSetAttribute(attn_prefill_mfma) failed: %s", hipGetErrorString(e));
-                return AWQ_ERR_HIP;
-            }
-        }
-        hipLaunchKernelGGL(pf::attn_prefill_mfma_kernel, dim3(8 * ((nh + 7) / 8) * div_up(M, pf::AQ)), dim3(256), lds, ctx->stream, out, q, kc, vc,
-                           nh, kv_mul, M, pos0, s_stride, out_perm);
-        return awq_check_launch("attn_prefill_mfma");
-    }
-    const int nk_max = (pos0 + M + 7) & ~7;
-    const size_t lds = (size_t)pf::BQ * hs * 2 + (size_t)pf::BQ * nk_max * 2 + pf::BQ * 8;
-    if (lds > 160 * 1024) {
-        awq_set_error("prefill attention: context of %d positions does not fit in LDS", pos0 + M);
-        return AWQ_ERR_SHAPE;
-    }
-    const dim3 grid(div_up(M, pf::BQ), nh);
-#define AWQ_ATTN_PF(LPV)                                                                                                  \
-    do {                                                                                                                  \
-        if (lds > 64 * 1024) {                                                                                            \
-            hipError_t e = hipFuncSetAttribute((const void*)pf::attn_prefill_kernel<LPV>,                                 \
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);                  \
-            if (e != hipSuccess) {                                                                                        \
-                awq_set_error("hipFuncSetAttribute(attn_prefill) failed: %s", hipGetErrorString(e));                      \
-                return AWQ_ERR_HIP;                                                                                       \
-            }                                                                                                             \
-        }                                                                                                                 \
-        hipLaunchKernelGGL((pf::attn_prefill_kernel<LPV>), grid, dim3(256), lds, ctx->stream, out, q, kc, vc, nh, hs, kv_mul, \
-                           M, pos0, out_perm);                                                                            \
-    } while (0)
-    switch (hs) {
-        case 64: AWQ_ATTN_PF(8); break;
-        case 128: AWQ_ATTN_PF(16); break;
-        case 256: AWQ_ATTN_PF(32); break;
-        default: awq_set_error("prefill attention: head_size %d unsupported", hs); return AWQ_ERR_SHAPE;
-    }
-#undef AWQ_ATTN_PF
-    return awq_check_launch("attn_prefill");
 }
 
 int awq_launch_set_pos(awq_ctx* ctx, int* pos_dev, volatile int* pos_host, int value) {

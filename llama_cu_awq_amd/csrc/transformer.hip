@@ -49,7 +49,6 @@ int awq_launch_rope_rows(awq_ctx* ctx, uint16_t* q, uint16_t* kcache_layer, int 
 int awq_launch_attn_prefill(awq_ctx* ctx, uint16_t* out, const uint16_t* q, const uint16_t* kc, const uint16_t* vc, int nh, int hs,
                             int kv_mul, int M, int pos0, int out_perm);
 int awq_launch_set_pos(awq_ctx* ctx, int* pos_dev, volatile int* pos_host, int value);
-int awq_prefill_attention_max_positions(int head_size);
 int awq_launch_copy_row(awq_ctx* ctx, uint16_t* dst, const uint16_t* src, int n);
 
 namespace {
@@ -828,14 +827,8 @@ int awq_transformer_prefill(awq_transformer* t, int n_tokens, int gen_token) {
     }
     const int pos_start = t->issued_pos;
     AWQ_REQUIRE(pos_start + n_tokens <= p.seq_len, AWQ_ERR_ARG, "prompt runs past seq_len");
-    // The batched attention keeps a score row per query in LDS, which bounds the context it can take; tokens past
-    // that bound go through the matrix-vector path one at a time (the definition of what prefill must leave behind).
-    const int max_ctx = awq_prefill_attention_max_positions(hs);
-    int n_batched = max_ctx - pos_start;
-    if (n_batched > n_tokens) n_batched = n_tokens;
-    if (n_batched < 0) n_batched = 0;
     const int chunk = 512;
-    if (n_batched > 0 && t->pf_rows == 0) {
+    if (t->pf_rows == 0) {
         const int rows = p.seq_len < chunk ? p.seq_len : chunk;
         uint16_t** bufs[5] = {&t->pf_x, &t->pf_xb, &t->pf_q, &t->pf_att, &t->pf_hb};
         const size_t widths[5] = {(size_t)dim, (size_t)dim, (size_t)dim, (size_t)dim, (size_t)hidden};
@@ -854,8 +847,8 @@ int awq_transformer_prefill(awq_transformer* t, int n_tokens, int gen_token) {
         t->pf_rows = rows;
     }
     int r;
-    for (int done = 0; done < n_batched; done += t->pf_rows) {
-        const int M = (n_batched - done < t->pf_rows) ? n_batched - done : t->pf_rows;
+    for (int done = 0; done < n_tokens; done += t->pf_rows) {
+        const int M = (n_tokens - done < t->pf_rows) ? n_tokens - done : t->pf_rows;
         const int pos0 = pos_start + done;
         if ((r = awq_launch_embed_rows(ctx, t->pf_x, t->embed, dim, t->tokens_dev, pos0, M))) return r;
         // The activations that feed a GEMM (xb, att, hb) are written with every 8 values in the order the packed weights
@@ -888,15 +881,6 @@ int awq_transformer_prefill(awq_transformer* t, int n_tokens, int gen_token) {
             if ((r = awq_launch_matvec_f16(ctx, t->s.logits, t->s.x, t->wcls, dim, p.vocab_size, t->rms_final, nullptr))) return r;
             if ((r = awq_launch_argmax(ctx, t->s.logits, p.vocab_size, t->s.shared_tokens, t->s.shared_pos, t->s.pos, gen_token,
                                        t->tokens_dev)))
-                return r;
-        }
-    }
-    if (n_batched < n_tokens) {
-        if (n_batched > 0 && (r = awq_launch_set_pos(ctx, t->s.pos, t->s.shared_pos, pos_start + n_batched))) return r;
-        for (int i = n_batched; i < n_tokens; i++) {
-            if ((r = network(t, pos_start + i + 1, AWQ_SCHEDULE_FUSED))) return r;
-            if ((r = awq_launch_argmax(ctx, t->s.logits, p.vocab_size, t->s.shared_tokens, t->s.shared_pos, t->s.pos,
-                                       i == n_tokens - 1 ? gen_token : 0, t->tokens_dev)))
                 return r;
         }
     }
