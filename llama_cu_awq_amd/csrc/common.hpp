@@ -26,12 +26,9 @@ struct awq_ctx {
     hipStream_t stream;
     bool owns_stream;
     awq_launch_probe* probe;  // null outside awq_transformer_time_launches
-    // Workspace of the prefill GEMM's split-K form (allocated on first use): fp32 partial tiles and per-tile arrival
-    // counters (self-resetting).
+    // Split-K workspace of the batched GEMMs (allocated on first use): fp32 partial tiles, then per-tile arrival counters
+    // (self-resetting).
     float* gemm_part;
-    size_t gemm_part_bytes;
-    unsigned int* gemm_counter;
-    size_t gemm_counter_count;
 };
 
 constexpr int kAttnMaxHeads = 256;

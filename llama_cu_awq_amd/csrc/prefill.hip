@@ -1,6 +1,6 @@
 // Multi-token prefill: every projection of M prompt tokens as one int4-weight x fp16-activation GEMM on the
-// fp16 matrix cores (weights dequantised into LDS), with batched RMSNorm and RoPE around it (the causal
-// attention is in prefill_attention.hip).
+// fp16 matrix cores, with batched RMSNorm and RoPE around it (most forms of the GEMM are in gemm_rows.hip, the causal
+// attention in prefill_attention.hip).
 //
 // The reference has no such path: it feeds prompt tokens through its matrix-VECTOR kernels one at a time
 // (llama2_q4.cu:716-735).  The contract here is therefore the result of that token-by-token run: after
@@ -16,67 +16,9 @@
 #include <mutex>
 
 #include "common.hpp"
-
-typedef _Float16 h16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+#include "gemm_tile.hpp"
 
 namespace pf {
-
-constexpr int BM = 128;  // tokens per tile
-constexpr int BN = 128;  // weight rows per tile
-constexpr int BK = 64;   // K per step: 128 bytes of fp16 per LDS tile row
-
-enum Epi { EPI_STORE = 0, EPI_RESID = 1, EPI_QKV = 2, EPI_FFN = 3 };
-
-struct GemmParams {
-    const uint16_t* A;  // [M][lda] fp16 activations
-    int lda, M, K;
-    const uint32_t* w[3];
-    const uint32_t* z[3];
-    const uint16_t* s[3];
-    int N[3];  // rows of each matrix
-    int C, pzh, sh;
-    int epi;
-    int mtiles, ntiles;
-    int ksplit;                  // 1, or 2: two workgroups share a tile, each taking half of K
-    float* part;                 // ksplit == 2: fp32 partial tiles [tile][2][128 x 128]
-    unsigned int* part_counter;  // ksplit == 2: arrivals per tile, zero between launches
-    // QKV with 128-wide heads: RoPE of the q and k tiles (one head each) in the epilogue, (cos, sin) from the table
-    // [position][pair]; row m of the GEMM is position rope_pos0 + m.  Null: no rotation.
-    const float2* rope;
-    int rope_pos0;
-    // FFN form: write the output with every 8 columns in the order (0,4,1,5,2,6,3,7), the order a permuted-A GEMM reads
-    int out_perm;
-    uint16_t* out[3];
-    long long ldo[3];       // output row stride in elements
-    long long out_off[3];   // element offset of output row 0 (KV cache: loff + pos0 * kv_dim)
-};
-
-// (h0,h1)(h2,h3)(h4,h5)(h6,h7) -> (h0,h4)(h1,h5)(h2,h6)(h3,h7): the order in which one packed dword unpacks
-__device__ __forceinline__ u32x4 permute8(const u32x4 v) {
-    u32x4 o;
-    o[0] = __builtin_amdgcn_perm(v[2], v[0], 0x05040100u);
-    o[1] = __builtin_amdgcn_perm(v[2], v[0], 0x07060302u);
-    o[2] = __builtin_amdgcn_perm(v[3], v[1], 0x05040100u);
-    o[3] = __builtin_amdgcn_perm(v[3], v[1], 0x07060302u);
-    return o;
-}
-
-// 8 nibbles of one dword -> 8 dequantised fp16 weights in the order (w0,w4)(w1,w5)(w2,w6)(w3,w7).
-// magic = 0x64006400 held in a vector register: v_and_or_b32 takes no literal, and with the constant in a register
-// the mask-and-merge of a nibble pair is one instruction.
-__device__ __forceinline__ u32x4 dequant8(uint32_t d, uint32_t z, h16x2 s2, uint32_t magic) {
-    const h16x2 zlo = as_h2(0xE400E400u | (z * 0x00010001u));  // -(1024 + z)
-    const h16x2 zhi = as_h2(0xD400D400u | (z * 0x00100010u));  // -(64 + z)
-    const h16x2 sixteenth = {(h16_t)0.0625f, (h16_t)0.0625f};
-    const uint32_t d8 = d >> 8;
-    const h16x2 t0 = as_h2((d & 0x000F000Fu) | magic) + zlo;                                      // exact q - z
-    const h16x2 t1 = __builtin_elementwise_fma(as_h2((d & 0x00F000F0u) | magic), sixteenth, zhi);  // exact
-    const h16x2 t2 = as_h2((d8 & 0x000F000Fu) | magic) + zlo;
-    const h16x2 t3 = __builtin_elementwise_fma(as_h2((d8 & 0x00F000F0u) | magic), sixteenth, zhi);
-    return u32x4{as_u32(t0 * s2), as_u32(t1 * s2), as_u32(t2 * s2), as_u32(t3 * s2)};  // one rounding each
-}
 
 // A tile's 128 columns are four blocks of 32 weight rows.  Which matrix a block belongs to and its first row:
 // single / QKV: consecutive rows of one matrix; FFN: blocks alternate gate, up over the same 32 row indices, so that a
@@ -108,40 +50,12 @@ __device__ __forceinline__ BlockMap block_map(const GemmParams& p, int tile, int
     return m;
 }
 
-// The activation tile in LDS is [128 rows][64 halves] with the 16-byte chunk index XOR-ed with a key of the row, so
-// that a wave's fragment reads (32 consecutive rows, one chunk) spread over all banks without padding.
-__device__ __forceinline__ int lds_key(int row) { return (row ^ (row >> 3)) & 7; }
-__device__ __forceinline__ int lds_off(int row, int chunk) { return row * BK + ((chunk ^ lds_key(row)) << 3); }
-
 constexpr int A_STAGES = 3;                   // activation tiles in the LDS ring (2 steps ahead)
 constexpr int W_STAGES = 3;                   // pairs of steps (one quantisation group) of packed weights in the LDS ring
 constexpr int TILE_BYTES = BM * BK * 2;       // 16 KB
 constexpr int W_WAVE_BYTES = 32 * 64 + 256 + 256;  // per wave and pair of steps: 32 rows x 64 packed bytes, zeros, scales
 constexpr int W_STAGE_BYTES = 4 * W_WAVE_BYTES;
 constexpr int GEMM_LDS_BYTES = A_STAGES * TILE_BYTES + W_STAGES * W_STAGE_BYTES;
-
-// Direct global -> LDS loads: lane L's 16 (4) bytes land at lds_byte_off + 16 (4) * L.  Issued as inline assembly,
-// so the compiler's wait-count bookkeeping does not see them; the kernel counts and waits for them itself.
-__device__ __forceinline__ void dma16(const void* gptr, uint32_t lds_byte_off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_byte_off), "v"(gptr) : "memory");
-}
-// Same with the address as a wave-uniform base plus a 32-bit byte offset per lane (no 64-bit vector arithmetic).
-__device__ __forceinline__ void dma16(const void* sbase, uint32_t voff, uint32_t lds_byte_off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_byte_off), "v"(voff), "s"(sbase) : "memory");
-}
-__device__ __forceinline__ void dma4(const void* gptr, uint32_t lds_byte_off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_byte_off), "v"(gptr) : "memory");
-}
-
-// inverse of permute8: (h0,h4)(h1,h5)(h2,h6)(h3,h7) -> (h0,h1)(h2,h3)(h4,h5)(h6,h7)
-__device__ __forceinline__ u32x4 unpermute8(const u32x4 v) {
-    u32x4 o;
-    o[0] = __builtin_amdgcn_perm(v[1], v[0], 0x05040100u);
-    o[1] = __builtin_amdgcn_perm(v[3], v[2], 0x05040100u);
-    o[2] = __builtin_amdgcn_perm(v[1], v[0], 0x07060302u);
-    o[3] = __builtin_amdgcn_perm(v[3], v[2], 0x07060302u);
-    return o;
-}
 
 // C[m][n] = sum_k A[m][k] * half((q[n][k] - z) * s), tile 128 x 128, K step 64.
 //  * Workgroup = 4 waves; wave w owns tile columns 32w .. 32w+31 and all 128 rows: four 32x32x16 fp16 MFMA
@@ -247,11 +161,10 @@ __global__ __launch_bounds__(256, 2) void gemm_int4_kernel(const GemmParams p) {
         const uint32_t z = (zw >> (4 * (g & 7))) & 0xFu;
         const uint16_t sbits = (uint16_t)(((s_row + g) & 1) ? (sw >> 16) : (sw & 0xFFFFu));
         const bool live = step * BK + lhalf * 32 < p.K;  // past K: zero scale, zero products
-        const h16_t sh = __builtin_bit_cast(h16_t, live ? sbits : (uint16_t)0);
-        const h16x2 s2 = {sh, sh};
+        const Group gc = group_consts(z, live ? sbits : (uint16_t)0);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const u32x4 dq = dequant8(wq[j], z, s2, magic);
+            const u32x4 dq = dequant8(wq[j], gc, magic);
             const h16x8 bf = __builtin_bit_cast(h16x8, APERM ? dq : unpermute8(dq));
             const int chunk = j + 4 * lhalf;
 #pragma unroll
@@ -553,10 +466,8 @@ __global__ __launch_bounds__(256) void copy_row_kernel(uint16_t* dst, const uint
 // at its own address until the process ends.  In host code the array's name is only a stand-in for the symbol: the
 // device address is looked up once per device with hipGetSymbolAddress and kept in g_scratch_ptr, and that pointer is
 // what kernels and clears receive.
-constexpr int kStaticTiles = 256;  // the split form is taken below 256 tiles only
-constexpr size_t kStaticPartBytes = (size_t)kStaticTiles * 2 * pf::BM * pf::BN * sizeof(float);  // 32 MiB
-constexpr size_t kStaticScratchBytes = kStaticPartBytes + kStaticTiles * sizeof(unsigned int);
-static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
+constexpr size_t kScratchBytes = kPartBytes + kPartTiles * sizeof(unsigned int);
+static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mutex;
@@ -588,6 +499,7 @@ int awq_gemm_device_setup(int device) {
             awq_set_error("hipFuncSetAttribute(gemm_int4) failed: %s", hipGetErrorString(e));
             return AWQ_ERR_HIP;
         }
+        if (int r = awq_gemm_rows_setup()) return r;
         g_gemm_lds_raised[device] = true;
     }
     if (!g_scratch_ptr[device]) {
@@ -603,63 +515,73 @@ int awq_gemm_device_setup(int device) {
 }
 
 // ---------------------------------------------------------------- launchers (internal)
+// The split-K workspace of a launch over `tiles` output tiles: the file-scope device array (static_ws; no allocation) or
+// the context's, allocated whole on first use, so that it never moves.
+static int bind_workspace(awq_ctx* ctx, pf::GemmParams& p, int tiles, bool static_ws, const char* what) {
+    if (static_ws) {
+        unsigned char* ws = static_cast<unsigned char*>(g_scratch_ptr[ctx->device]);
+        if (!ws) {
+            awq_set_error("%s: the static workspace was not set up on device %d", what, ctx->device);
+            return AWQ_ERR_HIP;
+        }
+        p.part = reinterpret_cast<float*>(ws);
+        p.part_counter = reinterpret_cast<unsigned int*>(ws + kPartBytes);
+        // the array keeps whatever the previous call on this GPU left: the arrival counters must start at zero
+        // (a fill kernel rather than a memset node, so that the call can be recorded into a graph)
+        hipLaunchKernelGGL(pf::clear_words_kernel, dim3(div_up(tiles, 256)), dim3(256), 0, ctx->stream, p.part_counter, tiles);
+        return awq_check_launch("clear_words");
+    }
+    if (!ctx->gemm_part) {
+        void* block = nullptr;
+        AWQ_HIP_TRY(hipMalloc(&block, kScratchBytes));
+        ctx->gemm_part = static_cast<float*>(block);
+        unsigned int* counter = reinterpret_cast<unsigned int*>(static_cast<uint8_t*>(block) + kPartBytes);
+        hipLaunchKernelGGL(pf::clear_words_kernel, dim3(1), dim3(kPartTiles), 0, ctx->stream, counter, kPartTiles);
+        if (int r = awq_check_launch("clear_words")) return r;
+    }
+    p.part = ctx->gemm_part;
+    p.part_counter = reinterpret_cast<unsigned int*>(reinterpret_cast<uint8_t*>(ctx->gemm_part) + kPartBytes);
+    return AWQ_OK;
+}
+
+// Expected time of the 128 x 128 kernel, to be weighed against the forms of gemm_rows.hip.  It is the best one where about
+// one of its workgroups comes to a compute unit (512 rows against 4096 columns: 33 us, the best other form 36).
+static float general_us(int cus, long long tiles, int K, int ksplit) {
+    const float split = ksplit > 1 ? 2.0f + 0.5e-6f * tiles * ksplit * (pf::BM * pf::BN * sizeof(float)) : 0.0f;
+    return awq_gemm_us(cus, 2, tiles * ksplit, div_up(div_up(K, pf::BK), ksplit), awq_step_us{0.52f, 0.58f, 1.1f}) + split;
+}
+
 // static_ws: take the split-K workspace from the file-scope device array (no allocation) instead of the context's.
 // a_perm: A holds every 8 activations in the order (0,4,1,5,2,6,3,7).
-static int launch_gemm(awq_ctx* ctx, pf::GemmParams& p, int ntiles, const char* what, bool a_perm, bool static_ws = false) {
-    // the kernel's 80 KB of LDS exceed the default dynamic limit; raised per device when a context is created
+// *rotated (QKV): whether the epilogue did what p.rope asks for.
+static int launch_gemm(awq_ctx* ctx, pf::GemmParams& p, int ntiles, const char* what, bool a_perm, bool static_ws = false,
+                       bool* rotated = nullptr) {
+    // the kernels' LDS exceeds the default dynamic limit; raised per device when a context is created
     // (contexts on a caller's stream included), here only for a device that was missed
     if (ctx->device < 0 || ctx->device >= kMaxDevices || !g_gemm_lds_raised[ctx->device]) {
         if (int r = awq_gemm_device_setup(ctx->device)) return r;
     }
-    if ((size_t)p.M * (size_t)p.lda * 2 >= ((size_t)1 << 32)) {  // the kernel addresses A by 32-bit byte offsets
+    if ((size_t)p.M * (size_t)p.lda * 2 >= ((size_t)1 << 32)) {  // the kernels address A by 32-bit byte offsets
         awq_set_error("%s: activation block of %d x %d halves exceeds 4 GB", what, p.M, p.lda);
         return AWQ_ERR_SHAPE;
     }
     p.mtiles = div_up(p.M, pf::BM);
     p.ntiles = ntiles;
-    p.ksplit = 1;
-    // A single matrix with fewer tiles than compute units: two workgroups per tile, each half of K.
-    if ((p.epi == pf::EPI_STORE || p.epi == pf::EPI_RESID) && p.mtiles * ntiles < 256 && p.K >= 8 * pf::BK) {
-        const size_t tiles = (size_t)p.mtiles * ntiles;
-        const size_t need = tiles * 2 * pf::BM * pf::BN * sizeof(float);
-        if (static_ws) {
-            if (tiles > (size_t)kStaticTiles) {
-                awq_set_error("%s: %zu output tiles of 128 x 128 exceed the %d the static split-K workspace holds", what, tiles,
-                              kStaticTiles);
-                return AWQ_ERR_SHAPE;
-            }
-            unsigned char* ws = static_cast<unsigned char*>(g_scratch_ptr[ctx->device]);
-            if (!ws) {
-                awq_set_error("%s: the static workspace was not set up on device %d", what, ctx->device);
-                return AWQ_ERR_HIP;
-            }
-            p.ksplit = 2;
-            p.part = reinterpret_cast<float*>(ws);
-            p.part_counter = reinterpret_cast<unsigned int*>(ws + kStaticPartBytes);
-            // the array keeps whatever the previous call on this GPU left: the arrival counters must start at zero
-            // (a fill kernel rather than a memset node, so that the call can be recorded into a graph)
-            hipLaunchKernelGGL(pf::clear_words_kernel, dim3(div_up((int)tiles, 256)), dim3(256), 0, ctx->stream, p.part_counter,
-                               (int)tiles);
-            if (int r = awq_check_launch("clear_words")) return r;
-        } else if (ctx->gemm_part_bytes < need || ctx->gemm_counter_count < tiles) {
-            AWQ_HIP_TRY(hipStreamSynchronize(ctx->stream));
-            if (ctx->gemm_part) (void)hipFree(ctx->gemm_part);
-            if (ctx->gemm_counter) (void)hipFree(ctx->gemm_counter);
-            ctx->gemm_part = nullptr;
-            ctx->gemm_counter = nullptr;
-            ctx->gemm_part_bytes = 0;
-            ctx->gemm_counter_count = 0;
-            AWQ_HIP_TRY(hipMalloc((void**)&ctx->gemm_part, need));
-            AWQ_HIP_TRY(hipMalloc((void**)&ctx->gemm_counter, tiles * sizeof(unsigned int)));
-            AWQ_HIP_TRY(hipMemset(ctx->gemm_counter, 0, tiles * sizeof(unsigned int)));
-            ctx->gemm_part_bytes = need;
-            ctx->gemm_counter_count = tiles;
-        }
-        if (!static_ws) {
-            p.ksplit = 2;
-            p.part = ctx->gemm_part;
-            p.part_counter = ctx->gemm_counter;
-        }
+    const long long tiles = (long long)p.mtiles * ntiles;
+    // a single matrix with fewer tiles than compute units: two workgroups per tile, each half of K
+    p.ksplit = (p.epi == pf::EPI_STORE || p.epi == pf::EPI_RESID) && tiles < 256 && p.K >= 8 * pf::BK ? 2 : 1;
+    const bool may_split = p.ksplit == 2 || (p.epi != pf::EPI_STORE && p.epi != pf::EPI_RESID);
+    const awq_rows_plan plan = awq_plan_gemm_rows(ctx->cus, p.M, p.K, ntiles * 2, may_split);
+    if (plan.form >= 0 && plan.us < general_us(ctx->cus, tiles, p.K, p.ksplit) && (!a_perm || (p.K & 127) == 0)) {
+        if (plan.ksplit > 1)
+            if (int r = bind_workspace(ctx, p, kPartTiles, static_ws, what)) return r;
+        return awq_launch_gemm_rows(ctx, p, ntiles * 2, plan, a_perm, what);
+    }
+    if (p.ksplit == 2)
+        if (int r = bind_workspace(ctx, p, (int)tiles, static_ws, what)) return r;
+    if (p.rope && p.head_size != 128) {
+        p.rope = nullptr;
+        *rotated = false;
     }
     // ids go round-robin over the 8 XCDs; each XCD takes every 8th weight tile with all of its M tiles (and K halves)
     const int grid = 8 * p.mtiles * p.ksplit * div_up(ntiles, 8);
@@ -700,17 +622,24 @@ int awq_launch_gemm_single(awq_ctx* ctx, uint16_t* out, long long ldo, const uin
     return launch_gemm(ctx, p, N / pf::BN, "gemm_int4", a_perm, static_ws);
 }
 
-int awq_launch_gemm_qkv(awq_ctx* ctx, uint16_t* q, uint16_t* key_cache, uint16_t* value_cache, long long kv_row0_off,
-                        const uint16_t* A, int lda, int M, const awq_qweight* qw, const awq_qweight* kw, const awq_qweight* vw,
-                        int K, int Nq, int Nkv, const float2* rope128, int pos0, bool a_perm) {
+int awq_launch_rope_rows(awq_ctx* ctx, uint16_t* q, uint16_t* kcache_layer, int nh, int nkv, int hs, int pos0, float theta, int M,
+                         const float2* table);
+
+// q rows and K, V cache rows of M positions from pos0 on, q and k rotated
+int awq_launch_gemm_qkv(awq_ctx* ctx, uint16_t* q, uint16_t* kcache_layer, uint16_t* vcache_layer, const uint16_t* A, int lda, int M,
+                        const awq_qweight* qw, const awq_qweight* kw, const awq_qweight* vw, int K, int Nq, int Nkv, int head_size,
+                        const float2* rope, float theta, int pos0, bool a_perm) {
     pf::GemmParams p;
     gemm_common(p, A, lda, M, K, pf::EPI_QKV);
-    p.rope = rope128;  // non-null only with 128-wide heads
+    bool rotated = rope != nullptr && (head_size == 64 || head_size == 128 || head_size == 256);
+    p.rope = rotated ? rope : nullptr;
+    p.head_size = head_size;
     p.rope_pos0 = pos0;
     set_mat(p, 0, qw, Nq, q, Nq, 0);
-    set_mat(p, 1, kw, Nkv, key_cache, Nkv, kv_row0_off);
-    set_mat(p, 2, vw, Nkv, value_cache, Nkv, kv_row0_off);
-    return launch_gemm(ctx, p, (Nq + 2 * Nkv) / pf::BN, "gemm_int4_qkv", a_perm);
+    set_mat(p, 1, kw, Nkv, kcache_layer, Nkv, (long long)pos0 * Nkv);
+    set_mat(p, 2, vw, Nkv, vcache_layer, Nkv, (long long)pos0 * Nkv);
+    if (int r = launch_gemm(ctx, p, (Nq + 2 * Nkv) / pf::BN, "gemm_int4_qkv", a_perm, false, &rotated)) return r;
+    return rotated ? AWQ_OK : awq_launch_rope_rows(ctx, q, kcache_layer, Nq / head_size, Nkv / head_size, head_size, pos0, theta, M, rope);
 }
 
 int awq_launch_gemm_ffn(awq_ctx* ctx, uint16_t* hb, const uint16_t* A, int lda, int M, const awq_qweight* gate_w,

@@ -74,9 +74,6 @@ static int ctx_init(int device, hipStream_t stream, bool owns, awq_ctx** out) {
     c->owns_stream = owns;
     c->probe = nullptr;
     c->gemm_part = nullptr;
-    c->gemm_part_bytes = 0;
-    c->gemm_counter = nullptr;
-    c->gemm_counter_count = 0;
     *out = c;
     return AWQ_OK;
 }
@@ -102,7 +99,6 @@ int awq_ctx_destroy(awq_ctx* ctx) {
     if (int r = awq_bind(ctx)) return r;
     (void)hipStreamSynchronize(ctx->stream);
     if (ctx->gemm_part) (void)hipFree(ctx->gemm_part);
-    if (ctx->gemm_counter) (void)hipFree(ctx->gemm_counter);
     if (ctx->owns_stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return AWQ_OK;

@@ -1,0 +1,109 @@
+"""The batched int4 GEMM at the edges of its row forms (one workgroup tile of 32, 64, 96 or 128 rows by 64, 128 or 256
+columns, K slices inside a workgroup and over workgroups): rows and K ranges around tile ends, K that is no multiple of a
+quantisation group, K past eight groups (scales and zeros travel for eight at a time), against the product in 64 bits.
+
+Bar: the weights are exact fp16 values, sums are fp32 and the result is rounded once: rel-L2 2.1e-4 by the rounding alone;
+1e-3 as for the other GEMM tests."""
+import numpy as np
+import pytest
+
+import llama_cu_awq_amd as A
+from llama_cu_awq_amd import synth
+from tests.helpers import f16, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    (1, 128, 128), (31, 160, 384), (32, 1120, 1152), (33, 2048, 128), (1, 4096, 384), (16, 4128, 256),  # 32 x 64, split or not
+    (65, 512, 6144), (97, 416, 4224), (33, 3072, 1152), (97, 4096, 384), (64, 1184, 8192),  # 64 x 64
+    (65, 256, 6144), (65, 160, 6144), (129, 2080, 4096), (300, 1056, 4096),  # 64 x 128
+    (257, 128, 12288), (300, 96, 12288), (257, 1184, 12288),  # 64 x 256
+    (700, 128, 6144), (513, 96, 8192), (700, 1152, 6144),  # 96 x 256
+    (385, 128, 16384), (385, 96, 16384), (513, 1120, 12288),  # 128 x 256
+]
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
+def test_against_fp64(ctx, M, K, N):
+    key = synth.stream_key(52, M, K, N)
+    w, z, s = synth.make_qweight(key, K, N)
+    a = synth.normal_f16(synth.stream_key(key, "a"), M * K)
+    resid = synth.normal_f16(synth.stream_key(key, "r"), M * N)
+    qw, da = A.QWeight.upload(ctx, w, z, s), ctx.upload(a)
+    w16 = synth.dequantize(w, z, s, K).astype(np.float32).astype(np.float16).astype(np.float64)
+    truth = a.astype(np.float64).reshape(M, K) @ w16.T
+    outs = []
+    for fn in (A.gemm_q, A.gemm_q_static, A.gemm_q):  # the arrival counters are back at zero for the second call
+        dout = ctx.zeros(M * N * 2)
+        fn(ctx, dout, N, da, K, M, qw, K, N)
+        outs.append(dout.download(np.uint16))
+    got = f16(outs[0]).reshape(M, N)
+    assert rel_l2(got, truth) <= 1e-3
+    assert rel_l2(got[-1], truth[-1]) <= 1e-3 and rel_l2(got[:, -32:], truth[:, -32:]) <= 1e-3
+    assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
+    dout = ctx.upload(resid)
+    A.gemm_q(ctx, dout, N, da, K, M, qw, K, N, accum=True)
+    assert rel_l2(f16(dout.download(np.uint16)).reshape(M, N), truth + resid.astype(np.float64).reshape(M, N)) <= 1e-3
+
+
+def test_infinite_activation_stays_in_its_row(ctx):
+    """K that ends in the middle of a step: nothing of a neighbouring row (or of the memory behind the last one) enters."""
+    M, K, N = 40, 1056, 256
+    key = synth.stream_key(53, M, K, N)
+    w, z, s = synth.make_qweight(key, K, N)
+    a = synth.normal_f16(synth.stream_key(key, "a"), M * K).reshape(M, K).copy()
+    qw = A.QWeight.upload(ctx, w, z, s)
+    outs = []
+    for value in (None, np.float16(np.inf)):
+        b = a.copy()
+        if value is not None:
+            b[20, 0] = value
+        dout = ctx.zeros(M * N * 2)
+        A.gemm_q(ctx, dout, N, ctx.upload(b.reshape(-1)), K, M, qw, K, N)
+        outs.append(dout.download(np.uint16).reshape(M, N))
+    rest = [m for m in range(M) if m != 20]
+    assert np.array_equal(outs[0][rest], outs[1][rest])
+    w16 = synth.dequantize(w, z, s, K).astype(np.float32)
+    got = f16(outs[1][20])
+    assert np.array_equal(np.isposinf(got), w16[:, 0] > 0) and np.array_equal(np.isneginf(got), w16[:, 0] < 0)
+
+
+# 64-wide heads, sizes at which the QKV and gate/up products take the 64 to 128 row forms by 128 and 256 columns
+SMALL = dict(dim=2048, hidden_dim=5632, n_layers=2, n_heads=32, n_kv_heads=4, vocab_size=512, seq_len=1280, rope_theta=10000.0)
+
+
+@pytest.fixture(scope="module")
+def small(ctx):
+    img = synth.make_model_image(SMALL, seed=54, scale_mult=0.25)
+    prompt = synth.prompt_tokens(54, 1000, SMALL["vocab_size"])
+    t = A.Transformer(ctx, image=img)
+    t.reset(prompt)
+    for i in range(1000):
+        t.forward(i == 999, use_graph=True)
+    ctx.sync()
+    want = _rows(t, 1000)
+    t.close()
+    return img, prompt, want
+
+
+def _rows(t, n):
+    kv_dim = SMALL["dim"] * SMALL["n_kv_heads"] // SMALL["n_heads"]
+    size = SMALL["n_layers"] * SMALL["seq_len"] * kv_dim
+    return [f16(t.download(name, size)).reshape(SMALL["n_layers"], SMALL["seq_len"], kv_dim)[:, :n].copy() for name in ("key_cache", "value_cache")]
+
+
+@pytest.mark.parametrize("parts", [(20, 45), (100, 129), (300, 400), (1000,)], ids=str)
+def test_prefill_epilogues_against_token_by_token(ctx, small, parts):
+    img, prompt, want = small
+    n = sum(parts)
+    t = A.Transformer(ctx, image=img)
+    t.reset(prompt[:n])
+    for p in parts:
+        t.prefill(p, gen_token=False)
+    ctx.sync()
+    got = _rows(t, n)
+    t.close()
+    for a, b in zip(got, want):
+        for l in range(SMALL["n_layers"]):
+            assert rel_l2(a[l], b[l][:n]) <= 1e-2, l
+            assert rel_l2(a[l][-3:], b[l][n - 3 : n]) <= 1e-2, l
