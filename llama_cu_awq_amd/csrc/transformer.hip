@@ -115,10 +115,9 @@ struct awq_transformer {
     tk::Sync* tk_sync;
     int* tk_err_host;
     long long* tk_trace;  // device buffer of per-phase time stamps when tracing is on, else null
-    // prefill workspace: activations of up to pf_rows tokens, one allocation (grown to the longest prompt met, at most
-    // kPrefillChunk rows)
+    // prefill workspace: activations of up to pf_rows tokens, in the last of pf_blocks
     int pf_rows;
-    uint8_t* pf_block;
+    std::vector<void*> pf_blocks;
     uint16_t *pf_x, *pf_xb, *pf_q, *pf_att, *pf_hb;
 };
 
@@ -247,7 +246,7 @@ void release(awq_transformer* t) {
     (void)hipFree(t->tk_phases);
     (void)hipFree(t->tk_sync);
     (void)hipFree(t->tk_trace);
-    (void)hipFree(t->pf_block);
+    for (void* b : t->pf_blocks) (void)hipFree(b);
     if (t->tk_err_host) (void)hipHostFree(t->tk_err_host);
     delete t;
 }
@@ -268,7 +267,6 @@ awq_transformer* new_transformer(awq_ctx* ctx) {
     t->tk_err_host = nullptr;
     t->tk_trace = nullptr;
     t->pf_rows = 0;
-    t->pf_block = nullptr;
     t->pf_x = t->pf_xb = t->pf_q = t->pf_att = t->pf_hb = nullptr;
     t->issued_pos = 0;
     memset(&t->s, 0, sizeof(t->s));
@@ -812,36 +810,49 @@ int awq_transformer_set_pos(awq_transformer* t, int pos, int token) {
 
 namespace {
 
-// Prompt tokens of one batched pass: a longer prompt streams the weights once per this many tokens.  2000 tokens at the 7B
-// shape: 41.3 ms in chunks of 512 (four passes, each GEMM with its own ramp and tail), 32.3 ms in one (0.84 PFLOP/s);
-// 700 tokens of a small model 5.7 -> 3.8 ms, 650 + 150 tokens at the 70B shape 18.2 -> 17.3 ms a slice of 8 layers.
+// Prompt tokens of one batched pass: a longer prompt streams the weights once per this many tokens, and each GEMM has its
+// ramp and tail in each.  With the 128 x 128 GEMM alone, chunks of 512 -> one pass: 2000 tokens at the 7B shape 41.3 -> 32.3
+// ms, 700 tokens of a small model 5.7 -> 3.8, 650 + 150 tokens on 8 layers of the 70B shape 18.2 -> 17.3.
 constexpr int kPrefillChunk = 2048;
 
+constexpr int kPrefillMinRows = 512;  // of the first allocation
+
+// A workspace for passes of up to min(n_tokens, kPrefillChunk) rows, or of fewer where it cannot be had (the prompt then
+// goes in more passes).  Smaller ones met before stay until the model is released (together less than the largest): a
+// recorded prefill may still replay on them.
 int ensure_prefill_rows(awq_transformer* t, int n_tokens) {
     const awq_config& p = t->cfg;
     int rows = n_tokens < kPrefillChunk ? n_tokens : kPrefillChunk;
     if (rows <= t->pf_rows) return AWQ_OK;
-    if (rows < 2 * t->pf_rows) rows = 2 * t->pf_rows;  // a prompt that grows by a few tokens per call must not reallocate each time
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (t->pf_rows > 0 && (hipStreamIsCapturing(t->ctx->stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone))
+        return AWQ_OK;
+    int least = p.seq_len < kPrefillMinRows ? p.seq_len : kPrefillMinRows;
+    if (least < 2 * t->pf_rows) least = 2 * t->pf_rows;  // a prompt that grows by a few tokens per call must not allocate each time
+    if (rows < least) rows = least;
     rows = (rows + 127) & ~127;
     if (rows > kPrefillChunk) rows = kPrefillChunk;
-    uint16_t** bufs[5] = {&t->pf_x, &t->pf_xb, &t->pf_q, &t->pf_att, &t->pf_hb};
     const size_t widths[5] = {(size_t)p.dim, (size_t)p.dim, (size_t)p.dim, (size_t)p.dim, (size_t)p.hidden_dim};
-    size_t bytes = 0;
-    for (size_t w : widths) bytes += (size_t)rows * w * 2;  // rows of 128 x 128 halves and more: every part stays aligned
-    if (t->pf_block) {
-        AWQ_HIP_TRY(hipStreamSynchronize(t->ctx->stream));
-        (void)hipFree(t->pf_block);
-        t->pf_block = nullptr;
-        t->pf_rows = 0;
-    }
-    hipError_t e = hipMalloc((void**)&t->pf_block, bytes);
+    size_t row_bytes = 0;
+    for (size_t w : widths) row_bytes += w * 2;
+    void* block = nullptr;
+    hipError_t e = hipMalloc(&block, (size_t)rows * row_bytes);
     if (e != hipSuccess) {
-        t->pf_block = nullptr;
-        awq_set_error("prefill workspace allocation failed: %s", hipGetErrorString(e));
-        return AWQ_ERR_HIP;
+        (void)hipGetLastError();
+        if (t->pf_rows > 0) return AWQ_OK;
+        if (rows > kPrefillMinRows) {
+            rows = kPrefillMinRows;
+            e = hipMalloc(&block, (size_t)rows * row_bytes);
+        }
+        if (e != hipSuccess) {
+            awq_set_error("prefill workspace allocation failed: %s", hipGetErrorString(e));
+            return AWQ_ERR_HIP;
+        }
     }
-    uint8_t* at = t->pf_block;
-    for (int i = 0; i < 5; i++) {
+    t->pf_blocks.push_back(block);
+    uint16_t** bufs[5] = {&t->pf_x, &t->pf_xb, &t->pf_q, &t->pf_att, &t->pf_hb};
+    uint8_t* at = static_cast<uint8_t*>(block);
+    for (int i = 0; i < 5; i++) {  // (rows and widths are multiples of 128: every part stays aligned)
         *bufs[i] = reinterpret_cast<uint16_t*>(at);
         at += (size_t)rows * widths[i] * 2;
     }
