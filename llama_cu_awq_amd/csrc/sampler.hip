@@ -281,12 +281,29 @@ __device__ __forceinline__ void select_in_index_order(const uint16_t* probs, int
 // sampler.h:94-107 + gpu_kernels.h:562-592, top-p: position in the descending stable order of the probabilities at
 // which the exact prefix sum, rounded to fp16, first reaches the threshold; the last position when none does.
 // The items come from the thread's rows (vocabularies up to 65535: counters of 16 bits, two to a dword) or, WIDE, straight
-// from global memory with one 32-bit counter per value (larger vocabularies: plain loops, no staging).
+// from global memory with one 32-bit counter per value (larger vocabularies).
+// COUNTED (with WIDE): the histogram is there already, in global memory.
 struct GlobalItems {
     const uint16_t* bits;
 };
-template <bool WIDE, class Items>
-__device__ __forceinline__ void select_in_sorted_order(const Items& x, int n, float threshold, unsigned int* hist32, const SampleOut out) {
+__device__ __forceinline__ void count_wide(unsigned int* hist, unsigned int& zeros, uint32_t bits) {
+    const int b = min((int)bits, kProbBins - 1);
+    if (b == 0)
+        zeros++;
+    else
+        atomicAdd(&hist[b], 1u);
+}
+// the threads' counts of zeros into word 0 of an LDS histogram; ends and begins with a barrier
+__device__ __forceinline__ void add_zeros(unsigned int* hist, unsigned int zeros) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) zeros += __shfl_xor(zeros, off);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0 && zeros) atomicAdd(&hist[0], zeros);
+    __syncthreads();
+}
+template <bool WIDE, bool COUNTED = false, class Items>
+__device__ __forceinline__ void select_in_sorted_order(const Items& x, int n, float threshold, unsigned int* hist32, const SampleOut out,
+                                                       const unsigned int* counted = nullptr) {
     auto hcount = [&](int b) -> unsigned int { return WIDE ? hist32[b] : (hist32[b >> 1] >> (16 * (b & 1))) & 0xFFFFu; };
     __shared__ unsigned long long wave_totals[16];
     __shared__ unsigned int counts[kSampleThreads];
@@ -304,31 +321,29 @@ __device__ __forceinline__ void select_in_sorted_order(const Items& x, int n, fl
     }
     // histogram of the probability values.  Zeros (most of a peaked distribution) are counted per thread instead of
     // through the one LDS word they would all hit.
-    for (int b = tid; b < (WIDE ? kProbBins : (kProbBins + 1) / 2); b += kSampleThreads) hist32[b] = 0u;
-    __syncthreads();
-    unsigned int zeros = 0;
-    auto count_value = [&](uint32_t bits) {
-        const int b = min((int)bits, kProbBins - 1);
-        if (b == 0)
-            zeros++;
-        else if (WIDE)
-            atomicAdd(&hist32[b], 1u);
-        else
-            atomicAdd(&hist32[b >> 1], (b & 1) ? 0x10000u : 1u);
-    };
-    if constexpr (WIDE) {
-        for (int i = tid; i < n; i += kSampleThreads) count_value(x.bits[i]);
+    if (COUNTED) {
+        for (int b = tid; b < kProbBins; b += kSampleThreads) hist32[b] = counted[b];
+        __syncthreads();
     } else {
+        for (int b = tid; b < (WIDE ? kProbBins : (kProbBins + 1) / 2); b += kSampleThreads) hist32[b] = 0u;
+        __syncthreads();
+        unsigned int zeros = 0;
+        if constexpr (WIDE) {
+            for (int i = tid; i < n; i += kSampleThreads) count_wide(hist32, zeros, x.bits[i]);
+        } else {
 #pragma unroll
-        for (int r = 0; r < (int)(sizeof(x.bits) / sizeof(x.bits[0])); r++) {
-            if (r * kSampleThreads + tid < n) count_value(x.bits[r]);
+            for (int r = 0; r < (int)(sizeof(x.bits) / sizeof(x.bits[0])); r++) {
+                if (r * kSampleThreads + tid < n) {
+                    const int b = min((int)x.bits[r], kProbBins - 1);
+                    if (b == 0)
+                        zeros++;
+                    else
+                        atomicAdd(&hist32[b >> 1], (b & 1) ? 0x10000u : 1u);
+                }
+            }
         }
+        add_zeros(hist32, zeros);  // bin 0 is word 0, or its low half
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) zeros += __shfl_xor(zeros, off);
-    __syncthreads();
-    if (lane == 0 && zeros) atomicAdd(&hist32[0], zeros);  // bin 0 is word 0, or its low half
-    __syncthreads();
     // bins in descending order, a contiguous run per thread: thread 0 owns the largest values
     constexpr int BPT = (kProbBins + kSampleThreads - 1) / kSampleThreads;
     const int hi = kProbBins - 1 - tid * BPT;              // first (largest) bin of this thread
@@ -420,19 +435,49 @@ __device__ __forceinline__ void select_in_sorted_order(const Items& x, int n, fl
     }
     if (unique) {
     } else if constexpr (WIDE) {
-        // a contiguous run of items per thread: matches counted per run, the counts scanned, and the thread whose run
-        // holds the wanted match walks it
-        const int per = (n + kSampleThreads - 1) / kSampleThreads;
-        const int i0 = min(tid * per, n), i1 = min(i0 + per, n);
+        // Matches become a bit per element in LDS (over the histogram, which is done with), read from memory 16 bytes per
+        // lane; then a contiguous run of bytes per thread, the counts scanned, and the thread whose run holds the wanted
+        // match walks it.  Vocabularies whose bits do not fit are walked in memory.
+        const int bytes = (n + 7) >> 3;
+        const bool in_lds = bytes <= kProbBins * 4;
+        unsigned char* mask = reinterpret_cast<unsigned char*>(hist32);
+        __syncthreads();
+        if (in_lds) {
+            const bool vec = aligned16(x.bits);
+            for (int e = tid; e < bytes; e += kSampleThreads) {
+                unsigned int m = 0;
+                if (vec && e * 8 + 8 <= n) {
+                    const u32x4 v = reinterpret_cast<const u32x4*>(x.bits)[e];
+#pragma unroll
+                    for (int k = 0; k < 8; k++) m |= (min((int)((v[k >> 1] >> (16 * (k & 1))) & 0xFFFFu), kProbBins - 1) == target_bin ? 1u : 0u) << k;
+                } else {
+                    for (int k = 0; k < 8 && e * 8 + k < n; k++) m |= (min((int)x.bits[e * 8 + k], kProbBins - 1) == target_bin ? 1u : 0u) << k;
+                }
+                mask[e] = (unsigned char)m;
+            }
+            __syncthreads();
+        }
+        auto matches = [&](int e) -> unsigned int {
+            if (in_lds) return mask[e];
+            unsigned int m = 0;
+            for (int k = 0; k < 8 && e * 8 + k < n; k++) m |= (min((int)x.bits[e * 8 + k], kProbBins - 1) == target_bin ? 1u : 0u) << k;
+            return m;
+        };
+        const int per = (bytes + kSampleThreads - 1) / kSampleThreads;
+        const int e0 = min(tid * per, bytes), e1 = min(e0 + per, bytes);
         unsigned int mine = 0;
-        for (int i = i0; i < i1; i++) mine += (min((int)x.bits[i], kProbBins - 1) == target_bin);
+        for (int e = e0; e < e1; e++) mine += __popc(matches(e));
         unsigned int seen = (unsigned int)block_exclusive_scan_1024((unsigned long long)mine, wave_totals);
         if (seen < target_rank && seen + mine >= target_rank) {
-            for (int i = i0; i < i1; i++) {
-                if (min((int)x.bits[i], kProbBins - 1) == target_bin && ++seen == target_rank) {
-                    s_index = i;
+            for (int e = e0; e < e1; e++) {
+                unsigned int m = matches(e);
+                const unsigned int c = __popc(m);
+                if (seen + c >= target_rank) {
+                    for (unsigned int skip = target_rank - seen - 1; skip; skip--) m &= m - 1u;
+                    s_index = e * 8 + __ffs((int)m) - 1;
                     break;
                 }
+                seen += c;
             }
         }
     } else {
@@ -505,6 +550,126 @@ __global__ __launch_bounds__(kSampleThreads) void sample_sorted_large_kernel(con
     select_in_sorted_order<true>(GlobalItems{probs}, n, threshold, dyn_lds, SampleOut{result, pPos, pPosGpu, mirror});
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// The same for a sampler, which holds scratch memory: the vocabulary over many workgroups, in four launches.  One
+// workgroup's passes over a large vocabulary are bound by their own round trips (65535 entries 46 us, 128256 entries, two
+// bytes per lane, softmax 84 us and selection 90 us); here 33 and 40 us, most of it the four launches.  Sums keep the order of the one-workgroup kernel (column t = elements t, t + 1024,
+// ..., one after the other, then the tree over the 1024 columns), so the probabilities are the same bits.
+constexpr int kWideVocab = 32768;  // beyond: one workgroup 40 us and more, this 29 (40000 entries); 32000: 26 against 28
+constexpr int kWideMaxGroups = 64;
+constexpr int kWideColumns = 32;    // columns per workgroup of the second kernel
+constexpr int kWideChunkRows = 128;  // rows whose exponentials are in LDS at a time
+struct WideScratch {
+    float max_part[kWideMaxGroups];
+    float column_sum[kSampleThreads];
+    unsigned int hist[kProbBins];
+};
+
+// maximum of the logits per workgroup (rounding and a positive temperature keep the order); clears the histogram
+__global__ __launch_bounds__(256) void wide_max_kernel(const uint16_t* logits, int n, WideScratch* ws) {
+    __shared__ float red[4];
+    const int gid = blockIdx.x * 256 + threadIdx.x, stride = kWideMaxGroups * 256;
+    static_assert(kWideMaxGroups * 256 >= kProbBins, "a thread clears at most one word");
+    if (gid < kProbBins) ws->hist[gid] = 0u;
+    float m = -INFINITY;
+    const int n8 = aligned16(logits) ? n >> 3 : 0;
+    for (int e = gid; e < n8; e += stride) {
+        const u32x4 v = reinterpret_cast<const u32x4*>(logits)[e];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const h16x2 h = as_h2(v[k]);
+            m = fmaxf(m, fmaxf((float)h[0], (float)h[1]));
+        }
+    }
+    for (int i = n8 * 8 + gid; i < n; i += stride) m = fmaxf(m, half_bits_to_float(logits[i]));
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) ws->max_part[blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+}
+
+// exponentials (rounded, in place of the logits) and the columns' sums of the unrounded ones
+__global__ __launch_bounds__(kSampleThreads) void wide_exp_kernel(uint16_t* logits, int n, float temperature, WideScratch* ws) {
+    __shared__ float vals[kWideChunkRows * kWideColumns];
+    static_assert(kWideMaxGroups == 64, "a lane per partial maximum");
+    const int tid = threadIdx.x, column = tid % kWideColumns, row0 = tid / kWideColumns;
+    const float raw = wave_max(ws->max_part[tid & 63]);
+    const float max_val = fmaxf(-3.402823466e+38f, half_bits_to_float(float_to_half_bits(raw / temperature)));
+    const int rows = (n + kSampleThreads - 1) / kSampleThreads;
+    constexpr int STEP = kSampleThreads / kWideColumns, PER = kWideChunkRows / STEP;
+    uint16_t* mine = logits + blockIdx.x * kWideColumns + column;
+    const int first = blockIdx.x * kWideColumns + column;
+    float sum = 0.0f;
+    for (int base = 0; base < rows; base += kWideChunkRows) {
+        uint16_t l[PER];
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const long long i = (long long)(base + row0 + k * STEP) * kSampleThreads;
+            l[k] = first + i < n ? mine[i] : (uint16_t)0;
+        }
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int r = base + row0 + k * STEP;
+            const long long i = (long long)r * kSampleThreads;
+            if (first + i < n) {
+                const uint16_t h = float_to_half_bits(half_bits_to_float(l[k]) / temperature);
+                const float v = expf(half_bits_to_float(h) - max_val);
+                mine[i] = float_to_half_bits(v);
+                vals[(r - base) * kWideColumns + column] = v;
+            }
+        }
+        __syncthreads();
+        if (tid < kWideColumns) {
+            const int end = min(rows - base, kWideChunkRows);
+            for (int r = 0; r < end; r++)
+                if (first + (long long)(base + r) * kSampleThreads < n) sum += vals[r * kWideColumns + column];
+        }
+        __syncthreads();
+    }
+    if (tid < kWideColumns) ws->column_sum[first] = sum;
+}
+
+// probabilities in place of the exponentials and, for the top-p selection, their histogram
+__global__ __launch_bounds__(kSampleThreads) void wide_divide_kernel(uint16_t* logits, int n, int count, WideScratch* ws) {
+    extern __shared__ unsigned int dyn_lds[];  // the workgroup's histogram
+    __shared__ float red[16];
+    const int tid = threadIdx.x, gid = blockIdx.x * kSampleThreads + tid, stride = gridDim.x * kSampleThreads;
+    if (count)
+        for (int b = tid; b < kProbBins; b += kSampleThreads) dyn_lds[b] = 0u;
+    const float sum = block_sum_1024(ws->column_sum[tid], red);  // (its barriers also publish the cleared histogram)
+    unsigned int zeros = 0;
+    const int n8 = aligned16(logits) ? n >> 3 : 0;
+    for (int e = gid; e < n8; e += stride) {
+        u32x4 v = reinterpret_cast<const u32x4*>(logits)[e];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const h16x2 h = as_h2(v[k]);
+            const uint32_t lo = float_to_half_bits((float)h[0] / sum), hi = float_to_half_bits((float)h[1] / sum);
+            v[k] = lo | (hi << 16);
+            if (count) {
+                count_wide(dyn_lds, zeros, lo);
+                count_wide(dyn_lds, zeros, hi);
+            }
+        }
+        reinterpret_cast<u32x4*>(logits)[e] = v;
+    }
+    for (int i = n8 * 8 + gid; i < n; i += stride) {
+        const uint16_t h = float_to_half_bits(half_bits_to_float(logits[i]) / sum);
+        logits[i] = h;
+        if (count) count_wide(dyn_lds, zeros, h);
+    }
+    if (!count) return;
+    add_zeros(dyn_lds, zeros);
+    for (int b = tid; b < kProbBins; b += kSampleThreads)
+        if (dyn_lds[b]) atomicAdd(&ws->hist[b], dyn_lds[b]);
+}
+
+__global__ __launch_bounds__(kSampleThreads) void wide_select_kernel(const uint16_t* probs, int n, float threshold, const WideScratch* ws,
+                                                                     int* result, volatile int* pPos, int* pPosGpu, int* mirror) {
+    extern __shared__ unsigned int dyn_lds[];
+    select_in_sorted_order<true, true>(GlobalItems{probs}, n, threshold, dyn_lds, SampleOut{result, pPos, pPosGpu, mirror}, ws->hist);
+}
+
 __global__ __launch_bounds__(kSampleThreads) void sample_plain_kernel(const uint16_t* probs, int n, float threshold, int vec,
                                                                       int* result, volatile int* pPos, int* pPosGpu, int* mirror) {
     extern __shared__ unsigned int dyn_lds[];  // the values, for vocabularies up to kLdsVocab
@@ -561,6 +726,7 @@ struct awq_sampler {
     float temperature;
     float topp;
     unsigned long long rng_state;
+    WideScratch* wide;  // scratch of the many-workgroup kernels; null: small vocabulary, or no memory for it
 };
 
 // xorshift* (sampler.h:65-74)
@@ -674,9 +840,23 @@ int awq_sampler_run(awq_sampler* s, uint16_t* logits, int* tokens, volatile int*
         return awq_launch_argmax(s->ctx, logits, s->vocab_size, tokens, pos_host, pos_dev, gen_token, mirror);
     const bool nucleus = s->topp > 0.0f && s->topp < 1.0f;
     const float threshold = nucleus ? coin * s->topp : coin;
-    if (nucleus ? s->vocab_size <= 65535 : s->vocab_size <= kLdsVocab)  // softmax and selection in one launch
+    if (nucleus ? !s->wide && s->vocab_size <= 65535 : s->vocab_size <= kLdsVocab)  // softmax and selection in one launch
         return launch_softmax_sample(s->ctx, logits, s->vocab_size, s->temperature, threshold, nucleus ? 1 : 0, tokens, pos_host,
                                      pos_dev, mirror);
+    if (s->wide) {
+        const size_t hist = nucleus ? (size_t)kProbBins * sizeof(unsigned int) : 0;
+        const int n = s->vocab_size;
+        hipLaunchKernelGGL(wide_max_kernel, dim3(kWideMaxGroups), dim3(256), 0, s->ctx->stream, logits, n, s->wide);
+        hipLaunchKernelGGL(wide_exp_kernel, dim3(kSampleThreads / kWideColumns), dim3(kSampleThreads), 0, s->ctx->stream, logits, n,
+                           s->temperature, s->wide);
+        hipLaunchKernelGGL(wide_divide_kernel, dim3(16), dim3(kSampleThreads), hist, s->ctx->stream, logits, n, nucleus ? 1 : 0, s->wide);
+        if (nucleus)
+            hipLaunchKernelGGL(wide_select_kernel, dim3(1), dim3(kSampleThreads), hist, s->ctx->stream, logits, n, threshold, s->wide, tokens,
+                               pos_host, pos_dev, mirror);
+        if (int r = awq_check_launch("sample (wide)")) return r;
+        if (nucleus) return AWQ_OK;
+        return launch_sample(s->ctx, logits, n, threshold, 0, tokens, pos_host, pos_dev, mirror);
+    }
     if (int r = launch_softmax_logits(s->ctx, logits, s->vocab_size, s->temperature)) return r;
     return launch_sample(s->ctx, logits, s->vocab_size, threshold, nucleus ? 1 : 0, tokens, pos_host, pos_dev, mirror);
 }
@@ -711,11 +891,17 @@ int awq_sampler_create(awq_ctx* ctx, int vocab_size, float temperature, float to
     s->temperature = temperature;
     s->topp = topp;
     s->rng_state = rng_seed;
+    s->wide = nullptr;
+    if (vocab_size > kWideVocab && temperature > 0.0f && hipMalloc((void**)&s->wide, sizeof(WideScratch)) != hipSuccess) {
+        (void)hipGetLastError();
+        s->wide = nullptr;  // (the one-workgroup kernels need none)
+    }
     *out = s;
     return AWQ_OK;
 }
 
 int awq_sampler_destroy(awq_sampler* s) {
+    if (s && s->wide) (void)hipFree(s->wide);
     delete s;
     return AWQ_OK;
 }

@@ -126,6 +126,50 @@ def test_sampler_object_follows_reference_sample(ctx, temperature, topp, V):
     pin.close()
 
 
+@pytest.mark.parametrize("topp", [0.6, 0.95, 1.0])
+@pytest.mark.parametrize("n", [32769, 40000, 50000, 65535, 65537, 100003, 128256, 500001, 1 << 20])
+def test_sampler_object_equals_the_two_entry_points(ctx, n, topp):
+    """The sampler spreads a large vocabulary over workgroups; the stand-alone softmax and selection run in one.  Same bits:
+    probabilities, token, positions, for aligned and unaligned logits, flat and peaked distributions and values that are
+    not finite."""
+    rng = np.random.default_rng(n)
+    cases = [(_logits(1, n, 3.0), 0.5), (_logits(2, n, 0.1), 1.3), (_logits(3, n, 12.0), 0.7)]
+    peak = _logits(4, n, 1.0)
+    peak[n - 1] = 60.0
+    inf = _logits(5, n, 1.0)
+    inf[rng.integers(0, n, 50)] = -np.inf
+    nan = _logits(6, n, 1.0)
+    nan[n // 2] = np.nan
+    cases += [(peak, 0.5), (inf, 0.8), (nan, 0.8), (np.full(n, -np.inf, np.float16), 0.8), (np.full(n, 60000, np.float16), 0.5)]
+    pin = Pinned(ctx)
+    for step, (logits, temperature) in enumerate(cases):
+        offset = step % 2  # an odd element: no 16-byte loads
+        padded = np.concatenate([np.zeros(offset, np.float16), logits])
+        s = A.Sampler(ctx, n, temperature, topp, 77 + step)
+        got = []
+        for alone in (False, True):
+            d = ctx.upload(padded.view(np.uint16))
+            pin.set_pos(3)
+            pin.tokens[4] = -1
+            at = d.ptr + 2 * offset
+            if alone:
+                coin = np.float32(oracle.random_f32(np.array([77 + step], dtype=np.uint64)))
+                nucleus = topp < 1.0
+                A.softmax_logits(ctx, at, n, temperature)
+                A.sample_top_p(ctx, at, n, float(coin * np.float32(topp)) if nucleus else float(coin), int(nucleus), pin.host + 16, pin.host, pin.dpos)
+            else:
+                s.sample(at, pin.host + 16, pin.host, pin.dpos, True)
+            ctx.sync()
+            assert pin.pos.value == 4 and pin.dpos.download(np.int32)[0] == 4
+            got.append((d.download(np.uint16), pin.tokens[4]))
+        s.close()
+        assert np.array_equal(got[0][0], got[1][0]), step
+        assert got[0][1] == got[1][1], step
+        if step < 5:
+            assert got[0][1] == _oracle_pick(f16(got[0][0])[offset:], float(coin * np.float32(topp)) if nucleus else float(coin), int(nucleus)), step
+    pin.close()
+
+
 @pytest.mark.parametrize("use_graph", [False, True])
 def test_transformer_sample_loop(ctx, use_graph):
     """forward_logits + sample on a small model: greedy sampler == the fused forward; stochastic sampler picks what
