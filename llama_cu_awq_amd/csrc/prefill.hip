@@ -515,6 +515,17 @@ int awq_gemm_device_setup(int device) {
 }
 
 // ---------------------------------------------------------------- launchers (internal)
+// The context's split-K workspace, allocated whole the first time.
+int awq_reserve_gemm_workspace(awq_ctx* ctx) {
+    if (ctx->gemm_part) return AWQ_OK;
+    void* block = nullptr;
+    AWQ_HIP_TRY(hipMalloc(&block, kScratchBytes));
+    ctx->gemm_part = static_cast<float*>(block);
+    unsigned int* counter = reinterpret_cast<unsigned int*>(static_cast<uint8_t*>(block) + kPartBytes);
+    hipLaunchKernelGGL(pf::clear_words_kernel, dim3(1), dim3(kPartTiles), 0, ctx->stream, counter, kPartTiles);
+    return awq_check_launch("clear_words");
+}
+
 // The split-K workspace of a launch over `tiles` output tiles: the file-scope device array (static_ws; no allocation) or
 // the context's, allocated whole on first use, so that it never moves.
 static int bind_workspace(awq_ctx* ctx, pf::GemmParams& p, int tiles, bool static_ws, const char* what) {
@@ -531,14 +542,7 @@ static int bind_workspace(awq_ctx* ctx, pf::GemmParams& p, int tiles, bool stati
         hipLaunchKernelGGL(pf::clear_words_kernel, dim3(div_up(tiles, 256)), dim3(256), 0, ctx->stream, p.part_counter, tiles);
         return awq_check_launch("clear_words");
     }
-    if (!ctx->gemm_part) {
-        void* block = nullptr;
-        AWQ_HIP_TRY(hipMalloc(&block, kScratchBytes));
-        ctx->gemm_part = static_cast<float*>(block);
-        unsigned int* counter = reinterpret_cast<unsigned int*>(static_cast<uint8_t*>(block) + kPartBytes);
-        hipLaunchKernelGGL(pf::clear_words_kernel, dim3(1), dim3(kPartTiles), 0, ctx->stream, counter, kPartTiles);
-        if (int r = awq_check_launch("clear_words")) return r;
-    }
+    if (int r = awq_reserve_gemm_workspace(ctx)) return r;
     p.part = ctx->gemm_part;
     p.part_counter = reinterpret_cast<unsigned int*>(reinterpret_cast<uint8_t*>(ctx->gemm_part) + kPartBytes);
     return AWQ_OK;
@@ -571,6 +575,10 @@ static int launch_gemm(awq_ctx* ctx, pf::GemmParams& p, int ntiles, const char* 
     // a single matrix with fewer tiles than compute units: two workgroups per tile, each half of K
     p.ksplit = (p.epi == pf::EPI_STORE || p.epi == pf::EPI_RESID) && tiles < 256 && p.K >= 8 * pf::BK ? 2 : 1;
     const bool may_split = p.ksplit == 2 || (p.epi != pf::EPI_STORE && p.epi != pf::EPI_RESID);
+    // reserved by every product of few tiles, whether its form splits K or not: a smaller one of the same weights, which
+    // may be recorded into a graph where nothing can be allocated, may split
+    if (p.ksplit == 2 && !static_ws)
+        if (int r = awq_reserve_gemm_workspace(ctx)) return r;
     const awq_rows_plan plan = awq_plan_gemm_rows(ctx->cus, p.M, p.K, ntiles * 2, may_split);
     if (plan.form >= 0 && plan.us < general_us(ctx->cus, tiles, p.K, p.ksplit) && (!a_perm || (p.K & 127) == 0)) {
         if (plan.ksplit > 1)

@@ -35,6 +35,7 @@ int awq_launch_argmax(awq_ctx* ctx, const uint16_t* logits, int size, int* token
 int awq_sampler_run(awq_sampler* s, uint16_t* logits, int* tokens, volatile int* pos_host, int* pos_dev, int gen_token,
                     int* mirror);
 // prefill.hip
+int awq_reserve_gemm_workspace(awq_ctx* ctx);
 int awq_launch_gemm_single(awq_ctx* ctx, uint16_t* out, long long ldo, const uint16_t* A, int lda, int M, const awq_qweight* w,
                            int K, int N, int accum, bool static_ws, bool a_perm);
 int awq_launch_gemm_qkv(awq_ctx* ctx, uint16_t* q, uint16_t* kcache_layer, uint16_t* vcache_layer, const uint16_t* A, int lda, int M,
@@ -832,6 +833,9 @@ int ensure_prefill_rows(awq_transformer* t, int n_tokens) {
     if (rows < least) rows = least;
     rows = (rows + 127) & ~127;
     if (rows > kPrefillChunk) rows = kPrefillChunk;
+    // with the first pass, whether its products split K or not: that of a shorter prompt, which may be recorded, may
+    // (where it cannot be had, the products that do split say so)
+    if (t->pf_rows == 0 && awq_reserve_gemm_workspace(t->ctx)) (void)hipGetLastError();
     const size_t widths[5] = {(size_t)p.dim, (size_t)p.dim, (size_t)p.dim, (size_t)p.dim, (size_t)p.hidden_dim};
     size_t row_bytes = 0;
     for (size_t w : widths) row_bytes += w * 2;

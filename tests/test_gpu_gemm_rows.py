@@ -4,11 +4,14 @@ quantisation group, K past eight groups (scales and zeros travel for eight at a 
 
 Bar: the weights are exact fp16 values, sums are fp32 and the result is rounded once: rel-L2 2.1e-4 by the rounding alone;
 1e-3 as for the other GEMM tests."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import llama_cu_awq_amd as A
 from llama_cu_awq_amd import synth
+from llama_cu_awq_amd._lib import lib
 from tests.helpers import f16, rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -107,3 +110,44 @@ def test_prefill_epilogues_against_token_by_token(ctx, small, parts):
         for l in range(SMALL["n_layers"]):
             assert rel_l2(a[l], b[l][:n]) <= 1e-2, l
             assert rel_l2(a[l][-3:], b[l][n - 3 : n]) <= 1e-2, l
+
+
+def test_short_prefill_recorded_after_a_long_one():
+    """1100 rows by 4096 columns split no K, 37 do: what that takes is there before the short prompt is recorded."""
+    cfg = dict(dim=4096, hidden_dim=1024, n_layers=1, n_heads=32, n_kv_heads=4, vocab_size=512, seq_len=1152, rope_theta=10000.0)
+    img = synth.make_model_image(cfg, seed=55, scale_mult=0.25)
+    prompt = synth.prompt_tokens(55, 1137, cfg["vocab_size"])
+    ctx = A.Context(0)
+    t = A.Transformer(ctx, image=img)
+
+    def caches():
+        return [t.download(name, cfg["seq_len"] * 512) for name in ("key_cache", "value_cache")]
+
+    # (looked up through the library: the HIP runtime it is linked with)
+    def hip(name, *args):
+        assert getattr(lib, name)(*args) == 0, name
+
+    stream, graph, runnable = C.c_void_p(lib.awq_ctx_stream(ctx.h)), C.c_void_p(), C.c_void_p()
+    t.reset(prompt)
+    t.prefill(1100, gen_token=False)
+    hip("hipStreamBeginCapture", stream, 0)
+    t.prefill(37, gen_token=False)
+    hip("hipStreamEndCapture", stream, C.byref(graph))
+    hip("hipGraphInstantiate", C.byref(runnable), graph, None, None, C.c_size_t(0))
+    recorded = []
+    for _ in range(3):
+        hip("hipGraphLaunch", runnable, stream)
+        ctx.sync()
+        recorded.append(caches())
+    t.reset(prompt)
+    t.prefill(1100, gen_token=False)
+    t.prefill(37, gen_token=False)
+    ctx.sync()
+    want = caches()
+    for got in recorded:
+        for a, b in zip(got, want):
+            assert np.array_equal(a, b) and f16(b).reshape(-1, 512)[1100:1137].any(axis=1).all()
+    hip("hipGraphExecDestroy", runnable)
+    hip("hipGraphDestroy", graph)
+    t.close()
+    ctx.close()
