@@ -2,6 +2,8 @@
 // KV-cache attention, the fp16 classifier matrix-vector product and the greedy
 // sampler.  Arithmetic and rounding points follow the reference kernels cited
 // at each entry point; launch geometry and data movement are this library's.
+#include <type_traits>
+
 #include "attention.hpp"
 #include "common.hpp"
 
@@ -391,7 +393,8 @@ __global__ __launch_bounds__(1024) void attn_fused_kernel(uint16_t* output, uint
 
 // ------------------------------------------------------------------ fp16 matvec
 // out[r] = half(sum_j w[r*n + j] * x[j]).  x staged in LDS in natural order;
-// a lane owns the same 16-byte column slices for the R rows of its wave.
+// a lane owns the same 16-byte column slices for the R rows of its wave.  A row's sums do not depend on R.  Bound by memory:
+// 6.2-7.1 TB/s from 100 MB on.
 template <int R, bool NORM>
 __global__ __launch_bounds__(256) void gemv_f16_kernel(uint16_t* out, const uint16_t* x, const uint16_t* w, int n, int d,
                                                        const uint16_t* norm_w, uint16_t* norm_out) {
@@ -636,13 +639,24 @@ int awq_launch_attention_partial(awq_ctx* ctx, float* part, int* chunks_out, con
 // Internal: fp16 matvec with optional fused RMSNorm of x (norm_out must not alias x).
 int awq_launch_matvec_f16(awq_ctx* ctx, uint16_t* out, const uint16_t* x, const uint16_t* w, int n, int d,
                           const uint16_t* norm_w, uint16_t* norm_out) {
-    constexpr int R = 4;
-    const dim3 grid(div_up(d, 4 * R));
-    const size_t lds = (size_t)n * 2;
-    if (norm_w)
-        awq_launch(ctx, gemv_f16_kernel<R, true>, grid, dim3(256), lds, out, x, w, n, d, norm_w, norm_out);
+    const auto launch = [&](auto rows) {
+        constexpr int R = decltype(rows)::value;
+        const dim3 grid(div_up(d, 4 * R));
+        const size_t lds = (size_t)n * 2;
+        if (norm_w)
+            awq_launch(ctx, gemv_f16_kernel<R, true>, grid, dim3(256), lds, out, x, w, n, d, norm_w, norm_out);
+        else
+            awq_launch(ctx, gemv_f16_kernel<R, false>, grid, dim3(256), lds, out, x, w, n, d, norm_w, norm_out);
+    };
+    // Rows a power of two apart: the four rows that a wave asks for together, and those of its neighbours, fall on the same
+    // memory channels, and two rows a wave spread better.  us, four rows | two rows, weights from memory: n = 2048, 32000
+    // rows 23.9 | 21.2, 128256 rows 80.6 | 74.1; 8192, 32000 rows 89.6 | 80.5, 128256 rows 331 | 305; 16384, 32000 rows
+    // 185 | 172.  n = 4096 is the exception (41.1 | 42.1).  Other lengths want four (fewer workgroups to stage x): 1536 16.7 |
+    // 17.6, 3072 30.0 | 30.8, 5120 48.9 | 50.6, 7168 68.0 | 69.6, 24576 236 | 245; below 2048 too (1024: 12.0 | 13.0).
+    if (n >= 2048 && (n & (n - 1)) == 0 && n != 4096)
+        launch(std::integral_constant<int, 2>{});
     else
-        awq_launch(ctx, gemv_f16_kernel<R, false>, grid, dim3(256), lds, out, x, w, n, d, norm_w, norm_out);
+        launch(std::integral_constant<int, 4>{});
     return awq_check_launch("gemv_f16");
 }
 

@@ -559,6 +559,23 @@ def test_matvec_f16(ctx, n, d):
     assert_close_f16(got, want, ulps=2)
 
 
+# power-of-two row lengths take two rows per wave: row counts around a wave's and a workgroup's share, and the lengths on
+# either side of the rule.  Bars as above: one fp16 rounding of an fp32 sum.
+@pytest.mark.parametrize("n", [1024, 2048, 4096, 8192, 16384])
+@pytest.mark.parametrize("d", [8, 24, 1032])
+def test_matvec_f16_power_of_two_rows(ctx, n, d):
+    key = synth.stream_key(70, n, d)
+    w = synth.normal_f16(synth.stream_key(key, "w"), n * d, 0.0, 0.02)
+    x = synth.normal_f16(synth.stream_key(key, "x"), n)
+    guard = np.full(d + 8, 0x7E01, dtype=np.uint16)
+    dout = ctx.upload(guard)
+    A.matmul(ctx, dout, ctx.upload(x), ctx.upload(w), n, d)
+    got = dout.download(np.uint16)
+    assert np.array_equal(got[d:], guard[d:])
+    truth = w.astype(np.float64).reshape(d, n) @ x.astype(np.float64)
+    assert rel_l2(f16(got[:d]), truth) <= 1e-3
+
+
 def test_argmax_advance_and_ties(ctx):
     V = 32000
     logits = synth.normal_f16(synth.stream_key(8, "l"), V)
