@@ -552,9 +552,10 @@ __global__ __launch_bounds__(kSampleThreads) void sample_sorted_large_kernel(con
 
 // ---------------------------------------------------------------------------------------------------------------
 // The same for a sampler, which holds scratch memory: the vocabulary over many workgroups, in four launches.  One
-// workgroup's passes over a large vocabulary are bound by their own round trips (65535 entries 46 us, 128256 entries, two
-// bytes per lane, softmax 84 us and selection 90 us); here 33 and 40 us, most of it the four launches.  Sums keep the order of the one-workgroup kernel (column t = elements t, t + 1024,
-// ..., one after the other, then the tree over the 1024 columns), so the probabilities are the same bits.
+// workgroup's passes over a large vocabulary are bound by their own round trips (65535 entries 46 us; 128256 entries, two
+// bytes per lane, softmax 84 us and selection 90 us); here 33 and 40 us, most of it the four launches.  Sums keep the order
+// of the one-workgroup kernel (column t = elements t, t + 1024, ..., one after the other, then the tree over the 1024
+// columns), so the probabilities are the same bits.
 constexpr int kWideVocab = 32768;  // beyond: one workgroup 40 us and more, this 29 (40000 entries); 32000: 26 against 28
 constexpr int kWideMaxGroups = 64;
 constexpr int kWideColumns = 32;    // columns per workgroup of the second kernel
