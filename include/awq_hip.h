@@ -311,6 +311,11 @@ int awq_gemm_int4(awq_ctx* ctx, uint16_t* out, int ldo, const uint16_t* a, int l
 int awq_gemm_int4_static(awq_ctx* ctx, uint16_t* out, int ldo, const uint16_t* a, int lda, int M, const awq_qweight* w, int K,
                          int N, int accum);
 
+/* Diagnostic (no counterpart in the reference, no device work): how the two calls above run a product on a GPU of
+ * `compute_units`: form = {rows, columns of a workgroup's tile, K slices inside a workgroup, workgroups per tile along K};
+ * {128, 128, 1, ...} is the 128 x 128 kernel.  AWQ_ERR_SHAPE where they would refuse the sizes. */
+int awq_gemm_int4_form(int compute_units, int M, int K, int N, int form[4]);
+
 /* Consume the n_tokens tokens at positions pos .. pos+n_tokens-1 of the shared token list in one batched pass:
  * afterwards the KV cache rows, the logits (of the last token), the token list and the position are those that
  * n_tokens calls of awq_transformer_forward (gen_token false for all but the last, `gen_token` for the last) would

@@ -12,6 +12,7 @@ from .ops import (  # noqa: F401
     copy_embedding,
     dequant,
     ffn_matvec_silu,
+    gemm_form,
     gemm_q,
     gemm_q_static,
     matmul,

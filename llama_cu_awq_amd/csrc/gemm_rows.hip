@@ -515,6 +515,12 @@ awq_rows_plan awq_plan_gemm_rows(int cus, int M, int K, int groups, bool may_spl
     return best;
 }
 
-int awq_launch_gemm_rows(awq_ctx* ctx, pf::GemmParams& p, int groups, const awq_rows_plan& plan, bool a_perm, const char* what) {
-    return kForms[plan.form].launch(ctx, p, groups, plan.ksplit, a_perm, what);
+int awq_launch_gemm_rows(awq_ctx* ctx, pf::GemmParams& p, int groups, int form, int ksplit, bool a_perm, const char* what) {
+    return kForms[form].launch(ctx, p, groups, ksplit, a_perm, what);
+}
+
+void awq_rows_form(int form, int* tile) {
+    tile[0] = kForms[form].rows;
+    tile[1] = kForms[form].nw * 64;
+    tile[2] = kForms[form].kw;
 }

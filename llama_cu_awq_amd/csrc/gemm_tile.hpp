@@ -125,4 +125,5 @@ struct awq_step_us {
 float awq_gemm_us(int cus, int per_cu, long long wgs, int steps, const awq_step_us& t);
 int awq_gemm_rows_setup();  // once per device, with that device current
 awq_rows_plan awq_plan_gemm_rows(int cus, int M, int K, int groups, bool may_split);
-int awq_launch_gemm_rows(awq_ctx* ctx, pf::GemmParams& p, int groups, const awq_rows_plan& plan, bool a_perm, const char* what);
+int awq_launch_gemm_rows(awq_ctx* ctx, pf::GemmParams& p, int groups, int form, int ksplit, bool a_perm, const char* what);
+void awq_rows_form(int form, int* tile);  // rows, columns, K slices inside a workgroup

@@ -555,6 +555,23 @@ static float general_us(int cus, long long tiles, int K, int ksplit) {
     return awq_gemm_us(cus, 2, tiles * ksplit, div_up(div_up(K, pf::BK), ksplit), awq_step_us{0.52f, 0.58f, 1.1f}) + split;
 }
 
+// How a product over `ntiles` tiles of 128 weight rows runs.
+struct GemmRoute {
+    int form;    // of gemm_rows.hip; -1: the 128 x 128 kernel
+    int ksplit;  // workgroups per tile along K
+};
+// The 128 x 128 kernel gives a single matrix with fewer tiles than compute units two workgroups per tile, each half of K.
+static bool general_splits(int M, int K, int ntiles, bool single) {
+    return single && (long long)div_up(M, pf::BM) * ntiles < 256 && K >= 8 * pf::BK;
+}
+// single: one matrix (plain or residual form); the QKV and gate/up products split K in the row forms only
+static GemmRoute route_gemm(int cus, int M, int K, int ntiles, bool single) {
+    const int ksplit = general_splits(M, K, ntiles, single) ? 2 : 1;
+    const awq_rows_plan plan = awq_plan_gemm_rows(cus, M, K, ntiles * 2, ksplit == 2 || !single);
+    if (plan.form >= 0 && plan.us < general_us(cus, (long long)div_up(M, pf::BM) * ntiles, K, ksplit)) return GemmRoute{plan.form, plan.ksplit};
+    return GemmRoute{-1, ksplit};
+}
+
 // static_ws: take the split-K workspace from the file-scope device array (no allocation) instead of the context's.
 // a_perm: A holds every 8 activations in the order (0,4,1,5,2,6,3,7).
 // *rotated (QKV): whether the epilogue did what p.rope asks for.
@@ -569,24 +586,18 @@ static int launch_gemm(awq_ctx* ctx, pf::GemmParams& p, int ntiles, const char* 
         awq_set_error("%s: activation block of %d x %d halves exceeds 4 GB", what, p.M, p.lda);
         return AWQ_ERR_SHAPE;
     }
-    p.mtiles = div_up(p.M, pf::BM);
-    p.ntiles = ntiles;
-    const long long tiles = (long long)p.mtiles * ntiles;
-    // a single matrix with fewer tiles than compute units: two workgroups per tile, each half of K
-    p.ksplit = (p.epi == pf::EPI_STORE || p.epi == pf::EPI_RESID) && tiles < 256 && p.K >= 8 * pf::BK ? 2 : 1;
-    const bool may_split = p.ksplit == 2 || (p.epi != pf::EPI_STORE && p.epi != pf::EPI_RESID);
+    const bool single = p.epi == pf::EPI_STORE || p.epi == pf::EPI_RESID;
     // reserved by every product of few tiles, whether its form splits K or not: a smaller one of the same weights, which
     // may be recorded into a graph where nothing can be allocated, may split
-    if (p.ksplit == 2 && !static_ws)
+    if (general_splits(p.M, p.K, ntiles, single) && !static_ws)
         if (int r = awq_reserve_gemm_workspace(ctx)) return r;
-    const awq_rows_plan plan = awq_plan_gemm_rows(ctx->cus, p.M, p.K, ntiles * 2, may_split);
-    if (plan.form >= 0 && plan.us < general_us(ctx->cus, tiles, p.K, p.ksplit) && (!a_perm || (p.K & 127) == 0)) {
-        if (plan.ksplit > 1)
-            if (int r = bind_workspace(ctx, p, kPartTiles, static_ws, what)) return r;
-        return awq_launch_gemm_rows(ctx, p, ntiles * 2, plan, a_perm, what);
-    }
-    if (p.ksplit == 2)
-        if (int r = bind_workspace(ctx, p, (int)tiles, static_ws, what)) return r;
+    const GemmRoute route = route_gemm(ctx->cus, p.M, p.K, ntiles, single);
+    p.mtiles = div_up(p.M, pf::BM);
+    p.ntiles = ntiles;
+    p.ksplit = route.ksplit;
+    if (p.ksplit > 1)
+        if (int r = bind_workspace(ctx, p, route.form >= 0 ? kPartTiles : p.mtiles * ntiles, static_ws, what)) return r;
+    if (route.form >= 0) return awq_launch_gemm_rows(ctx, p, ntiles * 2, route.form, route.ksplit, a_perm, what);
     if (p.rope && p.head_size != 128) {
         p.rope = nullptr;
         *rotated = false;
@@ -712,6 +723,21 @@ int awq_gemm_int4_static(awq_ctx* ctx, uint16_t* out, int ldo, const uint16_t* a
     AWQ_REQUIRE(ctx->device >= 0 && ctx->device < kMaxDevices && g_scratch_ptr[ctx->device] && g_gemm_lds_raised[ctx->device],
                 AWQ_ERR_HIP, "the static workspace was not set up on this device when the context was created");
     return awq_launch_gemm_single(ctx, out, ldo, a, lda, M, w, K, N, accum, true, false);
+}
+
+int awq_gemm_int4_form(int compute_units, int M, int K, int N, int form[4]) {
+    AWQ_REQUIRE(form && compute_units > 0, AWQ_ERR_ARG, "null form or no compute units");
+    if (M <= 0 || K <= 0 || N <= 0 || (K & 31) || (N & 127)) {
+        awq_set_error("awq_gemm_int4_form: needs M > 0, K %% 32 == 0, N %% 128 == 0 (got M=%d K=%d N=%d)", M, K, N);
+        return AWQ_ERR_SHAPE;
+    }
+    const GemmRoute route = route_gemm(compute_units, M, K, N / pf::BN, true);
+    form[0] = pf::BM;
+    form[1] = pf::BN;
+    form[2] = 1;
+    if (route.form >= 0) awq_rows_form(route.form, form);
+    form[3] = route.ksplit;
+    return AWQ_OK;
 }
 
 }  // extern "C"

@@ -244,3 +244,11 @@ def gemm_q(ctx, out, ldo, a, lda, M, w, K, N, accum=False):
 def gemm_q_static(ctx, out, ldo, a, lda, M, w, K, N, accum=False):
     """gemm_q() with the split-K workspace in the library's own device array: allocates nothing (for callers under graph capture)."""
     check(lib.awq_gemm_int4_static(ctx.h, _addr(out), ldo, _addr(a), lda, M, C.byref(w.c), K, N, int(accum)))
+
+
+def gemm_form(M, K, N, compute_units=256):
+    """How gemm_q() and gemm_q_static() run a product: (tile rows, tile columns, K slices inside a workgroup, workgroups per
+    tile along K); (128, 128, 1, ...) is the 128 x 128 kernel."""
+    form = (C.c_int * 4)()
+    check(lib.awq_gemm_int4_form(compute_units, M, K, N, form))
+    return tuple(form)
