@@ -32,8 +32,6 @@ __device__ __forceinline__ ColGroup col_group(const GemmParams& p, int g) {
     return ColGroup{mat, mat, g * 64, g * 64 + 32};
 }
 
-__device__ const uint32_t rows_zeros[4] = {0u, 0u, 0u, 0u};
-
 // The activation tile in LDS is [rows][64 halves], 16-byte chunks XOR-ed with a key of the row: the 32 rows of a fragment
 // read spread over all banks.
 __device__ __forceinline__ int rows_key(int row) { return (row ^ ((row & 31) >> 3)) & 7; }
@@ -149,7 +147,7 @@ __global__ __launch_bounds__(F::WAVES * 64, F::WAVES_PER_SIMD) void gemm_rows_ke
                 const int r = (wr * AL + q) * 8 + (lane >> 3);
                 const int k = step * BK + ((lane & 7) ^ rows_key(r)) * 8;
                 const void* src = reinterpret_cast<const uint8_t*>(p.A) + a_off[q] + (size_t)step * (BK * 2);
-                dma16(k < p.K ? src : (const void*)rows_zeros, dst + q * 1024);
+                dma16(k < p.K ? src : (const void*)zeros16, dst + q * 1024);
             }
         }
     };

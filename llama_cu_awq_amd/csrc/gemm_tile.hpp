@@ -78,6 +78,9 @@ __device__ __forceinline__ u32x4 dequant8(uint32_t d, const Group& g, uint32_t m
 __device__ __forceinline__ int lds_key(int row) { return (row ^ (row >> 3)) & 7; }
 __device__ __forceinline__ int lds_off(int row, int chunk) { return row * BK + ((chunk ^ lds_key(row)) << 3); }
 
+// what a 16-byte load of activations past K reads instead
+static __device__ const __align__(16) uint32_t zeros16[4] = {0u, 0u, 0u, 0u};
+
 // Direct global -> LDS loads: lane L's 16 (4) bytes land at lds_byte_off + 16 (4) * L.  Issued as inline assembly,
 // so the compiler's wait-count bookkeeping does not see them; the kernel counts and waits for them itself.
 __device__ __forceinline__ void dma16(const void* gptr, uint32_t lds_byte_off) {

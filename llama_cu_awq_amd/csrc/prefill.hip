@@ -67,8 +67,8 @@ constexpr int GEMM_LDS_BYTES = A_STAGES * TILE_BYTES + W_STAGES * W_STAGE_BYTES;
 //    (128 K = one quantisation group: 64 contiguous bytes per row, one zero-point dword and one scale) two pairs
 //    ahead into a ring that only the loading wave reads back, so they need no barrier.  LDS is the prefetch ring: no
 //    register carries a load across iterations and one hand-counted s_waitcnt per step covers everything.
-//  * One barrier per step.  The loop body has no conditional around its loads (steps past the end re-read the last
-//    ones with zero scales), so the number of loads between a request and its use is constant.
+//  * One barrier per step.  The loop body has no conditional around its loads (steps past the end are requested too), so
+//    the number of loads between a request and its use is constant.
 // Workgroup ids are mapped so that the M tiles sharing a weight tile run on one XCD (ids go round-robin over the 8
 // XCDs), which reads the weights from HBM once.
 //
@@ -76,7 +76,9 @@ constexpr int GEMM_LDS_BYTES = A_STAGES * TILE_BYTES + W_STAGES * W_STAGE_BYTES;
 // dword dequantises.  Both MFMA operands contract over K, so any order they agree on gives the same products; with A
 // already in that order the weights go into the MFMA as they come out of the dequantisation.  The prefill path writes
 // its intermediate activations that way; the public entry points take A in natural order.
-template <bool APERM>
+// WHOLE: K is a multiple of 128.  Otherwise activations past K are zeros that the loads fetch in their place: what lies there
+// is the next row (or the end of the allocation), and a zero scale does not make a product with infinity zero.
+template <bool APERM, bool WHOLE>
 __global__ __launch_bounds__(256, 2) void gemm_int4_kernel(const GemmParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_bytes[];  // [A ring][W ring]; nothing else is in LDS
     constexpr uint32_t W_RING = A_STAGES * TILE_BYTES;
@@ -128,16 +130,25 @@ __global__ __launch_bounds__(256, 2) void gemm_int4_kernel(const GemmParams p) {
         for (int j = 0; j < 16; j++) acc[i][j] = 0.0f;
 
     const int nsteps = (p.K + BK - 1) / BK;
-    const int k_last = (nsteps - 1) * BK;
     // split K: the halves meet at an even step, so that both start on a quantisation group
     const int s_split = (nsteps / 2) & ~1;
     const int s_begin = ks ? s_split : 0;
     const int s_end = (p.ksplit == 2 && ks == 0) ? s_split : nsteps;
     auto load_a = [&](int step) {  // 4 loads
-        const int k0 = min(step * BK, k_last);
         const uint32_t dst = (uint32_t)((step % A_STAGES) * TILE_BYTES + wave * 4096);
+        if (WHOLE) {
+            const uint16_t* base = p.A + min(step, nsteps - 1) * BK;
 #pragma unroll
-        for (int q = 0; q < 4; q++) dma16(p.A + k0, a_off[q], dst + q * 1024);
+            for (int q = 0; q < 4; q++) dma16(base, a_off[q], dst + q * 1024);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int r = (wave * 4 + q) * 8 + (lane >> 3);
+                const int k = step * BK + ((lane & 7) ^ lds_key(r)) * 8;
+                const void* src = reinterpret_cast<const uint8_t*>(p.A) + a_off[q] + (size_t)step * (BK * 2);
+                dma16(k < p.K ? src : (const void*)zeros16, dst + q * 1024);
+            }
+        }
     };
     auto load_w = [&](int pair) {  // 4 loads: K range [128 * pair, 128 * pair + 128) of the wave's 32 rows
         const uint32_t dst = W_RING + (uint32_t)((pair % W_STAGES) * W_STAGE_BYTES + wave * W_WAVE_BYTES);
@@ -490,14 +501,14 @@ int awq_gemm_device_setup(int device) {
     }
     std::lock_guard<std::mutex> lock(g_scratch_mutex);
     if (!g_gemm_lds_raised[device]) {
-        hipError_t e = hipFuncSetAttribute((const void*)pf::gemm_int4_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           pf::GEMM_LDS_BYTES);
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void*)pf::gemm_int4_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    pf::GEMM_LDS_BYTES);
-        if (e != hipSuccess) {
-            awq_set_error("hipFuncSetAttribute(gemm_int4) failed: %s", hipGetErrorString(e));
-            return AWQ_ERR_HIP;
+        const void* kernels[3] = {(const void*)pf::gemm_int4_kernel<true, true>, (const void*)pf::gemm_int4_kernel<false, true>,
+                                  (const void*)pf::gemm_int4_kernel<false, false>};
+        for (const void* k : kernels) {
+            const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, pf::GEMM_LDS_BYTES);
+            if (e != hipSuccess) {
+                awq_set_error("hipFuncSetAttribute(gemm_int4) failed: %s", hipGetErrorString(e));
+                return AWQ_ERR_HIP;
+            }
         }
         if (int r = awq_gemm_rows_setup()) return r;
         g_gemm_lds_raised[device] = true;
@@ -604,10 +615,12 @@ static int launch_gemm(awq_ctx* ctx, pf::GemmParams& p, int ntiles, const char* 
     }
     // ids go round-robin over the 8 XCDs; each XCD takes every 8th weight tile with all of its M tiles (and K halves)
     const int grid = 8 * p.mtiles * p.ksplit * div_up(ntiles, 8);
-    if (a_perm)
-        hipLaunchKernelGGL(pf::gemm_int4_kernel<true>, dim3(grid), dim3(256), pf::GEMM_LDS_BYTES, ctx->stream, p);
+    if (a_perm)  // (K a multiple of 128, as in every model that prefills)
+        hipLaunchKernelGGL((pf::gemm_int4_kernel<true, true>), dim3(grid), dim3(256), pf::GEMM_LDS_BYTES, ctx->stream, p);
+    else if ((p.K & 127) == 0)
+        hipLaunchKernelGGL((pf::gemm_int4_kernel<false, true>), dim3(grid), dim3(256), pf::GEMM_LDS_BYTES, ctx->stream, p);
     else
-        hipLaunchKernelGGL(pf::gemm_int4_kernel<false>, dim3(grid), dim3(256), pf::GEMM_LDS_BYTES, ctx->stream, p);
+        hipLaunchKernelGGL((pf::gemm_int4_kernel<false, false>), dim3(grid), dim3(256), pf::GEMM_LDS_BYTES, ctx->stream, p);
     return awq_check_launch(what);
 }
 

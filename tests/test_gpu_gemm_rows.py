@@ -49,9 +49,13 @@ def test_against_fp64(ctx, M, K, N):
     assert rel_l2(f16(dout.download(np.uint16)).reshape(M, N), truth + resid.astype(np.float64).reshape(M, N)) <= 1e-3
 
 
-def test_infinite_activation_stays_in_its_row(ctx):
+# the row form and the 128 x 128 kernel; K that ends in the middle of a step (33 units of 32) or of a quantisation group
+@pytest.mark.parametrize("M,K,N,form", [(40, 1056, 256, (32, 64)), (512, 1056, 8192, (128, 128)), (512, 1088, 8192, (128, 128)), (512, 1120, 8192, (128, 128))])
+@pytest.mark.parametrize("last", [False, True], ids=["first-column", "last-column"])
+def test_infinite_activation_stays_in_its_row(ctx, M, K, N, form, last):
     """K that ends in the middle of a step: nothing of a neighbouring row (or of the memory behind the last one) enters."""
-    M, K, N = 40, 1056, 256
+    assert A.gemm_form(M, K, N)[:2] == form
+    col = K - 1 if last else 0
     key = synth.stream_key(53, M, K, N)
     w, z, s = synth.make_qweight(key, K, N)
     a = synth.normal_f16(synth.stream_key(key, "a"), M * K).reshape(M, K).copy()
@@ -60,7 +64,7 @@ def test_infinite_activation_stays_in_its_row(ctx):
     for value in (None, np.float16(np.inf)):
         b = a.copy()
         if value is not None:
-            b[20, 0] = value
+            b[20, col] = value
         dout = ctx.zeros(M * N * 2)
         A.gemm_q(ctx, dout, N, ctx.upload(b.reshape(-1)), K, M, qw, K, N)
         outs.append(dout.download(np.uint16).reshape(M, N))
@@ -68,7 +72,7 @@ def test_infinite_activation_stays_in_its_row(ctx):
     assert np.array_equal(outs[0][rest], outs[1][rest])
     w16 = synth.dequantize(w, z, s, K).astype(np.float32)
     got = f16(outs[1][20])
-    assert np.array_equal(np.isposinf(got), w16[:, 0] > 0) and np.array_equal(np.isneginf(got), w16[:, 0] < 0)
+    assert np.array_equal(np.isposinf(got), w16[:, col] > 0) and np.array_equal(np.isneginf(got), w16[:, col] < 0)
 
 
 # 64-wide heads, sizes at which the QKV and gate/up products take the 64 to 128 row forms by 128 and 256 columns
