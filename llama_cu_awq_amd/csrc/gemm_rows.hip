@@ -204,6 +204,10 @@ __global__ __launch_bounds__(F::WAVES * 64, F::WAVES_PER_SIMD) void gemm_rows_ke
         }
         const uint8_t* ws = lds_bytes + w_ring + (pair % WS) * F::W_BYTES + lrow * 64;
         const int unit = (step & 1) * 2 + lhalf;
+        if (!WHOLE && step * BK + lhalf * 32 >= p.K) {  // past K: zero scales (a weight that is not finite is not undone by a zero activation)
+            const h16x2 none = {(h16_t)0.0f, (h16_t)0.0f};
+            gc[0].s2 = gc[1].s2 = none;
+        }
 #pragma unroll
         for (int b = 0; b < 2; b++) wq[b] = *reinterpret_cast<const u32x4*>(ws + b * 2048 + ((unit ^ ((lrow >> 1) & 3)) << 4));
     };

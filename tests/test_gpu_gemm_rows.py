@@ -75,6 +75,26 @@ def test_infinite_activation_stays_in_its_row(ctx, M, K, N, form, last):
     assert np.array_equal(np.isposinf(got), w16[:, col] > 0) and np.array_equal(np.isneginf(got), w16[:, col] < 0)
 
 
+@pytest.mark.parametrize("M,K,N,form", [(40, 1056, 256, (32, 64)), (65, 1120, 6144, (64, 64)), (300, 1056, 4096, (64, 128)), (300, 96, 12288, (64, 256)), (700, 1120, 6144, (96, 256)),
+                                        (513, 1120, 12288, (128, 256)), (512, 1056, 8192, (128, 128))])
+def test_weights_past_the_range_of_fp16(ctx, M, K, N, form):
+    """(q - z) * s beyond 65504 is an infinite weight; against positive activations its column is infinite, and what a load
+    past the end of a row brings in does not make it NaN."""
+    assert A.gemm_form(M, K, N)[:2] == form
+    key = synth.stream_key(56, M, K, N)
+    w, z, s = synth.make_qweight(key, K, N)
+    pwh, pzh, sh = synth.strides(K)
+    w, z, s = w.reshape(N, pwh).copy(), z.reshape(N, pzh).copy(), s.reshape(N, sh).copy()
+    w[5, : K // 8] = 0xFFFFFFFF
+    z[5] = 0
+    s[5, -1] = np.float16(6000.0)  # 15 * 6000, in the last group only
+    a = np.abs(synth.normal_f16(synth.stream_key(key, "a"), M * K)) + np.float16(0.5)
+    dout = ctx.zeros(M * N * 2)
+    A.gemm_q(ctx, dout, N, ctx.upload(a.astype(np.float16)), K, M, A.QWeight.upload(ctx, w.reshape(-1), z.reshape(-1), s.reshape(-1)), K, N)
+    got = f16(dout.download(np.uint16)).reshape(M, N)
+    assert np.isposinf(got[:, 5]).all() and np.isfinite(np.delete(got, 5, 1)).all()
+
+
 # 64-wide heads, sizes at which the QKV and gate/up products take the 64 to 128 row forms by 128 and 256 columns
 SMALL = dict(dim=2048, hidden_dim=5632, n_layers=2, n_heads=32, n_kv_heads=4, vocab_size=512, seq_len=1280, rope_theta=10000.0)
 
