@@ -526,15 +526,34 @@ int awq_gemm_device_setup(int device) {
 }
 
 // ---------------------------------------------------------------- launchers (internal)
-// The context's split-K workspace, allocated whole the first time.
+// The context's split-K workspace, allocated whole the first time.  Its counters are cleared ahead of every product, also
+// where the context's stream is being recorded: what is recorded there runs when the graph does, and an eager product may
+// come first, so that they are cleared at once on a stream of their own.
 int awq_reserve_gemm_workspace(awq_ctx* ctx) {
     if (ctx->gemm_part) return AWQ_OK;
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess) (void)hipGetLastError();
     void* block = nullptr;
     AWQ_HIP_TRY(hipMalloc(&block, kScratchBytes));
-    ctx->gemm_part = static_cast<float*>(block);
     unsigned int* counter = reinterpret_cast<unsigned int*>(static_cast<uint8_t*>(block) + kPartBytes);
-    hipLaunchKernelGGL(pf::clear_words_kernel, dim3(1), dim3(kPartTiles), 0, ctx->stream, counter, kPartTiles);
-    return awq_check_launch("clear_words");
+    const bool recorded = capturing != hipStreamCaptureStatusNone;
+    hipStream_t stream = ctx->stream;
+    hipError_t e = recorded ? hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) : hipSuccess;
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(pf::clear_words_kernel, dim3(1), dim3(kPartTiles), 0, stream, counter, kPartTiles);
+        e = hipGetLastError();
+        if (recorded) {
+            if (e == hipSuccess) e = hipStreamSynchronize(stream);
+            (void)hipStreamDestroy(stream);
+        }
+    }
+    if (e != hipSuccess) {
+        (void)hipFree(block);
+        awq_set_error("clearing the split-K counters failed: %s", hipGetErrorString(e));
+        return AWQ_ERR_HIP;
+    }
+    ctx->gemm_part = static_cast<float*>(block);
+    return AWQ_OK;
 }
 
 // The split-K workspace of a launch over `tiles` output tiles: the file-scope device array (static_ws; no allocation) or

@@ -136,6 +136,48 @@ def test_prefill_epilogues_against_token_by_token(ctx, small, parts):
             assert rel_l2(a[l][-3:], b[l][n - 3 : n]) <= 1e-2, l
 
 
+# (looked up through the library: the HIP runtime it is linked with)
+def _hip(name, *args):
+    assert getattr(lib, name)(*args) == 0, name
+
+
+def test_split_workspace_made_while_recording(ctx):
+    """The first product of a context, recorded: the arrival counters are clear before the graph has run, and nothing but the
+    product is recorded."""
+    M, K, N = 33, 2048, 128
+    assert A.gemm_form(M, K, N)[3] > 1
+    key = synth.stream_key(57, M, K, N)
+    qw = A.QWeight.upload(ctx, *synth.make_qweight(key, K, N))
+    a = [ctx.upload(synth.normal_f16(synth.stream_key(key, i), M * K)) for i in range(2)]
+    out = [ctx.zeros(M * N * 2) for _ in a]
+    fresh = A.Context(0)
+    ctx.sync()
+    stream, graph, runnable, nodes = C.c_void_p(lib.awq_ctx_stream(fresh.h)), C.c_void_p(), C.c_void_p(), C.c_size_t()
+    _hip("hipStreamBeginCapture", stream, 2)  # relaxed: allocations are allowed
+    A.gemm_q(fresh, out[0], N, a[0], K, M, qw, K, N)
+    _hip("hipStreamEndCapture", stream, C.byref(graph))
+    _hip("hipGraphGetNodes", graph, None, C.byref(nodes))
+    assert nodes.value == 1
+    _hip("hipGraphInstantiate", C.byref(runnable), graph, None, None, C.c_size_t(0))
+    want = []
+    for x in a:
+        d = ctx.zeros(M * N * 2)
+        A.gemm_q_static(ctx, d, N, x, K, M, qw, K, N)
+        want.append(d.download(np.uint16))
+    for _ in range(3):  # an eager product before the first replay and between the others
+        A.gemm_q(fresh, out[1], N, a[1], K, M, qw, K, N)
+        fresh.sync()
+        assert np.array_equal(out[1].download(np.uint16), want[1])
+        _hip("hipGraphLaunch", runnable, stream)
+        fresh.sync()
+        assert np.array_equal(out[0].download(np.uint16), want[0])
+        for d in out:
+            d.write(np.zeros(M * N, np.uint16))
+    _hip("hipGraphExecDestroy", runnable)
+    _hip("hipGraphDestroy", graph)
+    fresh.close()
+
+
 def test_short_prefill_recorded_after_a_long_one():
     """1100 rows by 4096 columns split no K, 37 do: what that takes is there before the short prompt is recorded."""
     cfg = dict(dim=4096, hidden_dim=1024, n_layers=1, n_heads=32, n_kv_heads=4, vocab_size=512, seq_len=1152, rope_theta=10000.0)
@@ -147,20 +189,16 @@ def test_short_prefill_recorded_after_a_long_one():
     def caches():
         return [t.download(name, cfg["seq_len"] * 512) for name in ("key_cache", "value_cache")]
 
-    # (looked up through the library: the HIP runtime it is linked with)
-    def hip(name, *args):
-        assert getattr(lib, name)(*args) == 0, name
-
     stream, graph, runnable = C.c_void_p(lib.awq_ctx_stream(ctx.h)), C.c_void_p(), C.c_void_p()
     t.reset(prompt)
     t.prefill(1100, gen_token=False)
-    hip("hipStreamBeginCapture", stream, 0)
+    _hip("hipStreamBeginCapture", stream, 0)
     t.prefill(37, gen_token=False)
-    hip("hipStreamEndCapture", stream, C.byref(graph))
-    hip("hipGraphInstantiate", C.byref(runnable), graph, None, None, C.c_size_t(0))
+    _hip("hipStreamEndCapture", stream, C.byref(graph))
+    _hip("hipGraphInstantiate", C.byref(runnable), graph, None, None, C.c_size_t(0))
     recorded = []
     for _ in range(3):
-        hip("hipGraphLaunch", runnable, stream)
+        _hip("hipGraphLaunch", runnable, stream)
         ctx.sync()
         recorded.append(caches())
     t.reset(prompt)
@@ -171,7 +209,7 @@ def test_short_prefill_recorded_after_a_long_one():
     for got in recorded:
         for a, b in zip(got, want):
             assert np.array_equal(a, b) and f16(b).reshape(-1, 512)[1100:1137].any(axis=1).all()
-    hip("hipGraphExecDestroy", runnable)
-    hip("hipGraphDestroy", graph)
+    _hip("hipGraphExecDestroy", runnable)
+    _hip("hipGraphDestroy", graph)
     t.close()
     ctx.close()
