@@ -285,7 +285,9 @@ int awq_sampler_create(awq_ctx* ctx, int vocab_size, float temperature, float to
 int awq_sampler_destroy(awq_sampler* sampler);
 /* sample() (sampler.h:77-115): draws the coin (every call, as the reference does), then the greedy kernel when
  * temperature == 0 or gen_token == 0, else softmax + top-p (threshold coin * topp) or plain sampling (threshold coin
- * when topp <= 0 or >= 1).  logits are overwritten on the non-greedy branch. */
+ * when topp <= 0 or >= 1).  logits are overwritten on the non-greedy branch.  Above 32768 entries the call runs over many
+ * workgroups on scratch memory that the sampler owns; recorded into a graph it runs in one workgroup instead, with the
+ * same results and nothing of the sampler's, which may be destroyed before the graph. */
 int awq_sampler_sample(awq_sampler* sampler, uint16_t* logits, int* tokens, volatile int* pos_host, int* pos_dev,
                        int gen_token);
 /* The same on a transformer's own logits and token list (also keeps the device mirror of the token list current):

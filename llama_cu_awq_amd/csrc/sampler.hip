@@ -730,6 +730,16 @@ struct awq_sampler {
     WideScratch* wide;  // scratch of the many-workgroup kernels; null: small vocabulary, or no memory for it
 };
 
+// Allocating and freeing are allowed in its scope while some stream is being recorded (nothing of them is recorded).
+struct DuringCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    bool exchanged;
+    DuringCapture() : exchanged(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
+    ~DuringCapture() {
+        if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
 // xorshift* (sampler.h:65-74)
 static unsigned int random_u32(unsigned long long* state) {
     *state ^= *state >> 12;
@@ -841,18 +851,25 @@ int awq_sampler_run(awq_sampler* s, uint16_t* logits, int* tokens, volatile int*
         return awq_launch_argmax(s->ctx, logits, s->vocab_size, tokens, pos_host, pos_dev, gen_token, mirror);
     const bool nucleus = s->topp > 0.0f && s->topp < 1.0f;
     const float threshold = nucleus ? coin * s->topp : coin;
-    if (nucleus ? !s->wide && s->vocab_size <= 65535 : s->vocab_size <= kLdsVocab)  // softmax and selection in one launch
+    // a recorded call holds nothing of the sampler: the graph may outlive it (and replay beside its eager calls)
+    WideScratch* wide = s->wide;
+    if (wide) {
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s->ctx->stream, &capturing) != hipSuccess) (void)hipGetLastError();
+        if (capturing != hipStreamCaptureStatusNone) wide = nullptr;
+    }
+    if (nucleus ? !wide && s->vocab_size <= 65535 : s->vocab_size <= kLdsVocab)  // softmax and selection in one launch
         return launch_softmax_sample(s->ctx, logits, s->vocab_size, s->temperature, threshold, nucleus ? 1 : 0, tokens, pos_host,
                                      pos_dev, mirror);
-    if (s->wide) {
+    if (wide) {
         const size_t hist = nucleus ? (size_t)kProbBins * sizeof(unsigned int) : 0;
         const int n = s->vocab_size;
-        hipLaunchKernelGGL(wide_max_kernel, dim3(kWideMaxGroups), dim3(256), 0, s->ctx->stream, logits, n, s->wide);
+        hipLaunchKernelGGL(wide_max_kernel, dim3(kWideMaxGroups), dim3(256), 0, s->ctx->stream, logits, n, wide);
         hipLaunchKernelGGL(wide_exp_kernel, dim3(kSampleThreads / kWideColumns), dim3(kSampleThreads), 0, s->ctx->stream, logits, n,
-                           s->temperature, s->wide);
-        hipLaunchKernelGGL(wide_divide_kernel, dim3(16), dim3(kSampleThreads), hist, s->ctx->stream, logits, n, nucleus ? 1 : 0, s->wide);
+                           s->temperature, wide);
+        hipLaunchKernelGGL(wide_divide_kernel, dim3(16), dim3(kSampleThreads), hist, s->ctx->stream, logits, n, nucleus ? 1 : 0, wide);
         if (nucleus)
-            hipLaunchKernelGGL(wide_select_kernel, dim3(1), dim3(kSampleThreads), hist, s->ctx->stream, logits, n, threshold, s->wide, tokens,
+            hipLaunchKernelGGL(wide_select_kernel, dim3(1), dim3(kSampleThreads), hist, s->ctx->stream, logits, n, threshold, wide, tokens,
                                pos_host, pos_dev, mirror);
         if (int r = awq_check_launch("sample (wide)")) return r;
         if (nucleus) return AWQ_OK;
@@ -893,16 +910,22 @@ int awq_sampler_create(awq_ctx* ctx, int vocab_size, float temperature, float to
     s->topp = topp;
     s->rng_state = rng_seed;
     s->wide = nullptr;
-    if (vocab_size > kWideVocab && temperature > 0.0f && hipMalloc((void**)&s->wide, sizeof(WideScratch)) != hipSuccess) {
-        (void)hipGetLastError();
-        s->wide = nullptr;  // (the one-workgroup kernels need none)
+    if (vocab_size > kWideVocab && temperature > 0.0f) {
+        const DuringCapture scope;
+        if (hipMalloc((void**)&s->wide, sizeof(WideScratch)) != hipSuccess) {
+            (void)hipGetLastError();
+            s->wide = nullptr;  // (the one-workgroup kernels need none)
+        }
     }
     *out = s;
     return AWQ_OK;
 }
 
 int awq_sampler_destroy(awq_sampler* s) {
-    if (s && s->wide) (void)hipFree(s->wide);
+    if (s && s->wide) {
+        const DuringCapture scope;
+        (void)hipFree(s->wide);
+    }
     delete s;
     return AWQ_OK;
 }

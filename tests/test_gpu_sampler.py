@@ -11,7 +11,7 @@ import pytest
 
 import llama_cu_awq_amd as A
 from llama_cu_awq_amd import synth
-from llama_cu_awq_amd._lib import AWQ_ERR_SHAPE
+from llama_cu_awq_amd._lib import AWQ_ERR_SHAPE, lib
 from oracle import oracle
 from tests.helpers import f16, ulp_diff_f16
 
@@ -167,6 +167,57 @@ def test_sampler_object_equals_the_two_entry_points(ctx, n, topp):
         assert got[0][1] == got[1][1], step
         if step < 5:
             assert got[0][1] == _oracle_pick(f16(got[0][0])[offset:], float(coin * np.float32(topp)) if nucleus else float(coin), int(nucleus)), step
+    pin.close()
+
+
+@pytest.mark.parametrize("topp,n,launches", [(0.9, 32769, 1), (0.9, 65535, 1), (0.9, 128256, 2), (1.0, 49152, 1), (1.0, 100003, 2)])
+def test_recorded_sampler_may_be_destroyed_before_the_graph(ctx, topp, n, launches):
+    """Large vocabularies: a sampler created, recorded and destroyed while the stream is being recorded.  The graph holds the
+    one-workgroup kernels, which take nothing of the sampler's memory; replays between eager calls of another sampler give
+    the bits of the eager call."""
+    def hip(name, *args):
+        assert getattr(lib, name)(*args) == 0, name
+
+    l = [_logits(80 + i, n, 3.0).view(np.uint16) for i in range(2)]
+    d = [ctx.upload(x) for x in l]
+    pin = Pinned(ctx)
+    eager = A.Sampler(ctx, n, 0.8, topp, 5)
+    eager.sample(d[1], pin.host + 16, pin.host, pin.dpos, True)  # (what a first call sets up)
+    ctx.sync()
+    stream, graph, runnable, nodes = C.c_void_p(lib.awq_ctx_stream(ctx.h)), C.c_void_p(), C.c_void_p(), C.c_size_t()
+    for early in (True, False):  # created before the recording or in it
+        s = A.Sampler(ctx, n, 0.8, topp, 5) if early else None
+        hip("hipStreamBeginCapture", stream, 0)
+        s = s or A.Sampler(ctx, n, 0.8, topp, 5)
+        s.sample(d[0], pin.host + 16, pin.host, pin.dpos, True)
+        if not early:
+            s.close()
+        hip("hipStreamEndCapture", stream, C.byref(graph))
+        s.close()
+        hip("hipGraphGetNodes", graph, None, C.byref(nodes))
+        assert nodes.value == launches
+        hip("hipGraphInstantiate", C.byref(runnable), graph, None, None, C.c_size_t(0))
+        for _ in range(3):
+            got = []
+            for replay in (False, True):
+                d[0].write(l[0])
+                ctx.sync()
+                pin.pos.value, pin.tokens[4] = 3, -1
+                pin.dpos.write(np.array([3], np.int32))  # (in place: the graph holds its address)
+                if replay:
+                    hip("hipGraphLaunch", runnable, stream)
+                else:
+                    again = A.Sampler(ctx, n, 0.8, topp, 5)
+                    again.sample(d[0], pin.host + 16, pin.host, pin.dpos, True)
+                ctx.sync()
+                got.append((d[0].download(np.uint16), pin.tokens[4], pin.pos.value))
+                if replay:
+                    again.close()
+                eager.sample(d[1], pin.host + 16, pin.host, pin.dpos, True)
+            assert np.array_equal(got[0][0], got[1][0]) and got[0][1:] == got[1][1:] and got[0][2] == 4
+        hip("hipGraphExecDestroy", runnable)
+        hip("hipGraphDestroy", graph)
+    eager.close()
     pin.close()
 
 
