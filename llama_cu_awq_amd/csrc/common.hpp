@@ -74,6 +74,16 @@ static inline int awq_check_launch(const char* what) {
     return AWQ_OK;
 }
 
+// Allocating and freeing are allowed in its scope while some stream is being recorded (nothing of them is recorded).
+struct awq_during_capture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    bool exchanged;
+    awq_during_capture() : exchanged(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
+    ~awq_during_capture() {
+        if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
 // Launch on the context's stream; with a probe set, through the extension launch that time-stamps the kernel itself.
 template <typename... Args, typename F = void (*)(Args...)>
 static inline void awq_launch(awq_ctx* ctx, F kernel, dim3 grid, dim3 block, size_t lds, Args... args) {

@@ -730,16 +730,6 @@ struct awq_sampler {
     WideScratch* wide;  // scratch of the many-workgroup kernels; null: small vocabulary, or no memory for it
 };
 
-// Allocating and freeing are allowed in its scope while some stream is being recorded (nothing of them is recorded).
-struct DuringCapture {
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    bool exchanged;
-    DuringCapture() : exchanged(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
-    ~DuringCapture() {
-        if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
-    }
-};
-
 // xorshift* (sampler.h:65-74)
 static unsigned int random_u32(unsigned long long* state) {
     *state ^= *state >> 12;
@@ -911,7 +901,7 @@ int awq_sampler_create(awq_ctx* ctx, int vocab_size, float temperature, float to
     s->rng_state = rng_seed;
     s->wide = nullptr;
     if (vocab_size > kWideVocab && temperature > 0.0f) {
-        const DuringCapture scope;
+        const awq_during_capture scope;
         if (hipMalloc((void**)&s->wide, sizeof(WideScratch)) != hipSuccess) {
             (void)hipGetLastError();
             s->wide = nullptr;  // (the one-workgroup kernels need none)
@@ -923,7 +913,7 @@ int awq_sampler_create(awq_ctx* ctx, int vocab_size, float temperature, float to
 
 int awq_sampler_destroy(awq_sampler* s) {
     if (s && s->wide) {
-        const DuringCapture scope;
+        const awq_during_capture scope;
         (void)hipFree(s->wide);
     }
     delete s;

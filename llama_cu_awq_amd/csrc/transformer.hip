@@ -819,15 +819,20 @@ constexpr int kPrefillChunk = 2048;
 constexpr int kPrefillMinRows = 512;  // of the first allocation
 
 // A workspace for passes of up to min(n_tokens, kPrefillChunk) rows, or of fewer where it cannot be had (the prompt then
-// goes in more passes).  Smaller ones met before stay until the model is released (together less than the largest): a
-// recorded prefill may still replay on them.
+// goes in more passes).  Smaller ones met before stay until the model is released (at most two, of less than 1.5
+// kPrefillChunk rows together): a recorded prefill may still replay on them.
 int ensure_prefill_rows(awq_transformer* t, int n_tokens) {
     const awq_config& p = t->cfg;
     int rows = n_tokens < kPrefillChunk ? n_tokens : kPrefillChunk;
     if (rows <= t->pf_rows) return AWQ_OK;
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (t->pf_rows > 0 && (hipStreamIsCapturing(t->ctx->stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone))
-        return AWQ_OK;
+    if (t->pf_rows > 0) {
+        if (hipStreamIsCapturing(t->ctx->stream, &capturing) != hipSuccess) {
+            (void)hipGetLastError();
+            return AWQ_OK;
+        }
+        if (capturing != hipStreamCaptureStatusNone) return AWQ_OK;
+    }
     int least = p.seq_len < kPrefillMinRows ? p.seq_len : kPrefillMinRows;
     if (least < 2 * t->pf_rows) least = 2 * t->pf_rows;  // a prompt that grows by a few tokens per call must not allocate each time
     if (rows < least) rows = least;
@@ -840,10 +845,14 @@ int ensure_prefill_rows(awq_transformer* t, int n_tokens) {
     size_t row_bytes = 0;
     for (size_t w : widths) row_bytes += w * 2;
     void* block = nullptr;
-    hipError_t e = hipMalloc(&block, (size_t)rows * row_bytes);
-    if (e != hipSuccess) {
+    if (t->pf_rows > 0) {  // growing: some other stream may be being recorded
+        const awq_during_capture scope;
+        if (hipMalloc(&block, (size_t)rows * row_bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            return AWQ_OK;
+        }
+    } else if (hipError_t e = hipMalloc(&block, (size_t)rows * row_bytes); e != hipSuccess) {
         (void)hipGetLastError();
-        if (t->pf_rows > 0) return AWQ_OK;
         if (rows > kPrefillMinRows) {
             rows = kPrefillMinRows;
             e = hipMalloc(&block, (size_t)rows * row_bytes);

@@ -1,10 +1,13 @@
 """GPU parity of the multi-token prefill path: the int4 x fp16 MFMA GEMM against fp64, and a whole prefill against
 the oracle's token-by-token run (KV cache contents and last-token logits within rel-L2 1e-2, same next token)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import llama_cu_awq_amd as A
 from llama_cu_awq_amd import synth
+from llama_cu_awq_amd._lib import lib
 from oracle import oracle
 from tests.helpers import f16, rel_l2
 
@@ -106,6 +109,32 @@ def test_prefill_in_two_parts_equals_one(ctx):
     a, b = states
     assert a[3] == b[3] == 70 and a[4] == b[4]
     assert rel_l2(f16(a[0]), f16(b[0])) <= 1e-3 and rel_l2(f16(a[1]), f16(b[1])) <= 1e-3 and rel_l2(f16(a[2]), f16(b[2])) <= 2e-3
+
+
+def test_longer_prompt_while_another_stream_is_recorded(ctx):
+    """The workspace of a longer prompt is allocated without ending a recording of some other stream."""
+    img = synth.make_model_image(CFG_LONG128, seed=34)
+    prompt = synth.prompt_tokens(34, 800, CFG_LONG128["vocab_size"])
+    kv = CFG_LONG128["n_layers"] * CFG_LONG128["seq_len"] * CFG_LONG128["dim"]
+    other = A.Context(0)
+    states = []
+    for recording in (False, True):
+        t = A.Transformer(ctx, image=img)
+        t.reset(prompt)
+        t.prefill(100, gen_token=False)
+        stream, graph = C.c_void_p(lib.awq_ctx_stream(other.h)), C.c_void_p()
+        if recording:
+            assert lib.hipStreamBeginCapture(stream, 0) == 0
+        t.prefill(700)
+        if recording:
+            assert lib.hipStreamEndCapture(stream, C.byref(graph)) == 0
+            assert lib.hipGraphDestroy(graph) == 0
+        ctx.sync()
+        states.append([t.download("key_cache", kv), t.download("value_cache", kv), t.download("logits", CFG_LONG128["vocab_size"]), t.token(800)])
+        t.close()
+    other.close()
+    for a, b in zip(*states):
+        assert np.array_equal(a, b)
 
 
 # 128-wide heads and a context past what the batched attention keeps in LDS (1920 positions): the tokens beyond that bound
