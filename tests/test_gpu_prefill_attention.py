@@ -78,3 +78,112 @@ def test_long_contexts_against_token_by_token(ctx, cfg, parts):
     want = _rows(t, cfg, n), f16(t.download("logits", cfg["vocab_size"]))
     t.close()
     _compare(_prefill(ctx, img, cfg, prompt, parts), want)
+
+
+# ---------------------------------------------------------------- scores by design
+def _designed(cfg, seed, reach):
+    """A model whose first layer's scores are known: a query's is `reach` times the key token's level, -1 .. 1 in 65 steps
+    (token v has level (v % 65) / 32 - 1), at every distance (the only pair of dimensions in use turns least)."""
+    dim, hid, heads, kv, vocab = (cfg[k] for k in ("dim", "hidden_dim", "n_heads", "n_kv_heads", "vocab_size"))
+    hs = dim // heads
+    img = synth.make_model_image(cfg, seed=seed, scale_mult=0.25)
+    rng = np.random.default_rng(seed)
+    # columns 0 .. 127 of every embedding are 1, of the next 128 as many are +1 as the level says, the others +-1 in pairs
+    embed = img[32 : 32 + 2 * vocab * dim].view(np.float16).reshape(vocab, dim)
+    embed[:, :128] = 1
+    for v in range(vocab):
+        ups = 2 * (v % 65)  # of 128
+        embed[v, 128:256] = rng.permutation(np.repeat([1.0, -1.0], [ups, 128 - ups]))
+        embed[v, 256:] = rng.choice([-1.0, 1.0], dim - 256)
+    off = 32 + 4 * vocab * dim + 2 * dim
+
+    def matrix(K, N):
+        nonlocal off
+        pwh, pzh, sh = synth.strides(K)
+        parts = []
+        for width, dtype in ((pwh, np.uint32), (pzh, np.uint32), (sh, np.float16)):
+            n = N * width * np.dtype(dtype).itemsize
+            parts.append(img[off : off + n].view(dtype).reshape(N, width))
+            off += n
+        return parts
+
+    def functional(m, rows, first, scale):
+        """`rows` of a matrix become scale times the sum over 128 columns."""
+        w, z, s = m
+        w[rows], z[rows], s[rows] = 0, 0, scale
+        w[rows, first // 8 : first // 8 + 16] = 0x11111111
+
+    alpha = hs**-0.5
+    q, k = matrix(dim, dim), matrix(dim, kv * hs)
+    matrix(dim, kv * hs)
+    for m in (q, k):
+        m[0][:], m[1][:] = 0, 0
+    functional(q, np.arange(heads) * hs + hs // 2 - 1, 0, 1 / 128)  # 1 for every token
+    functional(k, np.arange(kv) * hs + hs // 2 - 1, 128, reach / alpha / 128)
+    matrix(dim, dim)
+    for K, N in ((dim, hid), (dim, hid), (hid, dim)):
+        matrix(K, N)
+    img[off : off + 2 * dim].view(np.float16)[:] = 1  # the first norm's weights
+    return img
+
+
+def _token(level, rng, vocab):
+    """A token of the level nearest to `level`."""
+    v = int(np.clip(np.round((level + 1) * 32), 0, 64))
+    return int(v + 65 * rng.integers(0, vocab // 65))
+
+
+def _token_by_token(ctx, img, cfg, prompt):
+    t = A.Transformer(ctx, image=img)
+    t.reset(prompt)
+    for i in range(len(prompt)):
+        t.forward(i == len(prompt) - 1, use_graph=True)
+    ctx.sync()
+    out = _rows(t, cfg, len(prompt)), f16(t.download("logits", cfg["vocab_size"]))
+    t.close()
+    return out
+
+
+def _oracle(img, cfg, prompt):
+    o = oracle.Model(img)
+    o.reset(prompt)
+    for i in range(len(prompt)):
+        o.forward(i >= len(prompt) - 1)
+    kv_dim = cfg["dim"] * cfg["n_kv_heads"] // cfg["n_heads"]
+    size = cfg["n_layers"] * cfg["seq_len"] * kv_dim
+    rows = [f16(o.buffer(name, size)).reshape(cfg["n_layers"], cfg["seq_len"], kv_dim)[:, : len(prompt)].copy() for name in ("key_cache", "value_cache")]
+    out = rows, f16(o.buffer("logits", cfg["vocab_size"])).copy()
+    o.close()
+    return out
+
+
+# one profile of scores over the positions: the maximum grows by more than the rescale's threshold again and again; stands in the
+# first tile; differs by 40 and more between the key slices of a tile
+PROFILES = {
+    "ascending": lambda i, n: 2 * i / n - 1,
+    "descending": lambda i, n: 1 - 2 * i / n,
+    "by-slice": lambda i, n: (-0.7, 0.1, 0.9, 0.4)[(i // 32) % 4] + 0.05 * (i % 3),
+}
+# every form of the dispatch: (heads, prompt): one tile, 64 queries by 2 slices, 32 queries by 4 slices, 128 queries
+FORMS = [(H64, (64,)), (H64, (300,)), (H64, (600, 40)), (H128, (64,)), (H128, (300,)), (H128, (600, 40)), (H256, (64,)), (H256, (300,)), (H256, (600, 40)),
+         (H128_WIDE, (1030,))]
+FORM_IDS = [f"{c['n_heads']}x{c['dim'] // c['n_heads']}-{'+'.join(map(str, p))}" for c, p in FORMS]
+
+
+@pytest.mark.parametrize("profile", PROFILES)
+@pytest.mark.parametrize("cfg,parts", FORMS, ids=FORM_IDS)
+def test_maxima_that_move(ctx, cfg, parts, profile):
+    """Scores from -60 to 60 in known order, so that single keys carry the result.  One product makes a score, so both sides
+    round the same one; what differs is rounded to fp16 five times on the way to the second layer's rows (p, the output, the
+    residual, the norm, the product: 2^-11 / sqrt(3) each, 6e-4 together): 3e-3."""
+    n = sum(parts)
+    img = _designed(cfg, 61, 60.0)
+    rng = np.random.default_rng(62)
+    prompt = [_token(PROFILES[profile](i, n), rng, cfg["vocab_size"]) for i in range(n)]
+    want = _token_by_token(ctx, img, cfg, prompt) if cfg is H128_WIDE else _oracle(img, cfg, prompt)
+    got = _prefill(ctx, img, cfg, prompt, parts)
+    for a, b in zip(got[0], want[0]):
+        assert rel_l2(a[1], b[1]) <= 3e-3
+        for at in range(0, n, 32):
+            assert rel_l2(a[1][at : at + 32], b[1][at : at + 32]) <= 3e-3, at
+    assert rel_l2(got[1], want[1]) <= 1e-2
