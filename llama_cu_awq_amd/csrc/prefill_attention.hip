@@ -23,6 +23,42 @@ __device__ __forceinline__ h16x8 read_tr8(const uint16_t* p0, const uint16_t* p1
     return __builtin_bit_cast(h16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
+// One query by one wave, for blocks with values that are not finite: only the keys it sees take part.
+template <int HS>
+__device__ __forceinline__ void attn_row(uint16_t* out, const uint16_t* q, const uint16_t* kh, const uint16_t* vh, size_t kv_dim, int keys,
+                                         float alpha, int out_perm) {
+    constexpr int D = HS / 64;
+    const int lane = threadIdx.x & 63;
+    float o[D], m = -INFINITY, l = 0.0f;
+#pragma unroll
+    for (int d = 0; d < D; d++) o[d] = 0.0f;
+#pragma unroll 1
+    for (int t0 = 0; t0 < keys; t0 += 64) {
+        float s = 0.0f;
+        const uint16_t* k = kh + (size_t)min(t0 + lane, keys - 1) * kv_dim;
+#pragma unroll 1
+        for (int i = 0; i < HS; i++) s = fmaf(half_bits_to_float(q[i]), half_bits_to_float(k[i]), s);
+        s = t0 + lane < keys ? half_bits_to_float(float_to_half_bits(s * alpha)) : -INFINITY;
+        const float m_new = fmaxf(m, wave_max(s));
+        const float f = m_new == -INFINITY ? 1.0f : expf(m - m_new);
+        const float e = expf(s - (m_new == -INFINITY ? 0.0f : m_new));
+        m = m_new;
+        l = fmaf(l, f, wave_sum(e));
+        const float p = half_bits_to_float(float_to_half_bits(e));
+#pragma unroll
+        for (int d = 0; d < D; d++) o[d] *= f;
+#pragma unroll 1
+        for (int i = 0; i < 64 && t0 + i < keys; i++) {
+            const float pi = __shfl(p, i);
+#pragma unroll
+            for (int d = 0; d < D; d++) o[d] = fmaf(pi, half_bits_to_float(vh[(size_t)(t0 + i) * kv_dim + d * 64 + lane]), o[d]);
+        }
+    }
+    const int at = out_perm ? (lane & 56) | ((lane & 3) << 1) | ((lane >> 2) & 1) : lane;  // (0,4,1,5,2,6,3,7)
+#pragma unroll
+    for (int d = 0; d < D; d++) out[d * 64 + at] = float_to_half_bits(o[d] / l);
+}
+
 // A workgroup owns 32 * QW consecutive query tokens of one head: wave (qs, ks) takes the qs-th 32 queries and, of every
 // tile of 32 * NSUB * KW keys, the ks-th NSUB blocks of 32.
 //  * S^T = K Q^T: with the queries as columns a lane holds 16 scores of ONE query, so the row statistics are in-lane
@@ -33,6 +69,8 @@ __device__ __forceinline__ h16x8 read_tr8(const uint16_t* p0, const uint16_t* p1
 //    fp16 or fp32), which after the first tiles is never.
 //  * K and V tiles travel through registers into LDS one tile ahead (BUF buffers; rows padded so that fragment reads and
 //    transposed reads are free of bank conflicts).
+//  * The matrix product gives queries zero times the values past them, which is NaN where such a value is not finite: blocks
+//    that staged one past their first query do their queries one by one instead (attn_row).
 //  * KW > 1: the key slices' (maximum, sum, output) meet in LDS at the end.
 // What bounds it: the vector instructions between the two products (about 10 per score, an exponential among them, against
 // two matrix instructions per 16 scores of a lane); with two workgroups per compute unit one's products run under the
@@ -87,13 +125,20 @@ __global__ __launch_bounds__(QW * KW * 64, HS == 256 ? 1 : 2) void attn_kernel(u
             vr[i] = *reinterpret_cast<const u32x4*>(vh + row);
         }
     };
-    auto store = [&](int buf) {
+    uint32_t wild = 0;  // bits 15 and 31: a value that is not finite (an exponent of all ones carries) in a tile on the diagonal
+    auto store = [&](int t0, int buf) {
 #pragma unroll
         for (int i = 0; i < NP; i++) {
             const int idx = i * NT + tid;
             const int row = idx / (HS / 8), c = idx % (HS / 8);
             *reinterpret_cast<u32x4*>(Kt + (buf * TK + row) * KS + c * 8) = kr[i];
             *reinterpret_cast<u32x4*>(Vt + (buf * TK + row) * VS + c * 8) = vr[i];
+        }
+        if (t0 + TK > pos0 + mq0) {
+#pragma unroll
+            for (int i = 0; i < NP; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) wild |= (vr[i][e] & 0x7C007C00u) + 0x04000400u;
         }
     };
     load(0);
@@ -177,20 +222,25 @@ __global__ __launch_bounds__(QW * KW * 64, HS == 256 ? 1 : 2) void attn_kernel(u
     };
 
     const int ntiles = (nk + TK - 1) / TK;
-    store(0);
+    store(0, 0);
     __syncthreads();
     for (int it = 0; it < ntiles; it++) {
         const int t0 = it * TK;
         load(t0 + TK);  // (past the end: the last row again)
         if (BUF == 2) {
             compute(t0, it & 1);
-            store((it + 1) & 1);
+            store(t0 + TK, (it + 1) & 1);
         } else {
             compute(t0, 0);
             __syncthreads();
-            store(0);
+            store(t0 + TK, 0);
         }
         __syncthreads();
+    }
+    if (__syncthreads_or((wild & 0x80008000u) != 0)) {
+        for (int m = mq0 + wave; m < min(mq0 + 32 * QW, M); m += QW * KW)
+            attn_row<HS>(out + ((size_t)m * num_heads + h) * HS, q + ((size_t)m * num_heads + h) * HS, kh, vh, kv_dim, pos0 + m + 1, alpha, out_perm);
+        return;
     }
     {
         float other = l;

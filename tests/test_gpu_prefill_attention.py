@@ -187,3 +187,32 @@ def test_maxima_that_move(ctx, cfg, parts, profile):
         for at in range(0, n, 32):
             assert rel_l2(a[1][at : at + 32], b[1][at : at + 32]) <= 3e-3, at
     assert rel_l2(got[1], want[1]) <= 1e-2
+
+
+@pytest.mark.parametrize("cfg,parts", FORMS, ids=FORM_IDS)
+def test_infinite_values_stay_with_the_queries_that_see_them(ctx, cfg, parts):
+    """One token's value row overflows to infinity; the rows of the tokens before it are those of the prompt without it."""
+    n, vocab, dim = sum(parts), cfg["vocab_size"], cfg["dim"]
+    at = n - parts[-1] // 3 - 1  # of the last call, in the middle of a block of queries
+    img = synth.make_model_image(cfg, seed=63, scale_mult=0.5)
+    embed = img[32 : 32 + 2 * vocab * dim].view(np.float16).reshape(vocab, dim)
+    embed[:] = np.sign(embed) + (embed == 0)
+    embed[:, 0] = 0
+    embed[vocab - 1, 0] = 4
+    # row 0 of the first layer's values: 60000 times column 0
+    off = 32 + 4 * vocab * dim + 2 * dim
+    kv_dim = dim * cfg["n_kv_heads"] // cfg["n_heads"]
+    pwh, pzh, sh = synth.strides(dim)
+    off += (dim + kv_dim) * (4 * pwh + 4 * pzh + 2 * sh)
+    w, z, s = off, off + 4 * kv_dim * pwh, off + 4 * kv_dim * (pwh + pzh)
+    img[w : w + 4 * pwh].view(np.uint32)[:] = [0xF] + [0] * (pwh - 1)
+    img[z : z + 4 * pzh].view(np.uint32)[:] = 0
+    img[s : s + 2 * sh].view(np.float16)[:] = 4000
+    prompt = [int(v) % (vocab - 1) for v in synth.prompt_tokens(63, n, vocab)]
+    want = _prefill(ctx, img, cfg, prompt, parts)[0]
+    prompt[at] = vocab - 1
+    got = _prefill(ctx, img, cfg, prompt, parts)[0]
+    assert np.isposinf(got[1][0, at, 0]) and np.isfinite(got[1][0]).sum() == got[1][0].size - 1
+    for a, b in zip(got, want):
+        assert rel_l2(a[1, :at], b[1, :at]) <= 1e-3  # (the tokens before are the same ones; only the order of sums may differ)
+        assert not np.isfinite(a[1, at:]).all(axis=1).any()
