@@ -1,6 +1,6 @@
-"""The batched int4 GEMM at the edges of its row forms (one workgroup tile of 32, 64, 96 or 128 rows by 64, 128 or 256
-columns, K slices inside a workgroup and over workgroups): rows and K ranges around tile ends, K that is no multiple of a
-quantisation group, K past eight groups (scales and zeros travel for eight at a time), against the product in 64 bits.
+"""The batched int4 GEMM in each of its forms (one workgroup tile of 32, 64, 96 or 128 rows by 64, 128 or 256 columns, K
+slices inside a workgroup and over workgroups): rows and K ranges around tile ends, K that is no multiple of a quantisation
+group, K past eight groups (scales and zeros travel for eight at a time), against the product in 64 bits.
 
 Bar: the weights are exact fp16 values, sums are fp32 and the result is rounded once: rel-L2 2.1e-4 by the rounding alone;
 1e-3 as for the other GEMM tests."""
@@ -16,18 +16,23 @@ from tests.helpers import f16, rel_l2
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [
-    (1, 128, 128), (31, 160, 384), (32, 1120, 1152), (33, 2048, 128), (1, 4096, 384), (16, 4128, 256),  # 32 x 64, split or not
-    (65, 512, 6144), (97, 416, 4224), (33, 3072, 1152), (97, 4096, 384), (64, 1184, 8192),  # 64 x 64
-    (65, 256, 6144), (65, 160, 6144), (129, 2080, 4096), (300, 1056, 4096),  # 64 x 128
-    (257, 128, 12288), (300, 96, 12288), (257, 1184, 12288),  # 64 x 256
-    (700, 128, 6144), (513, 96, 8192), (700, 1152, 6144),  # 96 x 256
-    (385, 128, 16384), (385, 96, 16384), (513, 1120, 12288),  # 128 x 256
-]
+# per form (rows, columns of a workgroup's tile): products whose K is one piece, and parts of K that meet in the workspace
+SHAPES = {
+    (32, 64): {1: [(31, 160, 384), (32, 1120, 1152), (64, 1184, 8192)], 2: [(33, 2048, 128)], 3: [(16, 4128, 256)], 4: [(1, 4096, 384)]},
+    (64, 64): {1: [(65, 512, 6144), (97, 416, 4224), (129, 2080, 4096)], 2: [(33, 5152, 6144)], 3: [(33, 3072, 1152)], 4: [(97, 4096, 384)]},
+    (64, 128): {1: [(65, 256, 6144), (65, 160, 6144), (300, 1056, 4096), (257, 1184, 12288)], 2: [(129, 8224, 9216)], 3: [(513, 4128, 2048)]},
+    (64, 256): {1: [(257, 128, 12288), (300, 96, 12288), (385, 1184, 18432)], 3: [(289, 8192, 8192)]},
+    (96, 256): {1: [(700, 128, 6144), (513, 96, 8192), (700, 1152, 6144)], 2: [(898, 6176, 2304)], 3: [(65, 4128, 18432)], 4: [(65, 6176, 12288)]},
+    (128, 256): {1: [(385, 128, 16384), (385, 96, 16384), (513, 1120, 12288)], 3: [(324, 6176, 6144)]},
+    (128, 128): {1: [(1, 128, 128), (385, 1184, 8192)], 2: [(324, 4096, 3072), (65, 4128, 12288)]},
+}
+CASES = [(*shape, form, parts) for form, by_parts in SHAPES.items() for parts, shapes in by_parts.items() for shape in shapes]
 
 
-@pytest.mark.parametrize("M,K,N", SHAPES)
-def test_against_fp64(ctx, M, K, N):
+@pytest.mark.parametrize("M,K,N,form,parts", CASES, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_against_fp64(ctx, M, K, N, form, parts):
+    rows, cols, _, split = A.gemm_form(M, K, N)
+    assert ((rows, cols), split) == (form, parts)
     key = synth.stream_key(52, M, K, N)
     w, z, s = synth.make_qweight(key, K, N)
     a = synth.normal_f16(synth.stream_key(key, "a"), M * K)
