@@ -1,9 +1,9 @@
 """The batched int4 GEMM entry point that allocates nothing (awq_gemm_int4_static) against awq_gemm_int4.
 
 Both run the same kernel with the same work split; only where the split-K workspace lives differs (a device array
-inside the library instead of memory allocated on first use), and the two-term sum of the K halves does not depend
-on which half arrives first, so the outputs must agree bit for bit.  Two calls in a row share the array: the second
-is smaller and must not see anything the first left behind.
+inside the library instead of memory allocated on first use), and the parts of K are added in an order that does not
+depend on which arrives first, so the outputs must agree bit for bit.  Calls in a row share the array: each is smaller
+than the one before and must not see anything that it left behind.
 """
 import numpy as np
 import pytest
@@ -29,14 +29,15 @@ def _run(fn, ctx, qw, da, resid, M, K, N, accum):
     return dout.download(np.uint16)
 
 
-def test_static_workspace_matches_allocating_entry_point_twice_in_a_row(ctx):
-    # (512, 4096, 4096): 128 output tiles < 256, K = 64 steps -> the split-K form, every tile of the workspace the
-    # 7B-shape O projection uses; then (130, 1024, 384): 6 tiles, ragged last row tile, a fraction of the array
-    shapes = [(512, 4096, 4096), (130, 1024, 384)]
+# the 128 x 128 kernel with K in two parts (128 tiles, the 7B shape's down projection), then a row form in three parts with a
+# ragged last row tile and one in two that takes a fraction of the array; forms that split no K
+@pytest.mark.parametrize("shapes,parts", [([(512, 11008, 4096), (130, 4128, 1152), (33, 2048, 128)], [2, 3, 2]), ([(512, 4096, 4096), (130, 1024, 384)], [1, 1])])
+def test_static_workspace_matches_allocating_entry_point_twice_in_a_row(ctx, shapes, parts):
+    assert [A.gemm_form(*shape)[3] for shape in shapes] == parts
     for accum in (False, True):
         static_out, plain_out, truth = [], [], []
         cases = [_case(ctx, M, K, N, int(accum)) for M, K, N in shapes]
-        # the two static calls back to back on the same stream, nothing in between
+        # the static calls back to back on the same stream, nothing in between
         for (M, K, N), (qw, da, resid, _) in zip(shapes, cases):
             static_out.append(_run(A.gemm_q_static, ctx, qw, da, resid, M, K, N, accum))
         for (M, K, N), (qw, da, resid, host) in zip(shapes, cases):
@@ -53,6 +54,7 @@ def test_static_workspace_matches_allocating_entry_point_twice_in_a_row(ctx):
 def test_static_workspace_without_split(ctx):
     """More than 255 output tiles: no split, no workspace; still the same result."""
     M, K, N = 256, 256, 16384  # 2 x 128 tiles
+    assert A.gemm_form(M, K, N)[3] == 1
     qw, da, resid, _ = _case(ctx, M, K, N, 9)
     got = _run(A.gemm_q_static, ctx, qw, da, resid, M, K, N, False)
     want = _run(A.gemm_q, ctx, qw, da, resid, M, K, N, False)
