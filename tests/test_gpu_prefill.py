@@ -50,8 +50,7 @@ CFG_GQA = dict(dim=512, hidden_dim=1280, n_layers=2, n_heads=8, n_kv_heads=2, vo
 CFG_GQA128 = dict(dim=1024, hidden_dim=1536, n_layers=2, n_heads=8, n_kv_heads=2, vocab_size=512, seq_len=128, rope_theta=10000.0)
 
 
-# 128-wide heads and a prompt longer than one 512-token chunk: the second chunk attends to more than 512 keys (several
-# rounds of key blocks per wave, the two-pass softmax, more than two rounds of value tiles)
+# 128-wide heads and hundreds of keys: many tiles of them per block of queries
 CFG_LONG128 = dict(dim=256, hidden_dim=512, n_layers=2, n_heads=2, n_kv_heads=2, vocab_size=512, seq_len=1024, rope_theta=10000.0)
 
 
@@ -137,9 +136,8 @@ def test_longer_prompt_while_another_stream_is_recorded(ctx):
         assert np.array_equal(a, b)
 
 
-# 128-wide heads and a context past what the batched attention keeps in LDS (1920 positions): the tokens beyond that bound
-# go through the matrix-vector path one at a time inside the same call (position hand-over, token list, the
-# position-split attention from 1024 positions on).
+# 128-wide heads and a long context, in one call, in two and token by token (there the position-split attention from 1024
+# positions on).
 CFG_LONG2K = dict(dim=256, hidden_dim=512, n_layers=2, n_heads=2, n_kv_heads=2, vocab_size=512, seq_len=2176, rope_theta=10000.0)
 
 
@@ -149,7 +147,7 @@ CFG_LONG2K_GQA = dict(dim=512, hidden_dim=512, n_layers=2, n_heads=4, n_kv_heads
 
 
 @pytest.mark.parametrize("cfg", [CFG_LONG2K, CFG_LONG2K_GQA], ids=["2-heads", "grouped-queries"])
-def test_prefill_past_the_batched_attention_bound(ctx, cfg):
+def test_long_prefill(ctx, cfg):
     n_prompt = 2000
     img = synth.make_model_image(cfg, seed=33, scale_mult=0.5)
     prompt = synth.prompt_tokens(33, n_prompt, cfg["vocab_size"])
@@ -183,7 +181,7 @@ def test_prefill_past_the_batched_attention_bound(ctx, cfg):
         for n in ("key_cache", "value_cache"):
             for l in range(L):
                 assert rel_l2(kv[n][l], want_kv[n][l]) <= 1e-2, (name, n, l)
-                # the rows written one at a time past the bound, on their own
+                # the last rows, on their own
                 assert rel_l2(kv[n][l][1920:], want_kv[n][l][1920:]) <= 1e-2, (name, n, l)
         assert rel_l2(logits, want_logits) <= 1e-2, name
         assert nxt == want_next, name
@@ -201,3 +199,65 @@ def test_prefill_past_the_batched_attention_bound(ctx, cfg):
     for name, r in results.items():
         assert r[4] == want_more, name
     o.close()
+
+
+def test_prompts_of_more_than_one_pass(ctx):
+    """2048 tokens go in one pass at most: a call of 2210 takes two, behind 40 tokens of another call."""
+    cfg = dict(CFG_LONG2K, seq_len=2304)
+    n, L, seq, kv_dim, vocab = 2250, cfg["n_layers"], cfg["seq_len"], cfg["dim"], cfg["vocab_size"]
+    img = synth.make_model_image(cfg, seed=35, scale_mult=0.5)
+    prompt = synth.prompt_tokens(35, n, vocab)
+    o = oracle.Model(img)
+    o.reset(prompt)
+    for i in range(n):
+        o.forward(i >= n - 1)
+    t = A.Transformer(ctx, image=img)
+    t.reset(prompt)
+    t.prefill(40, gen_token=False)
+    t.prefill(2210)
+    ctx.sync()
+    assert t.pos == n and t.token(n) == o.tokens(n + 1)[n]
+    for name in ("key_cache", "value_cache"):
+        got, want = (f16(b).reshape(L, seq, kv_dim)[:, :n] for b in (t.download(name, L * seq * kv_dim), o.buffer(name, L * seq * kv_dim)))
+        for l in range(L):
+            for rows in (slice(None), slice(2040, 2088), slice(2088, 2096), slice(2096, None)):  # the second pass begins at 2088
+                assert rel_l2(got[l, rows], want[l, rows]) <= 1e-2, (name, l, rows)
+    assert rel_l2(f16(t.download("logits", vocab)), f16(o.buffer("logits", vocab))) <= 1e-2
+    t.close()
+    o.close()
+
+
+def test_recorded_prompt_longer_than_the_workspace(ctx):
+    """No workspace grows while the stream is recorded: a prompt that is longer goes in several passes (512 + 88 tokens)."""
+    img = synth.make_model_image(CFG_LONG128, seed=36)
+    n, vocab = 700, CFG_LONG128["vocab_size"]
+    prompt = synth.prompt_tokens(36, n, vocab)
+    kv = CFG_LONG128["n_layers"] * CFG_LONG128["seq_len"] * CFG_LONG128["dim"]
+
+    def state():
+        ctx.sync()
+        return [t.download("key_cache", kv), t.download("value_cache", kv), t.download("logits", vocab), t.token(n), t.pos]
+
+    t = A.Transformer(ctx, image=img)
+    t.reset(prompt)
+    t.prefill(100, gen_token=False)
+    ctx.sync()
+    stream, graph, runnable = C.c_void_p(lib.awq_ctx_stream(ctx.h)), C.c_void_p(), C.c_void_p()
+    assert lib.hipStreamBeginCapture(stream, 0) == 0
+    t.prefill(600)
+    assert lib.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert lib.hipGraphInstantiate(C.byref(runnable), graph, None, None, C.c_size_t(0)) == 0
+    replays = []
+    for _ in range(3):
+        assert lib.hipGraphLaunch(runnable, stream) == 0
+        replays.append(state())
+    t.reset(prompt)
+    t.prefill(100, gen_token=False)
+    t.prefill(600)
+    want = state()
+    for got in replays:
+        assert got[3:] == want[3:] and got[4] == n
+        for a, b in zip(got[:3], want[:3]):
+            assert rel_l2(f16(a), f16(b)) <= 2e-3
+    assert lib.hipGraphExecDestroy(runnable) == 0 and lib.hipGraphDestroy(graph) == 0
+    t.close()
