@@ -36,12 +36,12 @@ __device__ __forceinline__ ColGroup col_group(const GemmParams& p, int g) {
 // read spread over all banks.
 __device__ __forceinline__ int rows_key(int row) { return (row ^ ((row & 31) >> 3)) & 7; }
 
-template <int MT_, int MW_, int NW_, int KW_, int AS_, int WS_>
+template <int MT_, int NW_, int KW_, int AS_, int WS_>
 struct RowsForm {
-    static constexpr int MT = MT_, MW = MW_, NW = NW_, KW = KW_;  // row blocks per wave; waves along rows, columns, K
-    static constexpr int AS = AS_, WS = WS_;                      // slots of the activation (steps) and weight (pairs of steps) rings
-    static constexpr int WAVES = MW * NW * KW;
-    static constexpr int BMR = MT * MW * 32;   // tile rows
+    static constexpr int MT = MT_, NW = NW_, KW = KW_;  // row blocks per wave; waves along columns, K
+    static constexpr int AS = AS_, WS = WS_;            // slots of the activation (steps) and weight (pairs of steps) rings
+    static constexpr int WAVES = NW * KW;
+    static constexpr int BMR = MT * 32;        // tile rows
     static constexpr int A_BYTES = BMR * 128;  // activation tile of a step and K slice
     static constexpr int W_BYTES = 4096;       // packed weights of 64 rows for a pair of steps
     static constexpr int ZS_BYTES = 6 * 256;   // scales (5 dwords a row) and zeros (one) of 64 rows for 8 pairs
@@ -59,8 +59,8 @@ struct RowsForm {
 // C[m][n] = sum_k A[m][k] * half((q[n][k] - z) * s): prefill.hip's product, rounding points and epilogues, in tiles whose
 // waves own 64 columns, so that an activation fragment read from LDS feeds two matrix instructions (in the 128 x 128
 // kernel's waves of 32 columns it feeds one, which takes the LDS's whole bandwidth at full matrix rate).
-//  * A wave's tile is 32 MT rows x 64 columns; MW x NW waves make the workgroup's tile and KW such groups take a slice of
-//    K each and meet in LDS at the end (few rows: the chip is filled along K without partial tiles in memory).
+//  * A wave's tile is 32 MT rows x 64 columns; NW waves side by side make the workgroup's tile and KW such groups take a
+//    slice of K each and meet in LDS at the end (few rows: the chip is filled along K without partial tiles in memory).
 //  * Activations and packed weights travel global -> LDS directly into rings of AS steps and WS pairs of steps; the rings
 //    are as short as two workgroups per compute unit need (128 x 256: two slots each, 76 KB; what a third slot would hide,
 //    the other workgroup hides).  One barrier per step where waves share a tile, none where they do not.
@@ -77,15 +77,15 @@ struct RowsForm {
 // APERM: A's chunks of 8 are in the order a packed dword dequantises in; WHOLE: K is a multiple of 128 (nothing to mask).
 template <class F, bool APERM, bool WHOLE>
 __global__ __launch_bounds__(F::WAVES * 64, F::WAVES_PER_SIMD) void gemm_rows_kernel(const GemmParams p) {
-    constexpr int MT = F::MT, MW = F::MW, NW = F::NW, KW = F::KW, AS = F::AS, WS = F::WS;
+    constexpr int MT = F::MT, NW = F::NW, KW = F::KW, AS = F::AS, WS = F::WS;
     constexpr int NT = F::WAVES * 64;
     constexpr int AL = 4 * MT / NW;           // activation loads per wave and step
-    constexpr int WL = MW == 1 ? 4 : 2;       // weight loads per wave and pair of steps
-    constexpr bool SHARED = MW * NW > 1;      // waves read what other waves loaded: a barrier per step
+    constexpr int WL = 4;                     // weight loads per wave and pair of steps
+    constexpr bool SHARED = NW > 1;           // waves read what other waves loaded: a barrier per step
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_bytes[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int kw = wave / (MW * NW), wr = wave % (MW * NW), nw = wr / MW, mw = wr % MW;
+    const int kw = wave / NW, nw = wave % NW;
     // Workgroup ids go round-robin over the 8 XCDs; each XCD takes an eighth of the workgroups, in an order that keeps the
     // row tiles and K parts of a weight tile together (its rows leave memory once).  Whole weight tiles per XCD would
     // leave some XCDs a round more than the others (44 tiles of 11 row tiles, 64 places per XCD: 62 us instead of 41).
@@ -100,12 +100,12 @@ __global__ __launch_bounds__(F::WAVES * 64, F::WAVES_PER_SIMD) void gemm_rows_ke
     const uint32_t a_ring = (uint32_t)(kw * F::A_RING);
     const uint32_t w_ring = (uint32_t)(KW * F::A_RING + (kw * NW + nw) * F::W_RING);
 
-    // activation loader: instruction q of the slice's wave wr covers tile rows (wr * AL + q) * 8 .. + 8, 8 lanes x 16 bytes
+    // activation loader: instruction q of the slice's wave nw covers tile rows (nw * AL + q) * 8 .. + 8, 8 lanes x 16 bytes
     // per row; the lane's LDS chunk is lane & 7, so it fetches the source chunk that the swizzle maps there
     uint32_t a_off[AL];  // byte offset from p.A of the lane's chunk in the first step
 #pragma unroll
     for (int q = 0; q < AL; q++) {
-        const int r = (wr * AL + q) * 8 + (lane >> 3);
+        const int r = (nw * AL + q) * 8 + (lane >> 3);
         a_off[q] = (uint32_t)(((size_t)min(m0 + r, p.M - 1) * p.lda + ((lane & 7) ^ rows_key(r)) * 8) * 2);  // rows past M are computed, never stored
     }
     // weight loader: 16 rows of a block per instruction, 4 lanes x 16 bytes per row; 16-byte unit u of a row's 64 bytes
@@ -136,7 +136,7 @@ __global__ __launch_bounds__(F::WAVES * 64, F::WAVES_PER_SIMD) void gemm_rows_ke
     const int p_begin = (int)((long long)slice * npairs / slices), p_end = (int)((long long)(slice + 1) * npairs / slices);
     const int trips = (SHARED && KW > 1) ? (npairs + slices - 1) / slices : p_end - p_begin;
     auto load_a = [&](int step) {
-        const uint32_t dst = a_ring + (uint32_t)((step % AS) * F::A_BYTES + wr * (AL * 1024));
+        const uint32_t dst = a_ring + (uint32_t)((step % AS) * F::A_BYTES + nw * (AL * 1024));
         if (WHOLE) {
             const uint16_t* base = p.A + min(step, 2 * npairs - 1) * BK;
 #pragma unroll
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(F::WAVES * 64, F::WAVES_PER_SIMD) void gemm_rows_ke
         } else {  // chunks past K are zero
 #pragma unroll
             for (int q = 0; q < AL; q++) {
-                const int r = (wr * AL + q) * 8 + (lane >> 3);
+                const int r = (nw * AL + q) * 8 + (lane >> 3);
                 const int k = step * BK + ((lane & 7) ^ rows_key(r)) * 8;
                 const void* src = reinterpret_cast<const uint8_t*>(p.A) + a_off[q] + (size_t)step * (BK * 2);
                 dma16(k < p.K ? src : (const void*)zeros16, dst + q * 1024);
@@ -156,16 +156,14 @@ __global__ __launch_bounds__(F::WAVES * 64, F::WAVES_PER_SIMD) void gemm_rows_ke
         const uint32_t g = (uint32_t)min(pair, npairs - 1);
 #pragma unroll
         for (int b = 0; b < 2; b++)
-            if (MW == 1 || mw == b) {
 #pragma unroll
-                for (int q = 0; q < 2; q++) {
-                    if (WHOLE) {
-                        dma16(wblk[b] + g * 16, w_off[q], dst + b * 2048 + q * 1024);
-                    } else {  // units past the row's end re-read its last one (against activations that are zero)
-                        const int r = 16 * q + (lane >> 2);
-                        const uint32_t unit = g * 4 + ((lane & 3) ^ ((r >> 1) & 3));
-                        dma16(wblk[b], ((uint32_t)(r * p.C) + min(unit, (uint32_t)p.C - 1)) * 16, dst + b * 2048 + q * 1024);
-                    }
+            for (int q = 0; q < 2; q++) {
+                if (WHOLE) {
+                    dma16(wblk[b] + g * 16, w_off[q], dst + b * 2048 + q * 1024);
+                } else {  // units past the row's end re-read its last one (against activations and scales that are zero)
+                    const int r = 16 * q + (lane >> 2);
+                    const uint32_t unit = g * 4 + ((lane & 3) ^ ((r >> 1) & 3));
+                    dma16(wblk[b], ((uint32_t)(r * p.C) + min(unit, (uint32_t)p.C - 1)) * 16, dst + b * 2048 + q * 1024);
                 }
             }
     };
@@ -177,7 +175,6 @@ __global__ __launch_bounds__(F::WAVES * 64, F::WAVES_PER_SIMD) void gemm_rows_ke
         asm volatile("" : "+v"(l));  // (or its addresses would be kept in registers across the K loop)
 #pragma unroll
         for (int i = 0; i < 6; i++) {
-            if (MW == 2 && (i < 3) != (mw == 0)) continue;
             if (i < 5) {
                 const int idx = i * 64 + l, r = idx / 5;
                 const size_t first = (size_t)row_of(r) * p.sh;
@@ -217,7 +214,7 @@ __global__ __launch_bounds__(F::WAVES * 64, F::WAVES_PER_SIMD) void gemm_rows_ke
         h16x8 a[MT], b[2];
     };
     auto fetch = [&](Frag& f, int step, int j) {
-        const uint16_t* at = reinterpret_cast<const uint16_t*>(lds_bytes + a_ring + (step % AS) * F::A_BYTES) + mw * MT * 32 * BK;
+        const uint16_t* at = reinterpret_cast<const uint16_t*>(lds_bytes + a_ring + (step % AS) * F::A_BYTES);
 #pragma unroll
         for (int i = 0; i < MT; i++) f.a[i] = *reinterpret_cast<const h16x8*>(&at[i * 32 * BK + lrow * BK + (((j + 4 * lhalf) ^ rows_key(lrow)) << 3)]);
 #pragma unroll
@@ -293,7 +290,7 @@ __global__ __launch_bounds__(F::WAVES * 64, F::WAVES_PER_SIMD) void gemm_rows_ke
     // ---- epilogue: the accumulators pass through the idle rings as fp32 [wave][RB * 32 rows][64 columns]; an item is 8
     // columns of a row in both blocks, the K slices of which the item's lane adds up in slice order.
     constexpr int REG = F::RB * 32 * 64;  // floats per wave
-    constexpr int ITEMS = F::ITEMS, PER = F::PER;  // items per wave position (mw, nw), shared by its KW slices
+    constexpr int ITEMS = F::ITEMS, PER = F::PER;  // items per column wave, shared by its KW slices
     float* tile_f = reinterpret_cast<float*>(lds_bytes);
     auto put = [&](int round) {
         float* mine = tile_f + wave * REG + (lane >> 5) * 256 + (lane & 31);
@@ -307,7 +304,7 @@ __global__ __launch_bounds__(F::WAVES * 64, F::WAVES_PER_SIMD) void gemm_rows_ke
     auto get = [&](int item, float (&v)[2][8]) {  // the sum over the workgroup's K slices
 #pragma unroll
         for (int k = 0; k < KW; k++) {
-            const float* src = tile_f + (k * MW * NW + wr) * REG + (item >> 2) * 64 + (item & 3) * 8;
+            const float* src = tile_f + (k * NW + nw) * REG + (item >> 2) * 64 + (item & 3) * 8;
 #pragma unroll
             for (int b = 0; b < 2; b++)
 #pragma unroll
@@ -365,7 +362,6 @@ __global__ __launch_bounds__(F::WAVES * 64, F::WAVES_PER_SIMD) void gemm_rows_ke
         *reinterpret_cast<u32x4*>(o0) = pack8(v[0]);
         *reinterpret_cast<u32x4*>(o1) = pack8(v[1]);
     };
-    const int mw0 = m0 + mw * MT * 32;
     // Split K: each workgroup writes its fp32 sums through to memory and counts itself in; the last one adds all of them in
     // slice order, so that the result does not depend on who that is.
     const size_t tile_id = (size_t)tile * p.mtiles + m_index;
@@ -382,7 +378,7 @@ __global__ __launch_bounds__(F::WAVES * 64, F::WAVES_PER_SIMD) void gemm_rows_ke
                 float v[2][8];
                 get(item, v);
                 if (p.ksplit == 1) {
-                    finish(mw0 + round * F::RB * 32 + (item >> 2), item & 3, v);
+                    finish(m0 + round * F::RB * 32 + (item >> 2), item & 3, v);
                 } else {
                     float* dst = tile_part + (size_t)ks * F::PART_FLOATS + (round * PER + it) * 16 * NT;
 #pragma unroll
@@ -414,7 +410,7 @@ __global__ __launch_bounds__(F::WAVES * 64, F::WAVES_PER_SIMD) void gemm_rows_ke
                 for (int k = 1; k < p.ksplit; k++)
 #pragma unroll
                     for (int e = 0; e < 16; e++) v[e >> 3][e & 7] += src[(size_t)k * F::PART_FLOATS + e * NT];
-                finish(mw0 + round * F::RB * 32 + (item >> 2), item & 3, v);
+                finish(m0 + round * F::RB * 32 + (item >> 2), item & 3, v);
             }
         }
 }
@@ -460,18 +456,18 @@ struct Form {
     int (*launch)(awq_ctx*, pf::GemmParams&, int, int, bool, const char*);
     hipError_t (*raise)();
 };
-template <int MT, int MW, int NW, int KW, int AS, int WS>
+template <int MT, int NW, int KW, int AS, int WS>
 constexpr Form form(awq_step_us step) {
-    using F = pf::RowsForm<MT, MW, NW, KW, AS, WS>;
+    using F = pf::RowsForm<MT, NW, KW, AS, WS>;
     return Form{F::BMR, NW, KW, F::PER_CU > 1 ? 2 : 1, step, (size_t)F::PART_FLOATS, launch_form<F>, raise_lds<F>};
 }
 const Form kForms[] = {
-    form<1, 1, 1, 4, 2, 2>({0.56f, 0.62f, 0.97f}),  // 32 x 64, four K slices
-    form<2, 1, 1, 4, 3, 3>({0.68f, 0.80f, 0.80f}),  // 64 x 64, four K slices
-    form<2, 1, 2, 2, 2, 2>({0.69f, 0.85f, 1.25f}),  // 64 x 128, two K slices
-    form<2, 1, 4, 1, 3, 2>({0.60f, 0.72f, 1.15f}),  // 64 x 256
-    form<3, 1, 4, 1, 3, 2>({0.68f, 0.85f, 1.50f}),  // 96 x 256
-    form<4, 1, 4, 1, 2, 2>({0.72f, 1.02f, 1.90f}),  // 128 x 256
+    form<1, 1, 4, 2, 2>({0.56f, 0.62f, 0.97f}),  // 32 x 64, four K slices
+    form<2, 1, 4, 3, 3>({0.68f, 0.80f, 0.80f}),  // 64 x 64, four K slices
+    form<2, 2, 2, 2, 2>({0.69f, 0.85f, 1.25f}),  // 64 x 128, two K slices
+    form<2, 4, 1, 3, 2>({0.60f, 0.72f, 1.15f}),  // 64 x 256
+    form<3, 4, 1, 3, 2>({0.68f, 0.85f, 1.50f}),  // 96 x 256
+    form<4, 4, 1, 2, 2>({0.72f, 1.02f, 1.90f}),  // 128 x 256
 };
 constexpr int kMaxSplit = 4;
 
