@@ -321,7 +321,9 @@ int awq_gemm_int4_form(int compute_units, int M, int K, int N, int form[4]);
 /* Consume the n_tokens tokens at positions pos .. pos+n_tokens-1 of the shared token list in one batched pass:
  * afterwards the KV cache rows, the logits (of the last token), the token list and the position are those that
  * n_tokens calls of awq_transformer_forward (gen_token false for all but the last, `gen_token` for the last) would
- * leave.  Needs dim, kv_dim and hidden_dim to be multiples of 128. */
+ * leave, up to rounding.  (Attention rows below 1024 positions whose scores all lie below about -87 are an exception: token
+ * by token their softmax underflows, down to 0 / 0, as the reference's does; here it does not.)  Needs dim, kv_dim and
+ * hidden_dim to be multiples of 128. */
 int awq_transformer_prefill(awq_transformer* t, int n_tokens, int gen_token);
 
 /* Diagnostics of the persistent schedule (no counterpart in the reference; its DUMP_PER_TOKEN_TIMINGS switch,

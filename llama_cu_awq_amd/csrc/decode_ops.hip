@@ -648,11 +648,12 @@ int awq_launch_matvec_f16(awq_ctx* ctx, uint16_t* out, const uint16_t* x, const 
         else
             awq_launch(ctx, gemv_f16_kernel<R, false>, grid, dim3(256), lds, out, x, w, n, d, norm_w, norm_out);
     };
-    // Rows a power of two apart: the four rows that a wave asks for together, and those of its neighbours, fall on the same
-    // memory channels, and two rows a wave spread better.  us, four rows | two rows, weights from memory: n = 2048, 32000
-    // rows 23.9 | 21.2, 128256 rows 80.6 | 74.1; 8192, 32000 rows 89.6 | 80.5, 128256 rows 331 | 305; 16384, 32000 rows
-    // 185 | 172.  n = 4096 is the exception (41.1 | 42.1).  Other lengths want four (fewer workgroups to stage x): 1536 16.7 |
-    // 17.6, 3072 30.0 | 30.8, 5120 48.9 | 50.6, 7168 68.0 | 69.6, 24576 236 | 245; below 2048 too (1024: 12.0 | 13.0).
+    // Rows a power of two apart are read faster two to a wave than four, by measurement only: that four of them meet on the
+    // same memory channels would explain it, but no counter has shown it, and n = 4096 gains nothing.  us, four rows | two
+    // rows, weights from memory: n = 2048, 32000 rows 23.9 | 21.2, 128256 rows 80.6 | 74.1; 8192, 32000 rows 89.6 | 80.5,
+    // 128256 rows 331 | 305; 16384, 32000 rows 185 | 172; 4096, 16000 rows 22.0 | 21.6, 32000 rows 41.1 | 42.1 and 40.5 |
+    // 40.2, 64000 rows 77.5 | 76.9, 128256 rows 152.7 | 152.1.  Other lengths want four (fewer workgroups to stage x): 1536
+    // 16.7 | 17.6, 3072 30.0 | 30.8, 5120 48.9 | 50.6, 7168 68.0 | 69.6, 24576 236 | 245; below 2048 too (1024: 12.0 | 13.0).
     if (n >= 2048 && (n & (n - 1)) == 0 && n != 4096)
         launch(std::integral_constant<int, 2>{});
     else

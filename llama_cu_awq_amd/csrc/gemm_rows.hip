@@ -448,7 +448,11 @@ hipError_t raise_lds() {
 
 // Measured over K 2048 .. 28672, N 2560 .. 57344 and 16 .. 2000 rows with weights from memory: us per K step of 64 with
 // single workgroups on few compute units, on all of them, and with two on each (where the LDS holds two).  The estimate
-// made of them is within 15 % of the launches it was fitted to; what matters is which form it puts first.
+// made of them was within 15 % of the time of 145 of 148 products besides those it was fitted to (1 .. 2048 rows; up to 18 %
+// low).  Forms closer together than that are a toss-up: between one and two workgroups on a compute unit the unsplit
+// 64 x 128 form is put up to 15 % too low, and at 600 to 1000 rows of long K is taken where the 128 x 128 kernel is 2 to 8 %
+// faster (879 x 11008 x 4096: 116 us, 107); step times that correct it lose as much where that kernel stalls (859 x 10592 x
+// 4352: 126 us, 159).
 struct Form {
     int rows, nw, kw, per_cu;
     awq_step_us step;

@@ -5,9 +5,10 @@
 // The reference has no such path: it feeds prompt tokens through its matrix-VECTOR kernels one at a time
 // (llama2_q4.cu:716-735).  The contract here is therefore the result of that token-by-token run: after
 // awq_transformer_prefill(t, M, gen) the KV cache rows, the logits of the last token, the token list and the
-// position equal what M calls of awq_transformer_forward would leave (same rounding points: q/k/v, scores,
-// probabilities, attention output, residual stream and hidden vector are rounded to fp16 where the reference
-// kernels round them; only fp32 summation order differs).
+// position equal what M calls of awq_transformer_forward would leave, up to fp32 summation order and one rounding:
+// q/k/v, scores, attention output, residual stream and hidden vector are rounded to fp16 where the reference kernels
+// round them, probabilities before their division by the row's sum instead of after it.  The attention differs in one
+// more point, which shows only where all scores of a query lie below about -87 (prefill_attention.hip).
 //
 // Dequantised weights are bit-exact: w16 = half_rne((q - z) * s) computed as an exact fp16 integer (q - z)
 // times the fp16 scale in one rounding.
@@ -578,8 +579,10 @@ static int bind_workspace(awq_ctx* ctx, pf::GemmParams& p, int tiles, bool stati
     return AWQ_OK;
 }
 
-// Expected time of the 128 x 128 kernel, to be weighed against the forms of gemm_rows.hip.  It is the best one where about
-// one of its workgroups comes to a compute unit (512 rows against 4096 columns: 33 us, the best other form 36).
+// Expected time of the 128 x 128 kernel, to be weighed against the forms of gemm_rows.hip (147 of 159 products within 15 %).
+// It is as good as any of them where about one of its workgroups comes to a compute unit and K is long: weights from memory,
+// 512 x 11008 x 4096 in two parts 67 us, 128 x 256 in four parts 64, 64 x 256 in four 70, 64 x 128 71; 77 x 5120 x 13824 in
+// two parts 37.5 us, 96 x 256 in four 34, 32 x 64 36, 64 x 128 36.  At K = 4096 it is not (512 x 4096 x 4096: 32 us, 64 x 128 28).
 static float general_us(int cus, long long tiles, int K, int ksplit) {
     const float split = ksplit > 1 ? 2.0f + 0.5e-6f * tiles * ksplit * (pf::BM * pf::BN * sizeof(float)) : 0.0f;
     return awq_gemm_us(cus, 2, tiles * ksplit, div_up(div_up(K, pf::BK), ksplit), awq_step_us{0.52f, 0.58f, 1.1f}) + split;

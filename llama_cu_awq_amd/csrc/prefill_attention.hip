@@ -4,6 +4,10 @@
 // Rounding points of the reference (llama2_q4.cu:410-427) that survive the one pass: scores are rounded to fp16, sums of
 // exponentials and of P V are fp32, the output is fp16.  The probability itself is rounded to fp16 before the division by
 // the row's sum instead of after it (the same relative step; small probabilities no longer become fp16 denormals).
+// One that does not: below 1024 positions the reference, and with it the token-by-token path, starts a row's maximum from 0
+// (the lanes of its block that hold no score).  Exponentials of a row whose scores all lie below -87 are then fp32 denormals,
+// below about -104 all zero and the output 0 / 0; here the maximum is that of the scores, and such rows
+// come out as any other.
 #include <atomic>
 
 #include "common.hpp"
@@ -66,11 +70,13 @@ __device__ __forceinline__ void attn_row(uint16_t* out, const uint16_t* q, const
 //    order of an accumulator (8 (j/4) + 4 (lane/32) + j%4) is taken for the contraction, and the value fragments are read
 //    from LDS in that order, transposed by the LDS itself.
 //  * The accumulated output is rescaled only when some row's maximum grows by more than 5 (a factor of e^5 is nothing to
-//    fp16 or fp32), which after the first tiles is never.
+//    fp16 or fp32): rarely after the first tiles where scores are within a few units of each other, again and again where
+//    they spread over tens.
 //  * K and V tiles travel through registers into LDS one tile ahead (BUF buffers; rows padded so that fragment reads and
 //    transposed reads are free of bank conflicts).
 //  * The matrix product gives queries zero times the values past them, which is NaN where such a value is not finite: blocks
-//    that staged one past their first query do their queries one by one instead (attn_row).
+//    that staged one past their first query do their queries one by one instead (attn_row).  Looking for them costs 512
+//    tokens x 32 heads 14.2 -> 15.1 us (under the profiler).
 //  * KW > 1: the key slices' (maximum, sum, output) meet in LDS at the end.
 // What bounds it: the vector instructions between the two products (about 10 per score, an exponential among them, against
 // two matrix instructions per 16 scores of a lane); with two workgroups per compute unit one's products run under the

@@ -11,8 +11,10 @@
 // the threshold" a monotone test.  The sorted order never has to be materialised: one workgroup histograms the at
 // most 15361 distinct probability values in LDS, walks the bins from the largest value down to the one where the
 // exact prefix crosses, works out how many equal values into that bin the crossing is, and picks that many-th
-// occurrence in index order (the radix sort is stable).  One launch for softmax and selection together, no temporary
-// storage, capturable in a graph.
+// occurrence in index order (the radix sort is stable).  Up to 32768 entries softmax and selection are one launch of one
+// workgroup without temporary storage; above that a sampler object spreads them over many workgroups and four launches, in
+// scratch memory of its own and with the same bits (while recording, and where that memory could not be had, one workgroup
+// does it).  Both can be captured in a graph.
 // (CUB's scan adds in fp16 in an order of its own, so the reference's prefix is one of several roundings of the same
 // sums; this one is the unambiguous member of that family.)
 #include <math.h>
