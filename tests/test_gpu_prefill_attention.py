@@ -81,9 +81,9 @@ def test_long_contexts_against_token_by_token(ctx, cfg, parts):
 
 
 # ---------------------------------------------------------------- scores by design
-def _designed(cfg, seed, reach):
+def _designed(cfg, seed, reach, offset=0.0):
     """A model whose first layer's scores are known: a query's is `reach` times the key token's level, -1 .. 1 in 65 steps
-    (token v has level (v % 65) / 32 - 1), at every distance (the only pair of dimensions in use turns least)."""
+    (token v has level (v % 65) / 32 - 1), plus `offset`, at every distance (the only pair of dimensions in use turns least)."""
     dim, hid, heads, kv, vocab = (cfg[k] for k in ("dim", "hidden_dim", "n_heads", "n_kv_heads", "vocab_size"))
     hs = dim // heads
     img = synth.make_model_image(cfg, seed=seed, scale_mult=0.25)
@@ -119,7 +119,9 @@ def _designed(cfg, seed, reach):
     for m in (q, k):
         m[0][:], m[1][:] = 0, 0
     functional(q, np.arange(heads) * hs + hs // 2 - 1, 0, 1 / 128)  # 1 for every token
-    functional(k, np.arange(kv) * hs + hs // 2 - 1, 128, reach / alpha / 128)
+    k_rows = np.arange(kv) * hs + hs // 2 - 1
+    functional(k, k_rows, 128, reach / alpha / 128)
+    k[0][k_rows, :16], k[2][k_rows, 0] = 0x11111111, offset / alpha / 128
     matrix(dim, dim)
     for K, N in ((dim, hid), (dim, hid), (hid, dim)):
         matrix(K, N)
@@ -187,6 +189,18 @@ def test_maxima_that_move(ctx, cfg, parts, profile):
         for at in range(0, n, 32):
             assert rel_l2(a[1][at : at + 32], b[1][at : at + 32]) <= 3e-3, at
     assert rel_l2(got[1], want[1]) <= 1e-2
+
+
+@pytest.mark.parametrize("cfg,parts", [(H64, (64,)), (H64, (100,)), (H256, (100,))], ids=["64x1", "64x2", "256"])
+def test_scores_far_below_zero(ctx, cfg, parts):
+    """A constant added to every score changes no softmax: scores of -166 .. -134, whose exponentials are zero in fp32, against
+    -16 .. 16.  Both are multiples of a half, which fp16 holds; over 100 positions the pair turns by 0.0133, and what the fp16
+    factors keep of that, 0.0133^2 of a score, is below the rounding of the far ones (0.03 of 0.06) and moves the near ones by
+    up to 16 x 0.0133^2 = 0.003, a probability by 3e-3.  With the five fp16 roundings of the test above (6e-4): 4e-3."""
+    prompt = [_token(PROFILES["by-slice"](i, sum(parts)), np.random.default_rng(64 + i), cfg["vocab_size"]) for i in range(sum(parts))]
+    near, far = (_prefill(ctx, _designed(cfg, 65, 16.0, offset), cfg, prompt, parts) for offset in (0.0, -150.0))
+    for a, b in ((near[0][0][1], far[0][0][1]), (near[0][1][1], far[0][1][1]), (near[1], far[1])):
+        assert np.isfinite(b).all() and rel_l2(a, b) <= 4e-3
 
 
 @pytest.mark.parametrize("cfg,parts", FORMS, ids=FORM_IDS)
