@@ -909,6 +909,22 @@ int awq_transformer_prefill(awq_transformer* t, int n_tokens, int gen_token) {
             if ((r = awq_launch_gemm_qkv(ctx, t->pf_q, t->s.key_cache + loff, t->s.value_cache + loff, t->pf_xb, dim, M, &L.wq_q, &L.wq_k,
                                          &L.wq_v, dim, dim, kv_dim, hs, t->rope_table, p.rope_theta, pos0, true)))
                 return r;
+            // Of the last layer only its K and V rows and the last token's way to the logits have a reader: one row goes
+            // through the attention and then through the matrix-vector kernels.  ms a call, all rows -> one: 7B shape, 37
+            // tokens 3.21 -> 3.16, 512 9.40 -> 9.21, 2000 28.14 -> 27.48; 8 layers of the 70B shape, 650 + 150 tokens
+            // 13.88 -> 12.56; 22 layers of 2048, 700 tokens 3.19 -> 3.11.
+            if (l == p.n_layers - 1) {
+                if (done + M < n_tokens) break;
+                if ((r = awq_launch_copy_row(ctx, t->s.x, t->pf_x + (size_t)(M - 1) * dim, dim))) return r;
+                if ((r = awq_launch_attn_prefill(ctx, t->s.xb, t->pf_q + (size_t)(M - 1) * dim, t->s.key_cache + loff,
+                                                 t->s.value_cache + loff, p.n_heads, hs, kv_mul, 1, pos0 + M - 1, 0)))
+                    return r;
+                if ((r = awq_launch_matvec_int4(ctx, t->s.x, t->s.xb, &L.wq_o, dim, dim, 1, 1, -1, nullptr, nullptr, nullptr))) return r;
+                if ((r = awq_launch_ffn(ctx, t->s.hb, t->s.x, &L.wq_gate, &L.wq_up, dim, hidden, L.rms_ffn_weight, nullptr))) return r;
+                if ((r = awq_launch_matvec_int4(ctx, t->s.x, t->s.hb, &L.wq_down, hidden, dim, 1, 1, -1, nullptr, nullptr, nullptr)))
+                    return r;
+                break;
+            }
             if ((r = awq_launch_attn_prefill(ctx, t->pf_att, t->pf_q, t->s.key_cache + loff, t->s.value_cache + loff, p.n_heads, hs,
                                              kv_mul, M, pos0, 1)))
                 return r;
@@ -919,7 +935,6 @@ int awq_transformer_prefill(awq_transformer* t, int n_tokens, int gen_token) {
         }
         if (done + M == n_tokens) {
             // last token: final norm, classifier and the greedy sampler exactly as the decode path does them
-            if ((r = awq_launch_copy_row(ctx, t->s.x, t->pf_x + (size_t)(M - 1) * dim, dim))) return r;
             if ((r = awq_launch_set_pos(ctx, t->s.pos, t->s.shared_pos, pos_start + n_tokens - 1))) return r;
             if ((r = awq_launch_matvec_f16(ctx, t->s.logits, t->s.x, t->wcls, dim, p.vocab_size, t->rms_final, nullptr))) return r;
             if ((r = awq_launch_argmax(ctx, t->s.logits, p.vocab_size, t->s.shared_tokens, t->s.shared_pos, t->s.pos, gen_token,

@@ -55,7 +55,9 @@ CFG_LONG128 = dict(dim=256, hidden_dim=512, n_layers=2, n_heads=2, n_kv_heads=2,
 
 
 @pytest.mark.parametrize("cfg,n_prompt", [(CFG, 130), (CFG, 16), (CFG, 1), (CFG, 97), (CFG_GQA, 70), (CFG_GQA128, 75),
-                                          (CFG_LONG128, 700), (CFG_LONG128, 1000)])
+                                          (CFG_LONG128, 700), (CFG_LONG128, 1000),
+                                          # the last layer is the only one: one row of it goes on to the logits
+                                          (dict(CFG, n_layers=1), 97), (dict(CFG_GQA, n_layers=1), 1), (dict(CFG_GQA128, n_layers=1), 75)])
 def test_prefill_matches_token_by_token_oracle(ctx, cfg, n_prompt):
     img = synth.make_model_image(cfg, seed=31)
     t = A.Transformer(ctx, image=img)
