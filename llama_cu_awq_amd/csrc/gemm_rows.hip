@@ -377,7 +377,18 @@ __global__ __launch_bounds__(F::WAVES * 64, F::WAVES_PER_SIMD) void gemm_rows_ke
             if (item < ITEMS) {
                 float v[2][8];
                 get(item, v);
-                if (p.ksplit == 1) {
+                if (p.epi == EPI_PART) {
+                    const int m = m0 + round * F::RB * 32 + (item >> 2);
+                    float* dst = p.part + ((size_t)ks * p.M + m) * p.N[0] + (item & 3) * 8;
+                    if (m < p.M) {
+#pragma unroll
+                        for (int b = 0; b < 2; b++)
+#pragma unroll
+                            for (int h = 0; h < 2; h++)
+                                *reinterpret_cast<f32x4*>(dst + (b ? cg.row1 : cg.row0) + h * 4) =
+                                    f32x4{v[b][h * 4], v[b][h * 4 + 1], v[b][h * 4 + 2], v[b][h * 4 + 3]};
+                    }
+                } else if (p.ksplit == 1) {
                     finish(m0 + round * F::RB * 32 + (item >> 2), item & 3, v);
                 } else {
                     float* dst = tile_part + (size_t)ks * F::PART_FLOATS + (round * PER + it) * 16 * NT;
@@ -388,7 +399,7 @@ __global__ __launch_bounds__(F::WAVES * 64, F::WAVES_PER_SIMD) void gemm_rows_ke
             }
         }
     }
-    if (p.ksplit == 1) return;
+    if (p.ksplit == 1 || p.epi == EPI_PART) return;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     unsigned int* arrival = reinterpret_cast<unsigned int*>(lds_bytes);
@@ -497,7 +508,7 @@ int awq_gemm_rows_setup() {
     return AWQ_OK;
 }
 
-awq_rows_plan awq_plan_gemm_rows(int cus, int M, int K, int groups, bool may_split) {
+awq_rows_plan awq_plan_gemm_rows(int cus, int M, int K, int groups, bool may_split, bool parts) {
     awq_rows_plan best{-1, 1, 1e30f};
     const int npairs = div_up(K, 128);
     for (int i = 0; i < (int)(sizeof(kForms) / sizeof(kForms[0])); i++) {
@@ -507,10 +518,12 @@ awq_rows_plan awq_plan_gemm_rows(int cus, int M, int K, int groups, bool may_spl
         for (int s = 1; s <= (may_split ? kMaxSplit : 1); s++) {
             const long long wgs = tiles * s;
             // a split is for matrices that leave compute units idle, and has to fit the workspace
-            const size_t part = s > 1 ? wgs * f.part_floats * sizeof(float) : 0;
-            if (s > 1 && (tiles >= cus || tiles > kPartTiles || part > kPartBytes || npairs < 2 * f.kw * s)) break;
-            // partial tiles through memory: 2 us and 0.65 per MB
-            const float us = awq_gemm_us(cus, f.per_cu, wgs, 2 * div_up(npairs, f.kw * s), f.step) + (s > 1 ? 2.0f + 0.65e-6f * part : 0.0f);
+            const size_t part = s == 1 ? 0 : (parts ? (size_t)s * M * groups * 64 : wgs * f.part_floats) * sizeof(float);
+            if (s > 1 && (tiles >= cus || (!parts && tiles > kPartTiles) || part > kPartBytes || npairs < 2 * f.kw * s)) break;
+            // partial tiles that meet in the launch cost it 2 us and 0.65 per MB; sums left to the next launch cost the two
+            // of them 0.5 us and 0.2 to 0.3 per MB (512 x 4096, four parts: its norm 5.1 -> 9.1 us)
+            const float extra = s == 1 ? 0.0f : (parts ? 0.5f + 0.3e-6f * part : 2.0f + 0.65e-6f * part);
+            const float us = awq_gemm_us(cus, f.per_cu, wgs, 2 * div_up(npairs, f.kw * s), f.step) + extra;
             if (us < best.us) best = awq_rows_plan{i, s, us};
         }
     }

@@ -14,7 +14,8 @@ constexpr int BM = 128;  // tokens per tile
 constexpr int BN = 128;  // weight rows per tile
 constexpr int BK = 64;   // K per step: 128 bytes of fp16 per LDS tile row
 
-enum Epi { EPI_STORE = 0, EPI_RESID = 1, EPI_QKV = 2, EPI_FFN = 3 };
+// EPI_PART: fp32 sums of each part of K, [part][row][column], for whoever reads the result to add up
+enum Epi { EPI_STORE = 0, EPI_RESID = 1, EPI_QKV = 2, EPI_FFN = 3, EPI_PART = 4 };
 
 struct GemmParams {
     const uint16_t* A;  // [M][lda] fp16 activations
@@ -127,6 +128,7 @@ struct awq_step_us {
 };
 float awq_gemm_us(int cus, int per_cu, long long wgs, int steps, const awq_step_us& t);
 int awq_gemm_rows_setup();  // once per device, with that device current
-awq_rows_plan awq_plan_gemm_rows(int cus, int M, int K, int groups, bool may_split);
+// parts: the K parts of a split stay apart (EPI_PART)
+awq_rows_plan awq_plan_gemm_rows(int cus, int M, int K, int groups, bool may_split, bool parts = false);
 int awq_launch_gemm_rows(awq_ctx* ctx, pf::GemmParams& p, int groups, int form, int ksplit, bool a_perm, const char* what);
 void awq_rows_form(int form, int* tile);  // rows, columns, K slices inside a workgroup

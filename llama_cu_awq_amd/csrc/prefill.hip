@@ -423,6 +423,105 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(uint16_t* o, const ui
     for (int e = NP * 256 + tid; e < n8; e += 256) orow[e] = scale(xr[e], wr[e], ss);
 }
 
+// x[m] += the fp32 partial sums of a product over x's columns (added up in order, one rounding, as the product's own epilogue
+// does it), then o[m] = the RMSNorm of x[m] as above.  Bound by latency: one workgroup per row, every load of a thread
+// requested at once (4 columns a piece; two pieces, rows of up to 8192, stay in registers).
+template <int PARTS>
+__global__ __launch_bounds__(1024) void rmsnorm_parts_kernel(uint16_t* o, uint16_t* x, const float* part, const uint16_t* weight, int size,
+                                                           int perm) {
+    __shared__ float red[16];
+    constexpr int NP = 2;
+    const int tid = threadIdx.x;
+    const int n4 = size >> 2;
+    u32x2* xr = reinterpret_cast<u32x2*>(x + (size_t)blockIdx.x * size);
+    const u32x2* wr = reinterpret_cast<const u32x2*>(weight);
+    u32x2* orow = reinterpret_cast<u32x2*>(o + (size_t)blockIdx.x * size);
+    const f32x4* pr = reinterpret_cast<const f32x4*>(part + (size_t)blockIdx.x * size);
+    const size_t stride = (size_t)gridDim.x * n4;  // from one part to the next
+    struct Piece {
+        u32x2 x, w;
+        f32x4 p[PARTS];
+    };
+    auto load = [&](Piece& v, int e) {
+        v.x = xr[e];
+        v.w = wr[e];
+#pragma unroll
+        for (int k = 0; k < PARTS; k++) v.p[k] = pr[(size_t)k * stride + e];
+    };
+    auto sum = [&](Piece& v) {  // the new x, rounded, in v.x; its squares
+        f32x4 t = v.p[0];
+#pragma unroll
+        for (int k = 1; k < PARTS; k++) t += v.p[k];
+        float sq = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            h16x2 h = as_h2(v.x[k]);
+            h[0] = (h16_t)(t[2 * k] + (float)h[0]);
+            h[1] = (h16_t)(t[2 * k + 1] + (float)h[1]);
+            v.x[k] = as_u32(h);
+            sq = fmaf((float)h[0], (float)h[0], sq);
+            sq = fmaf((float)h[1], (float)h[1], sq);
+        }
+        return sq;
+    };
+    auto put = [&](const Piece& v, int e, float ss) {
+        u32x2 r;
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const h16x2 h = as_h2(v.x[k]), hw = as_h2(v.w[k]);
+            h16x2 q;
+            q[0] = (h16_t)((float)h[0] * (ss * (float)hw[0]));
+            q[1] = (h16_t)((float)h[1] * (ss * (float)hw[1]));
+            r[k] = as_u32(q);
+        }
+        if (perm) {  // lanes 2i and 2i + 1 hold columns 0..3 and 4..7 of eight: (0,4)(1,5) to the one, (2,6)(3,7) to the other
+            const bool odd = e & 1;
+            const uint32_t give = odd ? r[0] : r[1];
+            const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)give, 0xB1, 0xF, 0xF, true);  // quad_perm [1,0,3,2]
+            const uint32_t lo = odd ? got : r[0], hi = odd ? r[1] : got;
+            r[0] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+            r[1] = __builtin_amdgcn_perm(hi, lo, 0x07060302u);
+        }
+        orow[e] = r;
+    };
+    Piece v[NP];
+#pragma unroll
+    for (int i = 0; i < NP; i++) load(v[i], min(i * 1024 + tid, n4 - 1));
+    float sq = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+        const float s = sum(v[i]);
+        if (i * 1024 + tid < n4) {
+            sq += s;
+            xr[i * 1024 + tid] = v[i].x;
+        }
+    }
+    for (int e = NP * 1024 + tid; e < n4; e += 1024) {
+        Piece u;
+        load(u, e);
+        sq += sum(u);
+        xr[e] = u.x;
+    }
+    sq = wave_sum(sq);
+    if ((tid & 63) == 0) red[tid >> 6] = sq;
+    __syncthreads();
+    float ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) ss += red[i];
+    ss /= (float)size;
+    ss += 1e-5f;
+    ss = 1.0f / sqrtf(ss);
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+        if (i * 1024 + tid < n4) put(v[i], i * 1024 + tid, ss);
+    for (int e = NP * 1024 + tid; e < n4; e += 1024) {
+        Piece u;
+        u.x = xr[e];
+        u.w = wr[e];
+        put(u, e, ss);
+    }
+}
+
 // RoPE of q rows [M][heads*hs] and of the K cache rows pos0..pos0+M-1 (gpu_kernels.h:340-363 per position).
 __global__ void rope_rows_kernel(uint16_t* q, uint16_t* kcache_layer, int num_heads, int num_kv_heads, int head_size, int pos0,
                                  float rope_theta, const float2* table) {
@@ -592,6 +691,7 @@ static float general_us(int cus, long long tiles, int K, int ksplit) {
 struct GemmRoute {
     int form;    // of gemm_rows.hip; -1: the 128 x 128 kernel
     int ksplit;  // workgroups per tile along K
+    float us;    // what the launch is expected to take
 };
 // The 128 x 128 kernel gives a single matrix with fewer tiles than compute units two workgroups per tile, each half of K.
 static bool general_splits(int M, int K, int ntiles, bool single) {
@@ -601,15 +701,12 @@ static bool general_splits(int M, int K, int ntiles, bool single) {
 static GemmRoute route_gemm(int cus, int M, int K, int ntiles, bool single) {
     const int ksplit = general_splits(M, K, ntiles, single) ? 2 : 1;
     const awq_rows_plan plan = awq_plan_gemm_rows(cus, M, K, ntiles * 2, ksplit == 2 || !single);
-    if (plan.form >= 0 && plan.us < general_us(cus, (long long)div_up(M, pf::BM) * ntiles, K, ksplit)) return GemmRoute{plan.form, plan.ksplit};
-    return GemmRoute{-1, ksplit};
+    const float general = general_us(cus, (long long)div_up(M, pf::BM) * ntiles, K, ksplit);
+    if (plan.form >= 0 && plan.us < general) return GemmRoute{plan.form, plan.ksplit, plan.us};
+    return GemmRoute{-1, ksplit, general};
 }
 
-// static_ws: take the split-K workspace from the file-scope device array (no allocation) instead of the context's.
-// a_perm: A holds every 8 activations in the order (0,4,1,5,2,6,3,7).
-// *rotated (QKV): whether the epilogue did what p.rope asks for.
-static int launch_gemm(awq_ctx* ctx, pf::GemmParams& p, int ntiles, const char* what, bool a_perm, bool static_ws = false,
-                       bool* rotated = nullptr) {
+static int gemm_ready(awq_ctx* ctx, const pf::GemmParams& p, const char* what) {
     // the kernels' LDS exceeds the default dynamic limit; raised per device when a context is created
     // (contexts on a caller's stream included), here only for a device that was missed
     if (ctx->device < 0 || ctx->device >= kMaxDevices || !g_gemm_lds_raised[ctx->device]) {
@@ -619,6 +716,15 @@ static int launch_gemm(awq_ctx* ctx, pf::GemmParams& p, int ntiles, const char* 
         awq_set_error("%s: activation block of %d x %d halves exceeds 4 GB", what, p.M, p.lda);
         return AWQ_ERR_SHAPE;
     }
+    return AWQ_OK;
+}
+
+// static_ws: take the split-K workspace from the file-scope device array (no allocation) instead of the context's.
+// a_perm: A holds every 8 activations in the order (0,4,1,5,2,6,3,7).
+// *rotated (QKV): whether the epilogue did what p.rope asks for.
+static int launch_gemm(awq_ctx* ctx, pf::GemmParams& p, int ntiles, const char* what, bool a_perm, bool static_ws = false,
+                       bool* rotated = nullptr) {
+    if (int r = gemm_ready(ctx, p, what)) return r;
     const bool single = p.epi == pf::EPI_STORE || p.epi == pf::EPI_RESID;
     // reserved by every product of few tiles, whether its form splits K or not: a smaller one of the same weights, which
     // may be recorded into a graph where nothing can be allocated, may split
@@ -674,6 +780,41 @@ int awq_launch_gemm_single(awq_ctx* ctx, uint16_t* out, long long ldo, const uin
     gemm_common(p, A, lda, M, K, accum ? pf::EPI_RESID : pf::EPI_STORE);
     set_mat(p, 0, w, N, out, ldo, 0);
     return launch_gemm(ctx, p, N / pf::BN, "gemm_int4", a_perm, static_ws);
+}
+
+int awq_launch_rmsnorm_rows(awq_ctx* ctx, uint16_t* o, const uint16_t* x, const uint16_t* w, int size, int M, int perm);
+
+// x += A . W, or (parts > 0) its partial sums in ctx->gemm_part, [part][M][N], for awq_launch_rmsnorm_parts to add to x: where
+// K is split, parts that meet in the launch cost it 6 to 8 us (written through, counted in, read back).  7B shape, us with
+// the parts in the launch -> left to the norm: 37 tokens O 14.2 -> 9.9, down 20.4 -> 16.7 (norm 4.0 -> 4.8), 512 tokens down
+// 67 -> 55 (norm 5.1 -> 9.1).
+int awq_launch_gemm_resid(awq_ctx* ctx, uint16_t* x, const uint16_t* A, int lda, int M, const awq_qweight* w, int K, int N, int* parts) {
+    *parts = 0;
+    const GemmRoute route = route_gemm(ctx->cus, M, K, N / pf::BN, true);
+    const awq_rows_plan plan = awq_plan_gemm_rows(ctx->cus, M, K, N / 64, true, true);
+    if (plan.form >= 0 && plan.ksplit > 1 && plan.us < route.us && awq_reserve_gemm_workspace(ctx) == AWQ_OK) {
+        pf::GemmParams p;
+        gemm_common(p, A, lda, M, K, pf::EPI_PART);
+        set_mat(p, 0, w, N, x, N, 0);
+        p.part = ctx->gemm_part;
+        if (int r = gemm_ready(ctx, p, "gemm_int4")) return r;
+        *parts = plan.ksplit;
+        return awq_launch_gemm_rows(ctx, p, N / 64, plan.form, plan.ksplit, true, "gemm_int4");
+    }
+    return awq_launch_gemm_single(ctx, x, N, A, lda, M, w, K, N, 1, false, true);
+}
+
+// o = RMSNorm of x, M rows of `size`; parts > 0: after adding those of the last awq_launch_gemm_resid to x
+int awq_launch_rmsnorm_parts(awq_ctx* ctx, uint16_t* o, uint16_t* x, const uint16_t* w, int size, int M, int perm, int parts) {
+    const float* part = ctx->gemm_part;
+    switch (parts) {
+        case 0: return awq_launch_rmsnorm_rows(ctx, o, x, w, size, M, perm);
+        case 2: hipLaunchKernelGGL((pf::rmsnorm_parts_kernel<2>), dim3(M), dim3(1024), 0, ctx->stream, o, x, part, w, size, perm); break;
+        case 3: hipLaunchKernelGGL((pf::rmsnorm_parts_kernel<3>), dim3(M), dim3(1024), 0, ctx->stream, o, x, part, w, size, perm); break;
+        case 4: hipLaunchKernelGGL((pf::rmsnorm_parts_kernel<4>), dim3(M), dim3(1024), 0, ctx->stream, o, x, part, w, size, perm); break;
+        default: awq_set_error("rmsnorm: %d parts", parts); return AWQ_ERR_ARG;
+    }
+    return awq_check_launch("rmsnorm_parts");
 }
 
 int awq_launch_rope_rows(awq_ctx* ctx, uint16_t* q, uint16_t* kcache_layer, int nh, int nkv, int hs, int pos0, float theta, int M,

@@ -36,15 +36,14 @@ int awq_sampler_run(awq_sampler* s, uint16_t* logits, int* tokens, volatile int*
                     int* mirror);
 // prefill.hip
 int awq_reserve_gemm_workspace(awq_ctx* ctx);
-int awq_launch_gemm_single(awq_ctx* ctx, uint16_t* out, long long ldo, const uint16_t* A, int lda, int M, const awq_qweight* w,
-                           int K, int N, int accum, bool static_ws, bool a_perm);
 int awq_launch_gemm_qkv(awq_ctx* ctx, uint16_t* q, uint16_t* kcache_layer, uint16_t* vcache_layer, const uint16_t* A, int lda, int M,
                         const awq_qweight* qw, const awq_qweight* kw, const awq_qweight* vw, int K, int Nq, int Nkv, int head_size,
                         const float2* rope, float theta, int pos0, bool a_perm);
 int awq_launch_gemm_ffn(awq_ctx* ctx, uint16_t* hb, const uint16_t* A, int lda, int M, const awq_qweight* gate_w,
                         const awq_qweight* up_w, int K, int N, bool a_perm, bool out_perm);
 int awq_launch_embed_rows(awq_ctx* ctx, uint16_t* x, const uint16_t* table, int dim, const int* tokens, int pos0, int M);
-int awq_launch_rmsnorm_rows(awq_ctx* ctx, uint16_t* o, const uint16_t* x, const uint16_t* w, int size, int M, int perm);
+int awq_launch_gemm_resid(awq_ctx* ctx, uint16_t* x, const uint16_t* A, int lda, int M, const awq_qweight* w, int K, int N, int* parts);
+int awq_launch_rmsnorm_parts(awq_ctx* ctx, uint16_t* o, uint16_t* x, const uint16_t* w, int size, int M, int perm, int parts);
 int awq_launch_attn_prefill(awq_ctx* ctx, uint16_t* out, const uint16_t* q, const uint16_t* kc, const uint16_t* vc, int nh, int hs,
                             int kv_mul, int M, int pos0, int out_perm);
 int awq_launch_set_pos(awq_ctx* ctx, int* pos_dev, volatile int* pos_host, int value);
@@ -902,10 +901,12 @@ int awq_transformer_prefill(awq_transformer* t, int n_tokens, int gen_token) {
         // The activations that feed a GEMM (xb, att, hb) are written with every 8 values in the order the packed weights
         // dequantise in, so that the GEMMs multiply them without reordering either operand; x, q and the KV cache
         // keep the natural order.
+        // The O and down products may leave their result as partial sums; the norm that follows adds them to x.
+        int parts = 0;
         for (int l = 0; l < p.n_layers; l++) {
             const awq_layer_weights& L = t->layers[l];
             const long long loff = (long long)l * p.seq_len * kv_dim;
-            if ((r = awq_launch_rmsnorm_rows(ctx, t->pf_xb, t->pf_x, L.rms_att_weight, dim, M, 1))) return r;
+            if ((r = awq_launch_rmsnorm_parts(ctx, t->pf_xb, t->pf_x, L.rms_att_weight, dim, M, 1, parts))) return r;
             if ((r = awq_launch_gemm_qkv(ctx, t->pf_q, t->s.key_cache + loff, t->s.value_cache + loff, t->pf_xb, dim, M, &L.wq_q, &L.wq_k,
                                          &L.wq_v, dim, dim, kv_dim, hs, t->rope_table, p.rope_theta, pos0, true)))
                 return r;
@@ -928,10 +929,10 @@ int awq_transformer_prefill(awq_transformer* t, int n_tokens, int gen_token) {
             if ((r = awq_launch_attn_prefill(ctx, t->pf_att, t->pf_q, t->s.key_cache + loff, t->s.value_cache + loff, p.n_heads, hs,
                                              kv_mul, M, pos0, 1)))
                 return r;
-            if ((r = awq_launch_gemm_single(ctx, t->pf_x, dim, t->pf_att, dim, M, &L.wq_o, dim, dim, 1, false, true))) return r;
-            if ((r = awq_launch_rmsnorm_rows(ctx, t->pf_xb, t->pf_x, L.rms_ffn_weight, dim, M, 1))) return r;
+            if ((r = awq_launch_gemm_resid(ctx, t->pf_x, t->pf_att, dim, M, &L.wq_o, dim, dim, &parts))) return r;
+            if ((r = awq_launch_rmsnorm_parts(ctx, t->pf_xb, t->pf_x, L.rms_ffn_weight, dim, M, 1, parts))) return r;
             if ((r = awq_launch_gemm_ffn(ctx, t->pf_hb, t->pf_xb, dim, M, &L.wq_gate, &L.wq_up, dim, hidden, true, true))) return r;
-            if ((r = awq_launch_gemm_single(ctx, t->pf_x, dim, t->pf_hb, hidden, M, &L.wq_down, hidden, dim, 1, false, true))) return r;
+            if ((r = awq_launch_gemm_resid(ctx, t->pf_x, t->pf_hb, hidden, M, &L.wq_down, hidden, dim, &parts))) return r;
         }
         if (done + M == n_tokens) {
             // last token: final norm, classifier and the greedy sampler exactly as the decode path does them
