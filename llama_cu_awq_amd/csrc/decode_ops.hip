@@ -236,7 +236,7 @@ __global__ __launch_bounds__(1024) void attn_pv_sliced_kernel(uint16_t* output, 
     }
 }
 
-// Long contexts in the fused schedule: P.V split over positions as well, so that every compute unit pulls whole
+// awq_attention_partial: P.V split over positions as well, so that every compute unit pulls whole
 // cache lines.  A workgroup of 16 waves owns one head, one of `chunks` contiguous ranges of positions and one slice of
 // 64 value dimensions (128 bytes of every row: 8 lanes x 16 bytes); it computes the softmax statistics over ALL
 // positions from the fp16 scores (as every workgroup of the head does, in the same order, so they agree bit for bit),
@@ -367,6 +367,145 @@ __global__ __launch_bounds__(1024) void attn_pv_partial_kernel(float* part, cons
 #pragma unroll
             for (int i = 0; i < n / 2; i++) r[i] = r[2 * i] + r[2 * i + 1];
         part[(size_t)chunk * out_dim + (size_t)h * head_size + slice * 64 + tid] = r[0];
+    }
+}
+
+// Fused schedule, launch sizes above kAttnFusedMaxSeq: scores, softmax and P.V of one of `chunks` contiguous ranges of a head's
+// positions in a workgroup of 16 waves, one pass over its keys and values.  LP lanes (head_size / 8) share a position; each
+// such group of lanes keeps a running maximum, sum of exponentials and fp32 P.V of the positions it sees, the groups meet at
+// the end, and part[chunk][head * head_size + dim] with stat[head][chunk] = (maximum, sum) goes to the O projection, which
+// puts the ranges on one scale while it stages its input and rounds to fp16 there (the reference's rounding point;
+// gpu_kernels.h:368-451).  Scores are rounded to fp16 as the reference does and left in att; the probability, which the
+// reference rounds to fp16 after the division by the row's sum, stays fp32.  The maximum starts where the reference's does.
+// Bound by latency: launch, position word, one round trip for keys and values together, two reductions.  It replaces two
+// launches, scores and P.V (unsplit below 1024 positions; split over positions with the scores exchanged through memory above).
+// us a token, 4 layers, two launches -> one: 7B shape, position 300 167.5 -> 163.8, 700 172.5 -> 168.5, 2000 188.5 -> 181.5;
+// 13B shape 224.4 -> 210.1, 227.1 -> 216.9, 242.8 -> 232.7; 70B shape 391.8 -> 383.6, 407.2 -> 390.5, 423.1 -> 399.9; 32 heads
+// of 64 over 4 key heads 108.4 -> 103.3, 111.9 -> 104.5, 122.3 -> 108.1.
+template <int LP>
+__global__ __launch_bounds__(1024) void attn_ranges_kernel(float* part, float2* stat, uint16_t* att, const uint16_t* q,
+                                                           const uint16_t* key_cache, const uint16_t* value_cache, int num_heads,
+                                                           int kv_heads, int row_stride, float alpha, const int* pPos) {
+    constexpr int HS = LP * 8, PW = 64 / LP, ROUND = 16 * PW, R = 4;  // positions a wave and the workgroup take per load; loads in flight
+    __shared__ float red[16], red_l[16];
+    __shared__ float acc_lds[16][HS];
+    const int size = *pPos + 1;
+    // the query heads of a key head are gridDim-neighbours kv_heads apart: one XCD where kv_heads is a multiple of 8
+    const int kvh = blockIdx.x % kv_heads, h = kvh * (num_heads / kv_heads) + blockIdx.x / kv_heads;
+    const int chunk = blockIdx.y;
+    const int per = (size + (int)gridDim.y - 1) / (int)gridDim.y;
+    const int t_begin = chunk * per, t_end = min(size, t_begin + per);
+    const int t_last = min(max(t_end, t_begin + 1), size) - 1;  // what lies past the range re-reads its last row
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int j = lane % LP, mine = wave * PW + lane / LP;
+    const uint16_t* kh = key_cache + (size_t)kvh * HS + j * 8;
+    const uint16_t* vh = value_cache + (size_t)kvh * HS + j * 8;
+    uint16_t* att_head = att + (size_t)h * size;
+    const u32x4 qv = *reinterpret_cast<const u32x4*>(q + (size_t)h * HS + j * 8);
+    struct Rows {
+        u32x4 k[R], v[R];
+    };
+    auto request = [&](Rows& b, int t0) {
+#pragma unroll
+        for (int i = 0; i < R; i++) b.k[i] = *reinterpret_cast<const u32x4*>(kh + (size_t)min(t0 + mine + i * ROUND, t_last) * row_stride);
+#pragma unroll
+        for (int i = 0; i < R; i++) b.v[i] = *reinterpret_cast<const u32x4*>(vh + (size_t)min(t0 + mine + i * ROUND, t_last) * row_stride);
+    };
+    // below every fp16 score, and finite; the reference's idle-lane 0 when its 1024-thread softmax block is not full
+    float m = size < 1024 ? 0.0f : -1e5f, l = 0.0f;
+    float acc[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) acc[i] = 0.0f;
+    auto process = [&](const Rows& b, int t0) {
+        float s[R];
+        float top = m;
+#pragma unroll
+        for (int i = 0; i < R; i++) {
+            const int t = t0 + mine + i * ROUND;
+            float d = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) d = dot2(b.k[i][e], qv[e], d);
+            d = group_sum<LP>(d);
+            const uint16_t hb = float_to_half_bits(d * alpha);
+            if (j == 0 && t < t_end) att_head[t] = hb;
+            s[i] = t < t_end ? half_bits_to_float(hb) : -INFINITY;
+            top = fmaxf(top, s[i]);
+        }
+        const float fade = expf(m - top);
+        m = top;
+        l *= fade;
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc[e] *= fade;
+#pragma unroll
+        for (int i = 0; i < R; i++) {
+            if (t0 + mine + i * ROUND < t_end) {
+                const float p = expf(s[i] - m);
+                l += p;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const h16x2 hv = as_h2(b.v[i][e]);
+                    acc[2 * e] = fmaf((float)hv[0], p, acc[2 * e]);
+                    acc[2 * e + 1] = fmaf((float)hv[1], p, acc[2 * e + 1]);
+                }
+            }
+        }
+    };
+    // One request ahead of the one in hand.  Each request stands right before the rows it overtakes are used and every path
+    // counts its own loads (requested in a branch that joins again, they would be waited for with everything before them).
+    Rows a, b;
+    request(a, t_begin);
+    for (int t0 = t_begin;; t0 += 2 * R * ROUND) {
+        if (t0 + R * ROUND >= t_end) {
+            process(a, t0);
+            break;
+        }
+        request(b, t0 + R * ROUND);
+        process(a, t0);
+        if (t0 + 2 * R * ROUND >= t_end) {
+            process(b, t0 + R * ROUND);
+            break;
+        }
+        request(a, t0 + 2 * R * ROUND);
+        process(b, t0 + R * ROUND);
+    }
+    const float wm = wave_max(m);
+    if (lane == 0) red[wave] = wm;
+    __syncthreads();
+    float top = red[0];
+#pragma unroll
+    for (int w = 1; w < 16; w++) top = fmaxf(top, red[w]);
+    const float fade = expf(m - top);
+    auto groups_sum = [](float v) {
+        if (LP <= 8) v = lane_xor_sum<8>(v);
+        if (LP <= 16) v = lane_xor_sum<16>(v);
+        return lane_xor_sum<32>(v);
+    };
+    l = groups_sum(l * fade);
+#pragma unroll
+    for (int i = 0; i < 8; i++) acc[i] = groups_sum(acc[i] * fade);
+    if (lane == 0) red_l[wave] = l;
+    if (lane < LP) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) acc_lds[wave][lane * 8 + i] = acc[i];
+    }
+    __syncthreads();
+    auto tree = [](float (&r)[16]) {
+#pragma unroll
+        for (int n = 16; n > 1; n >>= 1)
+#pragma unroll
+            for (int i = 0; i < n / 2; i++) r[i] = r[2 * i] + r[2 * i + 1];
+        return r[0];
+    };
+    float r[16];
+    if (tid < HS) {
+#pragma unroll
+        for (int w = 0; w < 16; w++) r[w] = acc_lds[w][tid];
+        part[((size_t)chunk * num_heads + h) * HS + tid] = tree(r);
+    }
+    if (tid == 0) {
+#pragma unroll
+        for (int w = 0; w < 16; w++) r[w] = red_l[w];
+        stat[(size_t)h * kAttnMaxChunks + chunk] = make_float2(top, tree(r));
     }
 }
 
@@ -612,7 +751,7 @@ int awq_attention_partial_chunks(const awq_ctx* ctx, int num_heads, int head_siz
     return chunks;
 }
 
-// Internal (fused schedule, launch sizes above kAttnFusedMaxSeq): scores, then P.V as fp32 partial sums over
+// awq_attention_partial: scores, then P.V as fp32 partial sums over
 // `*chunks_out` ranges of positions, part[chunk][num_heads * head_size]; the consumer adds the chunks up in order and
 // rounds to fp16.  part must hold kAttnMaxChunks * num_heads * head_size floats.
 int awq_launch_attention_partial(awq_ctx* ctx, float* part, int* chunks_out, const uint16_t* q, const uint16_t* key_cache,
@@ -634,6 +773,35 @@ int awq_launch_attention_partial(awq_ctx* ctx, float* part, int* chunks_out, con
                row_stride, chunks, num_heads * head_size, pos);
     *chunks_out = chunks;
     return awq_check_launch("attn_pv_partial");
+}
+
+// Internal (fused schedule, launch sizes above kAttnFusedMaxSeq): attention in one launch, as parts of a softmax over
+// `*chunks_out` ranges of positions for awq_launch_matvec_int4_parts to put together.  part: kAttnMaxChunks * num_heads *
+// head_size floats; stat: kAttnMaxChunks * num_heads.
+int awq_launch_attention_ranges(awq_ctx* ctx, float* part, float2* stat, int* chunks_out, const uint16_t* q, const uint16_t* key_cache,
+                                const uint16_t* value_cache, uint16_t* att, int num_heads, int head_size, int kv_mul,
+                                int max_seq_len, const int* pos) {
+    const int kv_heads = num_heads / kv_mul, row_stride = kv_heads * head_size;
+    const float alpha = (float)(1.0 / sqrt((double)head_size));
+    // Ranges of what a workgroup requests at once (256 positions of 128-wide heads), at least two, at most about one workgroup
+    // per compute unit: a further range costs the staging of the O projection 0.3 to 0.8 us in every workgroup, positions that
+    // are requested late a round trip.  us per layer, 2 | 3 | 4 ranges: 7B shape (4 layers), position 300 40.9 | 41.2 | 41.5,
+    // 700 42.9 | 41.9 | 42.1, 1000 43.6 | 43.4 | 42.7, 2000 47.4 | 45.9 | 45.4; 70B shape 300 95.9 | 96.6 | 97.6, 2000 101.8 |
+    // 100.4 | 100.0; 32 heads of 64, 700 26.1 | 26.2 | 26.4, 2000 28.4 | 28.2 | 27.0.
+    const int round = 256 * 128 / head_size;
+    const int chunks = max(1, min(min(kAttnMaxChunks, ctx->cus / num_heads), max(2, div_up(max_seq_len, round))));
+    const dim3 grid(num_heads, chunks), block(1024);
+    auto go = [&](auto kernel) {
+        awq_launch(ctx, kernel, grid, block, 0, part, stat, att, q, key_cache, value_cache, num_heads, kv_heads, row_stride, alpha, pos);
+    };
+    switch (head_size) {
+        case 64: go(attn_ranges_kernel<8>); break;
+        case 128: go(attn_ranges_kernel<16>); break;
+        case 256: go(attn_ranges_kernel<32>); break;
+        default: awq_set_error("attention: head_size %d unsupported (64, 128 or 256)", head_size); return AWQ_ERR_SHAPE;
+    }
+    *chunks_out = chunks;
+    return awq_check_launch("attn_ranges");
 }
 
 // Internal: fp16 matvec with optional fused RMSNorm of x (norm_out must not alias x).

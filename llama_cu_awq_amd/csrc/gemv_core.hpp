@@ -13,9 +13,14 @@ struct XArgs {
     uint16_t* norm_out;      // optional: workgroup (0, 0) also stores the normalised vector here
     int K;
     int C;                   // 32-element chunks = ceil(K / 32)
-    const float* part;       // PARTS form: x = half(part[0][k] + part[1][k] + ...), rows K floats apart
+    const float* part;       // PARTS_SUM: x = half(part[0][k] + part[1][k] + ...), rows K floats apart
     int parts;               // 1 .. kMaxParts
+    const float2* stat;      // PARTS_SOFTMAX: (maximum, sum) of head k >> head_shift in each part, [head][kMaxParts]
+    int head_shift;
 };
+// How the activation vector arrives: as fp16; as fp32 sums to be added up; or as parts of a softmax, each relative to its
+// own maximum, to be put on one scale, added up and divided by the whole sum.
+enum { PARTS_NONE = 0, PARTS_SUM = 1, PARTS_SOFTMAX = 2 };
 constexpr int kMaxParts = 4;
 
 // 2^-20 * sum over the 32 consecutive K elements of one chunk of (q - z) * x.
@@ -97,16 +102,20 @@ __device__ __forceinline__ void load_x(XPieces<NORM, pieces_for(W)>& xr, const X
 // The PARTS form of load_x: the activation vector arrives as up to kMaxParts fp32 partial sums per element (the
 // chunks of the position-split attention); their sum, added in part order and rounded to fp16 once, is x.  The loads
 // are requested here, ahead of the packed weights; combine_x turns them into the pieces stage_x takes.
+constexpr int part_pieces_for(int waves) { return waves >= 16 ? 1 : XP; }  // of up to 8192 elements
+
+template <int NP>
 struct PartPieces {
-    u32x4 f[XP][kMaxParts][2];  // 8 floats per piece and part
+    u32x4 f[NP][kMaxParts][2];  // 8 floats per piece and part
+    u32x4 stat[NP][kMaxParts / 2];
 };
 
-template <int W>
-__device__ __forceinline__ void load_parts(PartPieces& pr, const XArgs& p) {
+template <int W, int PARTS>
+__device__ __forceinline__ void load_parts(PartPieces<part_pieces_for(W)>& pr, const XArgs& p) {
     constexpr int T = W * 64;
     const int n8 = p.K >> 3;
 #pragma unroll
-    for (int i = 0; i < XP; i++) {
+    for (int i = 0; i < part_pieces_for(W); i++) {
         if (i > 0 && i * T >= n8) break;
         const int e = min(i * T + (int)threadIdx.x, n8 - 1);
 #pragma unroll
@@ -116,23 +125,53 @@ __device__ __forceinline__ void load_parts(PartPieces& pr, const XArgs& p) {
             pr.f[i][s][0] = src[0];
             pr.f[i][s][1] = src[1];
         }
+        if constexpr (PARTS == PARTS_SOFTMAX) {  // (a head's record is whole whatever the number of parts)
+            const u32x4* src = reinterpret_cast<const u32x4*>(p.stat + (size_t)((e * 8) >> p.head_shift) * kMaxParts);
+#pragma unroll
+            for (int k = 0; k < kMaxParts / 2; k++) pr.stat[i][k] = src[k];
+        }
     }
 }
 
-template <int W>
-__device__ __forceinline__ void combine_x(XPieces<false, pieces_for(W)>& xr, const PartPieces& pr, const XArgs& p) {
+template <int W, int PARTS>
+__device__ __forceinline__ void combine_x(XPieces<false, pieces_for(W)>& xr, const PartPieces<part_pieces_for(W)>& pr, const XArgs& p) {
     constexpr int T = W * 64;
     const int n8 = p.K >> 3;
 #pragma unroll
-    for (int i = 0; i < XP; i++) {
+    for (int i = 0; i < part_pieces_for(W); i++) {
         if (i > 0 && i * T >= n8) break;
         // (a vector element goes through a scalar before the bit cast: cast directly, the element reference is
         // taken as the vector's storage and every lane of it reads element 0)
         float v[8];
+        float scale[kMaxParts];
+        if constexpr (PARTS == PARTS_SOFTMAX) {
+            float top = 0.0f, whole = 0.0f;
+            auto word = [&](int k) {
+                const uint32_t u = pr.stat[i][k >> 2][k & 3];
+                return __builtin_bit_cast(float, u);
+            };
+#pragma unroll
+            for (int s = 0; s < kMaxParts; s++) {
+                if (s >= p.parts) break;
+                top = s == 0 ? word(0) : fmaxf(top, word(2 * s));
+            }
+#pragma unroll
+            for (int s = 0; s < kMaxParts; s++) {
+                if (s >= p.parts) break;
+                scale[s] = expf(word(2 * s) - top);
+                whole = fmaf(scale[s], word(2 * s + 1), whole);
+            }
+#pragma unroll
+            for (int s = 0; s < kMaxParts; s++) {
+                if (s >= p.parts) break;
+                scale[s] /= whole;
+            }
+        }
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             const uint32_t u = pr.f[i][0][j >> 2][j & 3];
             v[j] = __builtin_bit_cast(float, u);
+            if constexpr (PARTS == PARTS_SOFTMAX) v[j] *= scale[0];
         }
 #pragma unroll
         for (int s = 1; s < kMaxParts; s++) {
@@ -140,7 +179,10 @@ __device__ __forceinline__ void combine_x(XPieces<false, pieces_for(W)>& xr, con
 #pragma unroll
             for (int j = 0; j < 8; j++) {
                 const uint32_t u = pr.f[i][s][j >> 2][j & 3];
-                v[j] += __builtin_bit_cast(float, u);
+                if constexpr (PARTS == PARTS_SOFTMAX)
+                    v[j] = fmaf(__builtin_bit_cast(float, u), scale[s], v[j]);
+                else
+                    v[j] += __builtin_bit_cast(float, u);
             }
         }
 #pragma unroll

@@ -52,6 +52,8 @@ struct GemvParams {
     int head_size;           // for the fused RoPE row pairing
     const float* xpart;      // PARTS form: x is the sum of `xparts` fp32 vectors K floats apart, rounded to fp16
     int xparts;
+    const float2* xstat;     // ... or of parts of a softmax, with their (maximum, sum) per head
+    int head_shift;          // log2 of the head size there
     // Filled in by launch().  Everything a wave needs before it can request its first packed weights is a handful of
     // scalar instructions on these: the compute unit's one scalar unit serves all of its waves, and with 16 to 24 waves
     // arriving at once every scalar instruction of the prologue costs all of them a cycle (a division by the grid size
@@ -88,9 +90,9 @@ __device__ __forceinline__ int map_row(int li, int half_shift) {
 // takes ceil(C * SPLIT / 64) passes per SPLIT rows instead of SPLIT * ceil(C / 64): the kernels' time follows the
 // number of passes, not the bytes (K = 11008 and K = 12288 took the same 6.9 us; 10240: 6.4).  R then counts the row
 // sets of a wave.
-template <int W, int R, int D, int KIND, bool NORM, bool ROPE, bool PARTS = false, int SPLIT = 1>
+template <int W, int R, int D, int KIND, bool NORM, bool ROPE, int PARTS = PARTS_NONE, int SPLIT = 1>
 __global__ __launch_bounds__(W * 64) void gemv_int4_kernel(const GemvParams p) {
-    static_assert(!PARTS || (!NORM && KIND == KIND_SINGLE), "partial-sum input only for the plain single-matrix form");
+    static_assert(PARTS == PARTS_NONE || (!NORM && KIND == KIND_SINGLE), "partial-sum input only for the plain single-matrix form");
     extern __shared__ u32x4 xs[];
     __shared__ float red[W + 1];
 #ifdef AWQ_STAMPS
@@ -312,11 +314,11 @@ __global__ __launch_bounds__(W * 64) void gemv_int4_kernel(const GemvParams p) {
 
     // Packed weights are requested before x is staged (all D stages in the plain forms, D - 1 in the norm-fused ones), so
     // that their HBM latency overlaps the staging (and the RMSNorm reduction).
-    const XArgs xa{p.x, p.norm_w, p.norm_out, p.K, p.C, p.xpart, p.xparts};
+    const XArgs xa{p.x, p.norm_w, p.norm_out, p.K, p.C, p.xpart, p.xparts, p.xstat, p.head_shift};
     XPieces<NORM, pieces_for(W)> xr;
-    PartPieces pr;
-    if constexpr (PARTS)
-        load_parts<W>(pr, xa);
+    PartPieces<part_pieces_for(W)> pr;
+    if constexpr (PARTS != PARTS_NONE)
+        load_parts<W, PARTS>(pr, xa);
     else
         load_x<W, NORM>(xr, xa);
     AWQ_STAMP(1);  // x requested
@@ -339,7 +341,7 @@ __global__ __launch_bounds__(W * 64) void gemv_int4_kernel(const GemvParams p) {
 #endif
     }
     AWQ_STAMP(3);  // the stages that go ahead of the staging requested
-    if constexpr (PARTS) combine_x<W>(xr, pr, xa);
+    if constexpr (PARTS != PARTS_NONE) combine_x<W, PARTS>(xr, pr, xa);
     stage_x<W, NORM>(xs, ca, xa, red, xr);
     AWQ_STAMP(4);  // x staged
 #pragma unroll
@@ -420,6 +422,8 @@ void fill_common(GemvParams& p, const uint16_t* x, int K, int N) {
     p.head_size = 0;
     p.xpart = nullptr;
     p.xparts = 0;
+    p.xstat = nullptr;
+    p.head_shift = 0;
 }
 
 Int4Mat to_mat(const awq_qweight* w) { return Int4Mat{w->weight, w->zeros, w->scales}; }
@@ -497,10 +501,12 @@ int launch(awq_ctx* ctx, GemvParams& p, int grid_y, const char* what) {
 #endif
     const dim3 grid(gx, grid_y);
     const size_t lds = (size_t)p.C * 68;  // activations + per-chunk constant
-    if constexpr (KIND == KIND_SINGLE && !ROPE && R == 1 && (W == 8 || W == 10 || W == 13)) {  // (partial-sum input comes with K <= 8192)
+    if constexpr (KIND == KIND_SINGLE && !ROPE && R == 1 && (W == 8 || W == 10 || W == 13 || W == 16)) {  // (partial-sum input comes with K <= 8192)
         if (p.xpart) {
-            if (int r = ensure_lds_limit(ctx, (const void*)gemv_int4_kernel<W, R, D, KIND, false, false, true, SPLIT>, lds, what)) return r;
-            awq_launch(ctx, gemv_int4_kernel<W, R, D, KIND, false, false, true, SPLIT>, grid, dim3(W * 64), lds, p);
+            auto kernel = p.xstat ? gemv_int4_kernel<W, R, D, KIND, false, false, PARTS_SOFTMAX, SPLIT>
+                                  : gemv_int4_kernel<W, R, D, KIND, false, false, PARTS_SUM, SPLIT>;
+            if (int r = ensure_lds_limit(ctx, (const void*)kernel, lds, what)) return r;
+            awq_launch(ctx, kernel, grid, dim3(W * 64), lds, p);
             return awq_check_launch(what);
         }
     }
@@ -509,11 +515,11 @@ int launch(awq_ctx* ctx, GemvParams& p, int grid_y, const char* what) {
         return AWQ_ERR_ARG;
     }
     if (p.norm_w) {
-        if (int r = ensure_lds_limit(ctx, (const void*)gemv_int4_kernel<W, R, D, KIND, true, ROPE, false, SPLIT>, lds, what)) return r;
-        awq_launch(ctx, gemv_int4_kernel<W, R, D, KIND, true, ROPE, false, SPLIT>, grid, dim3(W * 64), lds, p);
+        if (int r = ensure_lds_limit(ctx, (const void*)gemv_int4_kernel<W, R, D, KIND, true, ROPE, PARTS_NONE, SPLIT>, lds, what)) return r;
+        awq_launch(ctx, gemv_int4_kernel<W, R, D, KIND, true, ROPE, PARTS_NONE, SPLIT>, grid, dim3(W * 64), lds, p);
     } else {
-        if (int r = ensure_lds_limit(ctx, (const void*)gemv_int4_kernel<W, R, D, KIND, false, ROPE, false, SPLIT>, lds, what)) return r;
-        awq_launch(ctx, gemv_int4_kernel<W, R, D, KIND, false, ROPE, false, SPLIT>, grid, dim3(W * 64), lds, p);
+        if (int r = ensure_lds_limit(ctx, (const void*)gemv_int4_kernel<W, R, D, KIND, false, ROPE, PARTS_NONE, SPLIT>, lds, what)) return r;
+        awq_launch(ctx, gemv_int4_kernel<W, R, D, KIND, false, ROPE, PARTS_NONE, SPLIT>, grid, dim3(W * 64), lds, p);
     }
     return awq_check_launch(what);
 }
@@ -665,9 +671,10 @@ int awq_launch_matvec_int4(awq_ctx* ctx, uint16_t* out, const uint16_t* x, const
     return dispatch<KIND_SINGLE, false>(ctx, p, 1, "gemv_int4", plan_for(K, 1));
 }
 
-// out = half(W x [+ out]) with x = half(part[0] + part[1] + ...): the O projection behind the position-split attention.
+// out = half(W x [+ out]) with x = half(part[0] + part[1] + ...), or (stat) the parts of a softmax of awq_launch_attention_ranges
+// put together: the O projection behind the position-split attention.
 int awq_launch_matvec_int4_parts(awq_ctx* ctx, uint16_t* out, const float* part, int parts, const awq_qweight* w, int K, int N,
-                                 int accum) {
+                                 int accum, const float2* stat, int head_size) {
     if (parts < 1 || parts > kMaxParts || K > XP * 8 * 64 * 8) {  // every piece of x travels in registers (8-wave workgroups)
         awq_set_error("matvec with partial-sum input: %d parts, K = %d not supported", parts, K);
         return AWQ_ERR_SHAPE;
@@ -679,7 +686,13 @@ int awq_launch_matvec_int4_parts(awq_ctx* ctx, uint16_t* out, const float* part,
     p.accum = accum;
     p.xpart = part;
     p.xparts = parts;
-    return dispatch<KIND_SINGLE, false>(ctx, p, 1, "gemv_int4_parts", plan_for(K, 1));
+    p.xstat = stat;
+    while ((1 << p.head_shift) < head_size) p.head_shift++;
+    GemvPlan plan = plan_for(K, 1);
+    // Every workgroup stages all parts: workgroups of 16 waves where those of 8 would be two or more on a compute unit.  us a
+    // layer with 8 -> 16 waves: 70B shape, two ranges 99.3 -> 95.9, four 102.1 -> 97.6.
+    if (stat && div_up(N, 8) >= 2 * ctx->cus) plan.waves = 16;
+    return dispatch<KIND_SINGLE, false>(ctx, p, 1, "gemv_int4_parts", plan);
 }
 
 int awq_launch_qkv(awq_ctx* ctx, uint16_t* q, uint16_t* key_cache, uint16_t* value_cache, const uint16_t* x,
@@ -766,7 +779,7 @@ int awq_matvec_int4_parts(awq_ctx* ctx, uint16_t* out, const float* part, int pa
     if (int r = awq_bind(ctx)) return r;
     if (int r = check_shape(K, N)) return r;
     AWQ_REQUIRE(out && part && qw_ok(w), AWQ_ERR_ARG, "null pointer");
-    return awq_launch_matvec_int4_parts(ctx, out, part, parts, w, K, N, accum);
+    return awq_launch_matvec_int4_parts(ctx, out, part, parts, w, K, N, accum, nullptr, 0);
 }
 
 int awq_rmsnorm_ffn_matvec_silu(awq_ctx* ctx, uint16_t* out, const uint16_t* x, const uint16_t* norm_weight,

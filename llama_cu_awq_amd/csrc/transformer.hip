@@ -23,12 +23,11 @@ int awq_launch_ffn(awq_ctx* ctx, uint16_t* out, const uint16_t* x, const awq_qwe
                    int N, const uint16_t* norm_w, uint16_t* norm_out);
 int awq_launch_matvec_f16(awq_ctx* ctx, uint16_t* out, const uint16_t* x, const uint16_t* w, int n, int d,
                           const uint16_t* norm_w, uint16_t* norm_out);
-int awq_attention_partial_chunks(const awq_ctx* ctx, int num_heads, int head_size);
-int awq_launch_attention_partial(awq_ctx* ctx, float* part, int* chunks_out, const uint16_t* q, const uint16_t* key_cache,
-                                 const uint16_t* value_cache, uint16_t* att, int num_heads, int head_size, int kv_mul,
-                                 int max_seq_len, const int* pos);
+int awq_launch_attention_ranges(awq_ctx* ctx, float* part, float2* stat, int* chunks_out, const uint16_t* q, const uint16_t* key_cache,
+                                const uint16_t* value_cache, uint16_t* att, int num_heads, int head_size, int kv_mul,
+                                int max_seq_len, const int* pos);
 int awq_launch_matvec_int4_parts(awq_ctx* ctx, uint16_t* out, const float* part, int parts, const awq_qweight* w, int K, int N,
-                                 int accum);
+                                 int accum, const float2* stat, int head_size);
 int awq_launch_argmax(awq_ctx* ctx, const uint16_t* logits, int size, int* tokens, volatile int* pos_host, int* pos_dev,
                       int write_token, int* tokens_mirror);
 // sampler.hip
@@ -105,7 +104,7 @@ struct awq_transformer {
     bool captured_net[2][kMaxGraphs];
     int* tokens_dev;  // device mirror of SharedData.tokens (the persistent kernel reads its input token here)
     float2* rope_table;  // [seq_len][head_size/2] (cos, sin)
-    float* attn_part;    // [kAttnMaxChunks][dim] fp32 partial attention outputs of the position-split form
+    float* attn_part;    // [kAttnMaxChunks][dim] fp32 attention outputs of ranges of positions, [n_heads][kAttnMaxChunks] (maximum, sum)
     // plan of the persistent per-token kernel
     bool tk_ok;
     char tk_why[160];  // why the persistent kernel cannot run this model, when !tk_ok
@@ -213,7 +212,7 @@ int alloc_state(awq_transformer* t) {
     AWQ_HIP_TRY(hipMemset(t->tokens_dev, 0, (size_t)(c.seq_len + 8) * sizeof(int)));
     const int head = c.dim / c.n_heads;
     AWQ_HIP_TRY(hipMalloc((void**)&t->rope_table, (size_t)c.seq_len * (head / 2) * sizeof(float2)));
-    AWQ_HIP_TRY(hipMalloc((void**)&t->attn_part, (size_t)kAttnMaxChunks * c.dim * sizeof(float)));
+    AWQ_HIP_TRY(hipMalloc((void**)&t->attn_part, (size_t)kAttnMaxChunks * (c.dim * sizeof(float) + c.n_heads * sizeof(float2))));
     hipLaunchKernelGGL(rope_table_kernel, dim3(c.seq_len), dim3(head / 2), 0, t->ctx->stream, t->rope_table, head / 2, head, c.rope_theta);
     if (int r = awq_check_launch("rope_table")) return r;
     s.shared_pos = &t->shared->pos;
@@ -517,21 +516,17 @@ int network_fused(awq_transformer* t, int seq_len_bin) {
                                     L.rms_att_weight, nullptr, t->rope_table, head_size, kv_dim)))
                 return r;
         }
-        // Long launch sizes: P.V split over positions too, its fp32 partial sums added up (and rounded to fp16, the
-        // reference's rounding point) while the O projection stages its input; xb is not written on this path.
-        // (Measured: +1.4 % tokens/s at 1.6 K positions of the 13B shape; just above 256 positions the split costs
-        // 2 us per layer more than it saves, so it starts at the 1024 bin.)
-        // ... and it needs ranges long enough to pay for the partial sums: with four ranges (32 heads) the 1024 bin is
-        // faster unsplit (7B shape at positions 600-664: 743 against 719 tokens/s), with three (40 heads) it is not
-        // (13B shape: 448 against 453); from the 2048 bin on the split wins at both
-        const bool split = seq_len_bin >= kAttnSplitMinSeq && dim <= 8192 &&
-                           seq_len_bin / awq_attention_partial_chunks(ctx, p.n_heads, head_size) >= kAttnSplitMinRange;
+        // Launch sizes past the one-workgroup-per-head form: positions split over workgroups, the parts put together (and
+        // rounded to fp16, the reference's rounding point) while the O projection stages its input; xb is not written on this
+        // path.  (Larger vectors do not travel in the staging's registers.)
+        const bool split = seq_len_bin > kAttnFusedMaxSeq && dim <= 8192;
+        float2* stat = reinterpret_cast<float2*>(t->attn_part + (size_t)kAttnMaxChunks * dim);
         int parts = 0;
         {
             LaunchProbe probe(t, LK_ATTENTION);
             if (split)
-                r = awq_launch_attention_partial(ctx, t->attn_part, &parts, s.q, s.key_cache + loff, s.value_cache + loff, s.att,
-                                                 p.n_heads, head_size, kv_mul, seq_len_bin, pPos);
+                r = awq_launch_attention_ranges(ctx, t->attn_part, stat, &parts, s.q, s.key_cache + loff, s.value_cache + loff, s.att,
+                                                p.n_heads, head_size, kv_mul, seq_len_bin, pPos);
             else
                 r = awq_attention(ctx, s.xb, s.q, s.key_cache + loff, s.value_cache + loff, s.att, p.n_heads, head_size, kv_mul,
                                   seq_len_bin, pPos);
@@ -540,7 +535,7 @@ int network_fused(awq_transformer* t, int seq_len_bin) {
         {
             LaunchProbe probe(t, LK_OPROJ);
             if (split)
-                r = awq_launch_matvec_int4_parts(ctx, s.x, t->attn_part, parts, &L.wq_o, dim, dim, 1);
+                r = awq_launch_matvec_int4_parts(ctx, s.x, t->attn_part, parts, &L.wq_o, dim, dim, 1, stat, head_size);
             else
                 r = awq_launch_matvec_int4(ctx, s.x, s.xb, &L.wq_o, dim, dim, 1, 1, -1, nullptr, nullptr, nullptr);
             if (r) return r;

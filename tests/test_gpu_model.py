@@ -300,3 +300,38 @@ def test_fused_gate_up_with_more_row_groups_than_workgroups(ctx):
     finally:
         t.close()
         o.close()
+
+
+# heads, head size, key heads, positions: the launch sizes past one workgroup per head, where a head's positions are split over up
+# to four workgroups: the first of them, ranges that fill no or several rounds of requests (512, 256 and 128 positions for heads
+# of 64, 128 and 256), last ranges that are short, empty ones' neighbours, the reference's 1024 (the maximum's start), one range
+@pytest.mark.parametrize(
+    "heads,head,kv,positions",
+    [(4, 64, 2, (128, 256, 300, 1022, 1023, 2047, 4500)), (4, 128, 4, (129, 255, 256, 511, 1023, 1024, 3000, 5000)),
+     (8, 128, 1, (256, 257, 700)), (2, 256, 1, (256, 512, 1500, 2600)), (128, 64, 128, (257, 1100))],
+)
+def test_attention_of_long_contexts_in_one_launch(ctx, heads, head, kv, positions):
+    """The fused schedule's attention in ranges, put together by the O projection, against the reference schedule's separate
+    launches on the same cache.  fp16 activations behind it differ by single roundings (under 1e-3 in the norm); values that
+    grow with the position make a range that is missed or weighted wrongly a difference of several per cent."""
+    dim, seq = heads * head, 5120
+    cfg = dict(dim=dim, hidden_dim=256, n_layers=1, n_heads=heads, n_kv_heads=kv, vocab_size=512, seq_len=seq, rope_theta=10000.0)
+    t = A.Transformer(ctx, image=synth.make_model_image(cfg, seed=5))
+    rng = np.random.default_rng(heads * head + kv)
+    t.buffer("key_cache", seq * kv * head * 2).write(rng.standard_normal((seq, kv * head)).astype(np.float16))
+    rows = rng.standard_normal((seq, kv * head)) + 8 * np.arange(seq)[:, None] / seq - 2
+    t.buffer("value_cache", seq * kv * head * 2).write(rows.astype(np.float16))
+    for pos in positions:
+        logits, scores = {}, {}
+        for mode, graph in ((A.SCHEDULE_REFERENCE, False), (A.SCHEDULE_FUSED, False), (A.SCHEDULE_FUSED, True)):
+            t.set_pos(pos, 7)
+            t.forward_logits(use_graph=graph, mode=mode)
+            ctx.sync()
+            logits[mode, graph] = t.download("logits", cfg["vocab_size"]).view(np.float16).astype(np.float64)
+            scores[mode, graph] = t.download("att", heads * (pos + 1)).view(np.float16)
+        want = logits[A.SCHEDULE_REFERENCE, False]
+        assert np.isfinite(want).all()
+        for key in ((A.SCHEDULE_FUSED, False), (A.SCHEDULE_FUSED, True)):
+            assert rel_l2(logits[key], want) <= 4e-3, (pos, key)
+            assert rel_l2(scores[key], scores[A.SCHEDULE_REFERENCE, False]) <= 2e-3, (pos, key)
+    t.close()
