@@ -136,8 +136,8 @@ int awq_attention(awq_ctx* ctx, uint16_t* output, const uint16_t* q, const uint1
                   const uint16_t* value_cache, uint16_t* att, int num_heads, int head_size, int kv_mul,
                   int max_seq_len, const int* pos);
 
-/* The two halves of MultiHeadAttention + the O projection (llama2_q4.cu:410-427, 487) as the fused schedule runs them
- * at long contexts.  awq_attention_partial: scores as awq_attention, then the probability-weighted sum of the value
+/* MultiHeadAttention + the O projection (llama2_q4.cu:410-427, 487) in two halves, for drivers that call the launchers
+ * themselves at long contexts.  awq_attention_partial: scores as awq_attention, then the probability-weighted sum of the value
  * rows split over `*chunks` contiguous ranges of positions (chosen by the library, at most AWQ_ATTENTION_MAX_CHUNKS),
  * written as fp32 partial sums part[chunk][num_heads * head_size]; the probabilities are the reference's (softmax over
  * all positions, rounded to fp16).  awq_matvec_int4_parts: out = half(W x [+ out]) where x = half(part[0] + part[1] +
