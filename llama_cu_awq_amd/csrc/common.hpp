@@ -32,7 +32,10 @@ struct awq_ctx {
 };
 
 constexpr int kAttnMaxHeads = 256;
-constexpr int kAttnFusedMaxSeq = 256;  // up to this launch size attention runs as one workgroup per head
+// Up to this launch size attention runs as two workgroups per head that score all of its positions; past it the fused schedule takes
+// ranges of positions.  us a pass, this form | ranges: 7B shape, 16 tokens from 0 18426 | 18884; 16 grouped-query layers, 12
+// tokens from 200 9581 | 9543, which is what two runs differ by.
+constexpr int kAttnFusedMaxSeq = 256;
 constexpr int kAttnMaxChunks = 4;      // ranges of positions whose partial P.V sums the O projection adds up
 
 void awq_set_error(const char* fmt, ...);
