@@ -376,7 +376,9 @@ __global__ __launch_bounds__(1024) void attn_pv_partial_kernel(float* part, cons
 // the end, and part[chunk][head * head_size + dim] with stat[head][chunk] = (maximum, sum) goes to the O projection, which
 // puts the ranges on one scale while it stages its input and rounds to fp16 there (the reference's rounding point;
 // gpu_kernels.h:368-451).  Scores are rounded to fp16 as the reference does and left in att; the probability, which the
-// reference rounds to fp16 after the division by the row's sum, stays fp32.  The maximum starts where the reference's does.
+// reference rounds to fp16 after the division by the row's sum, stays fp32.  The maximum starts below every score: from the 0
+// that the reference starts at below 1024 positions, scores between -89 and -103 would leave sums so small that their reciprocal
+// is infinite.
 // Bound by latency: launch, position word, one round trip for keys and values together, two reductions.  It replaces two
 // launches, scores and P.V (unsplit below 1024 positions; split over positions with the scores exchanged through memory above).
 // us a token, 4 layers, two launches -> one: 7B shape, position 300 167.5 -> 163.8, 700 172.5 -> 168.5, 2000 188.5 -> 181.5;
@@ -411,8 +413,7 @@ __global__ __launch_bounds__(1024) void attn_ranges_kernel(float* part, float2* 
 #pragma unroll
         for (int i = 0; i < R; i++) b.v[i] = *reinterpret_cast<const u32x4*>(vh + (size_t)min(t0 + mine + i * ROUND, t_last) * row_stride);
     };
-    // below every fp16 score, and finite; the reference's idle-lane 0 when its 1024-thread softmax block is not full
-    float m = size < 1024 ? 0.0f : -1e5f, l = 0.0f;
+    float m = -1e5f, l = 0.0f;  // below every finite fp16 score, and finite itself
     float acc[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) acc[i] = 0.0f;

@@ -10,6 +10,7 @@ import llama_cu_awq_amd as A
 from llama_cu_awq_amd import synth
 from oracle import oracle
 from tests.helpers import f16, rel_l2
+from tests.test_gpu_prefill_attention import PROFILES, _designed, _rows, _token
 
 pytestmark = pytest.mark.gpu
 
@@ -335,3 +336,28 @@ def test_attention_of_long_contexts_in_one_launch(ctx, heads, head, kv, position
             assert rel_l2(logits[key], want) <= 4e-3, (pos, key)
             assert rel_l2(scores[key], scores[A.SCHEDULE_REFERENCE, False]) <= 2e-3, (pos, key)
     t.close()
+
+
+# sizes of the launch past one workgroup per head; 1024 is where the reference's maximum starts elsewhere
+@pytest.mark.parametrize("heads,head,kv", [(8, 64, 2), (2, 256, 1)], ids=["heads-of-64", "heads-of-256"])
+@pytest.mark.parametrize("size", [257, 301, 501, 1022, 1023, 1024])
+def test_decode_scores_far_below_zero(ctx, heads, head, kv, size):
+    """A constant added to every score changes no softmax: scores of -4 .. 4 and the same ones 20, 95 and 150 lower, whose
+    exponentials are small, denormal and zero in fp32.  All are multiples of an eighth, which fp16 and its key rows hold, and the
+    pair of dimensions in use turns by 1.5e-3 over the context, which moves a score by 1e-4 at most.  What may differ is five
+    roundings to fp16 on the way to the second layer's row (6e-4 together): 1e-3."""
+    cfg = dict(dim=heads * head, hidden_dim=256, n_layers=2, n_heads=heads, n_kv_heads=kv, vocab_size=512, seq_len=1280, rope_theta=1e6)
+    rng = np.random.default_rng(size)
+    prompt = [_token(PROFILES["by-slice"](i, size), rng, cfg["vocab_size"]) for i in range(size)]
+    outs = []
+    for offset in (0.0, -20.0, -95.0, -150.0):
+        t = A.Transformer(ctx, image=_designed(cfg, 66, 4.0, offset))
+        t.reset(prompt)
+        t.prefill(size - 1, gen_token=False)
+        t.forward(True, use_graph=True)
+        ctx.sync()
+        outs.append([rows[1, size - 1] for rows in _rows(t, cfg, size)] + [f16(t.download("logits", cfg["vocab_size"]))])
+        t.close()
+    for got in outs[1:]:
+        for a, b in zip(got, outs[0]):
+            assert np.isfinite(a).all() and rel_l2(a, b) <= 1e-3
