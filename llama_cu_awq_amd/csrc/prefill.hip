@@ -634,7 +634,11 @@ int awq_reserve_gemm_workspace(awq_ctx* ctx) {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess) (void)hipGetLastError();
     void* block = nullptr;
-    AWQ_HIP_TRY(hipMalloc(&block, kScratchBytes));
+    if (const hipError_t e = hipMalloc(&block, kScratchBytes); e != hipSuccess) {
+        (void)hipGetLastError();  // a caller that goes on without it must not find this behind its next launch
+        awq_set_error("split-K workspace allocation failed: %s", hipGetErrorString(e));
+        return AWQ_ERR_HIP;
+    }
     unsigned int* counter = reinterpret_cast<unsigned int*>(static_cast<uint8_t*>(block) + kPartBytes);
     const bool recorded = capturing != hipStreamCaptureStatusNone;
     hipStream_t stream = ctx->stream;

@@ -834,7 +834,7 @@ int ensure_prefill_rows(awq_transformer* t, int n_tokens) {
     if (rows > kPrefillChunk) rows = kPrefillChunk;
     // with the first pass, whether its products split K or not: that of a shorter prompt, which may be recorded, may
     // (where it cannot be had, the products that do split say so)
-    if (t->pf_rows == 0 && awq_reserve_gemm_workspace(t->ctx)) (void)hipGetLastError();
+    if (t->pf_rows == 0) (void)awq_reserve_gemm_workspace(t->ctx);
     const size_t widths[5] = {(size_t)p.dim, (size_t)p.dim, (size_t)p.dim, (size_t)p.dim, (size_t)p.hidden_dim};
     size_t row_bytes = 0;
     for (size_t w : widths) row_bytes += w * 2;

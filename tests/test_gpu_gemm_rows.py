@@ -5,6 +5,9 @@ group, K past eight groups (scales and zeros travel for eight at a time), agains
 Bar: the weights are exact fp16 values, sums are fp32 and the result is rounded once: rel-L2 2.1e-4 by the rounding alone;
 1e-3 as for the other GEMM tests."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -218,3 +221,53 @@ def test_short_prefill_recorded_after_a_long_one():
     _hip("hipGraphDestroy", graph)
     t.close()
     ctx.close()
+
+
+# hipMalloc fails for the split-K workspace's 32 MiB and its counters, and for nothing else, with the runtime's own error
+NO_WORKSPACE = """
+#include <dlfcn.h>
+#include <stddef.h>
+int hipMalloc(void** p, size_t n) {
+    static int (*real)(void**, size_t);
+    if (!real) real = (int (*)(void**, size_t))dlsym(dlopen("libamdhip64.so", RTLD_NOW), "hipMalloc");
+    return real(p, n == ((size_t)32 << 20) + 1024 ? (size_t)1 << 60 : n);
+}
+"""
+WITHOUT_WORKSPACE = """
+import ctypes as C, sys
+C.CDLL(sys.argv[1], C.RTLD_GLOBAL)
+import numpy as np
+import llama_cu_awq_amd as A
+from llama_cu_awq_amd import synth
+from llama_cu_awq_amd._lib import QWeightC, lib
+M, K, N = 900, 11008, 4096
+ctx = A.Context(0)
+key = synth.stream_key(58, M, K, N)
+qw = A.QWeight.upload(ctx, *synth.make_qweight(key, K, N))
+a = synth.normal_f16(synth.stream_key(key, "a"), M * K).reshape(M, K // 8, 8)
+x = synth.normal_f16(synth.stream_key(key, "x"), M * N)
+rows = [ctx.upload(np.ascontiguousarray(v).reshape(-1)) for v in (a, a[:, :, [0, 4, 1, 5, 2, 6, 3, 7]])]
+outs = [ctx.upload(x) for _ in rows]
+A.gemm_q_static(ctx, outs[0], N, rows[0], K, M, qw, K, N, accum=True)
+reserve, resid = lib["_Z26awq_reserve_gemm_workspaceP7awq_ctx"], lib["_Z21awq_launch_gemm_residP7awq_ctxPtPKtiiPK11awq_qweightiiPi"]
+reserve.argtypes = [C.c_void_p]
+resid.argtypes = [C.c_void_p] * 3 + [C.c_int] * 2 + [C.POINTER(QWeightC)] + [C.c_int] * 2 + [C.POINTER(C.c_int)]
+assert reserve(ctx.h) != 0, "the workspace was there"
+parts = C.c_int(-1)
+status = resid(ctx.h, outs[1].ptr, rows[1].ptr, K, M, C.byref(qw.c), K, N, C.byref(parts))
+assert (status, parts.value) == (0, 0), (status, parts.value, lib.awq_last_error())
+want, got = (o.download(np.uint16).view(np.float16).astype(np.float64) for o in outs)
+assert np.linalg.norm(got - want) <= 1e-3 * np.linalg.norm(want)
+print("same product")
+"""
+
+
+def test_residual_product_without_a_split_workspace(tmp_path):
+    """900 rows by 4096 columns would leave parts of K to the norm, but need not: where their workspace cannot be had, the
+    product runs unsplit, and the failed allocation is not taken for a failed launch."""
+    (tmp_path / "no_workspace.c").write_text(NO_WORKSPACE)
+    shim = str(tmp_path / "no_workspace.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", shim, str(tmp_path / "no_workspace.c"), "-ldl"], check=True)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", WITHOUT_WORKSPACE, shim], cwd=root, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "same product" in r.stdout, r.stdout + r.stderr
