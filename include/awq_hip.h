@@ -137,8 +137,8 @@ int awq_attention(awq_ctx* ctx, uint16_t* output, const uint16_t* q, const uint1
                   int max_seq_len, const int* pos);
 
 /* MultiHeadAttention + the O projection (llama2_q4.cu:410-427, 487) in two halves, for drivers that call the launchers
- * themselves at long contexts.  awq_attention_partial: scores as awq_attention, then the probability-weighted sum of the value
- * rows split over `*chunks` contiguous ranges of positions (chosen by the library, at most AWQ_ATTENTION_MAX_CHUNKS),
+ * themselves at long contexts (the fused schedule takes them where heads are few).  awq_attention_partial: scores as
+ * awq_attention, then the probability-weighted sum of the value rows split over `*chunks` contiguous ranges of positions (chosen by the library, at most AWQ_ATTENTION_MAX_CHUNKS),
  * written as fp32 partial sums part[chunk][num_heads * head_size]; the probabilities are the reference's (softmax over
  * all positions, rounded to fp16).  awq_matvec_int4_parts: out = half(W x [+ out]) where x = half(part[0] + part[1] +
  * ... ) is formed while the input vector is staged (the reference's fp16 rounding of the attention output).

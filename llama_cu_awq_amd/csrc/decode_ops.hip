@@ -776,6 +776,37 @@ int awq_launch_attention_partial(awq_ctx* ctx, float* part, int* chunks_out, con
     return awq_check_launch("attn_pv_partial");
 }
 
+// Ranges of positions a head's row is divided into, of what a workgroup requests at once (256 positions of 128-wide heads), at
+// least two, at most about one workgroup per compute unit: a further range costs the staging of the O projection 0.3 to 0.8 us
+// in every workgroup, positions that are requested late a round trip.  us per layer, 2 | 3 | 4 ranges: 7B shape (4 layers),
+// position 300 40.9 | 41.2 | 41.5, 700 42.9 | 41.9 | 42.1, 1000 43.6 | 43.4 | 42.7, 2000 47.4 | 45.9 | 45.4; 70B shape 300 95.9 |
+// 96.6 | 97.6, 2000 101.8 | 100.4 | 100.0; 32 heads of 64, 700 26.1 | 26.2 | 26.4, 2000 28.4 | 28.2 | 27.0.
+static int range_count(int cus, int num_heads, int head_size, int max_seq_len) {
+    const int round = 256 * 128 / head_size;
+    return max(1, min(min(kAttnMaxChunks, cus / num_heads), max(2, div_up(max_seq_len, round))));
+}
+
+// Internal (fused schedule, launch sizes above kAttnFusedMaxSeq): whether attention goes in ranges (awq_launch_attention_ranges)
+// or as scores and split P.V (awq_launch_attention_partial).  Ranges save a launch and the scores' way through memory, but there are
+// at most kAttnMaxChunks of them: where that leaves compute units idle, each takes its positions at 2 to 3 us per 128 KB of keys and
+// values, while the scores go 64 positions to a workgroup and P.V 64 dimensions to one (so heads of 256, which are four slices
+// there, turn first, and heads of 64, which are one, never did).  Query heads of one key head share its rows in the L2, which
+// only ranges make use of.  us a token of 4 layers, two launches | ranges; 8 heads of 128: launch size 1024 94.9 | 90.5, position
+// 2000 107.7 | 108.0 (2 key heads 99.8 | 106.4), 4000 118.8 | 123.6, 32000 343.2 | 471.6; 16 heads: 2000 125.3 | 121.9, 4000 138.3 |
+// 138.7, 8000 178.1 | 196.1; 32 heads: 4000 215.3 | 209.3, 8000 278.6 | 285.8 (8 key heads 223.4 | 208.9), 32000 650.4 | 708.3;
+// 40 heads: 8000 350.7 | 346.5, 32000 775.4 | 798.7; 52 heads: 32000 1031 | 975; 64 heads over 8 key heads: 32000 934 | 620; 16
+// heads of 256: 1100 177.4 | 176.9, 4000 214.8 | 240.6; 16 heads of 64: 8000 141.3 | 130.1, 32000 364.0 | 359.6.  A launch size
+// below four times 320 gives the two launches too little to do: 1220 positions, 4 heads of 128 96.5 | 93.7, 8 over one key head
+// 99.5 | 97.6.
+bool awq_attention_takes_ranges(int cus, int num_heads, int head_size, int kv_mul, int max_seq_len) {
+    if (max_seq_len < 1280 || head_size == 64) return true;
+    const int chunks = range_count(cus, num_heads, head_size, max_seq_len), wgs = num_heads * chunks;
+    if (4 * wgs >= 3 * cus || (8 * wgs >= 3 * cus && kv_mul >= 3)) return true;
+    // (at 256 compute units: 16 heads of 128 turn past 3000 positions, 32 past 7000, 40 past 9000)
+    const long long load = (long long)div_up(max_seq_len, chunks) * head_size * head_size >> 18;
+    return load <= wgs - 16;
+}
+
 // Internal (fused schedule, launch sizes above kAttnFusedMaxSeq): attention in one launch, as parts of a softmax over
 // `*chunks_out` ranges of positions for awq_launch_matvec_int4_parts to put together.  part: kAttnMaxChunks * num_heads *
 // head_size floats; stat: kAttnMaxChunks * num_heads.
@@ -784,13 +815,7 @@ int awq_launch_attention_ranges(awq_ctx* ctx, float* part, float2* stat, int* ch
                                 int max_seq_len, const int* pos) {
     const int kv_heads = num_heads / kv_mul, row_stride = kv_heads * head_size;
     const float alpha = (float)(1.0 / sqrt((double)head_size));
-    // Ranges of what a workgroup requests at once (256 positions of 128-wide heads), at least two, at most about one workgroup
-    // per compute unit: a further range costs the staging of the O projection 0.3 to 0.8 us in every workgroup, positions that
-    // are requested late a round trip.  us per layer, 2 | 3 | 4 ranges: 7B shape (4 layers), position 300 40.9 | 41.2 | 41.5,
-    // 700 42.9 | 41.9 | 42.1, 1000 43.6 | 43.4 | 42.7, 2000 47.4 | 45.9 | 45.4; 70B shape 300 95.9 | 96.6 | 97.6, 2000 101.8 |
-    // 100.4 | 100.0; 32 heads of 64, 700 26.1 | 26.2 | 26.4, 2000 28.4 | 28.2 | 27.0.
-    const int round = 256 * 128 / head_size;
-    const int chunks = max(1, min(min(kAttnMaxChunks, ctx->cus / num_heads), max(2, div_up(max_seq_len, round))));
+    const int chunks = range_count(ctx->cus, num_heads, head_size, max_seq_len);
     const dim3 grid(num_heads, chunks), block(1024);
     auto go = [&](auto kernel) {
         awq_launch(ctx, kernel, grid, block, 0, part, stat, att, q, key_cache, value_cache, num_heads, kv_heads, row_stride, alpha, pos);

@@ -303,13 +303,15 @@ def test_fused_gate_up_with_more_row_groups_than_workgroups(ctx):
         o.close()
 
 
-# heads, head size, key heads, positions: the launch sizes past one workgroup per head, where a head's positions are split over up
+# heads, head size, key heads, positions: the launch sizes past one workgroup per head, where a head's positions are split over two
 # to four workgroups: the first of them, ranges that fill no or several rounds of requests (512, 256 and 128 positions for heads
-# of 64, 128 and 256), last ranges that are short, empty ones' neighbours, the reference's 1024 (the maximum's start), one range
+# of 64, 128 and 256), last ranges that are short, two ranges a head (128 heads), 13 waves in the O projection (52 heads); few heads
+# of 128 and 256 past 1024, where P.V is a launch of its own
 @pytest.mark.parametrize(
     "heads,head,kv,positions",
     [(4, 64, 2, (128, 256, 300, 1022, 1023, 2047, 4500)), (4, 128, 4, (129, 255, 256, 511, 1023, 1024, 3000, 5000)),
-     (8, 128, 1, (256, 257, 700)), (2, 256, 1, (256, 512, 1500, 2600)), (128, 64, 128, (257, 1100))],
+     (8, 128, 1, (256, 257, 700)), (2, 256, 1, (256, 512, 1500, 2600)), (128, 64, 128, (257, 1100)),
+     (32, 128, 8, (1025, 2047, 4500)), (32, 256, 8, (1500, 2600)), (52, 128, 52, (300, 1100))],
 )
 def test_attention_of_long_contexts_in_one_launch(ctx, heads, head, kv, positions):
     """The fused schedule's attention in ranges, put together by the O projection, against the reference schedule's separate
