@@ -503,11 +503,13 @@ int launch(awq_ctx* ctx, GemvParams& p, int grid_y, const char* what) {
     const size_t lds = (size_t)p.C * 68;  // activations + per-chunk constant
     if constexpr (KIND == KIND_SINGLE && !ROPE && R == 1 && (W == 8 || W == 10 || W == 13 || W == 16)) {  // (partial-sum input comes with K <= 8192)
         if (p.xpart) {
-            auto kernel = p.xstat ? gemv_int4_kernel<W, R, D, KIND, false, false, PARTS_SOFTMAX, SPLIT>
-                                  : gemv_int4_kernel<W, R, D, KIND, false, false, PARTS_SUM, SPLIT>;
-            if (int r = ensure_lds_limit(ctx, (const void*)kernel, lds, what)) return r;
-            awq_launch(ctx, kernel, grid, dim3(W * 64), lds, p);
-            return awq_check_launch(what);
+            auto go = [&](auto kernel) {
+                if (int r = ensure_lds_limit(ctx, (const void*)kernel, lds, what)) return r;
+                awq_launch(ctx, kernel, grid, dim3(W * 64), lds, p);
+                return awq_check_launch(what);
+            };
+            if (p.xstat) return go(gemv_int4_kernel<W, R, D, KIND, false, false, PARTS_SOFTMAX, SPLIT>);
+            if constexpr (W != 16) return go(gemv_int4_kernel<W, R, D, KIND, false, false, PARTS_SUM, SPLIT>);  // (16: K > 8192, or softmax parts)
         }
     }
     if (p.xpart) {
