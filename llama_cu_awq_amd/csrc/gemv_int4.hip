@@ -585,6 +585,7 @@ int dispatch(awq_ctx* ctx, GemvParams& p, int grid_y, const char* what, GemvPlan
     // wave halve the workgroups of a matrix that has few rows to begin with.
     const int tail = p.C & 63;
     const bool split2 = tail != 0 && tail <= 32 && plan.rows <= 2 && p.K <= 8192;
+    if (split2 && plan.waves > 8) plan.waves = 8;  // these forms have no workgroups of 16
     if constexpr (KIND == KIND_SINGLE) {
         // The workgroups of a single-matrix product are all resident at once, and the kernel takes as long as the
         // compute unit that holds the most of them.  Workgroups of 10 or 13 waves are taken where they make the count a
@@ -691,8 +692,9 @@ int awq_launch_matvec_int4_parts(awq_ctx* ctx, uint16_t* out, const float* part,
     p.xstat = stat;
     while ((1 << p.head_shift) < head_size) p.head_shift++;
     GemvPlan plan = plan_for(K, 1);
-    // Every workgroup stages all parts: workgroups of 16 waves where those of 8 would be two or more on a compute unit.  us a
-    // layer with 8 -> 16 waves: 70B shape, two ranges 99.3 -> 95.9, four 102.1 -> 97.6.
+    // Every workgroup stages all parts: workgroups of 16 waves where those of 8 would be two or more on a compute unit (and are
+    // not of a form, or put more evenly on the compute units by a size, that dispatch() chooses).  us a launch with 8 -> 16 waves:
+    // 8192 rows 14.9 -> 11.2, 4096 rows 5.9 -> 5.5; a token of 4 layers from position 600 334.4 -> 318.5, 163.5 -> 162.0.
     if (stat && div_up(N, 8) >= 2 * ctx->cus) plan.waves = 16;
     return dispatch<KIND_SINGLE, false>(ctx, p, 1, "gemv_int4_parts", plan);
 }
