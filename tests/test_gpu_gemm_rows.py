@@ -14,7 +14,7 @@ import pytest
 
 import llama_cu_awq_amd as A
 from llama_cu_awq_amd import synth
-from llama_cu_awq_amd._lib import lib
+from llama_cu_awq_amd._lib import QWeightC, lib
 from tests.helpers import f16, rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -144,6 +144,51 @@ def test_prefill_epilogues_against_token_by_token(ctx, small, parts):
             assert rel_l2(a[l][-3:], b[l][n - 3 : n]) <= 1e-2, l
 
 
+class _Plan(C.Structure):  # of the row forms: which, into how many parts K is split over workgroups, the time expected
+    _fields_ = [("form", C.c_int), ("parts", C.c_int), ("us", C.c_float)]
+
+
+_plan = lib["_Z18awq_plan_gemm_rowsiiiibb"]  # compute units, rows, K, columns / 64, may split, the parts stay apart
+_plan.argtypes, _plan.restype = [C.c_int] * 4 + [C.c_bool] * 2, _Plan
+_resid = lib["_Z21awq_launch_gemm_residP7awq_ctxPtPKtiiPK11awq_qweightiiPi"]
+_resid.argtypes = [C.c_void_p] * 3 + [C.c_int] * 2 + [C.POINTER(QWeightC)] + [C.c_int] * 2 + [C.POINTER(C.c_int)]
+_norm_parts = lib["_Z24awq_launch_rmsnorm_partsP7awq_ctxPtS1_PKtiiii"]
+_norm_parts.argtypes = [C.c_void_p] * 4 + [C.c_int] * 4
+
+
+# (rows, K, columns) by the parts that K is split into: every form that splits, single and ragged rows, columns that end in the
+# first piece of a thread, in its second and past both (more than 8192: read and written twice)
+LEFT = {2: [(1, 2048, 128), (257, 2048, 1024), (385, 3072, 4096), (129, 2048, 12288), (200, 4096, 12288)],
+        3: [(1, 3072, 128), (450, 3072, 384), (97, 2048, 8320), (150, 6144, 12288), (129, 6144, 9216)],
+        4: [(1, 4096, 128), (321, 4096, 384), (257, 4096, 2048), (33, 4096, 8320), (97, 4096, 12288)]}
+
+
+@pytest.mark.parametrize("perm", [0, 1])
+@pytest.mark.parametrize("M,K,N,parts", [(*shape, n) for n, shapes in LEFT.items() for shape in shapes])
+def test_parts_left_to_the_norm(ctx, M, K, N, parts, perm):
+    """A residual product whose parts the norm adds up, against the one whose parts meet in the launch (held against 64 bits
+    above) and the plain norm behind it.  Both round the same fp32 sum once: apart from its order, under 1e-6, they differ where
+    that crosses a rounding, one element in some thousand by 2^-11: 1e-4."""
+    key = synth.stream_key(59, M, K, N)
+    qw = A.QWeight.upload(ctx, *synth.make_qweight(key, K, N))
+    a = synth.normal_f16(synth.stream_key(key, "a"), M * K).reshape(M, K // 8, 8)
+    da, da_perm = (ctx.upload(np.ascontiguousarray(v).reshape(-1)) for v in (a, a[:, :, [0, 4, 1, 5, 2, 6, 3, 7]]))
+    x = synth.normal_f16(synth.stream_key(key, "x"), M * N)
+    norm = ctx.upload(synth.normal_f16(synth.stream_key(key, "n"), N, 1.0, 0.02))
+    outs = []
+    for split in (False, True):
+        dx, do, left = ctx.upload(x), ctx.zeros(M * N * 2), C.c_int(0)
+        if split:
+            assert _resid(ctx.h, dx.ptr, da_perm.ptr, K, M, C.byref(qw.c), K, N, C.byref(left)) == 0 and left.value == parts
+        else:
+            A.gemm_q(ctx, dx, N, da, K, M, qw, K, N, accum=True)
+        assert _norm_parts(ctx.h, do.ptr, dx.ptr, norm.ptr, N, M, perm, left.value) == 0
+        outs.append([f16(d.download(np.uint16)).reshape(M, N) for d in (dx, do)])
+    for got, want in zip(outs[1], outs[0]):
+        assert np.isfinite(want).all() and rel_l2(got, want) <= 1e-4
+        assert rel_l2(got[-1], want[-1]) <= 1e-3 and rel_l2(got[:, -8:], want[:, -8:]) <= 1e-3
+
+
 # (looked up through the library: the HIP runtime it is linked with)
 def _hip(name, *args):
     assert getattr(lib, name)(*args) == 0, name
@@ -187,15 +232,16 @@ def test_split_workspace_made_while_recording(ctx):
 
 
 def test_short_prefill_recorded_after_a_long_one():
-    """1100 rows by 4096 columns split no K, 37 do: what that takes is there before the short prompt is recorded."""
-    cfg = dict(dim=4096, hidden_dim=1024, n_layers=1, n_heads=32, n_kv_heads=4, vocab_size=512, seq_len=1152, rope_theta=10000.0)
+    """1100 rows by 4096 columns split no K, 37 do (QKV and gate/up, whose parts meet in the launch, and of the first of two
+    layers O and down, whose parts the norm adds up): what that takes is there before the short prompt is recorded."""
+    cfg = dict(dim=4096, hidden_dim=2048, n_layers=2, n_heads=32, n_kv_heads=4, vocab_size=512, seq_len=1152, rope_theta=10000.0)
     img = synth.make_model_image(cfg, seed=55, scale_mult=0.25)
     prompt = synth.prompt_tokens(55, 1137, cfg["vocab_size"])
     ctx = A.Context(0)
     t = A.Transformer(ctx, image=img)
 
     def caches():
-        return [t.download(name, cfg["seq_len"] * 512) for name in ("key_cache", "value_cache")]
+        return [t.download(name, n) for name, n in (("key_cache", 2 * cfg["seq_len"] * 512), ("value_cache", 2 * cfg["seq_len"] * 512), ("logits", 512))]
 
     stream, graph, runnable = C.c_void_p(lib.awq_ctx_stream(ctx.h)), C.c_void_p(), C.c_void_p()
     t.reset(prompt)
@@ -216,7 +262,11 @@ def test_short_prefill_recorded_after_a_long_one():
     want = caches()
     for got in recorded:
         for a, b in zip(got, want):
-            assert np.array_equal(a, b) and f16(b).reshape(-1, 512)[1100:1137].any(axis=1).all()
+            assert np.array_equal(a, b)
+        for b in want[:2]:
+            assert f16(b).reshape(2, -1, 512)[:, 1100:1137].any(axis=2).all()
+    for M, K in ((37, 4096), (37, 2048)):
+        assert _plan(256, M, K, 4096 // 64, True, True).parts > 1
     _hip("hipGraphExecDestroy", runnable)
     _hip("hipGraphDestroy", graph)
     t.close()
