@@ -363,3 +363,39 @@ def test_decode_scores_far_below_zero(ctx, heads, head, kv, size):
     for got in outs[1:]:
         for a, b in zip(got, outs[0]):
             assert np.isfinite(a).all() and rel_l2(a, b) <= 1e-3
+
+
+@pytest.mark.parametrize("heads,head,kv,pos", [(4, 64, 2, 300), (8, 128, 2, 700), (2, 256, 1, 900), (32, 128, 8, 2100), (4, 128, 4, 2100)])
+def test_rows_past_the_position_do_not_enter(ctx, heads, head, kv, pos):
+    """Loads past a range's end repeat its last row, and what lies behind the position (an earlier, longer conversation) is not
+    read: NaN there changes no bit.  NaN and infinities of the rows that count reach the logits, as in the reference schedule."""
+    seq, row = 2304, kv * head
+    cfg = dict(dim=heads * head, hidden_dim=256, n_layers=1, n_heads=heads, n_kv_heads=kv, vocab_size=512, seq_len=seq, rope_theta=10000.0)
+    t = A.Transformer(ctx, image=synth.make_model_image(cfg, seed=6))
+    rng = np.random.default_rng(pos)
+    rows = {name: rng.standard_normal((seq, row)).astype(np.float16) for name in ("key_cache", "value_cache")}
+
+    def logits(mode, graph, **changes):
+        for name, r in rows.items():
+            r = r.copy()
+            for at, value in changes.get(name, ()):
+                r[at] = value
+            t.buffer(name, seq * row * 2).write(r)
+        t.set_pos(pos, 7)
+        t.forward_logits(use_graph=graph, mode=mode)
+        ctx.sync()
+        return f16(t.download("logits", cfg["vocab_size"])).copy()
+
+    behind = slice(pos + 1, None)
+    for graph in (False, True):
+        want = logits(A.SCHEDULE_FUSED, graph)
+        assert np.isfinite(want).all()
+        for value in (np.nan, np.inf):
+            got = logits(A.SCHEDULE_FUSED, graph, key_cache=[(behind, value)], value_cache=[(behind, value)])
+            assert np.array_equal(got.view(np.uint16), want.view(np.uint16))
+    # a key that is NaN, and a value that is infinite, in the first range and in the last
+    for at in (3, pos - 1):
+        for change in (dict(key_cache=[((at, row - 1), np.nan)]), dict(value_cache=[((at, row - 1), np.inf)])):
+            for mode in (A.SCHEDULE_REFERENCE, A.SCHEDULE_FUSED):
+                assert not np.isfinite(logits(mode, False, **change)).any(), (at, change, mode)
+    t.close()
