@@ -27,7 +27,8 @@ struct awq_ctx {
     bool owns_stream;
     awq_launch_probe* probe;  // null outside awq_transformer_time_launches
     // Split-K workspace of the batched GEMMs (allocated on first use): fp32 partial tiles, then per-tile arrival counters
-    // (self-resetting).
+    // (self-resetting).  The tiles are used inside one launch, but for awq_launch_gemm_resid: it may leave its parts there for
+    // awq_launch_rmsnorm_parts, and no other product of the context may be launched between the two.
     float* gemm_part;
 };
 

@@ -236,7 +236,7 @@ __global__ __launch_bounds__(1024) void attn_pv_sliced_kernel(uint16_t* output, 
     }
 }
 
-// awq_attention_partial: P.V split over positions as well, so that every compute unit pulls whole
+// awq_attention_partial and long contexts of few heads: P.V split over positions as well, so that every compute unit pulls whole
 // cache lines.  A workgroup of 16 waves owns one head, one of `chunks` contiguous ranges of positions and one slice of
 // 64 value dimensions (128 bytes of every row: 8 lanes x 16 bytes); it computes the softmax statistics over ALL
 // positions from the fp16 scores (as every workgroup of the head does, in the same order, so they agree bit for bit),
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(1024) void attn_pv_partial_kernel(float* part, cons
     }
 }
 
-// Fused schedule, launch sizes above kAttnFusedMaxSeq: scores, softmax and P.V of one of `chunks` contiguous ranges of a head's
+// Fused schedule, launch sizes above kAttnFusedMaxSeq (but see awq_attention_takes_ranges): scores, softmax and P.V of one of `chunks` contiguous ranges of a head's
 // positions in a workgroup of 16 waves, one pass over its keys and values.  LP lanes (head_size / 8) share a position; each
 // such group of lanes keeps a running maximum, sum of exponentials and fp32 P.V of the positions it sees, the groups meet at
 // the end, and part[chunk][head * head_size + dim] with stat[head][chunk] = (maximum, sum) goes to the O projection, which
@@ -752,7 +752,7 @@ int awq_attention_partial_chunks(const awq_ctx* ctx, int num_heads, int head_siz
     return chunks;
 }
 
-// awq_attention_partial: scores, then P.V as fp32 partial sums over
+// awq_attention_partial and, where awq_attention_takes_ranges says no, the fused schedule: scores, then P.V as fp32 partial sums over
 // `*chunks_out` ranges of positions, part[chunk][num_heads * head_size]; the consumer adds the chunks up in order and
 // rounds to fp16.  part must hold kAttnMaxChunks * num_heads * head_size floats.
 int awq_launch_attention_partial(awq_ctx* ctx, float* part, int* chunks_out, const uint16_t* q, const uint16_t* key_cache,

@@ -99,9 +99,10 @@ __device__ __forceinline__ void load_x(XPieces<NORM, pieces_for(W)>& xr, const X
     }
 }
 
-// The PARTS form of load_x: the activation vector arrives as up to kMaxParts fp32 partial sums per element (the
-// chunks of the position-split attention); their sum, added in part order and rounded to fp16 once, is x.  The loads
-// are requested here, ahead of the packed weights; combine_x turns them into the pieces stage_x takes.
+// The PARTS forms of load_x: the activation vector arrives as up to kMaxParts fp32 values per element (the chunks or ranges of
+// the position-split attention); their sum in part order, PARTS_SOFTMAX: each times exp(its maximum - the largest) / (the whole
+// sum), rounded to fp16 once, is x.  The loads are requested here, ahead of the packed weights; combine_x turns them into the
+// pieces stage_x takes.
 constexpr int part_pieces_for(int waves) { return waves >= 16 ? 1 : XP; }  // of up to 8192 elements
 
 template <int NP>

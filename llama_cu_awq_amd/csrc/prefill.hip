@@ -788,8 +788,8 @@ int awq_launch_gemm_single(awq_ctx* ctx, uint16_t* out, long long ldo, const uin
 
 int awq_launch_rmsnorm_rows(awq_ctx* ctx, uint16_t* o, const uint16_t* x, const uint16_t* w, int size, int M, int perm);
 
-// x += A . W, or (parts > 0) its partial sums in ctx->gemm_part, [part][M][N], for awq_launch_rmsnorm_parts to add to x: where
-// K is split, parts that meet in the launch cost it 6 to 8 us (written through, counted in, read back).  7B shape, us with
+// x += A . W, or (parts > 0) its partial sums in ctx->gemm_part, [part][M][N], for awq_launch_rmsnorm_parts to add to x (with no
+// other product of the context in between: its parts may take the same place).  Where K is split, parts that meet in the launch cost it 6 to 8 us (written through, counted in, read back).  7B shape, us with
 // the parts in the launch -> left to the norm: 37 tokens O 14.2 -> 9.9, down 20.4 -> 16.7 (norm 4.0 -> 4.8), 512 tokens down
 // 67 -> 55 (norm 5.1 -> 9.1).
 int awq_launch_gemm_resid(awq_ctx* ctx, uint16_t* x, const uint16_t* A, int lda, int M, const awq_qweight* w, int K, int N, int* parts) {

@@ -496,7 +496,7 @@ def test_attention(ctx, heads, head, kv_mul, pos, max_seq):
      (8, 128, 2, 9000, 16384), (64, 128, 8, 1500, 2048)],  # the last: Llama-2-70B's heads (8 share a KV head), K = 8192 into the O projection
 )
 def test_attention_split_over_positions_then_o_projection(ctx, heads, head, kv_mul, pos, max_seq):
-    """The long-context form of the fused schedule: P.V as fp32 partial sums per range of positions, added up and
+    """The two launchers for long contexts: P.V as fp32 partial sums per range of positions, added up and
     rounded to fp16 inside the O projection's staging.  The rounded sum of the partials must be the attention output
     (same probabilities, only the fp32 order of the sum over positions differs), and the product taken from the
     partials must be the product of that vector."""

@@ -138,13 +138,13 @@ def test_longer_prompt_while_another_stream_is_recorded(ctx):
         assert np.array_equal(a, b)
 
 
-# 128-wide heads and a long context, in one call, in two and token by token (there the position-split attention from 1024
-# positions on).
+# 128-wide heads and a long context, in one call, in two and token by token (there attention in ranges of positions
+# past 256, and as two launches past 1280).
 CFG_LONG2K = dict(dim=256, hidden_dim=512, n_layers=2, n_heads=2, n_kv_heads=2, vocab_size=512, seq_len=2176, rope_theta=10000.0)
 
 
-# the same with grouped queries: four heads share one KV head (the position-split attention and the single QKV launch
-# with fewer K and V rows, at long context)
+# the same with grouped queries: four heads share one KV head (those forms and the single QKV launch with fewer K and V
+# rows, at long context)
 CFG_LONG2K_GQA = dict(dim=512, hidden_dim=512, n_layers=2, n_heads=4, n_kv_heads=1, vocab_size=512, seq_len=2176, rope_theta=10000.0)
 
 
