@@ -370,15 +370,15 @@ __global__ __launch_bounds__(1024) void attn_pv_partial_kernel(float* part, cons
     }
 }
 
-// Fused schedule, launch sizes above kAttnFusedMaxSeq (but see awq_attention_takes_ranges): scores, softmax and P.V of one of `chunks` contiguous ranges of a head's
-// positions in a workgroup of 16 waves, one pass over its keys and values.  LP lanes (head_size / 8) share a position; each
-// such group of lanes keeps a running maximum, sum of exponentials and fp32 P.V of the positions it sees, the groups meet at
-// the end, and part[chunk][head * head_size + dim] with stat[head][chunk] = (maximum, sum) goes to the O projection, which
-// puts the ranges on one scale while it stages its input and rounds to fp16 there (the reference's rounding point;
-// gpu_kernels.h:368-451).  Scores are rounded to fp16 as the reference does and left in att; the probability, which the
-// reference rounds to fp16 after the division by the row's sum, stays fp32.  The maximum starts below every score: from the 0
-// that the reference starts at below 1024 positions, scores between -89 and -103 would leave sums so small that their reciprocal
-// is infinite.
+// Fused schedule, launch sizes above kAttnFusedMaxSeq (but see awq_attention_takes_ranges): scores, softmax and P.V of one of
+// `chunks` contiguous ranges of a head's positions in a workgroup of 16 waves, one pass over its keys and values.  LP lanes
+// (head_size / 8) share a position; each such group of lanes keeps a running maximum, sum of exponentials and fp32 P.V of the
+// positions it sees, the groups meet at the end, and part[chunk][head * head_size + dim] with stat[head][chunk] = (maximum, sum)
+// goes to the O projection, which puts the ranges on one scale while it stages its input and rounds to fp16 there (the
+// reference's rounding point; gpu_kernels.h:368-451).  Scores are rounded to fp16 as the reference does and left in att; the
+// probability, which the reference rounds to fp16 after the division by the row's sum, stays fp32.  The maximum starts below every
+// score: from the 0 that the reference starts at below 1024 positions, scores between -89 and -103 would leave sums so small
+// that their reciprocal is infinite.
 // Bound by latency: launch, position word, one round trip for keys and values together, two reductions.  It replaces two
 // launches, scores and P.V (unsplit below 1024 positions; split over positions with the scores exchanged through memory above).
 // us a token, 4 layers, two launches -> one: 7B shape, position 300 167.5 -> 163.8, 700 172.5 -> 168.5, 2000 188.5 -> 181.5;
