@@ -30,8 +30,8 @@ HBM_PEAK = 8.0e12  # MI355X published HBM3E bandwidth, bytes/s
 # from the rocprofv3 summaries committed under profiles/: the table rows of the kernels named here.
 TRACE_MD = "profiles/decode_7b_fused_kernel_trace.md"
 PMC_MD = "profiles/gemv_int4_ffn_7b_pmc.md"
-FFN_KERNEL = "gemv_int4_kernel<4, 1, 2, 2, true, false, false, 1>"  # norm-fused gate/up, the launch of the fused schedule
-GEMV_4096_KERNEL = "gemv_int4_kernel<8, 1, 2, 0, false, false, false, 1>"  # O projection and the 4096 x 4096 loops
+FFN_KERNEL = "gemv_int4_kernel<4, 1, 2, 2, true, false, 0, 1>"  # norm-fused gate/up, the launch of the fused schedule
+GEMV_4096_KERNEL = "gemv_int4_kernel<8, 1, 2, 0, false, false, 0, 1>"  # O projection and the 4096 x 4096 loops
 COPY_ROW = "__amd_rocclr_copyBuffer, 256 MiB"
 
 
