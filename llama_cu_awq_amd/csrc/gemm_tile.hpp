@@ -37,6 +37,9 @@ struct GemmParams {
     int rope_pos0;
     // FFN form: write the output with every 8 columns in the order (0,4,1,5,2,6,3,7), the order a permuted-A GEMM reads
     int out_perm;
+    // few-row form: 32-row tiles of A, which is in fragment order, and of the FFN form's output (0: rows, as out_perm says)
+    int a_tiles, out_tiles;
+    int few_per, few_extra;  // its K slices: quantisation groups of each, and how many of them have one more
     uint16_t* out[3];
     long long ldo[3];       // output row stride in elements
     long long out_off[3];   // element offset of output row 0 (KV cache: loff + pos0 * kv_dim)
@@ -50,6 +53,14 @@ __device__ __forceinline__ u32x4 permute8(const u32x4 v) {
     o[2] = __builtin_amdgcn_perm(v[3], v[1], 0x05040100u);
     o[3] = __builtin_amdgcn_perm(v[3], v[1], 0x07060302u);
     return o;
+}
+
+// Fragment order: activations as the few-row form's 32x32x16 products take them, the 64 lanes of an operand 1 KB in a row:
+// [column / 128][fragment][row / 32][half][row % 32][8 columns], where fragment f holds eighth f % 4 of quarters 2 (f / 4) and
+// 2 (f / 4) + 1 of the 128 columns (a lane's dwords of packed weights).  `tiles`: 32-row tiles of the block.
+__device__ __forceinline__ size_t fragment_offset(int row, int col, int tiles) {
+    const int f = ((col >> 6) & 1) * 4 + ((col >> 3) & 3);
+    return ((((size_t)(col >> 7) * 8 + f) * tiles + (row >> 5)) * 64 + ((col >> 5) & 1) * 32 + (row & 31)) * 8 + (col & 7);
 }
 
 // The constants of one quantisation group of a weight row.
@@ -132,3 +143,13 @@ int awq_gemm_rows_setup();  // once per device, with that device current
 awq_rows_plan awq_plan_gemm_rows(int cus, int M, int K, int groups, bool may_split, bool parts = false);
 int awq_launch_gemm_rows(awq_ctx* ctx, pf::GemmParams& p, int groups, int form, int ksplit, bool a_perm, const char* what);
 void awq_rows_form(int form, int* tile);  // rows, columns, K slices inside a workgroup
+
+// gemm_few.hip
+constexpr int kFewRows = 64;  // the most it takes
+struct awq_few_plan {
+    int units, ksplit;  // 32-row units of weights a workgroup; workgroups that share them, each with a part of K
+    float us;           // what the launch is expected to take
+};
+int awq_gemm_few_setup();  // once per device, with that device current
+awq_few_plan awq_plan_gemm_few(int cus, int M, int K, int N, bool may_split);
+int awq_launch_gemm_few(awq_ctx* ctx, pf::GemmParams& p, int N, const awq_few_plan& plan, const char* what);

@@ -368,15 +368,18 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(uint16_t* x, const uint
 // o[m] = half(x[m] * (rsqrt(mean(x[m]^2) + 1e-5) * w))  (gpu_kernels.h:72-105, one workgroup per token row).
 // 16-byte pieces; up to 4 per thread stay in registers between the two passes (rows of up to 8192), longer rows
 // re-read the rest.
-// perm: every 8 outputs are stored in the order (0,4,1,5,2,6,3,7) (what a permuted-A GEMM reads).
-__global__ __launch_bounds__(256) void rmsnorm_rows_kernel(uint16_t* o, const uint16_t* x, const uint16_t* weight, int size, int perm) {
+// perm: every 8 outputs are stored in the order (0,4,1,5,2,6,3,7) (what a permuted-A GEMM reads).  tiles: 32-row tiles of an
+// output in fragment order (the few-row GEMM's), 0: rows.
+__global__ __launch_bounds__(256) void rmsnorm_rows_kernel(uint16_t* o, const uint16_t* x, const uint16_t* weight, int size, int perm, int tiles) {
     __shared__ float red[4];
     constexpr int NP = 4;
     const int tid = threadIdx.x;
     const int n8 = size >> 3;
     const u32x4* xr = reinterpret_cast<const u32x4*>(x + (size_t)blockIdx.x * size);
     const u32x4* wr = reinterpret_cast<const u32x4*>(weight);
-    u32x4* orow = reinterpret_cast<u32x4*>(o + (size_t)blockIdx.x * size);
+    auto orow = [&](int e) -> u32x4& {
+        return *reinterpret_cast<u32x4*>(o + (tiles ? fragment_offset(blockIdx.x, e * 8, tiles) : (size_t)blockIdx.x * size + e * 8));
+    };
     u32x4 v[NP], w[NP];
 #pragma unroll
     for (int i = 0; i < NP; i++) {
@@ -419,8 +422,8 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(uint16_t* o, const ui
     ss = 1.0f / sqrtf(ss);
 #pragma unroll
     for (int i = 0; i < NP; i++)
-        if (i * 256 + tid < n8) orow[i * 256 + tid] = scale(v[i], w[i], ss);
-    for (int e = NP * 256 + tid; e < n8; e += 256) orow[e] = scale(xr[e], wr[e], ss);
+        if (i * 256 + tid < n8) orow(i * 256 + tid) = scale(v[i], w[i], ss);
+    for (int e = NP * 256 + tid; e < n8; e += 256) orow(e) = scale(xr[e], wr[e], ss);
 }
 
 // x[m] += the fp32 partial sums of a product over x's columns (added up in order, one rounding, as the product's own epilogue
@@ -428,14 +431,13 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(uint16_t* o, const ui
 // requested at once (4 columns a piece; two pieces, rows of up to 8192, stay in registers).
 template <int PARTS>
 __global__ __launch_bounds__(1024) void rmsnorm_parts_kernel(uint16_t* o, uint16_t* x, const float* part, const uint16_t* weight, int size,
-                                                           int perm) {
+                                                           int perm, int tiles) {
     __shared__ float red[16];
     constexpr int NP = 2;
     const int tid = threadIdx.x;
     const int n4 = size >> 2;
     u32x2* xr = reinterpret_cast<u32x2*>(x + (size_t)blockIdx.x * size);
     const u32x2* wr = reinterpret_cast<const u32x2*>(weight);
-    u32x2* orow = reinterpret_cast<u32x2*>(o + (size_t)blockIdx.x * size);
     const f32x4* pr = reinterpret_cast<const f32x4*>(part + (size_t)blockIdx.x * size);
     const size_t stride = (size_t)gridDim.x * n4;  // from one part to the next
     struct Piece {
@@ -482,7 +484,7 @@ __global__ __launch_bounds__(1024) void rmsnorm_parts_kernel(uint16_t* o, uint16
             r[0] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
             r[1] = __builtin_amdgcn_perm(hi, lo, 0x07060302u);
         }
-        orow[e] = r;
+        *reinterpret_cast<u32x2*>(o + (tiles ? fragment_offset(blockIdx.x, e * 4 & ~7, tiles) + (e & 1) * 4 : (size_t)blockIdx.x * size + e * 4)) = r;
     };
     Piece v[NP];
 #pragma unroll
@@ -611,6 +613,7 @@ int awq_gemm_device_setup(int device) {
             }
         }
         if (int r = awq_gemm_rows_setup()) return r;
+        if (int r = awq_gemm_few_setup()) return r;
         g_gemm_lds_raised[device] = true;
     }
     if (!g_scratch_ptr[device]) {
@@ -786,7 +789,25 @@ int awq_launch_gemm_single(awq_ctx* ctx, uint16_t* out, long long ldo, const uin
     return launch_gemm(ctx, p, N / pf::BN, "gemm_int4", a_perm, static_ws);
 }
 
-int awq_launch_rmsnorm_rows(awq_ctx* ctx, uint16_t* o, const uint16_t* x, const uint16_t* w, int size, int M, int perm);
+int awq_launch_rmsnorm_rows(awq_ctx* ctx, uint16_t* o, const uint16_t* x, const uint16_t* w, int size, int M, int perm, int tiles);
+
+// Whether a pass of M rows goes through a layer in the few-row form: its four products hand each other activations in
+// fragment order, so that they are weighed together.  Inside a pass they take 0.82 of the sum of their estimates where the row
+// forms take 1.04 of theirs.  Four layers and the logits, us, row forms -> few-row form, at 4, 32, 33 and 64 rows: dim 2048 by 5632
+// 245 -> 207, 252 -> 216, 256 -> 230, 261 -> 238; 4096 by 11008 339 -> 305, 351 -> 319, 396 -> 349, 409 -> 369; 6656 by 17920 574 ->
+// 530, 619 -> 573, 702 -> 634, 728 -> 675; but 8192 by 28672 649 -> 633, 703 -> 701, 761 -> 811, 793 -> 874.
+bool awq_prefill_takes_few(awq_ctx* ctx, int M, int dim, int kv_dim, int hidden) {
+    if (M > kFewRows) return false;
+    const auto few = [&](int K, int N, bool split) { return awq_plan_gemm_few(ctx->cus, M, K, N, split).us; };
+    const auto rows = [&](int K, int N, bool single) {
+        const float us = route_gemm(ctx->cus, M, K, N / pf::BN, single).us;
+        if (!single) return us;
+        const awq_rows_plan parts = awq_plan_gemm_rows(ctx->cus, M, K, N / 64, true, true);
+        return parts.form >= 0 && parts.us < us ? parts.us : us;
+    };
+    return 0.82f * (few(dim, dim + 2 * kv_dim, false) + few(dim, dim, true) + few(dim, 2 * hidden, false) + few(hidden, dim, true)) <
+           rows(dim, dim + 2 * kv_dim, false) + rows(dim, dim, true) + rows(dim, 2 * hidden, false) + rows(hidden, dim, true);
+}
 
 // x += A . W, or (parts > 0) its partial sums in ctx->gemm_part, [part][M][N], for awq_launch_rmsnorm_parts to add to x (with no
 // other product of the context in between: its parts may take the same place).  Where K is split, parts that meet in the launch cost it 6 to 8 us (written through, counted in, read back).  7B shape, us with
@@ -808,17 +829,37 @@ int awq_launch_gemm_resid(awq_ctx* ctx, uint16_t* x, const uint16_t* A, int lda,
     return awq_launch_gemm_single(ctx, x, N, A, lda, M, w, K, N, 1, false, true);
 }
 
-// o = RMSNorm of x, M rows of `size`; parts > 0: after adding those of the last awq_launch_gemm_resid to x
-int awq_launch_rmsnorm_parts(awq_ctx* ctx, uint16_t* o, uint16_t* x, const uint16_t* w, int size, int M, int perm, int parts) {
+// The same in the few-row form, A in fragment order.
+int awq_launch_gemm_few_resid(awq_ctx* ctx, uint16_t* x, const uint16_t* A, int M, const awq_qweight* w, int K, int N, int* parts) {
+    pf::GemmParams p;
+    gemm_common(p, A, K, M, K, pf::EPI_RESID);
+    set_mat(p, 0, w, N, x, N, 0);
+    awq_few_plan plan = awq_plan_gemm_few(ctx->cus, M, K, N, true);
+    if (plan.ksplit > 1 && awq_reserve_gemm_workspace(ctx) != AWQ_OK) plan = awq_plan_gemm_few(ctx->cus, M, K, N, false);
+    *parts = 0;
+    if (plan.ksplit > 1) {
+        p.epi = pf::EPI_PART;
+        p.part = ctx->gemm_part;
+        *parts = plan.ksplit;
+    }
+    return awq_launch_gemm_few(ctx, p, N, plan, "gemm_few");
+}
+
+// o = RMSNorm of x, M rows of `size`; parts > 0: after adding those of the last awq_launch_gemm_resid to x; tiles > 0: o in
+// fragment order
+int awq_launch_rmsnorm_parts(awq_ctx* ctx, uint16_t* o, uint16_t* x, const uint16_t* w, int size, int M, int perm, int parts, int tiles) {
     const float* part = ctx->gemm_part;
     switch (parts) {
-        case 0: return awq_launch_rmsnorm_rows(ctx, o, x, w, size, M, perm);
-        case 2: hipLaunchKernelGGL((pf::rmsnorm_parts_kernel<2>), dim3(M), dim3(1024), 0, ctx->stream, o, x, part, w, size, perm); break;
-        case 3: hipLaunchKernelGGL((pf::rmsnorm_parts_kernel<3>), dim3(M), dim3(1024), 0, ctx->stream, o, x, part, w, size, perm); break;
-        case 4: hipLaunchKernelGGL((pf::rmsnorm_parts_kernel<4>), dim3(M), dim3(1024), 0, ctx->stream, o, x, part, w, size, perm); break;
+        case 0: return awq_launch_rmsnorm_rows(ctx, o, x, w, size, M, perm, tiles);
+        case 2: hipLaunchKernelGGL((pf::rmsnorm_parts_kernel<2>), dim3(M), dim3(1024), 0, ctx->stream, o, x, part, w, size, perm, tiles); break;
+        case 3: hipLaunchKernelGGL((pf::rmsnorm_parts_kernel<3>), dim3(M), dim3(1024), 0, ctx->stream, o, x, part, w, size, perm, tiles); break;
+        case 4: hipLaunchKernelGGL((pf::rmsnorm_parts_kernel<4>), dim3(M), dim3(1024), 0, ctx->stream, o, x, part, w, size, perm, tiles); break;
         default: awq_set_error("rmsnorm: %d parts", parts); return AWQ_ERR_ARG;
     }
     return awq_check_launch("rmsnorm_parts");
+}
+int awq_launch_rmsnorm_parts(awq_ctx* ctx, uint16_t* o, uint16_t* x, const uint16_t* w, int size, int M, int perm, int parts) {
+    return awq_launch_rmsnorm_parts(ctx, o, x, w, size, M, perm, parts, 0);
 }
 
 int awq_launch_rope_rows(awq_ctx* ctx, uint16_t* q, uint16_t* kcache_layer, int nh, int nkv, int hs, int pos0, float theta, int M,
@@ -827,7 +868,7 @@ int awq_launch_rope_rows(awq_ctx* ctx, uint16_t* q, uint16_t* kcache_layer, int 
 // q rows and K, V cache rows of M positions from pos0 on, q and k rotated
 int awq_launch_gemm_qkv(awq_ctx* ctx, uint16_t* q, uint16_t* kcache_layer, uint16_t* vcache_layer, const uint16_t* A, int lda, int M,
                         const awq_qweight* qw, const awq_qweight* kw, const awq_qweight* vw, int K, int Nq, int Nkv, int head_size,
-                        const float2* rope, float theta, int pos0, bool a_perm) {
+                        const float2* rope, float theta, int pos0, bool a_perm, bool few) {
     pf::GemmParams p;
     gemm_common(p, A, lda, M, K, pf::EPI_QKV);
     bool rotated = rope != nullptr && (head_size == 64 || head_size == 128 || head_size == 256);
@@ -837,17 +878,20 @@ int awq_launch_gemm_qkv(awq_ctx* ctx, uint16_t* q, uint16_t* kcache_layer, uint1
     set_mat(p, 0, qw, Nq, q, Nq, 0);
     set_mat(p, 1, kw, Nkv, kcache_layer, Nkv, (long long)pos0 * Nkv);
     set_mat(p, 2, vw, Nkv, vcache_layer, Nkv, (long long)pos0 * Nkv);
-    if (int r = launch_gemm(ctx, p, (Nq + 2 * Nkv) / pf::BN, "gemm_int4_qkv", a_perm, false, &rotated)) return r;
+    if (few) {
+        if (int r = awq_launch_gemm_few(ctx, p, Nq + 2 * Nkv, awq_plan_gemm_few(ctx->cus, M, K, Nq + 2 * Nkv, false), "gemm_few_qkv")) return r;
+    } else if (int r = launch_gemm(ctx, p, (Nq + 2 * Nkv) / pf::BN, "gemm_int4_qkv", a_perm, false, &rotated)) return r;
     return rotated ? AWQ_OK : awq_launch_rope_rows(ctx, q, kcache_layer, Nq / head_size, Nkv / head_size, head_size, pos0, theta, M, rope);
 }
 
 int awq_launch_gemm_ffn(awq_ctx* ctx, uint16_t* hb, const uint16_t* A, int lda, int M, const awq_qweight* gate_w,
-                        const awq_qweight* up_w, int K, int N, bool a_perm, bool out_perm) {
+                        const awq_qweight* up_w, int K, int N, bool a_perm, bool out_perm, bool few) {
     pf::GemmParams p;
     gemm_common(p, A, lda, M, K, pf::EPI_FFN);
     p.out_perm = out_perm;
     set_mat(p, 0, gate_w, N, hb, N, 0);
     set_mat(p, 1, up_w, N, hb, N, 0);
+    if (few) return awq_launch_gemm_few(ctx, p, 2 * N, awq_plan_gemm_few(ctx->cus, M, K, 2 * N, false), "gemm_few_ffn");
     return launch_gemm(ctx, p, N / 64, "gemm_int4_ffn", a_perm);
 }
 
@@ -856,8 +900,8 @@ int awq_launch_embed_rows(awq_ctx* ctx, uint16_t* x, const uint16_t* table, int 
     return awq_check_launch("embed_rows");
 }
 
-int awq_launch_rmsnorm_rows(awq_ctx* ctx, uint16_t* o, const uint16_t* x, const uint16_t* w, int size, int M, int perm) {
-    hipLaunchKernelGGL(pf::rmsnorm_rows_kernel, dim3(M), dim3(256), 0, ctx->stream, o, x, w, size, perm);
+int awq_launch_rmsnorm_rows(awq_ctx* ctx, uint16_t* o, const uint16_t* x, const uint16_t* w, int size, int M, int perm, int tiles) {
+    hipLaunchKernelGGL(pf::rmsnorm_rows_kernel, dim3(M), dim3(256), 0, ctx->stream, o, x, w, size, perm, tiles);
     return awq_check_launch("rmsnorm_rows");
 }
 

@@ -11,9 +11,8 @@
 #include <atomic>
 
 #include "common.hpp"
+#include "gemm_tile.hpp"
 
-typedef _Float16 h16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 namespace pfa {
@@ -30,9 +29,11 @@ __device__ __forceinline__ h16x8 read_tr8(const uint16_t* p0, const uint16_t* p1
 // One query by one wave, for blocks with values that are not finite: only the keys it sees take part.  Bound by the round trips
 // of its loads; with 16 bytes of a key a lane and 8 value rows in flight, a 2000-token pass over two 7B layers whose every value
 // row is infinite somewhere takes 12.7 ms (46.6 with 2 bytes at a time; 1.9 where all values are finite).
-template <int HS>
-__device__ __forceinline__ void attn_row(uint16_t* out, const uint16_t* q, const uint16_t* kh, const uint16_t* vh, size_t kv_dim, int keys,
-                                         float alpha, int out_perm) {
+// FRAG: `out` is the whole block in fragment order (gemm_tile.hpp) of `tiles` 32-row tiles, in which the query's columns are those
+// of row `row` from `col0` on.
+template <int HS, bool FRAG>
+__device__ __forceinline__ void attn_row(uint16_t* out, const uint16_t* q, const uint16_t* kh, const uint16_t* vh, size_t kv_dim,
+                                         int keys, float alpha, int out_perm, int row, int col0, int tiles) {
     constexpr int D = HS / 64;
     const int lane = threadIdx.x & 63;
     float o[D], m = -INFINITY, l = 0.0f;
@@ -80,7 +81,9 @@ __device__ __forceinline__ void attn_row(uint16_t* out, const uint16_t* q, const
     }
     const int at = out_perm ? (lane & 56) | ((lane & 3) << 1) | ((lane >> 2) & 1) : lane;  // (0,4,1,5,2,6,3,7)
 #pragma unroll
-    for (int d = 0; d < D; d++) out[d * 64 + at] = float_to_half_bits(o[d] / l);
+    for (int d = 0; d < D; d++) {
+        out[FRAG ? pf::fragment_offset(row, col0 + d * 64 + at, tiles) : d * 64 + at] = float_to_half_bits(o[d] / l);
+    }
 }
 
 // A workgroup owns 32 * QW consecutive query tokens of one head: wave (qs, ks) takes the qs-th 32 queries and, of every
@@ -103,10 +106,10 @@ __device__ __forceinline__ void attn_row(uint16_t* out, const uint16_t* q, const
 // other's exponentials.  The form before this one held whole score rows in LDS (three passes, 32 queries per workgroup, at
 // most 1920 keys): 512 tokens x 32 heads 17.3 -> 13.2 us, 1920 tokens 97 us for the last 512 alone -> 63 us for all 2000;
 // heads of 64 and 256 dimensions ran without matrix cores (700 tokens x 32 heads of 64: 278 -> 12.3 us).
-template <int HS, int QW, int KW, int NSUB, int BUF>
+template <int HS, int QW, int KW, int NSUB, int BUF, bool FRAG>
 __global__ __launch_bounds__(QW * KW * 64, HS == 256 ? 1 : 2) void attn_kernel(uint16_t* out, const uint16_t* q, const uint16_t* key_cache,
                                                                              const uint16_t* value_cache, int num_heads, int kv_mul, int M,
-                                                                             int pos0, int out_perm) {
+                                                                             int pos0, int out_perm, int tiles) {
     constexpr int NT = QW * KW * 64;
     constexpr int TK = 32 * NSUB * KW;
     constexpr int KS = HS + 8, VS = HS + 16;  // halves per tile row: row strides of 4 and 8 dwords modulo the 32 banks
@@ -265,7 +268,8 @@ __global__ __launch_bounds__(QW * KW * 64, HS == 256 ? 1 : 2) void attn_kernel(u
     }
     if (__syncthreads_or((wild & 0x80008000u) != 0)) {
         for (int m = mq0 + wave; m < min(mq0 + 32 * QW, M); m += QW * KW)
-            attn_row<HS>(out + ((size_t)m * num_heads + h) * HS, q + ((size_t)m * num_heads + h) * HS, kh, vh, kv_dim, pos0 + m + 1, alpha, out_perm);
+            attn_row<HS, FRAG>(FRAG ? out : out + ((size_t)m * num_heads + h) * HS, q + ((size_t)m * num_heads + h) * HS, kh, vh, kv_dim, pos0 + m + 1, alpha, out_perm,
+                               m, h * HS, tiles);
         return;
     }
     {
@@ -339,20 +343,20 @@ __global__ __launch_bounds__(QW * KW * 64, HS == 256 ? 1 : 2) void attn_kernel(u
             } else {
                 r = u32x4{a0, a1, b0, b1};
             }
-            *reinterpret_cast<u32x4*>(orow + b * 32 + g * 8) = r;
+            *reinterpret_cast<u32x4*>(FRAG ? out + pf::fragment_offset(mq + l32, h * HS + lh * 8 + b * 32 + g * 8, tiles) : orow + b * 32 + g * 8) = r;
         }
 }
 
-template <int HS, int QW, int KW, int NSUB, int BUF>
+template <int HS, int QW, int KW, int NSUB, int BUF, bool FRAG>
 int launch(awq_ctx* ctx, uint16_t* out, const uint16_t* q, const uint16_t* kc, const uint16_t* vc, int nh, int kv_mul, int M, int pos0,
-           int out_perm) {
+           int out_perm, int tiles) {
     constexpr int TK = 32 * NSUB * KW;
-    constexpr int tiles = BUF * TK * (2 * HS + 24) * 2;
+    constexpr int staged = BUF * TK * (2 * HS + 24) * 2;
     constexpr int meet = (KW - 1) * QW * (HS / 2 + 2) * 256;
-    constexpr int lds = tiles > meet ? tiles : meet;
+    constexpr int lds = staged > meet ? staged : meet;
     static std::atomic<bool> raised[64];  // per device: the kernel may take more than the default 64 KB of LDS
     if (lds > 64 * 1024 && !(ctx->device < 64 && raised[ctx->device].load(std::memory_order_relaxed))) {
-        const hipError_t e = hipFuncSetAttribute((const void*)attn_kernel<HS, QW, KW, NSUB, BUF>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        const hipError_t e = hipFuncSetAttribute((const void*)attn_kernel<HS, QW, KW, NSUB, BUF, FRAG>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (e != hipSuccess) {
             awq_set_error("hipFuncSetAttribute(attn_prefill) failed: %s", hipGetErrorString(e));
             return AWQ_ERR_HIP;
@@ -360,16 +364,19 @@ int launch(awq_ctx* ctx, uint16_t* out, const uint16_t* q, const uint16_t* kc, c
         if (ctx->device < 64) raised[ctx->device].store(true, std::memory_order_relaxed);
     }
     const int nqb = div_up(M, 32 * QW), hpx = (nh + 7) / 8;
-    hipLaunchKernelGGL((attn_kernel<HS, QW, KW, NSUB, BUF>), dim3(8 * hpx * nqb), dim3(QW * KW * 64), lds, ctx->stream, out, q, kc, vc, nh,
-                       kv_mul, M, pos0, out_perm);
+    hipLaunchKernelGGL((attn_kernel<HS, QW, KW, NSUB, BUF, FRAG>), dim3(8 * hpx * nqb), dim3(QW * KW * 64), lds, ctx->stream, out, q, kc, vc, nh,
+                       kv_mul, M, pos0, out_perm, tiles);
     return awq_check_launch("attn_prefill");
 }
 
 }  // namespace pfa
 
+// tiles: 32-row tiles of an output in fragment order, 0: rows
 int awq_launch_attn_prefill(awq_ctx* ctx, uint16_t* out, const uint16_t* q, const uint16_t* kc, const uint16_t* vc, int nh, int hs,
-                            int kv_mul, int M, int pos0, int out_perm) {
-#define AWQ_FORM(HS, QW, KW, NSUB, BUF) return pfa::launch<HS, QW, KW, NSUB, BUF>(ctx, out, q, kc, vc, nh, kv_mul, M, pos0, out_perm)
+                            int kv_mul, int M, int pos0, int out_perm, int tiles) {
+#define AWQ_FORM(HS, QW, KW, NSUB, BUF)                                                                                      \
+    return tiles ? pfa::launch<HS, QW, KW, NSUB, BUF, true>(ctx, out, q, kc, vc, nh, kv_mul, M, pos0, out_perm, tiles)      \
+                 : pfa::launch<HS, QW, KW, NSUB, BUF, false>(ctx, out, q, kc, vc, nh, kv_mul, M, pos0, out_perm, 0)
     // Measured, us (128 queries x all keys | 64 queries x 2 key slices | 32 queries x 4 key slices, per workgroup):
     //   32 heads of 128: 512 tokens 16.9 | 13.2 | 14.1;  2000 tokens 62.6 | 68.5 | 99;  37 tokens 4.9 | 6.5 | 6.9, behind
     //   1500 cached ones 38 | 28 | 24;  64 heads: 650 tokens 24.9 | 26.0 | 36.6, 150 behind 650 24.2 | 18.8 | 22.5

@@ -41,14 +41,16 @@ int awq_sampler_run(awq_sampler* s, uint16_t* logits, int* tokens, volatile int*
 int awq_reserve_gemm_workspace(awq_ctx* ctx);
 int awq_launch_gemm_qkv(awq_ctx* ctx, uint16_t* q, uint16_t* kcache_layer, uint16_t* vcache_layer, const uint16_t* A, int lda, int M,
                         const awq_qweight* qw, const awq_qweight* kw, const awq_qweight* vw, int K, int Nq, int Nkv, int head_size,
-                        const float2* rope, float theta, int pos0, bool a_perm);
+                        const float2* rope, float theta, int pos0, bool a_perm, bool few);
 int awq_launch_gemm_ffn(awq_ctx* ctx, uint16_t* hb, const uint16_t* A, int lda, int M, const awq_qweight* gate_w,
-                        const awq_qweight* up_w, int K, int N, bool a_perm, bool out_perm);
+                        const awq_qweight* up_w, int K, int N, bool a_perm, bool out_perm, bool few);
 int awq_launch_embed_rows(awq_ctx* ctx, uint16_t* x, const uint16_t* table, int dim, const int* tokens, int pos0, int M);
 int awq_launch_gemm_resid(awq_ctx* ctx, uint16_t* x, const uint16_t* A, int lda, int M, const awq_qweight* w, int K, int N, int* parts);
-int awq_launch_rmsnorm_parts(awq_ctx* ctx, uint16_t* o, uint16_t* x, const uint16_t* w, int size, int M, int perm, int parts);
+int awq_launch_gemm_few_resid(awq_ctx* ctx, uint16_t* x, const uint16_t* A, int M, const awq_qweight* w, int K, int N, int* parts);
+bool awq_prefill_takes_few(awq_ctx* ctx, int M, int dim, int kv_dim, int hidden);
+int awq_launch_rmsnorm_parts(awq_ctx* ctx, uint16_t* o, uint16_t* x, const uint16_t* w, int size, int M, int perm, int parts, int tiles);
 int awq_launch_attn_prefill(awq_ctx* ctx, uint16_t* out, const uint16_t* q, const uint16_t* kc, const uint16_t* vc, int nh, int hs,
-                            int kv_mul, int M, int pos0, int out_perm);
+                            int kv_mul, int M, int pos0, int out_perm, int tiles);
 int awq_launch_set_pos(awq_ctx* ctx, int* pos_dev, volatile int* pos_host, int value);
 int awq_launch_copy_row(awq_ctx* ctx, uint16_t* dst, const uint16_t* src, int n);
 
@@ -905,14 +907,17 @@ int awq_transformer_prefill(awq_transformer* t, int n_tokens, int gen_token) {
         // The activations that feed a GEMM (xb, att, hb) are written with every 8 values in the order the packed weights
         // dequantise in, so that the GEMMs multiply them without reordering either operand; x, q and the KV cache
         // keep the natural order.
+        // Passes of few rows whose products take the few-row form have them in fragment order besides, `tiles` 32-row tiles.
         // The O and down products may leave their result as partial sums; the norm that follows adds them to x.
+        const bool few = awq_prefill_takes_few(ctx, M, dim, kv_dim, hidden);
+        const int tiles = few ? div_up(M, 32) : 0;
         int parts = 0;
         for (int l = 0; l < p.n_layers; l++) {
             const awq_layer_weights& L = t->layers[l];
             const long long loff = (long long)l * p.seq_len * kv_dim;
-            if ((r = awq_launch_rmsnorm_parts(ctx, t->pf_xb, t->pf_x, L.rms_att_weight, dim, M, 1, parts))) return r;
+            if ((r = awq_launch_rmsnorm_parts(ctx, t->pf_xb, t->pf_x, L.rms_att_weight, dim, M, 1, parts, tiles))) return r;
             if ((r = awq_launch_gemm_qkv(ctx, t->pf_q, t->s.key_cache + loff, t->s.value_cache + loff, t->pf_xb, dim, M, &L.wq_q, &L.wq_k,
-                                         &L.wq_v, dim, dim, kv_dim, hs, t->rope_table, p.rope_theta, pos0, true)))
+                                         &L.wq_v, dim, dim, kv_dim, hs, t->rope_table, p.rope_theta, pos0, true, few)))
                 return r;
             // Of the last layer only its K and V rows and the last token's way to the logits have a reader: one row goes
             // through the attention and then through the matrix-vector kernels.  ms a call, all rows -> one: 7B shape, 37
@@ -922,7 +927,7 @@ int awq_transformer_prefill(awq_transformer* t, int n_tokens, int gen_token) {
                 if (done + M < n_tokens) break;
                 if ((r = awq_launch_copy_row(ctx, t->s.x, t->pf_x + (size_t)(M - 1) * dim, dim))) return r;
                 if ((r = awq_launch_attn_prefill(ctx, t->s.xb, t->pf_q + (size_t)(M - 1) * dim, t->s.key_cache + loff,
-                                                 t->s.value_cache + loff, p.n_heads, hs, kv_mul, 1, pos0 + M - 1, 0)))
+                                                 t->s.value_cache + loff, p.n_heads, hs, kv_mul, 1, pos0 + M - 1, 0, 0)))
                     return r;
                 if ((r = awq_launch_matvec_int4(ctx, t->s.x, t->s.xb, &L.wq_o, dim, dim, 1, 1, -1, nullptr, nullptr, nullptr))) return r;
                 if ((r = awq_launch_ffn(ctx, t->s.hb, t->s.x, &L.wq_gate, &L.wq_up, dim, hidden, L.rms_ffn_weight, nullptr))) return r;
@@ -931,12 +936,16 @@ int awq_transformer_prefill(awq_transformer* t, int n_tokens, int gen_token) {
                 break;
             }
             if ((r = awq_launch_attn_prefill(ctx, t->pf_att, t->pf_q, t->s.key_cache + loff, t->s.value_cache + loff, p.n_heads, hs,
-                                             kv_mul, M, pos0, 1)))
+                                             kv_mul, M, pos0, 1, tiles)))
                 return r;
-            if ((r = awq_launch_gemm_resid(ctx, t->pf_x, t->pf_att, dim, M, &L.wq_o, dim, dim, &parts))) return r;
-            if ((r = awq_launch_rmsnorm_parts(ctx, t->pf_xb, t->pf_x, L.rms_ffn_weight, dim, M, 1, parts))) return r;
-            if ((r = awq_launch_gemm_ffn(ctx, t->pf_hb, t->pf_xb, dim, M, &L.wq_gate, &L.wq_up, dim, hidden, true, true))) return r;
-            if ((r = awq_launch_gemm_resid(ctx, t->pf_x, t->pf_hb, hidden, M, &L.wq_down, hidden, dim, &parts))) return r;
+            if ((r = few ? awq_launch_gemm_few_resid(ctx, t->pf_x, t->pf_att, M, &L.wq_o, dim, dim, &parts)
+                         : awq_launch_gemm_resid(ctx, t->pf_x, t->pf_att, dim, M, &L.wq_o, dim, dim, &parts)))
+                return r;
+            if ((r = awq_launch_rmsnorm_parts(ctx, t->pf_xb, t->pf_x, L.rms_ffn_weight, dim, M, 1, parts, tiles))) return r;
+            if ((r = awq_launch_gemm_ffn(ctx, t->pf_hb, t->pf_xb, dim, M, &L.wq_gate, &L.wq_up, dim, hidden, true, true, few))) return r;
+            if ((r = few ? awq_launch_gemm_few_resid(ctx, t->pf_x, t->pf_hb, M, &L.wq_down, hidden, dim, &parts)
+                         : awq_launch_gemm_resid(ctx, t->pf_x, t->pf_hb, hidden, M, &L.wq_down, hidden, dim, &parts)))
+                return r;
         }
         if (done + M == n_tokens) {
             // last token: final norm, classifier and the greedy sampler exactly as the decode path does them

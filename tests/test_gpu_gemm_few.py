@@ -1,0 +1,130 @@
+"""The few-row form of the batched int4 GEMM (prefills of up to 64 rows): activations in fragment order, K shared by the waves of a
+workgroup and by workgroups, against 64-bit products and against the token-by-token path."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import llama_cu_awq_amd as A
+from llama_cu_awq_amd import synth
+from llama_cu_awq_amd._lib import QWeightC, lib
+from tests.helpers import f16, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+class _Plan(C.Structure):  # 32-row units a workgroup, parts of K, the time expected
+    _fields_ = [("units", C.c_int), ("parts", C.c_int), ("us", C.c_float)]
+
+
+_plan = lib["_Z17awq_plan_gemm_fewiiiib"]  # compute units, rows, K, columns, may split
+_plan.argtypes, _plan.restype = [C.c_int] * 4 + [C.c_bool], _Plan
+_resid = lib["_Z25awq_launch_gemm_few_residP7awq_ctxPtPKtiPK11awq_qweightiiPi"]
+_resid.argtypes = [C.c_void_p] * 3 + [C.c_int] + [C.POINTER(QWeightC)] + [C.c_int] * 2 + [C.POINTER(C.c_int)]
+_norm_parts = lib["_Z24awq_launch_rmsnorm_partsP7awq_ctxPtS1_PKtiiii"]
+_norm_parts.argtypes = [C.c_void_p] * 4 + [C.c_int] * 4
+_takes_few = lib["_Z21awq_prefill_takes_fewP7awq_ctxiiii"]
+_takes_few.argtypes, _takes_few.restype = [C.c_void_p] + [C.c_int] * 4, C.c_bool
+
+
+def _fragments(a):
+    """[rows][K] in the order of gemm_tile.hpp's fragment_offset, each 8 columns as a packed dword unpacks; what no row fills is
+    not a number."""
+    M, K = a.shape
+    tiles = (M + 31) // 32
+    out = np.full((K // 128, 8, tiles, 2, 32, 8), np.nan, np.float16)
+    r, c = np.meshgrid(np.arange(M), np.arange(0, K, 8), indexing="ij")
+    f = ((c >> 6) & 1) * 4 + ((c >> 3) & 3)
+    out[c >> 7, f, r >> 5, (c >> 5) & 1, r & 31] = a.reshape(M, K // 8, 8)[:, :, [0, 4, 1, 5, 2, 6, 3, 7]]
+    return out.reshape(-1)
+
+
+# (rows, K, columns): edges of the row tiles; fewer groups than waves, one group more or less than a multiple of the waves, groups
+# that end in the middle of the four or eight that scales and zeros come in; a column tile that the last workgroup fills in part
+SHAPES = [(1, 256, 128), (31, 384, 256), (32, 1024, 2048), (33, 1152, 384), (37, 4096, 4096), (64, 896, 1280), (63, 2176, 640),
+          (5, 11008, 4096), (33, 11008, 4096), (64, 5248, 5120), (17, 4096, 24576), (48, 1024, 24576), (64, 8192, 16512)]
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
+def test_residual_product_against_fp64(ctx, M, K, N):
+    """fp16 weights and activations, fp32 sums, one rounding: apart from that rounding (2.1e-4 in the norm) sums differ by 1e-6.
+    Parts of K are added to x by the norm, one rounding too."""
+    key = synth.stream_key(61, M, K, N)
+    w, z, s = synth.make_qweight(key, K, N)
+    a = synth.normal_f16(synth.stream_key(key, "a"), M * K).reshape(M, K)
+    x = synth.normal_f16(synth.stream_key(key, "x"), M * N)
+    qw = A.QWeight.upload(ctx, w, z, s)
+    dense = synth.dequantize(w, z, s, K).astype(np.float32).astype(np.float16)
+    da, dx, do, left = ctx.upload(_fragments(a).view(np.uint16)), ctx.upload(x), ctx.zeros(M * N * 2), C.c_int(-1)
+    assert _resid(ctx.h, dx.ptr, da.ptr, M, C.byref(qw.c), K, N, C.byref(left)) == 0
+    plan = _plan(256, M, K, N, True)
+    assert left.value == (0 if plan.parts == 1 else plan.parts)
+    if left.value:
+        norm = ctx.upload(synth.normal_f16(synth.stream_key(key, "n"), N, 1.0, 0.02))
+        assert _norm_parts(ctx.h, do.ptr, dx.ptr, norm.ptr, N, M, 0, left.value) == 0
+    got = f16(dx.download(np.uint16)).reshape(M, N).astype(np.float64)
+    want = a.astype(np.float64) @ dense.astype(np.float64).T + x.astype(np.float64).reshape(M, N)
+    assert rel_l2(got, want) <= 4e-4
+    for at in (np.s_[-1], np.s_[0], np.s_[:, -8:], np.s_[:, :8]):
+        assert rel_l2(got[at], want[at]) <= 1e-3
+
+
+def test_every_form_is_taken():
+    taken = {(M > 32, p.units, p.parts > 1) for M, K, N in SHAPES for p in [_plan(256, M, K, N, True)]}
+    assert {t[:2] for t in taken} >= {(False, 1), (False, 2), (False, 3), (True, 1), (True, 2), (True, 3)} and any(t[2] for t in taken)
+
+
+def test_infinite_activation_stays_in_its_row(ctx):
+    M, K, N = 40, 1152, 384
+    key = synth.stream_key(62, M, K, N)
+    qw = A.QWeight.upload(ctx, *synth.make_qweight(key, K, N))
+    a = synth.normal_f16(synth.stream_key(key, "a"), M * K).reshape(M, K).copy()
+    a[39, K - 1] = np.inf  # the row that rows past the last read in its place
+    da, dx, left = ctx.upload(_fragments(a).view(np.uint16)), ctx.zeros(M * N * 2), C.c_int(-1)
+    assert _resid(ctx.h, dx.ptr, da.ptr, M, C.byref(qw.c), K, N, C.byref(left)) == 0 and left.value == 0
+    got = f16(dx.download(np.uint16)).reshape(M, N)
+    assert np.isfinite(got[:39]).all() and not np.isfinite(got[39]).all()
+
+
+MODELS = {"64": dict(dim=512, hidden_dim=1408, n_heads=8, n_kv_heads=2), "128": dict(dim=1024, hidden_dim=2816, n_heads=8, n_kv_heads=8),
+          "256": dict(dim=1536, hidden_dim=2048, n_heads=6, n_kv_heads=1), "wide": dict(dim=4096, hidden_dim=11008, n_heads=32, n_kv_heads=32)}
+
+
+@pytest.mark.parametrize("model", MODELS)
+def test_prefill_against_token_by_token(ctx, model):
+    """Passes at the edges of the row tiles, one behind another (the attention takes its forms for few and for many keys): cache rows
+    and logits of the token-by-token path within the tolerance of the batched one."""
+    m = MODELS[model]
+    cfg = dict(m, n_layers=2, vocab_size=512, seq_len=640, rope_theta=10000.0)
+    kv_dim = m["dim"] * m["n_kv_heads"] // m["n_heads"]
+    parts = (1, 31, 32, 33, 63, 64, 300, 40, 5)
+    n = sum(parts)
+    assert all(_takes_few(ctx.h, p, m["dim"], kv_dim, m["hidden_dim"]) for p in parts if p <= 64)
+    assert not _takes_few(ctx.h, 65, m["dim"], kv_dim, m["hidden_dim"])
+    img = synth.make_model_image(cfg, seed=63, scale_mult=0.25)
+    prompt = synth.prompt_tokens(63, n, cfg["vocab_size"])
+    t = A.Transformer(ctx, image=img)
+    size = 2 * cfg["seq_len"] * kv_dim
+
+    def state():
+        ctx.sync()
+        rows = [f16(t.download(name, size)).reshape(2, cfg["seq_len"], kv_dim)[:, :n].copy() for name in ("key_cache", "value_cache")]
+        return rows, f16(t.download("logits", cfg["vocab_size"])).copy()
+
+    t.reset(prompt)
+    for i in range(n):
+        t.forward(i == n - 1, use_graph=True)
+    want, want_logits = state()
+    t.reset(prompt)
+    for i, p in enumerate(parts):
+        t.prefill(p, gen_token=i == len(parts) - 1)
+    got, logits = state()
+    t.close()
+    for a, b in zip(got, want):
+        at = 0
+        for p in parts:
+            for l in range(2):
+                assert rel_l2(a[l, at : at + p], b[l, at : at + p]) <= 1e-2, (p, l)
+                assert rel_l2(a[l, at + p - 1], b[l, at + p - 1]) <= 2e-2, (p, l)
+            at += p
+    assert rel_l2(logits, want_logits) <= 1e-2
