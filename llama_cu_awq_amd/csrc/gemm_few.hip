@@ -10,16 +10,17 @@ struct FewForm {
     static constexpr int MT = MT_, NU = NU_;  // 32-row tiles; units of a workgroup
     static constexpr int WAVES = 8;
     static constexpr int SLOTS = 2;                      // quantisation groups of packed weights in a wave's ring
-    static constexpr int AD = 8;                         // activation fragments in flight (8 a group)
+    static constexpr int AD = MT <= 2 ? 8 : (MT * NU < 8 ? 4 : 2);  // activation fragments in flight (8 a group): what the registers hold
     static constexpr int W_BYTES = NU * 2048;            // a group of the workgroup's rows
     static constexpr int ROW = 36, TILE = 32 * ROW;      // floats of a sum's row and tile in LDS (rows padded: no bank conflicts)
-    static constexpr int RU = MT == 1 && NU % 2 == 0 ? 2 : 1, ROUNDS = NU / RU;  // units whose sums pass through LDS at a time
-    static constexpr int MEET = WAVES * RU * MT * TILE * 4;
+    // units and tiles whose sums pass through LDS at a time
+    static constexpr int RU = MT % 2 == 1 && NU % 2 == 0 ? 2 : 1, RT = MT % 2 == 0 ? 2 : 1, ROUNDS = (NU / RU) * (MT / RT);
+    static constexpr int MEET = WAVES * RU * RT * TILE * 4;
     static constexpr int RING = WAVES * SLOTS * W_BYTES;
     static constexpr int LDS = RING > (ROUNDS > 1 ? 2 : 1) * MEET ? RING : (ROUNDS > 1 ? 2 : 1) * MEET;
 };
 
-// C[m][n] = sum_k A[m][k] * half((q[n][k] - z) * s) of up to 64 rows: prefill.hip's product, rounding points and epilogues.  A
+// C[m][n] = sum_k A[m][k] * half((q[n][k] - z) * s) of up to 128 rows: prefill.hip's product, rounding points and epilogues.  A
 // workgroup of 8 waves owns NU units of 32 weight rows; its waves (and ksplit workgroups) share K, a contiguous run of
 // quantisation groups each, and their sums meet in LDS.
 //  * No wave reads what another one loaded, so there is no barrier before the sums meet and each wave waits for its own requests
@@ -33,7 +34,9 @@ struct FewForm {
 // each, with two waves a SIMD; about 4 us until the first activations and weights are there; 3 us until the sums have met.  More
 // waves of fewer registers, column groups that share A through L1, or weights left in cache change nothing.
 // Measured, us, the row forms -> this one: 7B shape, 37 rows QKV 17.9 -> 15.6, O 9.5 -> 8.5, gate/up 30.3 -> 21.5, down 16.5 ->
-// 14.5; 64 rows gate/up 30.2 -> 22.4.
+// 14.5; 64 rows gate/up 30.2 -> 22.4.  96 rows, from memory, QKV 26.9 -> 20.0, O 12.3 -> 10.2, 13824 columns of 5120 35.9 -> 24.5;
+// 128 rows QKV 27.8 -> 23.0, 13824 of 5120 36.3 -> 28.0, but gate/up 42.2 -> 44.2: two rounds of workgroups, since three units a workgroup
+// would need more registers than there are.
 // KIND: EPI_QKV, EPI_FFN (out in fragment order), or EPI_STORE for the single-matrix forms (p.epi says which).
 template <class F, int KIND>
 __global__ __launch_bounds__(F::WAVES * 64, 2) void gemm_few_kernel(const GemmParams p) {
@@ -41,7 +44,7 @@ __global__ __launch_bounds__(F::WAVES * 64, 2) void gemm_few_kernel(const GemmPa
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_bytes[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int first = (int)blockIdx.x * NU, ks = (int)blockIdx.z, m0 = (int)blockIdx.y * (MT * 32);
+    const int first = (int)blockIdx.x * NU, ks = (int)blockIdx.z;
 
     // A unit is 32 weight rows, two runs of 16 whose results meet in the epilogue: consecutive rows (single matrices, V), the gate
     // and up rows of the same indices (FFN), or the two halves of rotation pairs (Q and K with RoPE).
@@ -106,8 +109,8 @@ __global__ __launch_bounds__(F::WAVES * 64, 2) void gemm_few_kernel(const GemmPa
                 dma16(wu[u][b] + at, off, ring + slot * F::W_BYTES + u * 2048 + b * 1024);
     };
     // rows past M are computed, never stored: their lanes read the last row's line
-    const uint32_t a_lane = (uint32_t)lane * 16, a_last = (uint32_t)((lane & 32) + min(lane & 31, p.M - 1 - m0 - (MT - 1) * 32)) * 16;
-    const uint8_t* const abase = reinterpret_cast<const uint8_t*>(p.A) + (size_t)blockIdx.y * (MT * 1024);
+    const uint32_t a_lane = (uint32_t)lane * 16, a_last = (uint32_t)((lane & 32) + min(lane & 31, p.M - 1 - (MT - 1) * 32)) * 16;
+    const uint8_t* const abase = reinterpret_cast<const uint8_t*>(p.A);
     h16x8 a[AD][MT];
     auto load_a = [&](int f, int k) {
         k += f >> 3;
@@ -203,17 +206,18 @@ __global__ __launch_bounds__(F::WAVES * 64, 2) void gemm_few_kernel(const GemmPa
 
     // ---- epilogue: the waves' sums pass through LDS, [wave][unit][tile][row][32 columns], and are added in K order.  A lane takes
     // four columns of both runs: consecutive ones, or (FFN) those whose results are neighbours in the order a packed dword has.
+    constexpr int TR = MT / F::RT;  // rounds of a unit
     float* lds = reinterpret_cast<float*>(lds_bytes);
     auto put = [&](int round) {
-        float* mine = lds + (round & 1) * (F::MEET / 4) + wave * F::RU * MT * F::TILE + r32 * F::ROW + half * 4;
+        float* mine = lds + (round & 1) * (F::MEET / 4) + wave * F::RU * F::RT * F::TILE + r32 * F::ROW + half * 4;
 #pragma unroll
         for (int u = 0; u < F::RU; u++)
 #pragma unroll
-            for (int i = 0; i < MT; i++)
+            for (int i = 0; i < F::RT; i++)
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
-                    const f32x16& v = acc[round * F::RU + u][i];
-                    *reinterpret_cast<f32x4*>(mine + (u * MT + i) * F::TILE + q * 8) = f32x4{v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]};
+                    const f32x16& v = acc[round / TR * F::RU + u][round % TR * F::RT + i];
+                    *reinterpret_cast<f32x4*>(mine + (u * F::RT + i) * F::TILE + q * 8) = f32x4{v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]};
                 }
     };
     auto pack4 = [](const float (&v)[4]) {
@@ -267,15 +271,15 @@ __global__ __launch_bounds__(F::WAVES * 64, 2) void gemm_few_kernel(const GemmPa
     for (int round = 0; round < F::ROUNDS; round++) {
         __syncthreads();
         if (round + 1 < F::ROUNDS) put(round + 1);
-        if (tid < F::RU * MT * 128) {
-            const int q = tid & 3, r = (tid >> 2) % (MT * 32), u = tid / (MT * 128);
-            const float* src = lds + (round & 1) * (F::MEET / 4) + (u * MT + (r >> 5)) * F::TILE + (r & 31) * F::ROW;
+        if (tid < F::RU * F::RT * 128) {
+            const int q = tid & 3, r = (tid >> 2) % (F::RT * 32), u = tid / (F::RT * 128);
+            const float* src = lds + (round & 1) * (F::MEET / 4) + (u * F::RT + (r >> 5)) * F::TILE + (r & 31) * F::ROW;
             float v[2][4];
 #pragma unroll
             for (int k = 0; k < W; k++) {
 #pragma unroll
                 for (int b = 0; b < 2; b++) {
-                    const float* at = src + k * F::RU * MT * F::TILE + b * 16;
+                    const float* at = src + k * F::RU * F::RT * F::TILE + b * 16;
                     f32x4 t;
                     if (KIND == EPI_FFN) {
                         const f32x2 lo = *reinterpret_cast<const f32x2*>(at + (q >> 1) * 8 + (q & 1) * 2), hi = *reinterpret_cast<const f32x2*>(at + (q >> 1) * 8 + (q & 1) * 2 + 4);
@@ -287,8 +291,8 @@ __global__ __launch_bounds__(F::WAVES * 64, 2) void gemm_few_kernel(const GemmPa
                     for (int e = 0; e < 4; e++) v[b][e] = k == 0 ? t[e] : v[b][e] + t[e];
                 }
             }
-            const int unit = first + round * F::RU + u;
-            if (unit < p.ntiles && m0 + r < p.M) finish(unit_of(unit), q, m0 + r, v);
+            const int unit = first + round / TR * F::RU + u, m = round % TR * F::RT * 32 + r;
+            if (unit < p.ntiles && m < p.M) finish(unit_of(unit), q, m, v);
         }
     }
 }
@@ -306,16 +310,18 @@ struct FewFormInfo {
 };
 // Measured over 128 .. 504 workgroups, 1 .. 8 groups a wave, weights from memory; 2.5 us besides for the launch itself.
 constexpr int kFewForms = 3;
-const FewFormInfo kFew[2][kFewForms] = {
-    {{1, 0.9f, 1.6f}, {2, 1.2f, 2.7f}, {3, 1.6f, 4.0f}},  // up to 32 rows
-    {{1, 1.6f, 2.2f}, {2, 2.4f, 3.4f}, {3, 3.3f, 4.7f}},  // up to 64
+const FewFormInfo kFew[4][kFewForms] = {  // by 32-row tiles (four by three units: more registers than there are)
+    {{1, 0.9f, 1.6f}, {2, 1.2f, 2.7f}, {3, 1.6f, 4.0f}},
+    {{1, 1.6f, 2.2f}, {2, 2.4f, 3.4f}, {3, 3.3f, 4.7f}},
+    {{1, 1.3f, 3.0f}, {2, 1.9f, 4.0f}, {3, 2.6f, 5.6f}},
+    {{1, 1.2f, 3.5f}, {2, 2.2f, 4.6f}, {0, 0.0f, 0.0f}},
 };
 constexpr int kFewMaxSplit = 4;
 
 template <int MT, int NU>
 void few_launch(awq_ctx* ctx, const pf::GemmParams& p) {
     using F = pf::FewForm<MT, NU>;
-    const dim3 grid(div_up(p.ntiles, NU), div_up(p.a_tiles, MT), p.ksplit), block(F::WAVES * 64);
+    const dim3 grid(div_up(p.ntiles, NU), 1, p.ksplit), block(F::WAVES * 64);
     if (p.epi == pf::EPI_QKV)
         hipLaunchKernelGGL((pf::gemm_few_kernel<F, pf::EPI_QKV>), grid, block, F::LDS, ctx->stream, p);
     else if (p.epi == pf::EPI_FFN)
@@ -339,7 +345,8 @@ hipError_t few_raise() {
 }  // namespace
 
 int awq_gemm_few_setup() {
-    hipError_t (*const raise[])() = {few_raise<1, 1>, few_raise<1, 2>, few_raise<1, 3>, few_raise<2, 1>, few_raise<2, 2>, few_raise<2, 3>};
+    hipError_t (*const raise[])() = {few_raise<1, 1>, few_raise<1, 2>, few_raise<1, 3>, few_raise<2, 1>,
+                                    few_raise<2, 2>, few_raise<2, 3>, few_raise<3, 1>, few_raise<3, 2>, few_raise<3, 3>, few_raise<4, 1>, few_raise<4, 2>};
     for (auto f : raise) {
         const hipError_t e = f();
         if (e != hipSuccess) {
@@ -355,7 +362,8 @@ awq_few_plan awq_plan_gemm_few(int cus, int M, int K, int N, bool may_split) {
     if (M > kFewRows || K < 256 || (K & 127) || (N & 31)) return best;
     const int groups = K / 128, units = N / 32;
     for (int i = 0; i < kFewForms; i++) {
-        const FewFormInfo& f = kFew[M > 32][i];
+        const FewFormInfo& f = kFew[div_up(M, 32) - 1][i];
+        if (!f.units) break;
         for (int s = 1; s <= (may_split ? kFewMaxSplit : 1); s++) {
             const size_t part = s == 1 ? 0 : (size_t)s * M * N * sizeof(float);
             if (s > 1 && (part > kPartBytes || groups < 8 * s)) break;
@@ -375,13 +383,18 @@ int awq_launch_gemm_few(awq_ctx* ctx, pf::GemmParams& p, int N, const awq_few_pl
     p.out_tiles = p.a_tiles;
     p.few_per = p.sh / (8 * plan.ksplit);
     p.few_extra = p.sh % (8 * plan.ksplit);
-    switch ((p.M > 32) * 4 + plan.units) {
-        case 1: few_launch<1, 1>(ctx, p); break;
-        case 2: few_launch<1, 2>(ctx, p); break;
-        case 3: few_launch<1, 3>(ctx, p); break;
-        case 5: few_launch<2, 1>(ctx, p); break;
-        case 6: few_launch<2, 2>(ctx, p); break;
-        case 7: few_launch<2, 3>(ctx, p); break;
+    switch (p.a_tiles * 4 + plan.units) {
+        case 5: few_launch<1, 1>(ctx, p); break;
+        case 6: few_launch<1, 2>(ctx, p); break;
+        case 7: few_launch<1, 3>(ctx, p); break;
+        case 9: few_launch<2, 1>(ctx, p); break;
+        case 10: few_launch<2, 2>(ctx, p); break;
+        case 11: few_launch<2, 3>(ctx, p); break;
+        case 13: few_launch<3, 1>(ctx, p); break;
+        case 14: few_launch<3, 2>(ctx, p); break;
+        case 15: few_launch<3, 3>(ctx, p); break;
+        case 17: few_launch<4, 1>(ctx, p); break;
+        case 18: few_launch<4, 2>(ctx, p); break;
         default: awq_set_error("%s: no few-row form of %d units", what, plan.units); return AWQ_ERR_ARG;
     }
     return awq_check_launch(what);

@@ -145,7 +145,7 @@ int awq_launch_gemm_rows(awq_ctx* ctx, pf::GemmParams& p, int groups, int form, 
 void awq_rows_form(int form, int* tile);  // rows, columns, K slices inside a workgroup
 
 // gemm_few.hip
-constexpr int kFewRows = 64;  // the most it takes
+constexpr int kFewRows = 128;  // the most it takes
 struct awq_few_plan {
     int units, ksplit;  // 32-row units of weights a workgroup; workgroups that share them, each with a part of K
     float us;           // what the launch is expected to take

@@ -792,10 +792,13 @@ int awq_launch_gemm_single(awq_ctx* ctx, uint16_t* out, long long ldo, const uin
 int awq_launch_rmsnorm_rows(awq_ctx* ctx, uint16_t* o, const uint16_t* x, const uint16_t* w, int size, int M, int perm, int tiles);
 
 // Whether a pass of M rows goes through a layer in the few-row form: its four products hand each other activations in
-// fragment order, so that they are weighed together.  Inside a pass they take 0.82 of the sum of their estimates where the row
-// forms take 1.04 of theirs.  Four layers and the logits, us, row forms -> few-row form, at 4, 32, 33 and 64 rows: dim 2048 by 5632
-// 245 -> 207, 252 -> 216, 256 -> 230, 261 -> 238; 4096 by 11008 339 -> 305, 351 -> 319, 396 -> 349, 409 -> 369; 6656 by 17920 574 ->
-// 530, 619 -> 573, 702 -> 634, 728 -> 675; but 8192 by 28672 649 -> 633, 703 -> 701, 761 -> 811, 793 -> 874.
+// fragment order, so that they are weighed together.  Inside a pass they take 0.82 (up to 64 rows; 1.06 above) of the sum of their
+// estimates where the row forms take that of theirs.  Four layers and the logits, us, row forms -> few-row form, at 4, 32, 33 and 64
+// rows: dim 2048 by 5632 245 -> 207, 252 -> 216, 256 -> 230, 261 -> 238; 4096 by 11008 339 -> 305, 351 -> 319, 396 -> 349, 409 -> 369;
+// 6656 by 17920 574 -> 530, 619 -> 573, 702 -> 634, 728 -> 675; but 8192 by 28672 649 -> 633, 703 -> 701, 761 -> 811, 793 -> 874.
+// At 65, 96, 97 and 128 rows: 2048 308 -> 276, 307 -> 281, 314 -> 295, 316 -> 302; 4096 517 -> 434, 522 -> 447, 523 -> 508, 531 -> 534;
+// 5120 by 13824 656 -> 556, 667 -> 580, 679 -> 618, 685 -> 643; 6656 910 -> 790, 912 -> 821, 977 -> 960, 1000 -> 1013; 8192 1000 -> 989,
+// 1010 -> 1035, 1072 -> 1140, 1108 -> 1193.
 bool awq_prefill_takes_few(awq_ctx* ctx, int M, int dim, int kv_dim, int hidden) {
     if (M > kFewRows) return false;
     const auto few = [&](int K, int N, bool split) { return awq_plan_gemm_few(ctx->cus, M, K, N, split).us; };
@@ -805,7 +808,7 @@ bool awq_prefill_takes_few(awq_ctx* ctx, int M, int dim, int kv_dim, int hidden)
         const awq_rows_plan parts = awq_plan_gemm_rows(ctx->cus, M, K, N / 64, true, true);
         return parts.form >= 0 && parts.us < us ? parts.us : us;
     };
-    return 0.82f * (few(dim, dim + 2 * kv_dim, false) + few(dim, dim, true) + few(dim, 2 * hidden, false) + few(hidden, dim, true)) <
+    return (M <= 64 ? 0.82f : 1.06f) * (few(dim, dim + 2 * kv_dim, false) + few(dim, dim, true) + few(dim, 2 * hidden, false) + few(hidden, dim, true)) <
            rows(dim, dim + 2 * kv_dim, false) + rows(dim, dim, true) + rows(dim, 2 * hidden, false) + rows(hidden, dim, true);
 }
 

@@ -1,4 +1,4 @@
-"""The few-row form of the batched int4 GEMM (prefills of up to 64 rows): activations in fragment order, K shared by the waves of a
+"""The few-row form of the batched int4 GEMM (prefills of up to 128 rows): activations in fragment order, K shared by the waves of a
 workgroup and by workgroups, against 64-bit products and against the token-by-token path."""
 import ctypes as C
 
@@ -42,7 +42,9 @@ def _fragments(a):
 # (rows, K, columns): edges of the row tiles; fewer groups than waves, one group more or less than a multiple of the waves, groups
 # that end in the middle of the four or eight that scales and zeros come in; a column tile that the last workgroup fills in part
 SHAPES = [(1, 256, 128), (31, 384, 256), (32, 1024, 2048), (33, 1152, 384), (37, 4096, 4096), (64, 896, 1280), (63, 2176, 640),
-          (5, 11008, 4096), (33, 11008, 4096), (64, 5248, 5120), (17, 4096, 24576), (48, 1024, 24576), (64, 8192, 16512)]
+          (5, 11008, 4096), (33, 11008, 4096), (64, 5248, 5120), (17, 4096, 24576), (48, 1024, 24576), (64, 8192, 16512),
+          (65, 384, 256), (96, 4096, 4096), (77, 1152, 12288), (95, 2176, 22016), (65, 11008, 4096), (97, 384, 256), (128, 4096, 4096),
+          (127, 1152, 12288), (98, 11008, 4096)]
 
 
 @pytest.mark.parametrize("M,K,N", SHAPES)
@@ -70,8 +72,9 @@ def test_residual_product_against_fp64(ctx, M, K, N):
 
 
 def test_every_form_is_taken():
-    taken = {(M > 32, p.units, p.parts > 1) for M, K, N in SHAPES for p in [_plan(256, M, K, N, True)]}
-    assert {t[:2] for t in taken} >= {(False, 1), (False, 2), (False, 3), (True, 1), (True, 2), (True, 3)} and any(t[2] for t in taken)
+    taken = {((M + 31) // 32, p.units, p.parts > 1) for M, K, N in SHAPES for p in [_plan(256, M, K, N, True)]}
+    assert {t[:2] for t in taken} == {(m, u) for m in (1, 2, 3, 4) for u in (1, 2, 3)} - {(4, 3)}
+    assert {t[0] for t in taken if t[2]} == {1, 2, 3, 4}
 
 
 def test_infinite_activation_stays_in_its_row(ctx):
@@ -87,7 +90,8 @@ def test_infinite_activation_stays_in_its_row(ctx):
 
 
 MODELS = {"64": dict(dim=512, hidden_dim=1408, n_heads=8, n_kv_heads=2), "128": dict(dim=1024, hidden_dim=2816, n_heads=8, n_kv_heads=8),
-          "256": dict(dim=1536, hidden_dim=2048, n_heads=6, n_kv_heads=1), "wide": dict(dim=4096, hidden_dim=11008, n_heads=32, n_kv_heads=32)}
+          "256": dict(dim=1536, hidden_dim=2048, n_heads=6, n_kv_heads=1), "wide": dict(dim=4096, hidden_dim=11008, n_heads=32, n_kv_heads=32),
+          "64 wide": dict(dim=2048, hidden_dim=5632, n_heads=32, n_kv_heads=4)}
 
 
 @pytest.mark.parametrize("model", MODELS)
@@ -95,12 +99,13 @@ def test_prefill_against_token_by_token(ctx, model):
     """Passes at the edges of the row tiles, one behind another (the attention takes its forms for few and for many keys): cache rows
     and logits of the token-by-token path within the tolerance of the batched one."""
     m = MODELS[model]
-    cfg = dict(m, n_layers=2, vocab_size=512, seq_len=640, rope_theta=10000.0)
+    cfg = dict(m, n_layers=2, vocab_size=512, seq_len=1024, rope_theta=10000.0)
     kv_dim = m["dim"] * m["n_kv_heads"] // m["n_heads"]
-    parts = (1, 31, 32, 33, 63, 64, 300, 40, 5)
+    parts = (1, 31, 32, 33, 63, 64, 300, 40, 5, 65, 96, 97, 128)
     n = sum(parts)
     assert all(_takes_few(ctx.h, p, m["dim"], kv_dim, m["hidden_dim"]) for p in parts if p <= 64)
-    assert not _takes_few(ctx.h, 65, m["dim"], kv_dim, m["hidden_dim"])
+    assert all(_takes_few(ctx.h, p, m["dim"], kv_dim, m["hidden_dim"]) == ("wide" in model) for p in (65, 96, 97, 128))
+    assert not _takes_few(ctx.h, 129, m["dim"], kv_dim, m["hidden_dim"])
     img = synth.make_model_image(cfg, seed=63, scale_mult=0.25)
     prompt = synth.prompt_tokens(63, n, cfg["vocab_size"])
     t = A.Transformer(ctx, image=img)
