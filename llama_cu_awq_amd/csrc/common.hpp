@@ -33,9 +33,7 @@ struct awq_ctx {
 };
 
 constexpr int kAttnMaxHeads = 256;
-// Up to this launch size attention runs as two workgroups per head that score all of its positions; past it the fused schedule takes
-// ranges of positions.  us a pass, this form | ranges: 7B shape, 16 tokens from 0 18426 | 18884; 16 grouped-query layers, 12
-// tokens from 200 9581 | 9543, which is what two runs differ by.
+// Up to this launch size awq_attention runs as one launch, two workgroups per head that score all of its positions.
 constexpr int kAttnFusedMaxSeq = 256;
 constexpr int kAttnMaxChunks = 4;      // ranges of positions whose partial P.V sums the O projection adds up
 

@@ -370,7 +370,49 @@ __global__ __launch_bounds__(1024) void attn_pv_partial_kernel(float* part, cons
     }
 }
 
-// Fused schedule, launch sizes above kAttnFusedMaxSeq (but see awq_attention_takes_ranges): scores, softmax and P.V of one of
+// Maximum and sum over a wave's groups of LP lanes, of values that are the same within a group (the maximum) or stand for one lane of
+// each (the sum).
+template <int LP>
+__device__ __forceinline__ float groups_max(float v) {
+    if (LP <= 8) v = fmaxf(v, dpp_mov<0x128>(v));  // row_ror:8
+    float a = v, b = v;
+    if (LP <= 16) {
+        swap16(a, b);
+        a = b = fmaxf(a, b);
+    }
+    swap32(a, b);
+    return fmaxf(a, b);
+}
+template <int LP>
+__device__ __forceinline__ float groups_sum(float v) {
+    if (LP <= 8) v = lane_xor_sum<8>(v);
+    if (LP <= 16) v = lane_xor_sum<16>(v);
+    return lane_xor_sum<32>(v);
+}
+// Lane l (of 16) holds wave l's maximum and sum of exponentials: the row's maximum and sum, and what takes wave l's results to it.
+__device__ __forceinline__ float wave_scale(float2 w, float& top, float& sum) {
+    float t = w.x;
+    t = fmaxf(t, dpp_mov<0xB1>(t));
+    t = fmaxf(t, dpp_mov<0x4E>(t));
+    t = fmaxf(t, dpp_mov<0x124>(t));
+    top = fmaxf(t, dpp_mov<0x128>(t));
+    const float scale = expf(w.x - top);
+    sum = row16_sum(w.y * scale);
+    return scale;
+}
+// sum over 16 waves of acc[wave * stride], each on the scale that its lane holds
+__device__ __forceinline__ float scaled_waves(const float* acc, int stride, float scale) {
+    float r[16];
+#pragma unroll
+    for (int w = 0; w < 16; w++) r[w] = acc[w * stride] * read_lane(scale, w);
+#pragma unroll
+    for (int n = 16; n > 1; n >>= 1)
+#pragma unroll
+        for (int i = 0; i < n / 2; i++) r[i] = r[2 * i] + r[2 * i + 1];
+    return r[0];
+}
+
+// Fused schedule, launch sizes past awq_attention_takes_short (but see awq_attention_takes_ranges): scores, softmax and P.V of one of
 // `chunks` contiguous ranges of a head's positions in a workgroup of 16 waves, one pass over its keys and values.  LP lanes
 // (head_size / 8) share a position; each such group of lanes keeps a running maximum, sum of exponentials and fp32 P.V of the
 // positions it sees, the groups meet at the end, and part[chunk][head * head_size + dim] with stat[head][chunk] = (maximum, sum)
@@ -383,13 +425,14 @@ __global__ __launch_bounds__(1024) void attn_pv_partial_kernel(float* part, cons
 // launches, scores and P.V (unsplit below 1024 positions; split over positions with the scores exchanged through memory above).
 // us a token, 4 layers, two launches -> one: 7B shape, position 300 167.5 -> 163.8, 700 172.5 -> 168.5, 2000 188.5 -> 181.5;
 // 13B shape 224.4 -> 210.1, 227.1 -> 216.9, 242.8 -> 232.7; 70B shape 391.8 -> 383.6, 407.2 -> 390.5, 423.1 -> 399.9; 32 heads
-// of 64 over 4 key heads 108.4 -> 103.3, 111.9 -> 104.5, 122.3 -> 108.1.
+// of 64 over 4 key heads 108.4 -> 103.3, 111.9 -> 104.5, 122.3 -> 108.1.  (One barrier instead of two where the waves meet and a
+// quarter of the exponentials in each lane of a quad, 8 layers of the 7B shape, position 600 329.8 -> 325.7, 2000 370.4 -> 365.4.)
 template <int LP>
 __global__ __launch_bounds__(1024) void attn_ranges_kernel(float* part, float2* stat, uint16_t* att, const uint16_t* q,
                                                            const uint16_t* key_cache, const uint16_t* value_cache, int num_heads,
                                                            int kv_heads, int row_stride, float alpha, const int* pPos) {
     constexpr int HS = LP * 8, PW = 64 / LP, ROUND = 16 * PW, R = 4;  // positions a wave and the workgroup take per load; loads in flight
-    __shared__ float red[16], red_l[16];
+    __shared__ float2 waves[16];
     __shared__ float acc_lds[16][HS];
     const int size = *pPos + 1;
     // the query heads of a key head are gridDim-neighbours kv_heads apart: one XCD where kv_heads is a multiple of 8
@@ -437,16 +480,23 @@ __global__ __launch_bounds__(1024) void attn_ranges_kernel(float* part, float2* 
         l *= fade;
 #pragma unroll
         for (int e = 0; e < 8; e++) acc[e] *= fade;
+        // every lane of a group has its scores: lane i of a quad takes the exponential of score i for the others
+        float x = s[0];
+#pragma unroll
+        for (int i = 1; i < R; i++) x = (lane & 3) == i ? s[i] : x;
+        const float e = expf(x - m);
+        float el = e + dpp_mov<0xB1>(e);  // quad_perm [1,0,3,2]
+        el += dpp_mov<0x4E>(el);          // quad_perm [2,3,0,1]
+        l += el;
 #pragma unroll
         for (int i = 0; i < R; i++) {
+            const float p = i == 0 ? dpp_mov<0x00>(e) : i == 1 ? dpp_mov<0x55>(e) : i == 2 ? dpp_mov<0xAA>(e) : dpp_mov<0xFF>(e);
             if (t0 + mine + i * ROUND < t_end) {
-                const float p = expf(s[i] - m);
-                l += p;
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const h16x2 hv = as_h2(b.v[i][e]);
-                    acc[2 * e] = fmaf((float)hv[0], p, acc[2 * e]);
-                    acc[2 * e + 1] = fmaf((float)hv[1], p, acc[2 * e + 1]);
+                for (int d = 0; d < 4; d++) {
+                    const h16x2 hv = as_h2(b.v[i][d]);
+                    acc[2 * d] = fmaf((float)hv[0], p, acc[2 * d]);
+                    acc[2 * d + 1] = fmaf((float)hv[1], p, acc[2 * d + 1]);
                 }
             }
         }
@@ -469,48 +519,124 @@ __global__ __launch_bounds__(1024) void attn_ranges_kernel(float* part, float2* 
         request(a, t0 + 2 * R * ROUND);
         process(b, t0 + R * ROUND);
     }
-    const float wm = wave_max(m);
-    if (lane == 0) red[wave] = wm;
-    __syncthreads();
-    float top = red[0];
+    const float wm = groups_max<LP>(m), fade = expf(m - wm);
+    l = groups_sum<LP>(l * fade);
 #pragma unroll
-    for (int w = 1; w < 16; w++) top = fmaxf(top, red[w]);
-    const float fade = expf(m - top);
-    auto groups_sum = [](float v) {
-        if (LP <= 8) v = lane_xor_sum<8>(v);
-        if (LP <= 16) v = lane_xor_sum<16>(v);
-        return lane_xor_sum<32>(v);
-    };
-    l = groups_sum(l * fade);
-#pragma unroll
-    for (int i = 0; i < 8; i++) acc[i] = groups_sum(acc[i] * fade);
-    if (lane == 0) red_l[wave] = l;
+    for (int i = 0; i < 8; i++) acc[i] = groups_sum<LP>(acc[i] * fade);
+    if (lane == 0) waves[wave] = make_float2(wm, l);
     if (lane < LP) {
 #pragma unroll
         for (int i = 0; i < 8; i++) acc_lds[wave][lane * 8 + i] = acc[i];
     }
     __syncthreads();
-    auto tree = [](float (&r)[16]) {
-#pragma unroll
-        for (int n = 16; n > 1; n >>= 1)
-#pragma unroll
-            for (int i = 0; i < n / 2; i++) r[i] = r[2 * i] + r[2 * i + 1];
-        return r[0];
-    };
-    float r[16];
     if (tid < HS) {
-#pragma unroll
-        for (int w = 0; w < 16; w++) r[w] = acc_lds[w][tid];
-        part[((size_t)chunk * num_heads + h) * HS + tid] = tree(r);
-    }
-    if (tid == 0) {
-#pragma unroll
-        for (int w = 0; w < 16; w++) r[w] = red_l[w];
-        stat[(size_t)h * kAttnMaxChunks + chunk] = make_float2(top, tree(r));
+        float top, sum;
+        const float scale = wave_scale(waves[lane & 15], top, sum);
+        part[((size_t)chunk * num_heads + h) * HS + tid] = scaled_waves(&acc_lds[0][tid], HS, scale);
+        if (tid == 0) stat[(size_t)h * kAttnMaxChunks + chunk] = make_float2(top, sum);
     }
 }
 
-// Short contexts: a workgroup of 16 waves does scores, softmax and P.V of a head in a single launch (the work is a few
+// Fused schedule, short contexts (awq_attention_takes_short): all of a head's positions in one request, R rows of keys and values a
+// lane, the first of them asked for before the position is known; scores stay in registers.  Two workgroups a head take half of the
+// value dimensions each and compute the scores redundantly; those of a key head run on one XCD where key heads are 8 or more.
+// ROUNDED (up to 256 positions): the probability is rounded to fp16 after the division by the row's sum, as the reference does it
+// (gpu_kernels.h:368-451), so that maxima and sums of the 16 waves meet before P.V.  Past 256 positions, where ranges keep it fp32, it
+// stays fp32 and the waves meet once.  The maximum starts below every score, as in attn_ranges_kernel.
+// Bound by latency (launch, one round trip to memory, a barrier or two) and, at many rows, by exponentials, of which each lane of a
+// quad therefore takes a quarter.  us a token of 8 layers, scores in LDS between scores and statistics (attn_fused_kernel, which
+// looks at the whole row in every wave) -> this one, positions 40 and 200: 32 heads of 128 307.6 -> 296.9, 315.0 -> 305.2; 40 of 128
+// 403.2 -> 392.4, 412.5 -> 401.7; 32 heads of 64 over 4 key heads 196.6 -> 185.2, 215.9 -> 191.3; 8 heads of 128 166.7 -> 157.3,
+// 173.6 -> 166.9.  Exponentials in every lane: 32 heads of 128 at 200 312.
+template <int LP, int R, bool ROUNDED>
+__global__ __launch_bounds__(1024) void attn_short_kernel(uint16_t* output, uint16_t* att, const uint16_t* q, const uint16_t* key_cache,
+                                                          const uint16_t* value_cache, int kv_heads, int kv_mul, float alpha,
+                                                          const int* pPos, int max_seq_len) {
+    constexpr int HS = LP * 8, VS = HS / 2, PW = 64 / LP, ROUND = 16 * PW;
+    __shared__ float2 waves[16];
+    __shared__ __attribute__((aligned(16))) float acc_lds[16][VS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane % LP, mine = wave * PW + lane / LP;
+    const int kvh = min((int)blockIdx.x, kv_heads - 1), h = kvh * kv_mul + (blockIdx.y >> 1), slice = blockIdx.y & 1;
+    const int row_stride = kv_heads * HS;
+    const uint16_t* kh = key_cache + (size_t)kvh * HS + j * 8;
+    const uint16_t* vh = value_cache + (size_t)kvh * HS + slice * VS + j * 4;
+    const u32x4 qv = *reinterpret_cast<const u32x4*>(q + (size_t)h * HS + j * 8);
+    u32x4 k[R];
+    u32x2 v[R];
+    auto request = [&](int i, int t) {
+        k[i] = *reinterpret_cast<const u32x4*>(kh + (size_t)t * row_stride);
+        v[i] = *reinterpret_cast<const u32x2*>(vh + (size_t)t * row_stride);
+    };
+    // the first rows whatever the position, while its word is on its way (what lies past it is not looked at)
+    request(0, min(mine, max_seq_len - 1));
+    const int size = min(*pPos + 1, max_seq_len);  // (R rounds are max_seq_len positions or more)
+#pragma unroll
+    for (int i = 1; i < R; i++) request(i, min(mine + i * ROUND, size - 1));
+    float s[R], m = -1e5f;  // below every finite fp16 score, and finite itself
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+        const int t = mine + i * ROUND;
+        float d = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; e++) d = dot2(k[i][e], qv[e], d);
+        d = group_sum<LP>(d);
+        const uint16_t hb = float_to_half_bits(d * alpha);
+        if (slice == 0 && j == 0 && t < size && kvh == (int)blockIdx.x) att[(size_t)h * size + t] = hb;
+        s[i] = t < size ? half_bits_to_float(hb) : -INFINITY;
+        m = fmaxf(m, s[i]);
+    }
+    m = groups_max<LP>(m);
+    // every lane of a group has its scores: lane i of a quad takes the exponentials of scores i, i + 4, ... for the others
+    constexpr int G = (R + 3) / 4;
+    float e[G], l = 0.0f;
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+        float x = s[g * 4];
+#pragma unroll
+        for (int i = 1; i < 4 && R > 1; i++) x = (lane & 3) == i ? (g * 4 + i < R ? s[g * 4 + i] : -INFINITY) : x;
+        e[g] = expf(x - m);
+        l += e[g];
+    }
+    if (R > 1) {
+        l += dpp_mov<0xB1>(l);  // quad_perm [1,0,3,2]
+        l += dpp_mov<0x4E>(l);  // quad_perm [2,3,0,1]
+    }
+    l = groups_sum<LP>(l);
+    if (lane == 0) waves[wave] = make_float2(m, l);
+    float top, sum;
+    if (ROUNDED) {  // the row's maximum and sum first
+        __syncthreads();
+        const float scale = read_lane(wave_scale(waves[lane & 15], top, sum), wave) / sum;
+#pragma unroll
+        for (int g = 0; g < G; g++) e[g] = half_bits_to_float(float_to_half_bits(e[g] * scale));
+    }
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+        const float all = e[i / 4];
+        const float p = R == 1 ? all : i % 4 == 0 ? dpp_mov<0x00>(all) : i % 4 == 1 ? dpp_mov<0x55>(all) : i % 4 == 2 ? dpp_mov<0xAA>(all) : dpp_mov<0xFF>(all);
+        if (mine + i * ROUND < size) {
+#pragma unroll
+            for (int d = 0; d < 2; d++) {
+                const h16x2 hv = as_h2(v[i][d]);
+                acc[2 * d] = fmaf((float)hv[0], p, acc[2 * d]);
+                acc[2 * d + 1] = fmaf((float)hv[1], p, acc[2 * d + 1]);
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) acc[i] = groups_sum<LP>(acc[i]);
+    if (lane < LP) *reinterpret_cast<float4*>(&acc_lds[wave][lane * 4]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    __syncthreads();
+    if (tid < VS && kvh == (int)blockIdx.x) {
+        float scale = 1.0f;
+        if (!ROUNDED) scale = wave_scale(waves[lane & 15], top, sum) / sum;
+        output[(size_t)h * HS + slice * VS + tid] = float_to_half_bits(scaled_waves(&acc_lds[0][tid], VS, scale));
+    }
+}
+
+// Short contexts of the reference schedule and awq_attention: a workgroup of 16 waves does scores, softmax and P.V of a head in a single launch (the work is a few
 // hundred KB per head, so the launch count matters more than the parallelism); NS workgroups per head each take a
 // slice of the value dimensions and compute the scores redundantly.  Same arithmetic and
 // rounding points as the two-pass kernels above; the fp16 scores are also left in att.
@@ -776,6 +902,37 @@ int awq_launch_attention_partial(awq_ctx* ctx, float* part, int* chunks_out, con
     return awq_check_launch("attn_pv_partial");
 }
 
+// Internal (fused schedule): whether attention goes in the one request of attn_short_kernel (awq_launch_attention_short): up to what a
+// lane's registers hold.  Past 256 positions it pulls all keys of a head through each of two compute units, which ranges share, but
+// leaves the O projection no parts to put together.  us a token of 8 layers, ranges | one request, positions 300 and 500: 32 heads of
+// 128 316.6 | 308.4, 320.5 | 310.2; 40 of 128 409.2 | 407.6, 413.3 | 411.5; 64 of 128 771 | 768, 773 | 763; 8 of 128 176.8 | 173.5,
+// 178.4 | 175.5; 32 of 64 203.3 | 191.6, 205.7 | 193.4, at 600 and 1000 204.4 | 201.5, 209.7 | 209.0.
+bool awq_attention_takes_short(int head_size, int max_seq_len) {
+    return max_seq_len <= (head_size == 64 ? 1024 : head_size == 128 ? 512 : 256);
+}
+
+// Internal: attention in one launch where awq_attention_takes_short says so.
+int awq_launch_attention_short(awq_ctx* ctx, uint16_t* output, const uint16_t* q, const uint16_t* key_cache, const uint16_t* value_cache,
+                               uint16_t* att, int num_heads, int head_size, int kv_mul, int max_seq_len, const int* pos) {
+    const float alpha = (float)(1.0 / sqrt((double)head_size));
+    const int kv_heads = num_heads / kv_mul;
+    auto go = [&](auto kernel) {
+        awq_launch(ctx, kernel, dim3(kv_heads < 8 ? kv_heads : (kv_heads + 7) & ~7, 2 * kv_mul), dim3(1024), 0, output, att, q, key_cache,
+                   value_cache, kv_heads, kv_mul, alpha, pos, max_seq_len);
+    };
+    const int to = max_seq_len <= 128 ? 128 : max_seq_len <= 256 ? 256 : max_seq_len <= 512 ? 512 : 1024;  // positions that the kernel holds
+    switch (head_size) {
+        case 64:
+            to == 128 ? go(attn_short_kernel<8, 1, true>) : to == 256 ? go(attn_short_kernel<8, 2, true>)
+                    : to == 512 ? go(attn_short_kernel<8, 4, false>) : go(attn_short_kernel<8, 8, false>);
+            break;
+        case 128: to == 128 ? go(attn_short_kernel<16, 2, true>) : to == 256 ? go(attn_short_kernel<16, 4, true>) : go(attn_short_kernel<16, 8, false>); break;
+        case 256: to == 128 ? go(attn_short_kernel<32, 4, true>) : go(attn_short_kernel<32, 8, true>); break;
+        default: awq_set_error("attention: head_size %d unsupported (64, 128 or 256)", head_size); return AWQ_ERR_SHAPE;
+    }
+    return awq_check_launch("attn_short");
+}
+
 // Ranges of positions a head's row is divided into, of what a workgroup requests at once (256 positions of 128-wide heads), at
 // least two, at most about one workgroup per compute unit: a further range costs the staging of the O projection 0.3 to 0.8 us
 // in every workgroup, positions that are requested late a round trip.  us per layer, 2 | 3 | 4 ranges: 7B shape (4 layers),
@@ -786,7 +943,7 @@ static int range_count(int cus, int num_heads, int head_size, int max_seq_len) {
     return max(1, min(min(kAttnMaxChunks, cus / num_heads), max(2, div_up(max_seq_len, round))));
 }
 
-// Internal (fused schedule, launch sizes above kAttnFusedMaxSeq): whether attention goes in ranges (awq_launch_attention_ranges)
+// Internal (fused schedule, launch sizes past awq_attention_takes_short): whether attention goes in ranges (awq_launch_attention_ranges)
 // or as scores and split P.V (awq_launch_attention_partial).  Ranges save a launch and the scores' way through memory, but there are
 // at most kAttnMaxChunks of them: where that leaves compute units idle, each takes its positions at 2 to 3 us per 128 KB of keys and
 // values, while the scores go 64 positions to a workgroup and P.V 64 dimensions to one (so heads of 256, which are four slices
@@ -807,7 +964,7 @@ bool awq_attention_takes_ranges(int cus, int num_heads, int head_size, int kv_mu
     return load <= wgs - 16;
 }
 
-// Internal (fused schedule, launch sizes above kAttnFusedMaxSeq): attention in one launch, as parts of a softmax over
+// Internal (fused schedule, launch sizes past awq_attention_takes_short): attention in one launch, as parts of a softmax over
 // `*chunks_out` ranges of positions for awq_launch_matvec_int4_parts to put together.  part: kAttnMaxChunks * num_heads *
 // head_size floats; stat: kAttnMaxChunks * num_heads.
 int awq_launch_attention_ranges(awq_ctx* ctx, float* part, float2* stat, int* chunks_out, const uint16_t* q, const uint16_t* key_cache,

@@ -23,6 +23,9 @@ int awq_launch_ffn(awq_ctx* ctx, uint16_t* out, const uint16_t* x, const awq_qwe
                    int N, const uint16_t* norm_w, uint16_t* norm_out);
 int awq_launch_matvec_f16(awq_ctx* ctx, uint16_t* out, const uint16_t* x, const uint16_t* w, int n, int d,
                           const uint16_t* norm_w, uint16_t* norm_out);
+bool awq_attention_takes_short(int head_size, int max_seq_len);
+int awq_launch_attention_short(awq_ctx* ctx, uint16_t* output, const uint16_t* q, const uint16_t* key_cache, const uint16_t* value_cache,
+                               uint16_t* att, int num_heads, int head_size, int kv_mul, int max_seq_len, const int* pos);
 bool awq_attention_takes_ranges(int cus, int num_heads, int head_size, int kv_mul, int max_seq_len);
 int awq_launch_attention_partial(awq_ctx* ctx, float* part, int* chunks_out, const uint16_t* q, const uint16_t* key_cache,
                                  const uint16_t* value_cache, uint16_t* att, int num_heads, int head_size, int kv_mul,
@@ -526,7 +529,8 @@ int network_fused(awq_transformer* t, int seq_len_bin) {
         // rounded to fp16, the reference's rounding point) while the O projection stages its input; xb is not written on this
         // path.  (Larger vectors do not travel in the staging's registers.)  The parts are those of a softmax, each relative to its
         // own maximum, or, where ranges would leave too much of the chip idle, plain sums behind a launch of their own.
-        const bool split = seq_len_bin > kAttnFusedMaxSeq && dim <= 8192;
+        const bool whole = awq_attention_takes_short(head_size, seq_len_bin);
+        const bool split = !whole && dim <= 8192;
         const bool ranges = split && awq_attention_takes_ranges(ctx->cus, p.n_heads, head_size, kv_mul, seq_len_bin);
         float2* stat = ranges ? reinterpret_cast<float2*>(t->attn_part + (size_t)kAttnMaxChunks * dim) : nullptr;
         int parts = 0;
@@ -538,6 +542,9 @@ int network_fused(awq_transformer* t, int seq_len_bin) {
             else if (split)
                 r = awq_launch_attention_ranges(ctx, t->attn_part, stat, &parts, s.q, s.key_cache + loff, s.value_cache + loff, s.att,
                                                 p.n_heads, head_size, kv_mul, seq_len_bin, pPos);
+            else if (whole)
+                r = awq_launch_attention_short(ctx, s.xb, s.q, s.key_cache + loff, s.value_cache + loff, s.att, p.n_heads, head_size, kv_mul,
+                                               seq_len_bin, pPos);
             else
                 r = awq_attention(ctx, s.xb, s.q, s.key_cache + loff, s.value_cache + loff, s.att, p.n_heads, head_size, kv_mul,
                                   seq_len_bin, pPos);

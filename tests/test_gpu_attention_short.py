@@ -1,0 +1,91 @@
+"""The fused schedule's attention where a head's positions are one request (up to 1024 of them for heads of 64, 512 for 128, 256 for 256): at the
+edges of a request and of a lane's rows, against the reference schedule's form with the scores in LDS and on rows that must not count."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import llama_cu_awq_amd as A
+import tests.test_gpu_model as model
+from llama_cu_awq_amd import synth
+from llama_cu_awq_amd._lib import lib
+from tests.helpers import f16, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+takes_short = lib["_Z25awq_attention_takes_shortii"]
+takes_short.argtypes, takes_short.restype = [C.c_int] * 2, C.c_bool
+
+# heads, head size, key heads: one key head, fewer than 8, a number that is no multiple of 8
+HEADS = [(4, 64, 2), (32, 64, 4), (16, 128, 1), (24, 128, 12), (8, 128, 8), (4, 256, 2), (16, 256, 16)]
+POSITIONS = (0, 1, 15, 63, 64, 127, 128, 129, 255, 256, 300, 510, 511, 512, 1022, 1023)
+
+
+def _transformer(ctx, heads, head, kv, seed):
+    cfg = dict(dim=heads * head, hidden_dim=256, n_layers=1, n_heads=heads, n_kv_heads=kv, vocab_size=512, seq_len=1024, rope_theta=10000.0)
+    return cfg, A.Transformer(ctx, image=synth.make_model_image(cfg, seed=seed))
+
+
+@pytest.mark.parametrize("heads,head,kv", HEADS)
+def test_against_the_reference_schedule(ctx, heads, head, kv):
+    """Both round scores to fp16, and up to 256 positions the probabilities.  Activations of fp16 behind it differ by single roundings (under 1e-3
+    in the norm); values that grow with the position make a row that is missed or weighted wrongly a difference of several per cent."""
+    cfg, t = _transformer(ctx, heads, head, kv, 7)
+    seq = cfg["seq_len"]
+    rng = np.random.default_rng(heads * head + kv)
+    t.buffer("key_cache", seq * kv * head * 2).write(rng.standard_normal((seq, kv * head)).astype(np.float16))
+    rows = rng.standard_normal((seq, kv * head)) + 8 * np.arange(seq)[:, None] / seq - 2
+    t.buffer("value_cache", seq * kv * head * 2).write(rows.astype(np.float16))
+    assert [takes_short(head, n) for n in (256, 257, 512, 513, 1024, 1025)] == [True, head < 256, head < 256, head == 64, head == 64, False]
+    for pos in POSITIONS:
+        logits, scores = [], []
+        for mode, graph in ((A.SCHEDULE_REFERENCE, False), (A.SCHEDULE_FUSED, False), (A.SCHEDULE_FUSED, True)):
+            t.set_pos(pos, 7)
+            t.forward_logits(use_graph=graph, mode=mode)
+            ctx.sync()
+            logits.append(f16(t.download("logits", cfg["vocab_size"])).astype(np.float64))
+            scores.append(f16(t.download("att", heads * (pos + 1))).astype(np.float64))
+        assert np.isfinite(logits[0]).all()
+        for got, att in zip(logits[1:], scores[1:]):
+            assert rel_l2(got, logits[0]) <= 4e-3, pos
+            assert rel_l2(att, scores[0]) <= 2e-3, pos
+    t.close()
+
+
+@pytest.mark.parametrize("heads,head,kv", [(4, 64, 2), (16, 128, 4), (4, 256, 2)])
+@pytest.mark.parametrize("pos", [0, 5, 70, 200, 260, 520])
+def test_rows_past_the_position_do_not_enter(ctx, heads, head, kv, pos):
+    """The first rows are read before the position is known: NaN and infinities behind it change no bit.  Those of rows that count reach
+    the logits."""
+    cfg, t = _transformer(ctx, heads, head, kv, 8)
+    seq, row = cfg["seq_len"], kv * head
+    rng = np.random.default_rng(pos)
+    rows = {name: rng.standard_normal((seq, row)).astype(np.float16) for name in ("key_cache", "value_cache")}
+
+    def logits(graph, at=None, value=0.0, names=tuple(rows)):
+        for name, r in rows.items():
+            r = r.copy()
+            if at is not None and name in names:
+                r[at] = value
+            t.buffer(name, seq * row * 2).write(r)
+        t.set_pos(pos, 7)
+        t.forward_logits(use_graph=graph, mode=A.SCHEDULE_FUSED)
+        ctx.sync()
+        return f16(t.download("logits", cfg["vocab_size"])).copy()
+
+    for graph in (False, True):
+        want = logits(graph)
+        assert np.isfinite(want).all()
+        for value in (np.nan, np.inf):
+            assert np.array_equal(logits(graph, slice(pos + 1, None), value).view(np.uint16), want.view(np.uint16))
+        if pos:
+            assert not np.isfinite(logits(graph, (pos - 1, row - 1), np.nan, ("key_cache",))).any()
+            assert not np.isfinite(logits(graph, (0, row - 1), np.inf, ("value_cache",))).any()
+    t.close()
+
+
+@pytest.mark.parametrize("heads,head,kv", [(8, 64, 2), (2, 256, 1)])  # (1/sqrt(head size) is exact: scores stay multiples of an eighth)
+@pytest.mark.parametrize("size", [2, 64, 200, 256])
+def test_scores_far_below_zero(ctx, heads, head, kv, size):
+    """As at longer contexts: a constant added to every score changes no softmax, also where its exponentials are zero in fp32."""
+    model.test_decode_scores_far_below_zero(ctx, heads, head, kv, size)
