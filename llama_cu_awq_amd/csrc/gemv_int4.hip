@@ -332,7 +332,7 @@ __global__ __launch_bounds__(W * 64) void gemv_int4_kernel(const GemvParams p) {
     // ahead of the other workgroups' activations on the compute unit (7B shape +1.5 % tokens/s, 13B +0.6 %, 33B
     // unchanged; with nothing requested ahead of the staging the weights' own latency shows: -0.4 %; the plain forms lose
     // by any delay)
-    constexpr int DE = NORM ? D - 1 : D;  // stages requested before the staging
+    constexpr int DE = NORM && D > 1 ? D - 1 : D;  // stages requested before the staging
 #pragma unroll
     for (int d = 0; d < DE; d++) {
         issue(st[d]);
@@ -434,7 +434,7 @@ bool qw_ok(const awq_qweight* w) { return w && w->weight && w->zeros && w->scale
 struct GemvPlan {
     int waves;   // waves per workgroup (4, 8)
     int rows;    // rows per wave (1, 2, 4)
-    int depth;   // stages in flight per wave (2, 3, 4)
+    int depth;   // stages in flight per wave (2, 3, 4; rows of one pass: 1)
 };
 
 #ifdef AWQ_STAMPS
@@ -530,6 +530,8 @@ int launch(awq_ctx* ctx, GemvParams& p, int grid_y, const char* what) {
 // flight.
 template <int W, int KIND, bool ROPE, int SPLIT>
 int dispatch_split(awq_ctx* ctx, GemvParams& p, int grid_y, const char* what, int depth) {
+    if constexpr (KIND == KIND_SINGLE)
+        if (p.C <= 64 / SPLIT) return launch<W, 1, 1, KIND, ROPE, SPLIT>(ctx, p, grid_y, what);  // (see dispatch_depth)
     if (depth == 2) return launch<W, 1, 2, KIND, ROPE, SPLIT>(ctx, p, grid_y, what);
     return launch<W, 1, 3, KIND, ROPE, SPLIT>(ctx, p, grid_y, what);
 }
@@ -537,6 +539,10 @@ int dispatch_split(awq_ctx* ctx, GemvParams& p, int grid_y, const char* what, in
 template <int W, int R, int KIND, bool ROPE>
 int dispatch_depth(awq_ctx* ctx, GemvParams& p, int grid_y, const char* what, const GemvPlan& plan) {
     constexpr int NS = (KIND == KIND_FFN) ? 2 * R : R;
+    // A row of one pass, one row to a wave: nothing is in flight behind it, and padded to a depth of two it is requested twice (32 heads of
+    // 64, dim 2048: a token of 8 layers 184.7 -> 180.6 us).
+    if constexpr (KIND == KIND_SINGLE && R == 1)
+        if (p.C <= 64) return launch<W, R, 1, KIND, ROPE>(ctx, p, grid_y, what);
     int depth = plan.depth;
     while (depth > 2 && (NS * depth > 16 || depth > 4)) depth--;  // what the register file affords
     switch (depth) {
@@ -579,6 +585,9 @@ int dispatch(awq_ctx* ctx, GemvParams& p, int grid_y, const char* what, GemvPlan
         if (ceil(per_cu8) / per_cu8 < ceil(per_cu16) / per_cu16 - 0.05) plan.waves = 8;
     }
     if (ROPE && plan.rows < 2) plan.rows = 2;  // a rotation pair lives in one wave
+    // Q, K and V so small that workgroups of 8 waves leave compute units idle (dim 2048 with 256 K and V rows: 160; a token of 8 layers
+    // 184.7 -> 180.6 us; dim 1024: 192, 159.3 -> 158.0)
+    if (KIND == KIND_QKV && plan.waves == 8 && plan.rows == 2 && div_up(p.N, 16) + (grid_y - 1) * div_up(p.Nkv, 16) < ctx->cus) plan.waves = 4;
     // Rows that leave at most half of a 64-lane pass over go two to a wave, 32 lanes each (see the kernel).  Measured
     // at the 13B and 33B shapes (K = 5120, 6656): gate/up -6 %, O projection -7 %, QKV -2 % with two passes in flight
     // and even with three, tokens/s +3 %.  Rows above 8192 (K = 11008: 16 waves, or 8, at any depth) lose: two rows per

@@ -78,6 +78,22 @@ def test_matvec_int4_plain(ctx, K, N):
         assert (got != best).mean() <= max(2 * (f16(want) != best).mean(), 4e-3)
 
 
+@pytest.mark.parametrize("N", [8, 264, 2048])
+@pytest.mark.parametrize("K", [1024, 1032, 2040, 2048, 2056])
+def test_matvec_int4_rows_of_one_pass(ctx, K, N):
+    """Up to 2048 elements (1024 where two rows share a wave) a row is one request: one rounding behind fp32 sums, with and without x added."""
+    w, z, s, x = _case(K, N, 9)
+    qw = A.QWeight.upload(ctx, w, z, s)
+    dx, resid = ctx.upload(x), synth.normal_f16(synth.stream_key(9, K, N), N)
+    want = synth.dequantize(w, z, s, K) @ x.astype(np.float64)
+    dout = ctx.upload(resid)
+    A.matmul_q(ctx, dout, dx, qw, K, N)
+    assert rel_l2(f16(dout.download(np.uint16)), want) <= 4e-4
+    dout = ctx.upload(resid)
+    A.matmul_q(ctx, dout, dx, qw, K, N, accum=True)
+    assert rel_l2(f16(dout.download(np.uint16)), want + resid.astype(np.float64)) <= 4e-4
+
+
 # ---- shapes chosen to reach every branch of the launch geometry (waves per workgroup 4 / 8 / 10 / 13 / 16, one, two or
 # four rows side by side in a wave, two or three passes in flight, partly filled last workgroups and row groups, row
 # lengths that are no multiple of a pass or of a quantisation group), in the three forms.
