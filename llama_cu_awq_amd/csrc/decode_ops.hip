@@ -540,20 +540,21 @@ __global__ __launch_bounds__(1024) void attn_ranges_kernel(float* part, float2* 
 // Fused schedule, short contexts (awq_attention_takes_short): all of a head's positions in one request, R rows of keys and values a
 // lane, the first of them asked for before the position is known; scores stay in registers.  Two workgroups a head take half of the
 // value dimensions each and compute the scores redundantly; those of a key head run on one XCD where key heads are 8 or more.
-// ROUNDED (up to 256 positions): the probability is rounded to fp16 after the division by the row's sum, as the reference does it
-// (gpu_kernels.h:368-451), so that maxima and sums of the 16 waves meet before P.V.  Past 256 positions, where ranges keep it fp32, it
-// stays fp32 and the waves meet once.  The maximum starts below every score, as in attn_ranges_kernel.
+// ROUNDED (up to 256 positions): maximum (from 0, as the reference's idle lanes have it), sum, probabilities rounded to fp16 after their
+// division by it and all sums in attn_fused_kernel's order: its bits.  Past 256 positions, where ranges keep probabilities fp32 and start
+// the maximum below every score, so does this, and the waves meet once.
 // Bound by latency (launch, one round trip to memory, a barrier or two) and, at many rows, by exponentials, of which each lane of a
 // quad therefore takes a quarter.  us a token of 8 layers, scores in LDS between scores and statistics (attn_fused_kernel, which
-// looks at the whole row in every wave) -> this one, positions 40 and 200: 32 heads of 128 307.6 -> 296.9, 315.0 -> 305.2; 40 of 128
-// 403.2 -> 392.4, 412.5 -> 401.7; 32 heads of 64 over 4 key heads 196.6 -> 185.2, 215.9 -> 191.3; 8 heads of 128 166.7 -> 157.3,
-// 173.6 -> 166.9.  Exponentials in every lane: 32 heads of 128 at 200 312.
+// passes twice over the row and divides in every lane) -> this one, positions 40 and 200: 32 heads of 128 309.0 -> 299.6, 317.1 -> 308.1;
+// 40 of 128 413.3 -> 404.6, 421.2 -> 413.8; 32 heads of 64 over 4 key heads 195.3 -> 180.2, 213.4 -> 186.8 (1.6 and 2.1 us of these by
+// products of one pass); 8 heads of 128 167.0 -> 155.8, 177.7 -> 163.6.
 template <int LP, int R, bool ROUNDED>
 __global__ __launch_bounds__(1024) void attn_short_kernel(uint16_t* output, uint16_t* att, const uint16_t* q, const uint16_t* key_cache,
                                                           const uint16_t* value_cache, int kv_heads, int kv_mul, float alpha,
                                                           const int* pPos, int max_seq_len) {
     constexpr int HS = LP * 8, VS = HS / 2, PW = 64 / LP, ROUND = 16 * PW;
     __shared__ float2 waves[16];
+    __shared__ float scores[ROUNDED ? R * ROUND : 1];
     __shared__ __attribute__((aligned(16))) float acc_lds[16][VS];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane % LP, mine = wave * PW + lane / LP;
@@ -584,9 +585,28 @@ __global__ __launch_bounds__(1024) void attn_short_kernel(uint16_t* output, uint
         const uint16_t hb = float_to_half_bits(d * alpha);
         if (slice == 0 && j == 0 && t < size && kvh == (int)blockIdx.x) att[(size_t)h * size + t] = hb;
         s[i] = t < size ? half_bits_to_float(hb) : -INFINITY;
+        if (ROUNDED && j == 0) scores[t] = s[i];
         m = fmaxf(m, s[i]);
     }
-    m = groups_max<LP>(m);
+    float sum = 0.0f;
+    if (ROUNDED) {  // the row's maximum and sum first, in every wave alike
+        __syncthreads();
+        constexpr int N = R * ROUND / 64;
+        float x[N];
+        m = size < 1024 ? 0.0f : -INFINITY;  // the reference's idle-lane seed
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            x[i] = scores[lane + i * 64];
+            m = fmaxf(m, x[i]);
+        }
+        m = wave_max(m);
+#pragma unroll
+        for (int i = 0; i < N; i++)
+            if (i * 64 < size) sum += expf(x[i] - m);  // (0 past the position)
+        sum = wave_sum(sum);
+    } else {
+        m = groups_max<LP>(m);
+    }
     // every lane of a group has its scores: lane i of a quad takes the exponentials of scores i, i + 4, ... for the others
     constexpr int G = (R + 3) / 4;
     float e[G], l = 0.0f;
@@ -596,20 +616,8 @@ __global__ __launch_bounds__(1024) void attn_short_kernel(uint16_t* output, uint
 #pragma unroll
         for (int i = 1; i < 4 && R > 1; i++) x = (lane & 3) == i ? (g * 4 + i < R ? s[g * 4 + i] : -INFINITY) : x;
         e[g] = expf(x - m);
-        l += e[g];
-    }
-    if (R > 1) {
-        l += dpp_mov<0xB1>(l);  // quad_perm [1,0,3,2]
-        l += dpp_mov<0x4E>(l);  // quad_perm [2,3,0,1]
-    }
-    l = groups_sum<LP>(l);
-    if (lane == 0) waves[wave] = make_float2(m, l);
-    float top, sum;
-    if (ROUNDED) {  // the row's maximum and sum first
-        __syncthreads();
-        const float scale = read_lane(wave_scale(waves[lane & 15], top, sum), wave) / sum;
-#pragma unroll
-        for (int g = 0; g < G; g++) e[g] = half_bits_to_float(float_to_half_bits(e[g] * scale));
+        if (ROUNDED) e[g] = half_bits_to_float(float_to_half_bits(e[g] / sum));
+        else l += e[g];
     }
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -627,12 +635,30 @@ __global__ __launch_bounds__(1024) void attn_short_kernel(uint16_t* output, uint
     }
 #pragma unroll
     for (int i = 0; i < 4; i++) acc[i] = groups_sum<LP>(acc[i]);
+    if (!ROUNDED) {
+        if (R > 1) {
+            l += dpp_mov<0xB1>(l);  // quad_perm [1,0,3,2]
+            l += dpp_mov<0x4E>(l);  // quad_perm [2,3,0,1]
+        }
+        l = groups_sum<LP>(l);
+        if (lane == 0) waves[wave] = make_float2(m, l);
+    }
     if (lane < LP) *reinterpret_cast<float4*>(&acc_lds[wave][lane * 4]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
     __syncthreads();
     if (tid < VS && kvh == (int)blockIdx.x) {
-        float scale = 1.0f;
-        if (!ROUNDED) scale = wave_scale(waves[lane & 15], top, sum) / sum;
-        output[(size_t)h * HS + slice * VS + tid] = float_to_half_bits(scaled_waves(&acc_lds[0][tid], VS, scale));
+        float total = 0.0f;
+        if (ROUNDED) {
+            float r[16];
+#pragma unroll
+            for (int w = 0; w < 16; w++) r[w] = acc_lds[w][tid];
+#pragma unroll
+            for (int w = 0; w < 16; w++) total += r[w];
+        } else {
+            float top;
+            const float scale = wave_scale(waves[lane & 15], top, sum) / sum;
+            total = scaled_waves(&acc_lds[0][tid], VS, scale);
+        }
+        output[(size_t)h * HS + slice * VS + tid] = float_to_half_bits(total);
     }
 }
 

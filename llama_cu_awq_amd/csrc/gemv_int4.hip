@@ -585,9 +585,6 @@ int dispatch(awq_ctx* ctx, GemvParams& p, int grid_y, const char* what, GemvPlan
         if (ceil(per_cu8) / per_cu8 < ceil(per_cu16) / per_cu16 - 0.05) plan.waves = 8;
     }
     if (ROPE && plan.rows < 2) plan.rows = 2;  // a rotation pair lives in one wave
-    // Q, K and V so small that workgroups of 8 waves leave compute units idle (dim 2048 with 256 K and V rows: 160; a token of 8 layers
-    // 184.7 -> 180.6 us; dim 1024: 192, 159.3 -> 158.0)
-    if (KIND == KIND_QKV && plan.waves == 8 && plan.rows == 2 && div_up(p.N, 16) + (grid_y - 1) * div_up(p.Nkv, 16) < ctx->cus) plan.waves = 4;
     // Rows that leave at most half of a 64-lane pass over go two to a wave, 32 lanes each (see the kernel).  Measured
     // at the 13B and 33B shapes (K = 5120, 6656): gate/up -6 %, O projection -7 %, QKV -2 % with two passes in flight
     // and even with three, tokens/s +3 %.  Rows above 8192 (K = 11008: 16 waves, or 8, at any depth) lose: two rows per

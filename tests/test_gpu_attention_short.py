@@ -84,8 +84,8 @@ def test_rows_past_the_position_do_not_enter(ctx, heads, head, kv, pos):
     t.close()
 
 
-@pytest.mark.parametrize("heads,head,kv", [(8, 64, 2), (2, 256, 1)])  # (1/sqrt(head size) is exact: scores stay multiples of an eighth)
-@pytest.mark.parametrize("size", [2, 64, 200, 256])
+@pytest.mark.parametrize("heads,head,kv", [(8, 64, 2)])  # (1/sqrt(head size) is exact: scores stay multiples of an eighth)
+@pytest.mark.parametrize("size", [257, 300, 512])
 def test_scores_far_below_zero(ctx, heads, head, kv, size):
     """As at longer contexts: a constant added to every score changes no softmax, also where its exponentials are zero in fp32."""
     model.test_decode_scores_far_below_zero(ctx, heads, head, kv, size)
