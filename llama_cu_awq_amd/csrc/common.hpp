@@ -179,12 +179,13 @@ __device__ __forceinline__ float lane_xor_sum(float v) {
 }
 
 // Sum within each aligned group of 16 lanes (a DPP row); every lane of the
-// group ends up holding the group's sum.
+// group ends up holding the same bits, those of (quad 0 + quad 3) + (quad 1 + quad 2): each step adds two values that both lanes of a
+// pair have.  (Rotations by 4 and 8 would give odd quads another order of sums.)
 __device__ __forceinline__ float row16_sum(float v) {
     v += dpp_mov<0xB1>(v);   // quad_perm [1,0,3,2]
     v += dpp_mov<0x4E>(v);   // quad_perm [2,3,0,1]
-    v += dpp_mov<0x124>(v);  // row_ror:4
-    v += dpp_mov<0x128>(v);  // row_ror:8
+    v += dpp_mov<0x140>(v);  // row_mirror: quads 0<->3, 1<->2
+    v += dpp_mov<0x141>(v);  // row_half_mirror: quads 0<->1, 2<->3
     return v;
 }
 // Sum over the 64 lanes of the wave; the result is wave-uniform.
@@ -204,20 +205,18 @@ __device__ __forceinline__ float wave_max(float v) {
     swap32(a, b);
     return fmaxf(a, b);
 }
-// Sum within aligned groups of LP lanes (LP = 8, 16 or 32).
+// Sum within aligned groups of LP lanes (LP = 8, 16 or 32), the same bits in every lane of the group: a score that each of its lanes
+// rounds to fp16 for itself is one score.
 template <int LP>
 __device__ __forceinline__ float group_sum(float v) {
     static_assert(LP == 8 || LP == 16 || LP == 32, "unsupported group width");
-    v += dpp_mov<0xB1>(v);
-    v += dpp_mov<0x4E>(v);
     if (LP == 8) {
-        v += dpp_mov<0x141>(v);  // row_half_mirror: quads 0<->1 inside each 8 lanes
-    } else {
-        v += dpp_mov<0x124>(v);
-        v += dpp_mov<0x128>(v);
-        if (LP == 32) v = lane_xor_sum<16>(v);
+        v += dpp_mov<0xB1>(v);
+        v += dpp_mov<0x4E>(v);
+        return v + dpp_mov<0x141>(v);  // row_half_mirror: quads 0<->1 inside each 8 lanes
     }
-    return v;
+    v = row16_sum(v);
+    return LP == 32 ? lane_xor_sum<16>(v) : v;
 }
 
 #endif  // __HIPCC__

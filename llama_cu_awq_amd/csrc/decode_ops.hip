@@ -541,9 +541,8 @@ __global__ __launch_bounds__(1024) void attn_ranges_kernel(float* part, float2* 
 // lane, the first of them asked for before the position is known; scores stay in registers.  Two workgroups a head take half of the
 // value dimensions each and compute the scores redundantly; those of a key head run on one XCD where key heads are 8 or more.
 // ROUNDED (up to 256 positions): maximum (from 0, as the reference's idle lanes have it), sum, probabilities rounded to fp16 after their
-// division by it and all sums in attn_fused_kernel's order: its bits for heads of 64 and 256 (for 128 a score is scaled and rounded to
-// fp16 in one rounding here, in two there).  Past 256 positions, where ranges keep probabilities fp32 and start
-// the maximum below every score, so does this, and the waves meet once.
+// division by it and all sums in attn_fused_kernel's order, and its bits.  Past 256 positions, where ranges keep probabilities fp32 and
+// start the maximum below every score, so does this, and the waves meet once.
 // Bound by latency (launch, one round trip to memory, a barrier or two) and, at many rows, by exponentials, of which each lane of a
 // quad therefore takes a quarter.  us a token of 8 layers, scores in LDS between scores and statistics (attn_fused_kernel, which
 // passes twice over the row and divides in every lane) -> this one, positions 40 and 200: 32 heads of 128 309.0 -> 299.6, 317.1 -> 308.1;

@@ -16,6 +16,11 @@ pytestmark = pytest.mark.gpu
 takes_short = lib["_Z25awq_attention_takes_shortii"]
 takes_short.argtypes, takes_short.restype = [C.c_int] * 2, C.c_bool
 
+_short = lib["_Z26awq_launch_attention_shortP7awq_ctxPtPKtS3_S3_S1_iiiiPKi"]
+_short.argtypes = [C.c_void_p] * 6 + [C.c_int] * 4 + [C.c_void_p]
+_ranges = lib["_Z27awq_launch_attention_rangesP7awq_ctxPfP15HIP_vector_typeIfLj2EEPiPKtS7_S7_PtiiiiPKi"]
+_ranges.argtypes = [C.c_void_p] * 3 + [C.POINTER(C.c_int)] + [C.c_void_p] * 4 + [C.c_int] * 4 + [C.c_void_p]
+
 # heads, head size, key heads: one key head, fewer than 8, a number that is no multiple of 8
 HEADS = [(4, 64, 2), (32, 64, 4), (16, 128, 1), (24, 128, 12), (8, 128, 8), (4, 256, 2), (16, 256, 16)]
 POSITIONS = (0, 1, 15, 63, 64, 127, 128, 129, 255, 256, 300, 510, 511, 512, 1022, 1023)
@@ -89,3 +94,51 @@ def test_rows_past_the_position_do_not_enter(ctx, heads, head, kv, pos):
 def test_scores_far_below_zero(ctx, heads, head, kv, size):
     """As at longer contexts: a constant added to every score changes no softmax, also where its exponentials are zero in fp32."""
     model.test_decode_scores_far_below_zero(ctx, heads, head, kv, size)
+
+
+def _inputs(ctx, heads, head, kv, size, cancelling):
+    """Query, keys and values of one layer.  `cancelling`: the first 32 dimensions of a key add 2^24 to its score and the next 32 take it away
+    again, so that fp32 sums in another order give scores that are whole steps apart."""
+    rng = np.random.default_rng(heads * head + kv + size)
+    q = rng.standard_normal((heads, head)).astype(np.float16)
+    k, v = (rng.standard_normal((size, kv, head)).astype(np.float16) for _ in range(2))
+    if cancelling:
+        q[:, [0, 32]] = 4096
+        k[:, :, 0], k[:, :, 32] = 4096, -4096
+    return q, k, v
+
+
+@pytest.mark.parametrize("cancelling", [False, True], ids=["random", "cancelling"])
+@pytest.mark.parametrize("heads,head,kv", [(32, 64, 4), (32, 128, 32), (24, 128, 12), (16, 256, 16)])
+@pytest.mark.parametrize("size", [1, 64, 65, 128, 200, 256])
+def test_bits_of_the_form_with_scores_in_lds(ctx, heads, head, kv, size, cancelling):
+    """Up to 256 positions a sampled run takes the tokens that it takes through awq_attention: the same scores, weights and sums, bit for bit."""
+    dq, dk, dv = (ctx.upload(a) for a in _inputs(ctx, heads, head, kv, size, cancelling))
+    pos, got = ctx.upload(np.array([size - 1], np.int32)), []
+    for short in (False, True):
+        out, att = ctx.zeros(heads * head * 2), ctx.zeros(heads * size * 2)
+        if short:
+            assert _short(ctx.h, out.ptr, dq.ptr, dk.ptr, dv.ptr, att.ptr, heads, head, heads // kv, size, pos.ptr) == 0
+        else:
+            A.MultiHeadAttention(ctx, out, dq, dk, dv, att, heads, head, heads // kv, size, pos)
+        got.append([d.download(np.uint16) for d in (out, att)])
+    for a, b in zip(*got):
+        assert np.isfinite(f16(a)).all() and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("heads,head,kv,size", [(8, 64, 2, 200), (8, 64, 2, 700), (16, 128, 4, 100), (16, 128, 4, 256), (16, 128, 4, 300), (16, 128, 4, 512),
+                                                (8, 256, 2, 256)])
+@pytest.mark.parametrize("ranges", [False, True], ids=["short", "ranges"])
+def test_every_dimension_gives_a_position_one_weight(ctx, heads, head, kv, size, ranges):
+    """The lanes that share a position share its score: value rows with one number in every dimension come out with the same bits in every
+    dimension."""
+    q, k, v = _inputs(ctx, heads, head, kv, size, True)
+    v[:] = v[:, :1, :1]
+    dq, dk, dv, pos, att = (ctx.upload(a) for a in (q, k, v, np.array([size - 1], np.int32), np.zeros(heads * size, np.uint16)))
+    out, stat, n = ctx.zeros(4 * heads * head * 4), ctx.zeros(4 * heads * 8), C.c_int(1)
+    if ranges:
+        assert _ranges(ctx.h, out.ptr, stat.ptr, C.byref(n), dq.ptr, dk.ptr, dv.ptr, att.ptr, heads, head, heads // kv, size, pos.ptr) == 0 and n.value > 1
+    else:
+        assert _short(ctx.h, out.ptr, dq.ptr, dk.ptr, dv.ptr, att.ptr, heads, head, heads // kv, size, pos.ptr) == 0
+    got = out.download(np.uint32 if ranges else np.uint16, n.value * heads * head).reshape(-1, head)
+    assert got.any() and np.array_equal(got, np.repeat(got[:, :1], head, axis=1))
