@@ -792,15 +792,20 @@ int awq_launch_gemm_single(awq_ctx* ctx, uint16_t* out, long long ldo, const uin
 int awq_launch_rmsnorm_rows(awq_ctx* ctx, uint16_t* o, const uint16_t* x, const uint16_t* w, int size, int M, int perm, int tiles);
 
 // Whether a pass of M rows goes through a layer in the few-row form: its four products hand each other activations in
-// fragment order, so that they are weighed together.  Inside a pass they take 0.82 (up to 64 rows; 1.06 above) of the sum of their
-// estimates where the row forms take that of theirs.  Four layers and the logits, us, row forms -> few-row form, at 4, 32, 33 and 64
-// rows: dim 2048 by 5632 245 -> 207, 252 -> 216, 256 -> 230, 261 -> 238; 4096 by 11008 339 -> 305, 351 -> 319, 396 -> 349, 409 -> 369;
-// 6656 by 17920 574 -> 530, 619 -> 573, 702 -> 634, 728 -> 675; but 8192 by 28672 649 -> 633, 703 -> 701, 761 -> 811, 793 -> 874.
-// At 65, 96, 97 and 128 rows: 2048 308 -> 276, 307 -> 281, 314 -> 295, 316 -> 302; 4096 517 -> 434, 522 -> 447, 523 -> 508, 531 -> 534;
-// 5120 by 13824 656 -> 556, 667 -> 580, 679 -> 618, 685 -> 643; 6656 910 -> 790, 912 -> 821, 977 -> 960, 1000 -> 1013; 8192 1000 -> 989,
-// 1010 -> 1035, 1072 -> 1140, 1108 -> 1193.
+// fragment order, so that they are weighed together.  Inside a pass the sum of their estimates counts for kFewWeight (by 32-row
+// tiles) of the row forms': they start and end faster, and what they read of weights and activations overlaps better, the more so the
+// fewer the rows.  Four layers and the logits, us, row forms | few-row form, by key and value columns, at 4, 32, 33 and 64 rows:
+// dim 2048 (256) by 5632 246 | 207, 266 | 226, 270 | 246, 277 | 250; 4096 (4096) by 11008 361 | 327, 375 | 339, 422 | 372, 429 | 392;
+// 6656 (6656) by 17920 595 | 549, 641 | 592, 718 | 657, 743 | 698; 8192 (8192) by 22016 651 | 646, 695 | 686, 804 | 757, 826 | 811;
+// 8192 (1024) by 28672 666 | 647, 718 | 719, 778 | 826, 807 | 891; 8192 (8192) by 28672 728 | 714, 786 | 777, 866 | 890, 897 | 957.
+// At 65, 96, 97 and 128 rows: 2048 300 | 273, 299 | 278, 307 | 289, 311 | 301; 4096 517 | 439, 522 | 452, 523 | 511, 534 | 534; 5120
+// (5120) by 13824 637 | 544, 651 | 568, 655 | 609, 670 | 636; 6656 907 | 792, 916 | 826, 971 | 963, 984 | 1009; 8192 (1024) by 28672
+// 1004 | 994, 1019 | 1046, 1079 | 1137, 1102 | 1192; 8192 (8192) by 28672 1109 | 1080, 1135 | 1141, 1244 | 1306, 1267 | 1376.  The estimates
+// are too high for narrow products of several row tiles: 1536 (256) by 4096 stays with the row forms past 64 rows (288 | 265 at 65,
+// 275 | 267 at 128).
 bool awq_prefill_takes_few(awq_ctx* ctx, int M, int dim, int kv_dim, int hidden) {
     if (M > kFewRows) return false;
+    constexpr float kFewWeight[4] = {0.75f, 0.89f, 1.05f, 1.06f};
     const auto few = [&](int K, int N, bool split) { return awq_plan_gemm_few(ctx->cus, M, K, N, split).us; };
     const auto rows = [&](int K, int N, bool single) {
         const float us = route_gemm(ctx->cus, M, K, N / pf::BN, single).us;
@@ -808,7 +813,7 @@ bool awq_prefill_takes_few(awq_ctx* ctx, int M, int dim, int kv_dim, int hidden)
         const awq_rows_plan parts = awq_plan_gemm_rows(ctx->cus, M, K, N / 64, true, true);
         return parts.form >= 0 && parts.us < us ? parts.us : us;
     };
-    return (M <= 64 ? 0.82f : 1.06f) * (few(dim, dim + 2 * kv_dim, false) + few(dim, dim, true) + few(dim, 2 * hidden, false) + few(hidden, dim, true)) <
+    return kFewWeight[(M - 1) / 32] * (few(dim, dim + 2 * kv_dim, false) + few(dim, dim, true) + few(dim, 2 * hidden, false) + few(hidden, dim, true)) <
            rows(dim, dim + 2 * kv_dim, false) + rows(dim, dim, true) + rows(dim, 2 * hidden, false) + rows(hidden, dim, true);
 }
 
