@@ -593,7 +593,7 @@ __global__ __launch_bounds__(1024) void attn_short_kernel(uint16_t* output, uint
         __syncthreads();
         constexpr int N = R * ROUND / 64;
         float x[N];
-        m = size < 1024 ? 0.0f : -INFINITY;  // the reference's idle-lane seed
+        m = 0.0f;  // the reference's idle-lane seed, as below 1024 positions
 #pragma unroll
         for (int i = 0; i < N; i++) {
             x[i] = scores[lane + i * 64];

@@ -540,8 +540,8 @@ template <int W, int R, int KIND, bool ROPE>
 int dispatch_depth(awq_ctx* ctx, GemvParams& p, int grid_y, const char* what, const GemvPlan& plan) {
     constexpr int NS = (KIND == KIND_FFN) ? 2 * R : R;
     // A row of one pass, one row to a wave: nothing is in flight behind it, and padded to a depth of two it is requested twice (32 heads of
-    // 64, dim 2048: a token of 8 layers 184.7 -> 180.6 us).
-    if constexpr (KIND == KIND_SINGLE && R == 1)
+    // 64, dim 2048: a token of 8 layers 184.7 -> 180.6 us).  (Workgroups of more than 8 waves have rows of several passes.)
+    if constexpr (KIND == KIND_SINGLE && R == 1 && W <= 8)
         if (p.C <= 64) return launch<W, R, 1, KIND, ROPE>(ctx, p, grid_y, what);
     int depth = plan.depth;
     while (depth > 2 && (NS * depth > 16 || depth > 4)) depth--;  // what the register file affords
