@@ -103,7 +103,8 @@ def test_weights_past_the_range_of_fp16(ctx, M, K, N, form):
     assert np.isposinf(got[:, 5]).all() and np.isfinite(np.delete(got, 5, 1)).all()
 
 
-# 64-wide heads, sizes at which the QKV and gate/up products take the 64 to 128 row forms by 128 and 256 columns
+# 64-wide heads, sizes at which the QKV and gate/up products take the 64 to 128 row forms by 128 and 256 columns (passes of up to 128
+# rows go in the few-row form; the row forms' epilogues at few rows are held against 64-bit products below)
 SMALL = dict(dim=2048, hidden_dim=5632, n_layers=2, n_heads=32, n_kv_heads=4, vocab_size=512, seq_len=1280, rope_theta=10000.0)
 
 
@@ -189,6 +190,95 @@ def test_parts_left_to_the_norm(ctx, M, K, N, parts, perm):
         assert rel_l2(got[-1], want[-1]) <= 1e-3 and rel_l2(got[:, -8:], want[:, -8:]) <= 1e-3
 
 
+_qkv = lib["_Z19awq_launch_gemm_qkvP7awq_ctxPtS1_S1_PKtiiPK11awq_qweightS6_S6_iiiiPK15HIP_vector_typeIfLj2EEfibb"]
+_qkv.argtypes = [C.c_void_p] * 5 + [C.c_int] * 2 + [C.POINTER(QWeightC)] * 3 + [C.c_int] * 4 + [C.c_void_p, C.c_float, C.c_int, C.c_bool, C.c_bool]
+_ffn = lib["_Z19awq_launch_gemm_ffnP7awq_ctxPtPKtiiPK11awq_qweightS6_iibbb"]
+_ffn.argtypes = [C.c_void_p] * 3 + [C.c_int] * 2 + [C.POINTER(QWeightC)] * 2 + [C.c_int] * 2 + [C.c_bool] * 3
+_plan_few = lib["_Z17awq_plan_gemm_fewiiiib"]  # compute units, rows, K, columns, may split (its fields: see _Plan)
+_plan_few.argtypes, _plan_few.restype = [C.c_int] * 4 + [C.c_bool], _Plan
+_takes_few = lib["_Z21awq_prefill_takes_fewP7awq_ctxiiii"]
+_takes_few.argtypes, _takes_few.restype = [C.c_void_p] + [C.c_int] * 4, C.c_bool
+_tile = lib["_Z13awq_rows_formiPi"]
+_tile.argtypes, _tile.restype = [C.c_int, C.POINTER(C.c_int)], None
+
+
+def _form(M, K, N):
+    """Tile and parts of K of a product that is not a single matrix."""
+    plan, tile = _plan(256, M, K, N // 64, True, False), (C.c_int * 3)()
+    _tile(plan.form, tile)
+    return (tile[0], tile[1]), plan.parts
+
+
+# up to 128 rows, where passes whose products do not take the few-row form (matrices of 8192 by 28672, say) run QKV and gate/up: whole K
+# and parts of it that meet in the launch.  (rows, K, query columns, key and value columns, head size, tile, parts)
+QKV = [(20, 256, 128, 128, 64, (32, 64), 1), (1, 2048, 128, 128, 128, (32, 64), 2), (37, 3072, 128, 128, 64, (32, 64), 3), (33, 4096, 128, 128, 128, (32, 64), 4),
+       (64, 512, 6400, 1024, 256, (64, 64), 1), (65, 8192, 2048, 384, 128, (64, 64), 2), (48, 3072, 512, 256, 256, (64, 64), 3), (128, 4096, 640, 128, 64, (64, 64), 4),
+       (37, 256, 6272, 1024, 128, (64, 128), 1), (100, 4096, 6272, 1024, 64, (64, 128), 3)]
+# (rows, K, hidden, tile, parts)
+FFN = [(20, 256, 256, (32, 64), 1), (1, 2048, 256, (32, 64), 2), (33, 3072, 256, (32, 64), 3), (37, 4096, 256, (32, 64), 4), (64, 512, 4224, (64, 64), 1),
+       (65, 8192, 1408, (64, 64), 2), (48, 3072, 512, (64, 64), 3), (128, 4096, 384, (64, 64), 4), (37, 256, 4224, (64, 128), 1), (100, 4096, 4224, (64, 128), 3)]
+
+
+def _matrix(ctx, key, K, N):
+    """On the device, and as the kernels multiply it."""
+    w, z, s = synth.make_qweight(key, K, N)
+    return A.QWeight.upload(ctx, w, z, s), synth.dequantize(w, z, s, K).astype(np.float32).astype(np.float16).astype(np.float64)
+
+
+def _rows_in_packed_order(ctx, key, M, K):
+    a = synth.normal_f16(synth.stream_key(key, "a"), M * K)
+    return ctx.upload(np.ascontiguousarray(a.reshape(M, K // 8, 8)[:, :, [0, 4, 1, 5, 2, 6, 3, 7]]).reshape(-1)), a.astype(np.float64).reshape(M, K)
+
+
+def _near(got, want):
+    assert rel_l2(got, want) <= 4e-4
+    for at in (np.s_[-1], np.s_[0], np.s_[:, -32:], np.s_[:, :32]):
+        assert rel_l2(got[at], want[at]) <= 1e-3
+
+
+@pytest.mark.parametrize("M,K,Nq,Nkv,head,tile,parts", QKV)
+def test_qkv_of_few_rows_against_fp64(ctx, M, K, Nq, Nkv, head, tile, parts):
+    """Rotated q and k, v as it is, cache rows from a position on.  q and k are rounded to fp16 before the rotation and behind it, v once
+    (2.1e-4 in the norm each, 3.0e-4 together)."""
+    assert _form(M, K, Nq + 2 * Nkv) == (tile, parts)
+    key, pos0 = synth.stream_key(66, M, K, Nq), 5
+    mats = [_matrix(ctx, synth.stream_key(key, name), K, n) for name, n in (("q", Nq), ("k", Nkv), ("v", Nkv))]
+    da, a = _rows_in_packed_order(ctx, key, M, K)
+    angle = np.random.default_rng(M + Nq).uniform(0, 2 * np.pi, (pos0 + M, head // 2))
+    rope = np.stack([np.cos(angle), np.sin(angle)], axis=-1).astype(np.float32)
+    dr, runs = ctx.upload(rope), []
+    for _ in range(2):  # (the arrival counters are back at zero for the second launch)
+        outs = [ctx.upload(np.full((first + M + 1) * n, 0xFFFF, np.uint16)) for n, first in ((Nq, 0), (Nkv, pos0), (Nkv, pos0))]
+        assert _qkv(ctx.h, *(o.ptr for o in outs), da.ptr, K, M, *(C.byref(m.c) for m, _ in mats), K, Nq, Nkv, head, dr.ptr, 10000.0, pos0, True, False) == 0
+        runs.append([o.download(np.uint16) for o in outs])
+    for i, (n, first) in enumerate(((Nq, 0), (Nkv, pos0), (Nkv, pos0))):
+        assert np.array_equal(runs[0][i], runs[1][i])
+        bits = runs[0][i].reshape(-1, n)
+        assert (bits[:first] == 0xFFFF).all() and (bits[first + M :] == 0xFFFF).all()
+        want = a @ mats[i][1].T
+        if i < 2:
+            x, y = (want.reshape(M, -1, 2, head // 2)[:, :, j] for j in (0, 1))
+            c, s = (rope[pos0:, None, :, j].astype(np.float64) for j in (0, 1))
+            want = np.stack([x * c - y * s, x * s + y * c], axis=2).reshape(M, n)
+        _near(f16(bits[first : first + M]).astype(np.float64), want)
+
+
+@pytest.mark.parametrize("M,K,N,tile,parts", FFN)
+def test_gate_and_up_of_few_rows_against_fp64(ctx, M, K, N, tile, parts):
+    """silu(gate) * up in fp32, rounded once (2.1e-4 in the norm), every 8 columns in the order that a packed dword unpacks in."""
+    assert _form(M, K, 2 * N) == (tile, parts)
+    key = synth.stream_key(67, M, K, N)
+    (gate, gate64), (up, up64) = (_matrix(ctx, synth.stream_key(key, name), K, N) for name in ("gate", "up"))
+    (da, a), runs = _rows_in_packed_order(ctx, key, M, K), []
+    for _ in range(2):
+        dh = ctx.zeros(M * N * 2)
+        assert _ffn(ctx.h, dh.ptr, da.ptr, K, M, C.byref(gate.c), C.byref(up.c), K, N, True, True, False) == 0
+        runs.append(dh.download(np.uint16))
+    assert np.array_equal(*runs)
+    g, u = (a @ m.T for m in (gate64, up64))
+    _near(f16(runs[0]).reshape(M, N // 8, 8)[:, :, [0, 2, 4, 6, 1, 3, 5, 7]].reshape(M, N).astype(np.float64), g / (1 + np.exp(-g)) * u)
+
+
 # (looked up through the library: the HIP runtime it is linked with)
 def _hip(name, *args):
     assert getattr(lib, name)(*args) == 0, name
@@ -231,23 +321,26 @@ def test_split_workspace_made_while_recording(ctx):
     fresh.close()
 
 
-def test_short_prefill_recorded_after_a_long_one():
-    """1100 rows by 4096 columns split no K, 37 do (QKV and gate/up, whose parts meet in the launch, and of the first of two
-    layers O and down, whose parts the norm adds up): what that takes is there before the short prompt is recorded."""
-    cfg = dict(dim=4096, hidden_dim=2048, n_layers=2, n_heads=32, n_kv_heads=4, vocab_size=512, seq_len=1152, rope_theta=10000.0)
+@pytest.mark.parametrize("few,n,kv,hidden", [(True, 37, 4, 2048), (False, 100, 1, 1024)])
+def test_short_prefill_recorded_after_a_long_one(few, n, kv, hidden):
+    """1100 rows by 4096 columns split no K, the short prompt's do: 37 rows in the few-row form (O and down of the first of two layers,
+    whose parts the norm adds up), 100 in the row forms (gate/up, whose parts meet in the launch, and O, whose parts the norm adds up).
+    What that takes is there before the short prompt is recorded."""
+    cfg = dict(dim=4096, hidden_dim=hidden, n_layers=2, n_heads=32, n_kv_heads=kv, vocab_size=512, seq_len=1280, rope_theta=10000.0)
     img = synth.make_model_image(cfg, seed=55, scale_mult=0.25)
-    prompt = synth.prompt_tokens(55, 1137, cfg["vocab_size"])
+    prompt = synth.prompt_tokens(55, 1100 + n, cfg["vocab_size"])
     ctx = A.Context(0)
     t = A.Transformer(ctx, image=img)
+    kv_dim = kv * 128
 
     def caches():
-        return [t.download(name, n) for name, n in (("key_cache", 2 * cfg["seq_len"] * 512), ("value_cache", 2 * cfg["seq_len"] * 512), ("logits", 512))]
+        return [t.download(name, size) for name, size in (("key_cache", 2 * cfg["seq_len"] * kv_dim), ("value_cache", 2 * cfg["seq_len"] * kv_dim), ("logits", 512))]
 
     stream, graph, runnable = C.c_void_p(lib.awq_ctx_stream(ctx.h)), C.c_void_p(), C.c_void_p()
     t.reset(prompt)
     t.prefill(1100, gen_token=False)
     _hip("hipStreamBeginCapture", stream, 0)
-    t.prefill(37, gen_token=False)
+    t.prefill(n, gen_token=False)
     _hip("hipStreamEndCapture", stream, C.byref(graph))
     _hip("hipGraphInstantiate", C.byref(runnable), graph, None, None, C.c_size_t(0))
     recorded = []
@@ -257,16 +350,19 @@ def test_short_prefill_recorded_after_a_long_one():
         recorded.append(caches())
     t.reset(prompt)
     t.prefill(1100, gen_token=False)
-    t.prefill(37, gen_token=False)
+    t.prefill(n, gen_token=False)
     ctx.sync()
     want = caches()
     for got in recorded:
         for a, b in zip(got, want):
             assert np.array_equal(a, b)
         for b in want[:2]:
-            assert f16(b).reshape(2, -1, 512)[:, 1100:1137].any(axis=2).all()
-    for M, K in ((37, 4096), (37, 2048)):
-        assert _plan(256, M, K, 4096 // 64, True, True).parts > 1
+            assert f16(b).reshape(2, -1, kv_dim)[:, 1100 : 1100 + n].any(axis=2).all()
+    assert _takes_few(ctx.h, n, 4096, kv_dim, hidden) == few
+    if few:
+        assert all(_plan_few(256, n, K, 4096, True).parts > 1 for K in (4096, hidden))
+    else:
+        assert _form(n, 4096, 2 * hidden)[1] > 1 and _plan(256, n, 4096, 4096 // 64, True, True).parts > 1
     _hip("hipGraphExecDestroy", runnable)
     _hip("hipGraphDestroy", graph)
     t.close()
