@@ -303,15 +303,16 @@ def test_fused_gate_up_with_more_row_groups_than_workgroups(ctx):
         o.close()
 
 
-# heads, head size, key heads, positions: the launch sizes past one workgroup per head, where a head's positions are split over two
-# to four workgroups: the first of them, ranges that fill no or several rounds of requests (512, 256 and 128 positions for heads
-# of 64, 128 and 256), last ranges that are short, two ranges a head (128 heads), 13 waves in the O projection (52 heads); few heads
-# of 128 and 256 past 1024, where P.V is a launch of its own
+# heads, head size, key heads, positions: launch sizes past 256.  Up to 1024 (heads of 64) and 512 (of 128) positions are one request
+# of a head; past them, and for heads of 256 at once, they are split over two to four workgroups: the first such sizes, ranges that
+# fill no or several rounds of requests (512, 256 and 128 positions for heads of 64, 128 and 256), last ranges that are short, two
+# ranges a head (128 heads), 13 waves in the O projection (52 heads); few heads of 128 and 256 past 1279, where P.V is a launch of its own
 @pytest.mark.parametrize(
     "heads,head,kv,positions",
-    [(4, 64, 2, (128, 256, 300, 1022, 1023, 2047, 4500)), (4, 128, 4, (129, 255, 256, 511, 1023, 1024, 3000, 5000)),
-     (8, 128, 1, (256, 257, 700)), (2, 256, 1, (256, 512, 1500, 2600)), (128, 64, 128, (257, 1100)),
-     (32, 128, 8, (1025, 2047, 4500)), (32, 256, 8, (1500, 2600)), (52, 128, 52, (300, 1100))],
+    [(4, 64, 2, (128, 256, 300, 1022, 1023, 1024, 1025, 1100, 1535, 1536, 2047, 4500)),
+     (4, 128, 4, (129, 255, 256, 511, 512, 513, 767, 768, 1023, 1024, 3000, 5000)),
+     (8, 128, 1, (256, 257, 512, 700)), (2, 256, 1, (256, 512, 1500, 2600)), (128, 64, 128, (257, 1100)),
+     (32, 128, 8, (1025, 2047, 4500)), (32, 256, 8, (1500, 2600)), (52, 128, 52, (300, 600, 1100))],
 )
 def test_attention_of_long_contexts_in_one_launch(ctx, heads, head, kv, positions):
     """The fused schedule's attention in ranges, put together by the O projection, against the reference schedule's separate
@@ -340,9 +341,10 @@ def test_attention_of_long_contexts_in_one_launch(ctx, heads, head, kv, position
     t.close()
 
 
-# sizes of the launch past one workgroup per head; 1024 is where the reference's maximum starts elsewhere
+# sizes of the launch past 256 positions: ranges for heads of 256, for heads of 64 one request up to 1024; that is also where the reference's
+# maximum starts elsewhere
 @pytest.mark.parametrize("heads,head,kv", [(8, 64, 2), (2, 256, 1)], ids=["heads-of-64", "heads-of-256"])
-@pytest.mark.parametrize("size", [257, 301, 501, 1022, 1023, 1024])
+@pytest.mark.parametrize("size", [257, 301, 501, 1022, 1023, 1024, 1025, 1279])
 def test_decode_scores_far_below_zero(ctx, heads, head, kv, size):
     """A constant added to every score changes no softmax: scores of -4 .. 4 and the same ones 20, 95 and 150 lower, whose
     exponentials are small, denormal and zero in fp32.  All are multiples of an eighth, which fp16 and its key rows hold, and the
@@ -365,7 +367,7 @@ def test_decode_scores_far_below_zero(ctx, heads, head, kv, size):
             assert np.isfinite(a).all() and rel_l2(a, b) <= 1e-3
 
 
-@pytest.mark.parametrize("heads,head,kv,pos", [(4, 64, 2, 300), (8, 128, 2, 700), (2, 256, 1, 900), (32, 128, 8, 2100), (4, 128, 4, 2100)])
+@pytest.mark.parametrize("heads,head,kv,pos", [(4, 64, 2, 300), (4, 64, 2, 1100), (8, 128, 2, 700), (2, 256, 1, 900), (32, 128, 8, 2100), (4, 128, 4, 2100)])
 def test_rows_past_the_position_do_not_enter(ctx, heads, head, kv, pos):
     """Loads past a range's end repeat its last row, and what lies behind the position (an earlier, longer conversation) is not
     read: NaN there changes no bit.  NaN and infinities of the rows that count reach the logits, as in the reference schedule."""
