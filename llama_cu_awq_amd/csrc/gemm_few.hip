@@ -30,9 +30,10 @@ struct FewForm {
 //    lanes on different rows: 64 cycles an instruction instead of 16.
 //  * 32x32x16 products, weights as the first operand: between two of them another wave's dequantisation finds room.  (In 16x16x32
 //    products the two hardly overlap: 3 of them and 13 vector instructions take 81 ns a wave, 2 of 32x32x16 and the same 69.)
-// What bounds it: about 10 of 21 us (7B gate/up, 37 rows) the 13 vector instructions that dequantise a packed dword, at 5 cycles
-// each, with two waves a SIMD; about 4 us until the first activations and weights are there; 3 us until the sums have met.  More
-// waves of fewer registers, column groups that share A through L1, or weights left in cache change nothing.
+// What bounds it (7B gate/up, 37 rows, 22 us = 44 000 clocks, by counters): with two waves a SIMD its matrix core is busy 12 300
+// clocks and its vector instructions take 15 000, of which 10 000 are the 13 that dequantise a packed dword; the two overlap in part.
+// Waves wait a quarter of their life for memory or LDS: about 4 us until the first activations and weights are there, 3 us until the
+// sums have met.  More waves of fewer registers, column groups that share A through L1, or weights left in cache change nothing.
 // Measured, us, the row forms -> this one: 7B shape, 37 rows QKV 17.9 -> 15.6, O 9.5 -> 8.5, gate/up 30.3 -> 21.5, down 16.5 ->
 // 14.5; 64 rows gate/up 30.2 -> 22.4.  96 rows, from memory, QKV 26.9 -> 20.0, O 12.3 -> 10.2, gate/up 41.9 -> 33.2, 13824 columns of 5120 35.9 -> 24.5;
 // 128 rows QKV 27.8 -> 23.0, 13824 of 5120 36.3 -> 28.0, but gate/up 42.2 -> 44.2: two rounds of workgroups, since three units a workgroup
